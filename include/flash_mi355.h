@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define FA_ABI_VERSION 7
+#define FA_ABI_VERSION 8
 
 /* score_func_mode, flash_triton.py:20-22 */
 #define FA_SCORE_MODE0_NOPE 0
@@ -58,6 +58,14 @@ extern "C" {
    block (i / 64, j / 64) is non-zero and the causal / window / prefix terms hold. */
 #define FA_SCORE_MODE2_BLOCK 2
 #define FA_MASK_BLOCK 64
+/* Packed sequences (no counterpart in the reference, which takes ids directly, flash_triton.py:506): B = 1, the rows of
+   q and of k, v are `nseq` sequences back to back.  `eq` points to nseq + 1 cumulative lengths of the queries
+   (id_dtype, first element 0, non-decreasing, on the device), `ek` to those of the keys (the same pointer when they
+   are the same); the strides of ids are not used.  A row sees the keys of its own sequence only; with `causal` every
+   sequence is aligned at its end: row i of a sequence of m rows and n keys has its diagonal at its key n - m + i (a
+   row before the first key sees nothing).  Rows and keys behind the last boundary form one more sequence, aligned
+   at its start.  window is allowed, prefix and qpos are not; 16-bit types; fa_mask_plan writes the tile tables. */
+#define FA_SCORE_MODE3_PACKED 3
 
 /* element types */
 #define FA_DTYPE_BF16 0
@@ -84,6 +92,10 @@ extern "C" {
                                and also stores it to p->delta: the fa_bwd_delta launch is then not needed, and
                                fa_bwd_dkdv, which reads delta, goes after fa_bwd_dq on the stream.
                                Ignored by every other call. */
+#define FA_FLAG_SPLIT_KEYS 4    /* mode 0: fa_fwd and fa_bwd_dq may split the key range of a launch that is short of
+                               workgroups.  fa_workspace_* then may ask for a workspace in this mode too (0 bytes:
+                               nothing is split at these sizes); when they do, fa_mask_plan goes before fa_fwd.
+                               Set it in every call that shares the workspace, or in none. */
 #define FA_FLAG_DEBUG_NO_PAIR_WAIT 0x100
                             /* Diagnostic, for tests of the failure path below; never set it in production.
                                In fa_bwd_dkdv at D = 128 two waves share each block of 32 keys: one publishes P in
@@ -113,7 +125,7 @@ typedef struct fa_params {
   const void* eq;
   const void* ek;
   /* scratch written by fa_mask_plan and read by the compute kernels
-     (required when score_mode != 0; size from fa_workspace_bytes) */
+     (required when fa_workspace_bytes is not 0) */
   void*       workspace;
   uint64_t    workspace_bytes;
 
@@ -156,6 +168,8 @@ typedef struct fa_params {
      it from one call to the next; two launches that share it must be ordered on one stream. */
   void*       split_scratch;
   uint64_t    split_scratch_bytes;
+  int32_t     nseq;       /* FA_SCORE_MODE3_PACKED: number of sequences */
+  int32_t     reserved;
 } fa_params;
 
 /* ABI version of the loaded library (== FA_ABI_VERSION of the header it was built from). */
@@ -176,7 +190,7 @@ int fa_last_hip_error(void);
           3 = fa_bwd_dkdv (stage 1, and FA_FLAG_DEBUG_NO_PAIR_WAIT is accepted). */
 int fa_validate(const fa_params* p, int stage);
 
-/* Bytes of workspace fa_mask_plan needs for these sizes (0 when score_mode == 0). */
+/* Bytes of workspace fa_mask_plan needs for these sizes (0 when score_mode == 0 or 2, except with FA_FLAG_SPLIT_KEYS). */
 uint64_t fa_workspace_bytes(const fa_params* p);
 
 /* The first fa_workspace_plan_bytes() bytes of the workspace carry the plan from fa_mask_plan to

@@ -1,0 +1,152 @@
+"""The launch forms chosen by size: heads that share a tile, the decode form, split key ranges without ids, packed sequences.
+Each at the sizes where its tiles, chunks and tables have edges, against the CPU oracle on the same rounded inputs."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from tests._tol import check_close
+
+pytestmark = pytest.mark.gpu
+
+# B, H, Hk, M, N, D, dtype, causal, window, prefix
+FORWARD_CASES = [
+    (2, 8, 2, 1, 1, 128, torch.bfloat16, True, 0, 0),          # decode form: one key
+    (1, 8, 2, 1, 33, 128, torch.bfloat16, True, 0, 0),         # ... one key into the second block
+    (3, 4, 4, 1, 1000, 64, torch.float16, True, 0, 0),         # ... no groups
+    (1, 16, 2, 4, 4099, 128, torch.bfloat16, True, 0, 0),      # ... a full tile of 32 packed rows, split key range
+    (1, 3, 1, 7, 2048, 128, torch.bfloat16, False, 0, 0),      # ... a group of three heads, 21 rows
+    (2, 8, 8, 31, 600, 32, torch.bfloat16, True, 0, 0),
+    (1, 4, 2, 2, 5000, 16, torch.float16, True, 0, 0),
+    (1, 4, 1, 3, 3000, 128, torch.bfloat16, True, 700, 0),     # ... a window that leaves most blocks out
+    (1, 4, 1, 5, 900, 64, torch.bfloat16, True, 0, 890),       # ... a prefix past some diagonals
+    (1, 40, 1, 1, 777, 128, torch.bfloat16, True, 0, 0),       # a group larger than the decode tile
+    (1, 4, 2, 100, 9000, 128, torch.bfloat16, True, 0, 0),     # 64-row tiles, split key range
+    (1, 6, 2, 43, 2500, 64, torch.float16, True, 300, 0),
+    (1, 2, 2, 129, 20000, 128, torch.bfloat16, False, 0, 0),
+    (2, 12, 4, 333, 333, 128, torch.bfloat16, True, 0, 0),     # short prompt, groups of three
+]
+
+
+def _tensors(B, H, Hk, M, N, D, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, h, n, D, generator=g).to(dtype) for h, n in ((H, M), (Hk, N), (Hk, N), (H, M))]
+
+
+@pytest.mark.parametrize("case", FORWARD_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-%s-c%d-w%d-p%d" % (
+    *c[:6], str(c[6])[6:], *c[7:]))
+def test_forward_only_forms(case):
+    from flash_mi355 import attention_with_lse
+    from oracle import attention_oracle as O
+    B, H, Hk, M, N, D, dtype, causal, window, prefix = case
+    print("case", case, flush=True)
+    q, k, v, _ = _tensors(B, H, Hk, M, N, D, dtype, 5)
+    room = torch.full((B, Hk, N + 50, D), float("nan"), dtype=dtype, device="cuda")   # a cache: what lies behind the keys is not read
+    room_v = room.clone()
+    room[:, :, :N] = k.cuda()
+    room_v[:, :, :N] = v.cuda()
+    with torch.no_grad():
+        for scale in (None, -0.2):
+            o, lse = attention_with_lse(q.cuda(), room[:, :, :N], room_v[:, :, :N], causal, scale, window=window, prefix=prefix)
+            torch.cuda.synchronize()
+            ro, rl = O.attention_closed_form(q, k, v, causal, scale, None, None, 0, window=window, prefix=prefix)[:2]
+            check_close(f"o (scale {scale})", o, ro)
+            assert (lse.cpu() - rl).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("case", [(1, 8, 2, 200, 200, 128, True), (2, 6, 2, 75, 333, 64, True), (1, 8, 1, 150, 150, 128, False), (2, 16, 2, 1, 500, 128, True)])
+def test_heads_that_share_a_tile_backward(case):
+    from flash_mi355 import attention
+    from oracle import attention_oracle as O
+    B, H, Hk, M, N, D, causal = case
+    print("case", case, flush=True)
+    q, k, v, do = _tensors(B, H, Hk, M, N, D, torch.bfloat16, 6)
+    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    out = attention(qd, kd, vd, causal)
+    out.backward(do.cuda())
+    torch.cuda.synchronize()
+    ro, _, rdq, rdk, rdv = O.attention_autograd(q, k, v, do, causal, None, None, None, 0)
+    for name, got, ref in (("o", out.detach(), ro), ("dq", qd.grad, rdq), ("dk", kd.grad, rdk), ("dv", vd.grad, rdv)):
+        check_close(name, got, ref)
+
+
+# query lengths, key lengths (None: the queries'), tokens behind the last boundary, H, Hk, D, causal, window
+PACKED_CASES = [
+    ([64, 128, 1, 0, 65, 300], None, 0, 4, 2, 128, True, 0),
+    ([33, 31, 32], None, 17, 8, 2, 64, True, 0),
+    ([5, 260, 129], None, 3, 2, 2, 128, False, 0),
+    ([190, 64], None, 0, 6, 2, 128, True, 50),
+    ([1] * 40, [int(x) for x in np.random.default_rng(0).integers(1, 900, 40)], 0, 8, 2, 128, True, 0),    # decoding
+    ([1, 2, 1], [7000, 40, 3], 0, 4, 1, 64, True, 0),                                                       # one long range to split
+    ([128, 17, 70], [3000, 500, 70], 0, 8, 2, 128, True, 0),                                                # chunked prefill
+    ([40, 90, 12], [20, 300, 0], 5, 4, 4, 128, True, 0),                                                    # fewer keys than queries, none
+    ([40, 9, 12], [20, 300, 50], 0, 4, 2, 32, False, 0),                                                    # cross attention
+    ([100, 60], [400, 200], 0, 4, 2, 128, True, 128),
+]
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("i", range(len(PACKED_CASES)))
+def test_packed_sequences(i, grad):
+    from flash_mi355 import attention_varlen
+    from oracle import attention_oracle as O
+    lq, lk, tail, H, Hk, D, causal, window = PACKED_CASES[i]
+    print("case", PACKED_CASES[i], grad, flush=True)
+    same = lk is None
+    lk = lq if same else lk
+    cuq, cuk = (np.concatenate([[0], np.cumsum(x)]) for x in (lq, lk))
+    Tq, Tk = int(cuq[-1]) + tail, int(cuk[-1]) + tail
+    g = torch.Generator().manual_seed(40 + i)
+    q, k, v, do = (torch.randn(t, h, D, generator=g).to(torch.bfloat16) for t, h in ((Tq, H), (Tk, Hk), (Tk, Hk), (Tq, H)))
+    qd, kd, vd = (t.cuda().requires_grad_(grad) for t in (q, k, v))
+    cq = torch.from_numpy(cuq).to(torch.int32 if i % 2 else torch.int64).cuda()
+    ck = None if same else torch.from_numpy(cuk).to(cq.dtype).cuda()
+    out = attention_varlen(qd, kd, vd, cq, ck, causal=causal, window=window)
+    if grad:
+        out.backward(do.cuda())
+    torch.cuda.synchronize()
+    starts = [(int(a), int(b), int(c), int(d)) for a, b, c, d in zip(cuq[:-1], cuq[1:], cuk[:-1], cuk[1:])]
+    starts.append((int(cuq[-1]), Tq, int(cuk[-1]), Tk))   # what lies behind the last boundary is a sequence too
+    for a, b, c, d in starts:
+        if a == b or c == d:
+            assert out[a:b].abs().sum().item() == 0
+            if grad:
+                assert kd.grad[c:d].abs().sum().item() == 0 and vd.grad[c:d].abs().sum().item() == 0 and qd.grad[a:b].abs().sum().item() == 0
+            continue
+        sq = lambda t: t[a:b].transpose(0, 1)[None]
+        sk = lambda t: t[c:d].transpose(0, 1)[None]
+        m, n = b - a, d - c
+        ids = torch.zeros(1, H, m, dtype=torch.int32), torch.zeros(1, H, n, dtype=torch.int32)
+        pos = (torch.arange(m) + n - m).clamp(min=-1)[None].to(torch.int32) if causal else None
+        args = (causal, None, ids[0], ids[1], 1)
+        ro, _, rdq, rdk, rdv = O.attention_autograd(sq(q), sk(k), sk(v), sq(do), *args, window=window, qpos=pos)
+        check_close(f"o {a}:{b}", sq(out.detach().float().cpu()), ro, quiet=True)
+        if grad:
+            for name, got, ref, sl in (("dq", qd.grad, rdq, sq), ("dk", kd.grad, rdk, sk), ("dv", vd.grad, rdv, sk)):
+                check_close(f"{name} {a}:{b}", sl(got.float().cpu()), ref, quiet=True)
+
+
+def test_packed_graph_replay():
+    """A captured packed call is replayed with other boundaries in the same buffer: the tile tables are rebuilt on the device."""
+    from flash_mi355 import attention_varlen
+    H, Hk, D = 8, 2, 128
+    g = torch.Generator().manual_seed(9)
+    lens = [[1, 3, 1, 1], [2, 1, 2, 1]], [[700, 2500, 90, 30], [10, 310, 2000, 1000]]
+    Tq, Tk = sum(lens[0][0]), sum(lens[1][0])
+    q, k, v = (torch.randn(t, h, D, generator=g).to(torch.bfloat16).cuda() for t, h in ((Tq, H), (Tk, Hk), (Tk, Hk)))
+    cu = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device="cuda")
+    cq, ck = cu(lens[0][0]), cu(lens[1][0])
+    with torch.no_grad():
+        attention_varlen(q, k, v, cq, ck, causal=True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = attention_varlen(q, k, v, cq, ck, causal=True)
+        for rep in range(4):
+            cq.copy_(cu(lens[0][rep % 2])); ck.copy_(cu(lens[1][rep % 2]))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            got = out.clone()
+            assert torch.equal(got, attention_varlen(q, k, v, cq, ck, causal=True)), rep

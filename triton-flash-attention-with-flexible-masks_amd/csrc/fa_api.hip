@@ -50,14 +50,13 @@ extern "C" int fa_validate(const fa_params* p, int stage) {
   if (p->dtype != FA_DTYPE_BF16 && p->dtype != FA_DTYPE_FP16 && p->dtype != FA_DTYPE_FP32) return FA_ERR_DTYPE;
   if (p->B <= 0 || p->H <= 0 || p->Hk <= 0 || p->M <= 0 || p->N <= 0) return FA_ERR_SHAPE;
   if (p->H % p->Hk != 0) return FA_ERR_SHAPE;
-  if (p->causal && p->N < p->M && p->qpos == nullptr) return FA_ERR_SHAPE;
-  if (p->score_mode != FA_SCORE_MODE0_NOPE && p->score_mode != FA_SCORE_MODE1_DOC && p->score_mode != FA_SCORE_MODE2_BLOCK)
-    return FA_ERR_MODE;
+  if (p->causal && p->N < p->M && p->qpos == nullptr && p->score_mode != FA_SCORE_MODE3_PACKED) return FA_ERR_SHAPE;
+  if (p->score_mode < FA_SCORE_MODE0_NOPE || p->score_mode > FA_SCORE_MODE3_PACKED) return FA_ERR_MODE;
   if (p->score_mode == FA_SCORE_MODE2_BLOCK) {
     if (p->eq == nullptr) return FA_ERR_MODE;
     if (p->eq_stride[0] < 0 || p->eq_stride[1] < 0 || p->eq_stride[2] < (p->N + FA_MASK_BLOCK - 1) / FA_MASK_BLOCK) return FA_ERR_STRIDE;
   }
-  if ((p->flags & ~(FA_FLAG_DQ_DELTA | FA_FLAG_DEBUG_NO_PAIR_WAIT)) != 0) return FA_ERR_MODE;
+  if ((p->flags & ~(FA_FLAG_DQ_DELTA | FA_FLAG_SPLIT_KEYS | FA_FLAG_DEBUG_NO_PAIR_WAIT)) != 0) return FA_ERR_MODE;
   if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) != 0 && stage != 3) return FA_ERR_MODE;   // a diagnostic of fa_bwd_dkdv alone
   if (p->window < 0 || p->prefix < 0 || (p->window > 0 && p->prefix > 0)) return FA_ERR_MODE;
   if ((p->window > 0 || p->prefix > 0) && !p->causal) return FA_ERR_MODE;
@@ -65,6 +64,14 @@ extern "C" int fa_validate(const fa_params* p, int stage) {
   if (p->score_mode == FA_SCORE_MODE1_DOC) {
     if (p->eq == nullptr || p->ek == nullptr) return FA_ERR_MODE;
     if (p->id_dtype != FA_IDTYPE_I32 && p->id_dtype != FA_IDTYPE_I64) return FA_ERR_DTYPE;
+  }
+  if (p->score_mode == FA_SCORE_MODE3_PACKED) {
+    if (p->eq == nullptr || p->ek == nullptr || p->prefix > 0 || p->qpos != nullptr) return FA_ERR_MODE;
+    if (p->id_dtype != FA_IDTYPE_I32 && p->id_dtype != FA_IDTYPE_I64) return FA_ERR_DTYPE;
+    if (p->dtype == FA_DTYPE_FP32) return FA_ERR_DTYPE;
+    if (p->B != 1 || p->nseq <= 0 || (int64_t(p->M) * (p->H / p->Hk)) >> 31) return FA_ERR_SHAPE;
+  }
+  if (fa_workspace_bytes(p) > 0) {
     if (p->workspace == nullptr) return FA_ERR_WORKSPACE;
     if ((reinterpret_cast<uintptr_t>(p->workspace) & 255) != 0) return FA_ERR_ALIGN;
     if (p->split_scratch == nullptr) {
@@ -92,27 +99,34 @@ extern "C" int fa_validate(const fa_params* p, int stage) {
   return FA_OK;
 }
 
-extern "C" uint64_t fa_workspace_bytes(const fa_params* p) {
-  if (p == nullptr || p->score_mode != FA_SCORE_MODE1_DOC) return 0;
-  if (p->B <= 0 || p->H <= 0 || p->M <= 0 || p->N <= 0) return 0;
-  return ws_layout(p).total;
+// plan bytes, all bytes
+struct WsSize { uint64_t plan, total; };
+static WsSize ws_size(const fa_params* p) {
+  if (p == nullptr || p->B <= 0 || p->H <= 0 || p->Hk <= 0 || p->H % p->Hk != 0 || p->M <= 0 || p->N <= 0) return {0, 0};
+  if (p->score_mode == FA_SCORE_MODE1_DOC) {
+    const WsLayout w = ws_layout(p);
+    return {w.plan_bytes, w.total};
+  }
+  if (p->score_mode == FA_SCORE_MODE3_PACKED || (p->score_mode == FA_SCORE_MODE0_NOPE && (p->flags & FA_FLAG_SPLIT_KEYS))) {
+    const TabLayout w = tab_layout(p, fwd_config(p));
+    return {w.plan_bytes, w.total};
+  }
+  return {0, 0};
 }
 
-extern "C" uint64_t fa_workspace_plan_bytes(const fa_params* p) {
-  if (p == nullptr || p->score_mode != FA_SCORE_MODE1_DOC) return 0;
-  if (p->B <= 0 || p->H <= 0 || p->M <= 0 || p->N <= 0) return 0;
-  return ws_layout(p).plan_bytes;
-}
-
+extern "C" uint64_t fa_workspace_bytes(const fa_params* p) { return ws_size(p).total; }
+extern "C" uint64_t fa_workspace_plan_bytes(const fa_params* p) { return ws_size(p).plan; }
 extern "C" uint64_t fa_workspace_scratch_bytes(const fa_params* p) {
-  if (p == nullptr || p->score_mode != FA_SCORE_MODE1_DOC) return 0;
-  if (p->B <= 0 || p->H <= 0 || p->M <= 0 || p->N <= 0) return 0;
-  const WsLayout w = ws_layout(p);
-  return w.total - w.plan_bytes;
+  const WsSize w = ws_size(p);
+  return w.total - w.plan;
 }
 
 static KArgs make_args(const fa_params* p, uint64_t split_budget = kSplitScratchBudget) {
   KArgs a;
+  const FwdCfg fc = fwd_config(p);
+  a.pack = fc.pack; a.nHp = p->H / fc.pack;
+  a.bm = fc.bm; a.nTiles = fc.tiles; a.dsplit = fc.split;
+  a.shdr = nullptr; a.qtab = a.ktab = nullptr; a.nQent = a.nKent = 0;
   a.q = p->q; a.k = p->k; a.v = p->v; a.o = p->o; a.lse = p->lse;
   a.dout = p->dout; a.dq = p->dq; a.dk = p->dk; a.dv = p->dv; a.delta = p->delta;
   a.q_bs = p->q_stride[0]; a.q_hs = p->q_stride[1]; a.q_rs = p->q_stride[2];
@@ -143,6 +157,20 @@ static KArgs make_args(const fa_params* p, uint64_t split_budget = kSplitScratch
   if (p->score_mode == FA_SCORE_MODE2_BLOCK) {
     a.bmask = reinterpret_cast<const unsigned char*>(p->eq);
     a.bm_bs = p->eq_stride[0]; a.bm_hs = p->eq_stride[1]; a.bm_rs = p->eq_stride[2];
+  }
+  if (p->score_mode == FA_SCORE_MODE3_PACKED || (p->score_mode == FA_SCORE_MODE0_NOPE && a.dsplit > 1)) {
+    const TabLayout w = tab_layout(p, fc);
+    char* ws = reinterpret_cast<char*>(p->workspace);
+    char* sc_base = p->split_scratch != nullptr ? reinterpret_cast<char*>(p->split_scratch) - w.plan_bytes : ws;
+    a.sk_cnt = reinterpret_cast<int*>(ws + w.off_cnt);
+    a.sk_ml = reinterpret_cast<float*>(sc_base + w.off_ml);
+    a.sk_o = reinterpret_cast<float*>(sc_base + w.off_o);
+    if (p->score_mode == FA_SCORE_MODE3_PACKED) {
+      a.shdr = reinterpret_cast<const SeqHdr*>(ws + w.off_hdr);
+      a.qtab = reinterpret_cast<const SeqTile*>(ws + w.off_q);
+      a.ktab = reinterpret_cast<const SeqTile*>(ws + w.off_k);
+      a.nQent = w.nQ; a.nKent = w.nK;
+    }
   }
   if (p->score_mode == FA_SCORE_MODE1_DOC) {
     const WsLayout w = ws_layout(p, split_budget);
@@ -183,6 +211,16 @@ static int finish(int hip_rc) {
 extern "C" int fa_mask_plan(const fa_params* p, void* stream) {
   int rc = fa_validate(p, 2);
   if (rc != FA_OK) return rc;
+  if (p->score_mode == FA_SCORE_MODE3_PACKED) {
+    const FwdCfg c = fwd_config(p);
+    return finish(launch_seq_plan(p, c, tab_layout(p, c), reinterpret_cast<hipStream_t>(stream)));
+  }
+  if (p->score_mode == FA_SCORE_MODE0_NOPE && fa_workspace_bytes(p) > 0) {
+    const FwdCfg c = fwd_config(p);
+    const TabLayout w = tab_layout(p, c);
+    return finish(launch_zero_counters(reinterpret_cast<int*>(reinterpret_cast<char*>(p->workspace) + w.off_cnt), w.nCnt * (p->H / c.pack),
+                                       reinterpret_cast<hipStream_t>(stream)));
+  }
   if (p->score_mode != FA_SCORE_MODE1_DOC) return FA_OK;
   return finish(launch_mask_plan(p, ws_layout(p), reinterpret_cast<hipStream_t>(stream)));
 }
@@ -193,6 +231,7 @@ extern "C" int fa_fwd(const fa_params* p, void* stream) {
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p->dtype == FA_DTYPE_FP32) return finish(launch_fwd_f32(make_args(p), p->D, causal, doc, s));
+  if (fwd_config(p).dec) return finish(launch_decode(make_args(p), p->dtype, p->D, causal, s));
   return finish(launch_fwd(make_args(p), p->dtype, p->D, causal, doc, s));
 }
 
@@ -284,6 +323,7 @@ extern "C" int fa_mask_dump(const fa_params* p, uint8_t* out, void* stream) {
   int rc = fa_validate(p, 2);
   if (rc != FA_OK) return rc;
   if (out == nullptr) return FA_ERR_NULLPTR;
+  if (p->score_mode == FA_SCORE_MODE3_PACKED) return FA_ERR_NOT_IMPLEMENTED;
   return finish(launch_mask_dump(make_args(p), p->causal != 0, p->score_mode == FA_SCORE_MODE1_DOC, out,
                                  reinterpret_cast<hipStream_t>(stream)));
 }

@@ -84,7 +84,8 @@ void bwd_dkdv_kernel(const KArgs a) {
   // belong to the column form): a workgroup then takes kColsRun key tiles, nSlots tiles apart, and steps over
   // those -- a workgroup that only finds out that it is not needed costs the dispatcher as much as a short
   // useful one (8192 of them: 50 us), a skipped tile of a run costs a comparison.
-  const int nSlots = COLS ? (nKt + kColsRun - 1) / kColsRun : nKt;
+  const bool packed = !DOC && a.ktab != nullptr;   // packed sequences: the slots are the plan's key tiles, longest first
+  const int nSlots = COLS ? (nKt + kColsRun - 1) / kColsRun : (packed ? a.nKent : nKt);
   int bid = (int)blockIdx.x;   // index of the workgroup among those of its form
   if constexpr (COLS) {
     static_assert(DOC && (SPLIT ? 128 * NKB : 64 * NKB) == 256, "the column form runs with ids, 4 waves per workgroup");
@@ -103,8 +104,17 @@ void bwd_dkdv_kernel(const KArgs a) {
 
   // one workgroup per (key tile, batch, kv head) -- or per run of key tiles, see above
   int kt0, bhk;
-  if (!block_to_tile(nSlots, a.B * a.Hk, false, kt0, bhk, bid)) return;  // causal: the first key tiles see the most rows
+  if (!block_to_tile(nSlots, a.B * a.Hk, packed, kt0, bhk, bid)) return;  // causal: the first key tiles see the most rows
   const int b = bhk / a.Hk, hk = bhk % a.Hk;
+  int M = a.M, N = a.N, gap = a.gap;   // of the batch entry, or of the sequence
+  int64_t q0 = 0, k0 = 0;
+  if (packed) {
+    if (kt0 >= a.shdr->nk) return;
+    const SeqTile* __restrict__ e = a.ktab + kt0;
+    M = __builtin_amdgcn_readfirstlane(e->M); N = __builtin_amdgcn_readfirstlane(e->N); gap = __builtin_amdgcn_readfirstlane(e->gap);
+    q0 = __builtin_amdgcn_readfirstlane(e->q0); k0 = __builtin_amdgcn_readfirstlane(e->k0);
+    kt0 = __builtin_amdgcn_readfirstlane(e->tile);
+  }
   const int ncols = COLS ? gcol_info(a, b, hk).ncols : 0;   // leading keys that belong to the column form of this launch
   bool ran = false;
   for (int rr = 0; rr < (COLS ? kColsRun : 1); ++rr) {
@@ -116,18 +126,18 @@ void bwd_dkdv_kernel(const KArgs a) {
   pair_lost = 0;
   const int nw = n0 + kb * 32;
   const int key = nw + lq;
-  const int keyc = key < a.N ? key : a.N - 1;
+  const int keyc = key < N ? key : N - 1;
 
   // B operand held for the whole kernel: K^T for the score wave, V^T for the gradient wave.
   // Lane holds d = 16*ks + 8*g .. +7 of its key row.
-  const T* srcp = role == 0 ? reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + int64_t(keyc) * a.k_rs
-                            : reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + int64_t(keyc) * a.v_rs;
+  const T* srcp = role == 0 ? reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + (k0 + keyc) * a.k_rs
+                            : reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + (k0 + keyc) * a.v_rs;
   vec8 frag[KS];
   vec8 frag2[KS];   // V^T next to K^T when one wave does both roles
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) frag[ks] = *reinterpret_cast<const vec8*>(srcp + ks * 16 + g * 8);
   if (!SPLIT) {
-    const T* vsrc = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + int64_t(keyc) * a.v_rs;
+    const T* vsrc = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + (k0 + keyc) * a.v_rs;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) frag2[ks] = *reinterpret_cast<const vec8*>(vsrc + ks * 16 + g * 8);
   }
@@ -148,11 +158,11 @@ void bwd_dkdv_kernel(const KArgs a) {
   // Without ids a row is named by its index r and its diagonal sits at key gap + r; with ids rows are
   // named by the diagonal position the mask plan stored for them (gap + row, or the caller's per-row
   // position), so the offset is 0 and the names run up to kPosMax.
-  const int gk = DOC ? 0 : a.gap;
-  const int rcap = DOC ? kPosMax : a.M - 1;
+  const int gk = DOC ? 0 : gap;
+  const int rcap = DOC ? kPosMax : M - 1;
   const int row_lo = CAUSAL ? (key <= a.pfx_m1 ? 0 : max(0, key - gk)) : 0;
   const int row_hi = CAUSAL ? min(rcap, key - gk + a.win - 1) : rcap;
-  const unsigned row_span = (key < a.N && row_hi >= row_lo) ? (unsigned)(row_hi - row_lo + 1) : 0u;
+  const unsigned row_span = (key < N && row_hi >= row_lo) ? (unsigned)(row_hi - row_lo + 1) : 0u;
 
   // per query head state (set at the top of the head loop)
   const float* lsep = nullptr;
@@ -198,7 +208,7 @@ void bwd_dkdv_kernel(const KArgs a) {
       const int m0 = tile * BQ;
       ldQ.issue(m0, smem + bufi * TILE_BYTES);
       ldO.issue(m0, smem + (2 + bufi) * TILE_BYTES);
-      const int r = m0 + lane < a.M ? m0 + lane : a.M - 1;
+      const int r = m0 + lane < M ? m0 + lane : M - 1;
       if (wave == 0) glb_load_lds4(lsep + r, aux);
       if (wave == 1) glb_load_lds4(delp + r, aux + 256);
     } else {
@@ -519,12 +529,12 @@ void bwd_dkdv_kernel(const KArgs a) {
 
   for (int gi = 0; gi < a.G; ++gi) {
     const int h = hk * a.G + gi;
-    lsep = a.lse + (int64_t(b) * a.H + h) * a.M;
-    delp = a.delta + (int64_t(b) * a.H + h) * a.M;
-    ldQ.init(reinterpret_cast<const T*>(a.q) + b * a.q_bs + h * a.q_hs, a.q_rs, a.M);
-    ldO.init(reinterpret_cast<const T*>(a.dout) + b * a.do_bs + h * a.do_hs, a.do_rs, a.M);
+    lsep = a.lse + (int64_t(b) * a.H + h) * a.M + q0;
+    delp = a.delta + (int64_t(b) * a.H + h) * a.M + q0;
+    ldQ.init(reinterpret_cast<const T*>(a.q) + b * a.q_bs + h * a.q_hs + q0 * a.q_rs, a.q_rs, M);
+    ldO.init(reinterpret_cast<const T*>(a.dout) + b * a.do_bs + h * a.do_hs + q0 * a.do_rs, a.do_rs, M);
     int gk_lo = 0, gk_hi = 0;   // id interval of the workgroup's 128 keys
-    int nQtiles = (a.M + BQ - 1) / BQ;
+    int nQtiles = (M + BQ - 1) / BQ;
     int first = CAUSAL ? (n0 <= a.pfx_m1 ? 0 : max(0, n0 - gk) / BQ) : 0;
     // sliding window: the last row that sees a key of this workgroup
     const int wg_rhi = CAUSAL ? min(rcap, n0 + BK - 1 - gk + a.win - 1) : rcap;
@@ -542,7 +552,7 @@ void bwd_dkdv_kernel(const KArgs a) {
         const IdSummary s1 = ks[n0 / kSumRows + 1];
         gk_lo = min(gk_lo, s1.lo); gk_hi = max(gk_hi, s1.hi);
       }
-      const bool valid = key < a.N;
+      const bool valid = key < N;
       int lo_ = valid ? ek_j : 0x7fffffff, hi_ = valid ? ek_j : (int)0x80000000;
 #pragma unroll
       for (int off = 16; off >= 1; off >>= 1) {
@@ -561,10 +571,10 @@ void bwd_dkdv_kernel(const KArgs a) {
       bool skip, lim, doc = false, glob = false, col = false, none = false;
       if (!DOC) {
         const int m0 = t * BQ;
-        const int rmin = m0, rmax = min(m0 + BQ - 1, a.M - 1);
-        skip = (nw >= a.N) || (CAUSAL && ((a.gap + rmax < nw && nw > a.pfx_m1) || a.gap + rmin - a.win + 1 > nw + 31));
-        lim = (m0 + BQ > a.M) || (nw + 32 > a.N) ||
-              (CAUSAL && ((a.gap + rmin < nw + 31 && nw + 31 > a.pfx_m1) || a.gap + rmax - a.win + 1 > nw));
+        const int rmin = m0, rmax = min(m0 + BQ - 1, M - 1);
+        skip = (nw >= N) || (CAUSAL && ((gap + rmax < nw && nw > a.pfx_m1) || gap + rmin - a.win + 1 > nw + 31));
+        lim = (m0 + BQ > M) || (nw + 32 > N) ||
+              (CAUSAL && ((gap + rmin < nw + 31 && nw + 31 > a.pfx_m1) || gap + rmax - a.win + 1 > nw));
         if (bmk != nullptr) {
           const bool in = t < a.nBr;
           const unsigned char* r = bmk + int64_t(t) * a.bm_rs;
@@ -575,9 +585,9 @@ void bwd_dkdv_kernel(const KArgs a) {
           none = (b0 | b1) == 0;
         }
       } else {
-        skip = (nw >= a.N) || (CAUSAL && ((qs.rmax < nw && nw > a.pfx_m1) || qs.rmin - a.win + 1 > nw + 31)) ||
+        skip = (nw >= N) || (CAUSAL && ((qs.rmax < nw && nw > a.pfx_m1) || qs.rmin - a.win + 1 > nw + 31)) ||
                !doc_may_keep(qs.lo, qs.hi, qs.glob, wk_lo, wk_hi);
-        lim = (qs.nvalid < BQ) || (nw + 32 > a.N) ||
+        lim = (qs.nvalid < BQ) || (nw + 32 > N) ||
               (CAUSAL && ((qs.rmin < nw + 31 && nw + 31 > a.pfx_m1) || qs.rmax - a.win + 1 > nw));
         doc = !doc_all_keep(qs.lo, qs.hi, wk_lo, wk_hi);
         glob = qs.glob != 0;
@@ -640,13 +650,13 @@ void bwd_dkdv_kernel(const KArgs a) {
   FA_TRACE_ONLY(if (SPLIT && threadIdx.x == 64 * NKB && blockIdx.x < fa::kTraceWgs) g_trace_dkdv[blockIdx.x * 8 + 1] = tr_wait;)
   {
     // dK / dV rows leave through LDS (store_rows_through_lds), once every wave is done with the last query tile
-    T* dvp = reinterpret_cast<T*>(a.dv) + b * a.dv_bs + hk * a.dv_hs;
-    T* dkp = reinterpret_cast<T*>(a.dk) + b * a.dk_bs + hk * a.dk_hs;
+    T* dvp = reinterpret_cast<T*>(a.dv) + b * a.dv_bs + hk * a.dv_hs + k0 * a.dv_rs;
+    T* dkp = reinterpret_cast<T*>(a.dk) + b * a.dk_bs + hk * a.dk_hs + k0 * a.dk_rs;
     __syncthreads();
     char* patch = smem + wave * row_patch_bytes<D>();
     auto store = [&](T* base, const int64_t rs, const f32x16 (&v)[DBN], const float sc) __attribute__((always_inline)) {
       store_rows_through_lds<E, D, DBN>(patch, v, sc, [&](const int r) -> T* {
-        return nw + r < a.N ? base + int64_t(nw + r) * rs : nullptr;
+        return nw + r < N ? base + int64_t(nw + r) * rs : nullptr;
       });
     };
     if (SPLIT) {
@@ -679,7 +689,8 @@ static int launch_nkb(const KArgs& a, hipStream_t s) {
   auto kern = bwd_dkdv_kernel<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  const int blocks = COLS ? grid_blocks((nKt + kColsRun - 1) / kColsRun, a.B * a.Hk) + dkdv_cols_blocks(a) : grid_blocks(nKt, a.B * a.Hk);
+  const int slots = !DOC && a.ktab != nullptr ? a.nKent : nKt;
+  const int blocks = COLS ? grid_blocks((nKt + kColsRun - 1) / kColsRun, a.B * a.Hk) + dkdv_cols_blocks(a) : grid_blocks(slots, a.B * a.Hk);
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(SPLIT ? 128 * NKB : 64 * NKB), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -703,6 +714,7 @@ static int launch_one(const KArgs& a, hipStream_t s) {
   }
   if constexpr (D > 64) {
     if (DOC || a.bmask != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s);
+    if (a.ktab != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, kSeqKeyTile / 32>(a, s);
     int tiles = (a.M + 63) / 64;
     if (CAUSAL) tiles = a.win < 0x3fffffff ? min(tiles, a.win / 64 + 3) : (tiles + 1) / 2;
     tiles *= a.G;

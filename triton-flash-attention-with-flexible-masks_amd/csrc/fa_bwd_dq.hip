@@ -29,7 +29,7 @@ void bwd_dq_kernel(const KArgs a) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
-  constexpr int BM = 128, BN = 64, KS = D / 16;
+  constexpr int BN = 64, KS = D / 16;
   constexpr int DL = D < 32 ? 32 : D;  // LDS row width: D = 16 is staged as 32 columns, the upper 16 zero
   constexpr int DBN = DL / 32;
   constexpr int TILE_BYTES = BN * DL * 2;
@@ -40,33 +40,22 @@ void bwd_dq_kernel(const KArgs a) {
   FA_STAMP(g_trace_dq, 0, FA_CLOCK()); FA_STAMP(g_trace_dq, 4, 0); FA_STAMP(g_trace_dq, 6, 0); FA_STAMP(g_trace_dq, 7, -1);
   FA_TRACE_ONLY(int tr_tiles = 0;)
 
-  const int nQt = DOC ? a.Pp / BM : (a.M + BM - 1) / BM;
-  const int nSlots = nQt + (DOC ? split_extra(a) : 0);
-  int slot, bh;
-  if (!block_to_tile(nSlots, a.B * a.H, DOC && nQt >= 32, slot, bh)) return;
-  const int b = bh / a.H, h = bh % a.H, hk = h / a.G;
-  QWork wk;
-  QHeader hd = {};
-  if (DOC) hd = a.qhdr[b * a.qh_bs + h * a.qh_hs];
-  if (!q_work<DOC>(a, hd, nQt, slot, wk)) return;
+  TileGeo ge;
   QTileCtx<CAUSAL, DOC> qc;
-  if (!qc.init(a, b, h, wk.tile, threadIdx.x >> 6)) return;
-  q_work_finish(a, hd, wk);
-  int kt_first = qc.first_tile(a), kt_last = qc.last_tile(a);
-  const int nsplit = split_range(a, wk, kt_first, kt_last);
-  if (wk.split >= nsplit) return;
-  FA_STAMP(g_trace_dq, 1, FA_CLOCK()); FA_STAMP(g_trace_dq, 7, (long long)wk.tile | ((long long)wk.split << 16) | ((long long)nsplit << 24));
+  int kt_first, kt_last;
+  if (!tile_work(a, ge, qc, kt_first, kt_last)) return;
+  const int b = ge.b, h = ge.h0, hk = ge.hk, nsplit = ge.nchunk;
+  FA_STAMP(g_trace_dq, 1, FA_CLOCK()); FA_STAMP(g_trace_dq, 7, (long long)ge.tile | ((long long)ge.chunk << 16) | ((long long)nsplit << 24));
   const int row = qc.row, rowc = qc.rowc, eq_i = qc.eq_i;
   const int* ekp = qc.ekp;
 
-  const T* qp = reinterpret_cast<const T*>(a.q) + b * a.q_bs + h * a.q_hs;
-  const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs;
-  const T* vp = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs;
-  const T* dop = reinterpret_cast<const T*>(a.dout) + b * a.do_bs + h * a.do_hs;
-  T* dqp = reinterpret_cast<T*>(a.dq) + b * a.dq_bs + h * a.dq_hs;
-  const float* lsep = a.lse + (int64_t(b) * a.H + h) * a.M;
-  float* delp = a.delta + (int64_t(b) * a.H + h) * a.M;
-  const T* op = reinterpret_cast<const T*>(a.o) + b * a.o_bs + h * a.o_hs;
+  const T* qp = reinterpret_cast<const T*>(a.q) + b * a.q_bs + (h + qc.hg) * a.q_hs + ge.q0 * a.q_rs;
+  const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + ge.k0 * a.k_rs;
+  const T* vp = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + ge.k0 * a.v_rs;
+  const T* dop = reinterpret_cast<const T*>(a.dout) + b * a.do_bs + (h + qc.hg) * a.do_hs + ge.q0 * a.do_rs;
+  T* dqp = reinterpret_cast<T*>(a.dq) + b * a.dq_bs + h * a.dq_hs + ge.q0 * a.dq_rs;
+  const int64_t row_l = (int64_t(b) * a.H + h + qc.hg) * a.M + ge.q0 + rowc;   // of LSE and delta
+  const T* op = reinterpret_cast<const T*>(a.o) + b * a.o_bs + (h + qc.hg) * a.o_hs + ge.q0 * a.o_rs;
   const bool own_delta = a.dq_delta != 0;   // delta = rowsum(O * dO) is computed here instead of being read
 
   vec8 qf[KS], dof[KS];
@@ -81,12 +70,12 @@ void bwd_dq_kernel(const KArgs a) {
     for (int ks = 0; ks < KS; ++ks) of[ks] = *reinterpret_cast<const vec8*>(op + int64_t(rowc) * a.o_rs + ks * 16 + g * 8);
   }
   const float c = a.scale_log2e;
-  float L_i = lsep[rowc];
-  float delta_i = own_delta ? 0.f : delp[rowc];
+  float L_i = a.lse[row_l];
+  float delta_i = own_delta ? 0.f : a.delta[row_l];
 
   // decisions of this wave for key tile t, evaluated by the lane that tests the tile
   QBlockMask bmq;
-  bmq.init(a, b, h, wk.tile);
+  bmq.init(a, b, h, ge.tile);
   const bool halved = qc.halved;
   const int sub = __builtin_amdgcn_readfirstlane(qc.sub);   // halved tiles (QTileCtx): this wave computes keys 32 * sub .. of every key tile
   auto dec = [&](int t, const IdSummary& ks) {
@@ -109,13 +98,13 @@ void bwd_dq_kernel(const KArgs a) {
 #pragma unroll
       for (int t = 0; t < 8; ++t) part += float(of[ks][t]) * float(dof[ks][t]);
     delta_i = xhalf_sum(part);
-    if (row >= 0 && g == 0 && wk.split == 0 && sub == 0) delp[row] = delta_i;   // for the dk/dv kernel
+    if (row >= 0 && g == 0 && ge.chunk == 0 && sub == 0) a.delta[row_l] = delta_i;   // for the dk/dv kernel
   }
   if (L_i == -INFINITY) L_i = INFINITY;  // row without any kept key: P = exp2(-inf) = 0
 
   TileLoader<DL, BN, D> ldK, ldV;
-  ldK.init(kp, a.k_rs, a.N);
-  ldV.init(vp, a.v_rs, a.N);
+  ldK.init(kp, a.k_rs, ge.N);
+  ldV.init(vp, a.v_rs, ge.N);
   LdsOffsets<DL> lo;
   lo.init();
   int id_off = g * 16, key_off = 0;
@@ -267,48 +256,54 @@ void bwd_dq_kernel(const KArgs a) {
     }
   }
   const bool writer = !halved || sub == 0;   // the wave that holds the rows' result
-  if (DOC && nsplit > 1) {
+  if (nsplit > 1) {
     // This workgroup saw one chunk of the keys: store the partial sum; the last chunk to arrive
     // adds them up in a fixed order and writes dQ.
-    const int64_t tbase = (int64_t(b) * a.H + h) * a.split_tiles + wk.gt;
-    float* po = a.sk_o + (tbase * a.split_k + wk.split) * (128 * D);
+    const int rows = DOC ? 128 : a.bm;   // rows of a partial result
+    float* po = a.sk_o + (ge.part + int64_t(ge.chunk) * ge.pstride) * (rows * D);
 #pragma unroll
     for (int db = 0; db < DBN; ++db)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
-        if (32 * db + 8 * q4 >= D || !writer) continue;
+        if (32 * db + 8 * q4 >= D || !writer || 32 * qc.rb >= rows) continue;
         f32x4 x = {dq[db][4 * q4 + 0], dq[db][4 * q4 + 1], dq[db][4 * q4 + 2], dq[db][4 * q4 + 3]};
         store_dev(po + part_index<D>(qc.rb, 4 * db + q4, lane) * 4, x);
       }
-    if (!split_arrive(a.sk_cnt + tbase, nsplit)) { FA_STAMP(g_trace_dq, 4, FA_CLOCK()); return; }
+    if (!split_arrive(a.sk_cnt + ge.cnt, nsplit)) { FA_STAMP(g_trace_dq, 4, FA_CLOCK()); return; }
     FA_STAMP(g_trace_dq, 6, FA_CLOCK());
     // (up to eight chunks are requested together, four or two steps of them: every device-scope load is a
     // round trip of its own, so they are put in flight side by side instead of one after the other)
     constexpr int C4 = D / 4;
-    const float* bo = a.sk_o + tbase * a.split_k * (128 * D);
-    const int* prm = a.perm + b * a.pm_bs + h * a.pm_hs + wk.tile * 128;
-    auto finish_row = [&](int mrow, int c, f32x4 acc) __attribute__((always_inline)) {
+    const float* bo = a.sk_o + int64_t(ge.part) * (rows * D);
+    const int64_t so = int64_t(ge.pstride) * (rows * D);   // from chunk to chunk
+    const int* prm = DOC ? a.perm + b * a.pm_bs + h * a.pm_hs + ge.tile * 128 : nullptr;
+    // row of the tile -> row of the operands (with ids), or packed row (without), -1: no such row
+    auto row_of = [&](int r) __attribute__((always_inline)) {
+      return DOC ? prm[r] : (ge.tile * a.bm + r < ge.M * a.pack ? ge.tile * a.bm + r : -1);
+    };
+    auto finish_row = [&](int prow, int c, f32x4 acc) __attribute__((always_inline)) {
+      const int mrow = DOC ? prow : prow / a.pack, mh = DOC ? 0 : prow - mrow * a.pack;
       const typename E::vec2 x0 = E::cvt2(acc[0] * a.scale, acc[1] * a.scale);
       const typename E::vec2 x1 = E::cvt2(acc[2] * a.scale, acc[3] * a.scale);
       typename E::vec4 x = {x0[0], x0[1], x1[0], x1[1]};
-      *reinterpret_cast<typename E::vec4*>(dqp + int64_t(mrow) * a.dq_rs + 4 * c) = x;
+      *reinterpret_cast<typename E::vec4*>(dqp + mh * a.dq_hs + int64_t(mrow) * a.dq_rs + 4 * c) = x;
     };
     // NS chunk slots of IT steps each: 16 loads in flight per thread whatever the number of chunks
     auto merge_batched = [&](auto it_c, auto ns_c) __attribute__((always_inline)) {
       constexpr int IT = decltype(it_c)::value, NS = decltype(ns_c)::value;
-      for (int i0 = threadIdx.x; i0 < 128 * C4; i0 += 256 * IT) {
+      for (int i0 = threadIdx.x; i0 < rows * C4; i0 += 256 * IT) {
         f32x4 x[IT][NS];
         int mrow[IT], cc[IT];
 #pragma unroll
         for (int u = 0; u < IT; ++u) {
           const int i = i0 + 256 * u;
           int r, c;
-          part_coords<D>(min(i, 128 * C4 - 1), r, c);
+          part_coords<D>(min(i, rows * C4 - 1), r, c);
           cc[u] = c;
-          mrow[u] = i < 128 * C4 ? prm[r] : -1;
+          mrow[u] = i < rows * C4 ? row_of(r) : -1;
           if (mrow[u] < 0) continue;   // no such row: nothing to fetch
 #pragma unroll
-          for (int sp = 0; sp < NS; ++sp) x[u][sp] = load_dev4(bo + min(sp, nsplit - 1) * (128 * D) + i * 4);
+          for (int sp = 0; sp < NS; ++sp) x[u][sp] = load_dev4(bo + min(sp, nsplit - 1) * so + i * 4);
         }
 #pragma unroll
         for (int u = 0; u < IT; ++u) {
@@ -329,14 +324,14 @@ void bwd_dq_kernel(const KArgs a) {
       FA_STAMP(g_trace_dq, 4, FA_CLOCK());
       return;
     }
-    for (int i = threadIdx.x; i < 128 * C4; i += 256) {
+    for (int i = threadIdx.x; i < rows * C4; i += 256) {
       int r, c;
       part_coords<D>(i, r, c);
-      const int mrow = prm[r];
+      const int mrow = row_of(r);
       if (mrow < 0) continue;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
       for (int sp = 0; sp < nsplit; ++sp) {
-        const f32x4 x = load_dev4(bo + sp * (128 * D) + i * 4);
+        const f32x4 x = load_dev4(bo + sp * so + i * 4);
         acc[0] += x[0]; acc[1] += x[1]; acc[2] += x[2]; acc[3] += x[3];
       }
       finish_row(mrow, c, acc);
@@ -351,8 +346,8 @@ void bwd_dq_kernel(const KArgs a) {
   if (writer) {
     char* patch = smem + (halved ? qc.rb * (16 * DBN * 64 * 4) : wave * row_patch_bytes<D>());
     store_rows_through_lds<E, D, DBN>(patch, dq, a.scale, [&](const int r) -> T* {
-      const int rr = __shfl(row, r);
-      return rr >= 0 ? dqp + int64_t(rr) * a.dq_rs : nullptr;
+      const int rr = __shfl(row, r), hh = DOC ? 0 : __shfl(qc.hg, r);
+      return rr >= 0 ? dqp + hh * a.dq_hs + int64_t(rr) * a.dq_rs : nullptr;
     });
   }
   FA_STAMP(g_trace_dq, 4, FA_CLOCK());
@@ -361,13 +356,14 @@ void bwd_dq_kernel(const KArgs a) {
 
 template <typename Tag, int D, bool CAUSAL, bool DOC>
 static int launch_one(const KArgs& a, hipStream_t s) {
-  constexpr int BM = 128, BN = 64;
-  const int nQt = (DOC ? a.Pp / BM : (a.M + BM - 1) / BM) + (DOC ? split_extra(a) : 0);
+  constexpr int BN = 64;
+  const int slots = DOC ? a.Pp / 128 + split_extra(a) : dense_slots(a);
+  const int bhs = DOC ? a.B * a.H : (a.qtab != nullptr ? a.nHp : a.B * a.nHp);
   const size_t lds = 4 * BN * (D < 32 ? 32 : D) * 2 + 2 * BN * 4;  // K, V double buffered + key ids
   auto kern = bwd_dq_kernel<Tag, D, CAUSAL, DOC>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  hipLaunchKernelGGL(kern, dim3(grid_blocks(nQt, a.B * a.H)), dim3(256), lds, s, a);
+  hipLaunchKernelGGL(kern, dim3(grid_blocks(slots, bhs)), dim3(256), lds, s, a);
   return (int)hipGetLastError();
 }
 

@@ -95,6 +95,75 @@ inline SplitCfg split_config(int B, int H, int M, int N, int D, uint64_t budget 
   return c;
 }
 
+// ---------------------------------------------------------------------------
+// Shape of the launches without ids (and without a block map): how many query heads share a tile, how many rows a
+// tile has, whether the key range of a tile is cut.
+//   pack : the G query heads of one key head share their tiles: packed row r is query r / G of head r % G.  A tile
+//          then meets the diagonal with 128 / G queries instead of 128 (less of it is masked), all the heads that
+//          read the same K / V sit on one XCD, and a short query block fills tiles instead of padding them.
+//   bm   : 128 rows, or 64 when 128-row tiles would leave CUs without a workgroup (the 64-row form splits every key
+//          tile between two waves, see QTileCtx::halved).
+//   dec  : at most 32 packed rows: the form of fa_decode.hip.
+//   split: chunks of the key range; only with FA_FLAG_SPLIT_KEYS, which gives the launch a workspace for them.
+// ---------------------------------------------------------------------------
+constexpr int kCUs = 256;
+struct FwdCfg { int pack, bm, tiles, split; bool dec; };
+// Chunks for `wgs` tiles of `steps` steps each: the cheapest total by a model of rounds x (set-up + steps of a chunk)
+// + merging, in units of one step; `slots` workgroups run at a time.  A chunk keeps at least `min_steps` steps.
+inline int pick_split(int64_t wgs, int steps, int slots, float setup, float merge, int min_steps) {
+  int best = 1;
+  float best_t = 1e30f;
+  for (int s = 1; s <= kSplitKMaxFew && (s == 1 || steps / s >= min_steps); ++s) {
+    const int64_t rounds = (wgs * s + slots - 1) / slots;
+    // a launch that does not fill the chip streams faster per workgroup, but not without bound
+    const float fill = rounds > 1 ? 1.f : float(wgs * s) / slots;
+    const float step = fill > 0.4f ? fill : 0.4f;
+    const float t = rounds * (setup + float((steps + s - 1) / s) * step) + (s > 1 ? merge : 0.f);
+    if (t < best_t * 0.97f) { best_t = t; best = s; }
+  }
+  return best;
+}
+inline FwdCfg fwd_config(const fa_params* p) {
+  FwdCfg c = {1, 128, 0, 1, false};
+  if (p->score_mode == FA_SCORE_MODE3_PACKED) {
+    // the host knows the totals only: 32-row tiles when an average sequence fills no more
+    c.pack = p->H / p->Hk;
+    const int64_t rows = int64_t(p->M) * c.pack, avg = rows / (p->nseq > 0 ? p->nseq : 1);
+    c.dec = avg <= 32;
+    c.bm = c.dec ? 32 : (avg <= 64 || (rows / 128 + p->nseq) * p->Hk < kCUs ? 64 : 128);
+    return c;
+  }
+  if (p->score_mode != FA_SCORE_MODE0_NOPE || p->dtype == FA_DTYPE_FP32) { c.tiles = (p->M + 127) / 128; return c; }
+  c.pack = p->H / p->Hk;
+  const int64_t rows = int64_t(p->M) * c.pack, bh = int64_t(p->B) * p->Hk;
+  const int nk = p->window > 0 && p->causal && p->window + p->M < p->N ? p->window + p->M : p->N;   // keys a tile can see
+  if (rows <= 32) {
+    c.dec = true; c.bm = 32; c.tiles = 1;
+    // a step: four waves x 32 keys.  64 KB at D = 128 take a CU 3 us at the rate the whole card reads; setting a
+    // workgroup up takes about as long, handing the result over and merging one and a half steps
+    const float rel = 128.f / p->D;
+    if (p->flags & FA_FLAG_SPLIT_KEYS) c.split = pick_split(bh, (nk + 127) / 128, kCUs, 1.2f * rel, 1.5f * rel, 2);
+    return c;
+  }
+  c.tiles = int((rows + 127) / 128);
+  if (c.tiles * bh < kCUs) { c.bm = 64; c.tiles = int((rows + 63) / 64); }
+  // a step: one 64-key tile; two workgroups to a CU
+  if ((p->flags & FA_FLAG_SPLIT_KEYS) && c.tiles * bh < 2 * kCUs)
+    c.split = pick_split(c.tiles * bh, (nk + 63) / 64, 2 * kCUs, 3.f, 4.f, 8);
+  return c;
+}
+
+// Packed sequences (FA_SCORE_MODE3_PACKED): one entry of the tile tables the plan kernel writes (fa_seq.hip).
+struct SeqTile {
+  int q0, M, k0, N;      // the sequence's first query row and its rows, its first key and its keys
+  int gap;               // row i of the sequence has its diagonal at key gap + i
+  int tile;              // query tile (of bm packed rows) or key tile of the sequence
+  int chunk, nchunk;     // share of the key range (query tiles only)
+  int cnt, part;         // arrival counter and first partial result of a split tile, per head: times nHp, plus the head
+  int pad[6];
+};
+struct SeqHdr { int nq, nk, pad[2]; };   // entries in use
+
 // Compile-time integer handed to a generic lambda.
 template <int V> struct IntC { static constexpr int value = V; };
 
@@ -311,6 +380,15 @@ struct KArgs {
   int pfx_m1;   // prefix-LM: keys j <= pfx_m1 are seen by every row (-1: no prefix)
   int Pp;                 // entries of the permuted order per (b, h)
   int nQs, nKs;           // summary entries per (b, h)
+  // the launches without ids: see FwdCfg
+  int pack, nHp;          // query heads per tile, H / pack
+  int bm, nTiles;         // rows per query tile, tiles per (batch, head group)
+  int dsplit;             // chunks of the key range of every tile
+  // packed sequences: tables of the plan (null otherwise) and their capacities
+  const SeqHdr* shdr;
+  const SeqTile* qtab;
+  const SeqTile* ktab;
+  int nQent, nKent;
   int dq_delta;           // the dq kernel computes delta from O and dO itself and stores it
   int pair_spin;          // dk/dv, role-split form: polls of the pair flag before the gradient wave gives up
   // block mask (FA_SCORE_MODE2_BLOCK): bytes [B, H, nBr, nBc] per 64 x 64 block of (row, key) pairs, or null
@@ -368,6 +446,43 @@ inline WsLayout ws_layout(const fa_params* p, uint64_t split_budget = kSplitScra
   return w;
 }
 
+// Layouts without a mask plan.  Mode 0 with FA_FLAG_SPLIT_KEYS: arrival counters (the part called plan) and partial
+// results.  Packed sequences: header, tile tables, counters, and partial results.
+struct TabLayout {
+  uint64_t off_hdr, off_q, off_k, off_spill, off_cnt, plan_bytes, off_ml, off_o, total;
+  int nQ, nK, nCnt, nPart;   // entries per head group
+};
+// Keys per entry of the key-tile table: the 64-key role-split form at D = 128 (sequences are short), 128 keys below.
+constexpr int kSeqKeyTile = 64;
+FA_HD int seq_key_tile(int D) { return D > 64 ? kSeqKeyTile : 128; }
+constexpr int kSeqTargetWgs = 3 * kCUs;   // workgroups a split launch of packed sequences aims at
+inline TabLayout tab_layout(const fa_params* p, const FwdCfg& c) {
+  TabLayout w = {};
+  uint64_t o = 0;
+  auto take = [&](uint64_t bytes) { uint64_t r = o; o += (bytes + 255) & ~uint64_t(255); return r; };
+  const int nh = p->H / c.pack;
+  if (p->score_mode == FA_SCORE_MODE0_NOPE) {
+    if (c.split <= 1) return w;
+    w.nCnt = p->B * c.tiles; w.nPart = w.nCnt * c.split;
+    w.off_cnt = take(uint64_t(w.nCnt) * nh * 4);
+  } else {
+    w.off_hdr = take(sizeof(SeqHdr));
+    const int spare = kSeqTargetWgs / nh + 1;
+    w.nQ = int((int64_t(p->M) * c.pack) / c.bm) + p->nseq + 1 + spare;
+    w.nK = p->N / seq_key_tile(p->D) + p->nseq + 1;
+    w.nCnt = spare; w.nPart = 2 * spare;
+    w.off_q = take(uint64_t(w.nQ) * sizeof(SeqTile));
+    w.off_k = take(uint64_t(w.nK) * sizeof(SeqTile));
+    w.off_spill = take(p->nseq < 8000 ? 0 : uint64_t(p->nseq + 2) * 2 * 4);   // tile offsets of very many sequences (fa_seq.hip)
+    w.off_cnt = take(uint64_t(w.nCnt) * nh * 4);
+  }
+  w.plan_bytes = o;
+  w.off_ml = take(uint64_t(w.nPart) * nh * c.bm * 2 * 4);
+  w.off_o = take(uint64_t(w.nPart) * nh * c.bm * uint64_t(p->D) * 4);
+  w.total = o;
+  return w;
+}
+
 // Raise the dynamic LDS limit of a kernel once per device (the attribute is per device and per
 // kernel; a process may drive several GPUs).  `done` is the caller's per-kernel record.
 template <typename K>
@@ -385,6 +500,9 @@ static int allow_lds(K kern, size_t lds, bool (&done)[64]) {
 
 // Launchers implemented one per translation unit; each returns a hipError_t as int.
 int launch_fwd(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);
+int launch_decode(const KArgs& a, int dtype, int D, bool causal, hipStream_t s);   // at most 32 packed rows, or packed sequences with 32-row tiles
+int launch_zero_counters(int* cnt, int n, hipStream_t s);
+int launch_seq_plan(const fa_params* p, const FwdCfg& c, const TabLayout& w, hipStream_t s);
 int launch_bwd_delta(const KArgs& a, int dtype, int D, hipStream_t s);
 int launch_bwd_dq(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);
 int launch_bwd_dkdv(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);

@@ -41,7 +41,7 @@ void fwd_kernel(const KArgs a) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
-  constexpr int BM = 128, BN = 64, KS = D / 16;
+  constexpr int BN = 64, KS = D / 16;
   constexpr int DL = D < 32 ? 32 : D;  // LDS row width: D = 16 is staged as 32 columns, the upper 16 zero
   constexpr int DBN = DL / 32;
   constexpr int TILE_BYTES = BN * DL * 2;
@@ -54,30 +54,20 @@ void fwd_kernel(const KArgs a) {
 
   // heaviest tiles first: with ids the global-row tiles sit at the end of the permuted
   // order and see the longest key ranges; without ids the last rows do
-  const int nQt = DOC ? a.Pp / BM : (a.M + BM - 1) / BM;
-  const int nSlots = nQt + (DOC ? split_extra(a) : 0);
-  int slot, bh;
-  if (!block_to_tile(nSlots, a.B * a.H, DOC && nQt >= 32, slot, bh)) return;
-  const int b = bh / a.H, h = bh % a.H, hk = h / a.G;
-  QWork wk;
-  QHeader hd = {};
-  if (DOC) hd = a.qhdr[b * a.qh_bs + h * a.qh_hs];
-  if (!q_work<DOC>(a, hd, nQt, slot, wk)) return;
+  TileGeo ge;
   QTileCtx<CAUSAL, DOC> qc;
-  if (!qc.init(a, b, h, wk.tile, threadIdx.x >> 6)) return;
-  q_work_finish(a, hd, wk);
-  int kt_first = qc.first_tile(a), kt_last = qc.last_tile(a);
-  const int nsplit = split_range(a, wk, kt_first, kt_last);
-  if (wk.split >= nsplit) return;
-  FA_STAMP(g_trace_fwd, 1, FA_CLOCK()); FA_STAMP(g_trace_fwd, 7, (long long)wk.tile | ((long long)wk.split << 16) | ((long long)nsplit << 24));
+  int kt_first, kt_last;
+  if (!tile_work(a, ge, qc, kt_first, kt_last)) return;
+  const int b = ge.b, h = ge.h0, hk = ge.hk, nsplit = ge.nchunk;
+  FA_STAMP(g_trace_fwd, 1, FA_CLOCK()); FA_STAMP(g_trace_fwd, 7, (long long)ge.tile | ((long long)ge.chunk << 16) | ((long long)nsplit << 24));
   const int row = qc.row, rowc = qc.rowc, eq_i = qc.eq_i;
   const int* ekp = qc.ekp;
 
-  const T* qp = reinterpret_cast<const T*>(a.q) + b * a.q_bs + h * a.q_hs;
-  const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs;
-  const T* vp = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs;
-  T* op = reinterpret_cast<T*>(a.o) + b * a.o_bs + h * a.o_hs;
-  float* lsep = a.lse + (int64_t(b) * a.H + h) * a.M;
+  const T* qp = reinterpret_cast<const T*>(a.q) + b * a.q_bs + (h + qc.hg) * a.q_hs + ge.q0 * a.q_rs;
+  const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + ge.k0 * a.k_rs;
+  const T* vp = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + ge.k0 * a.v_rs;
+  T* op = reinterpret_cast<T*>(a.o) + b * a.o_bs + h * a.o_hs + ge.q0 * a.o_rs;
+  float* lsep = a.lse + (int64_t(b) * a.H + h) * a.M + ge.q0;
 
   // Q^T fragments (B operand): lane holds d = 16*ks + 8*g .. +7 of its query row.
   vec8 qf[KS];
@@ -87,7 +77,7 @@ void fwd_kernel(const KArgs a) {
 
   // decisions of this wave for key tile t, evaluated by the lane that tests the tile
   QBlockMask bmq;
-  bmq.init(a, b, h, wk.tile);
+  bmq.init(a, b, h, ge.tile);
   const bool halved = qc.halved;
   const int sub = __builtin_amdgcn_readfirstlane(qc.sub);   // halved tiles: this wave computes keys 32 * sub .. of every key tile
   auto dec = [&](int t, const IdSummary& ks) {
@@ -109,8 +99,8 @@ void fwd_kernel(const KArgs a) {
   }
 
   TileLoader<DL, BN, D> ldK, ldV;
-  ldK.init(kp, a.k_rs, a.N);
-  ldV.init(vp, a.v_rs, a.N);
+  ldK.init(kp, a.k_rs, ge.N);
+  ldV.init(vp, a.v_rs, ge.N);
   LdsOffsets<DL> lo;
   lo.init();
   int id_off = g * 16, key_off = 0;
@@ -363,43 +353,49 @@ void fwd_kernel(const KArgs a) {
   }
   const bool writer = !halved || sub == 0;   // the wave that holds the rows' result
   const float l_tot = xhalf_sum(l_run);
-  if (DOC && nsplit > 1) {
+  if (nsplit > 1) {
     // This workgroup saw one chunk of the keys: store the unnormalised partial result; the last
     // chunk to arrive combines them (log-sum-exp merge) and writes O and LSE.
-    const int64_t tbase = (int64_t(b) * a.H + h) * a.split_tiles + wk.gt;
-    float* po = a.sk_o + (tbase * a.split_k + wk.split) * (128 * D);
-    float* pml = a.sk_ml + (tbase * a.split_k + wk.split) * (128 * 2);
+    const int rows = DOC ? 128 : a.bm;   // rows of a partial result
+    float* po = a.sk_o + (ge.part + int64_t(ge.chunk) * ge.pstride) * (rows * D);
+    float* pml = a.sk_ml + (ge.part + int64_t(ge.chunk) * ge.pstride) * (rows * 2);
     const int rt = qc.rb * 32 + (lane & 31);   // row inside the tile
-    if (g == 0 && writer) store_dev(pml + rt * 2, m_ref, l_tot);
+    if (g == 0 && writer && rt < rows) store_dev(pml + rt * 2, m_ref, l_tot);
 #pragma unroll
     for (int db = 0; db < DBN; ++db)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
-        if (32 * db + 8 * q4 >= D || !writer) continue;
+        if (32 * db + 8 * q4 >= D || !writer || 32 * qc.rb >= rows) continue;
         f32x4 x = {o[db][4 * q4 + 0], o[db][4 * q4 + 1], o[db][4 * q4 + 2], o[db][4 * q4 + 3]};
         store_dev(po + part_index<D>(qc.rb, 4 * db + q4, lane) * 4, x);
       }
-    if (!split_arrive(a.sk_cnt + tbase, nsplit)) { FA_STAMP(g_trace_fwd, 4, FA_CLOCK()); return; }
+    if (!split_arrive(a.sk_cnt + ge.cnt, nsplit)) { FA_STAMP(g_trace_fwd, 4, FA_CLOCK()); return; }
     FA_STAMP(g_trace_fwd, 6, FA_CLOCK());
     // merge: the whole workgroup walks the tile, one float4 of one row per thread and step.  The
     // partial results come through device-scope loads, each a round trip of its own: up to eight chunks are
     // requested together, four or two steps of them (16 + 16 loads in flight per thread), instead of one by one.
     constexpr int C4 = D / 4;
-    const float* bo = a.sk_o + tbase * a.split_k * (128 * D);
-    const float* bml = a.sk_ml + tbase * a.split_k * (128 * 2);
-    const int* prm = a.perm + b * a.pm_bs + h * a.pm_hs + wk.tile * 128;
-    auto finish_row = [&](int mrow, int c, float mmax, float lsum, f32x4 acc) __attribute__((always_inline)) {
+    const float* bo = a.sk_o + int64_t(ge.part) * (rows * D);
+    const float* bml = a.sk_ml + int64_t(ge.part) * (rows * 2);
+    const int64_t so = int64_t(ge.pstride) * (rows * D), sml = int64_t(ge.pstride) * (rows * 2);   // from chunk to chunk
+    const int* prm = DOC ? a.perm + b * a.pm_bs + h * a.pm_hs + ge.tile * 128 : nullptr;
+    // row of the tile -> row of the operands (with ids), or packed row (without), -1: no such row
+    auto row_of = [&](int r) __attribute__((always_inline)) {
+      return DOC ? prm[r] : (ge.tile * a.bm + r < ge.M * a.pack ? ge.tile * a.bm + r : -1);
+    };
+    auto finish_row = [&](int prow, int c, float mmax, float lsum, f32x4 acc) __attribute__((always_inline)) {
       const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
-      if (c == 0) lsep[mrow] = lsum > 0.f ? mmax + fast_log2(lsum) : -INFINITY;
+      const int mrow = DOC ? prow : prow / a.pack, mh = DOC ? 0 : prow - mrow * a.pack;
+      if (c == 0) lsep[int64_t(mh) * a.M + mrow] = lsum > 0.f ? mmax + fast_log2(lsum) : -INFINITY;
       const typename E::vec2 x0 = E::cvt2(acc[0] * inv, acc[1] * inv);
       const typename E::vec2 x1 = E::cvt2(acc[2] * inv, acc[3] * inv);
       typename E::vec4 x = {x0[0], x0[1], x1[0], x1[1]};
-      *reinterpret_cast<typename E::vec4*>(op + int64_t(mrow) * a.o_rs + 4 * c) = x;
+      *reinterpret_cast<typename E::vec4*>(op + mh * a.o_hs + int64_t(mrow) * a.o_rs + 4 * c) = x;
     };
     // NS chunk slots of IT steps each: 16 + 16 loads in flight per thread whatever the number of chunks
     auto merge_batched = [&](auto it_c, auto ns_c) __attribute__((always_inline)) {
       constexpr int IT = decltype(it_c)::value, NS = decltype(ns_c)::value;
-      for (int i0 = threadIdx.x; i0 < 128 * C4; i0 += 256 * IT) {
+      for (int i0 = threadIdx.x; i0 < rows * C4; i0 += 256 * IT) {
         float m_[IT][NS], l_[IT][NS];
         f32x4 x[IT][NS];
         int mrow[IT], cc[IT];
@@ -407,15 +403,15 @@ void fwd_kernel(const KArgs a) {
         for (int u = 0; u < IT; ++u) {
           const int i = i0 + 256 * u;
           int r, c;
-          part_coords<D>(min(i, 128 * C4 - 1), r, c);
+          part_coords<D>(min(i, rows * C4 - 1), r, c);
           cc[u] = c;
-          mrow[u] = i < 128 * C4 ? prm[r] : -1;
+          mrow[u] = i < rows * C4 ? row_of(r) : -1;
           if (mrow[u] < 0) continue;   // no such row (a tile of a few dozen rows has mostly these): nothing to fetch
 #pragma unroll
           for (int sp = 0; sp < NS; ++sp) {
             const int spc = min(sp, nsplit - 1);   // chunks past the last one repeat it (weight 0 below)
-            load_dev(bml + spc * 256 + r * 2, m_[u][sp], l_[u][sp]);
-            x[u][sp] = load_dev4(bo + spc * (128 * D) + i * 4);
+            load_dev(bml + spc * sml + r * 2, m_[u][sp], l_[u][sp]);
+            x[u][sp] = load_dev4(bo + spc * so + i * 4);
           }
         }
 #pragma unroll
@@ -442,25 +438,25 @@ void fwd_kernel(const KArgs a) {
       FA_STAMP(g_trace_fwd, 4, FA_CLOCK());
       return;
     }
-    for (int i = threadIdx.x; i < 128 * C4; i += 256) {
+    for (int i = threadIdx.x; i < rows * C4; i += 256) {
       int r, c;
       part_coords<D>(i, r, c);
-      const int mrow = prm[r];
+      const int mrow = row_of(r);
       if (mrow < 0) continue;
       float mmax = -INFINITY;
       for (int sp = 0; sp < nsplit; ++sp) {
         float m_, l_;
-        load_dev(bml + sp * 256 + r * 2, m_, l_);
+        load_dev(bml + sp * sml + r * 2, m_, l_);
         mmax = fmaxf(mmax, m_);
       }
       float lsum = 0.f;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
       for (int sp = 0; sp < nsplit; ++sp) {
         float m_, l_;
-        load_dev(bml + sp * 256 + r * 2, m_, l_);
+        load_dev(bml + sp * sml + r * 2, m_, l_);
         const float w = m_ == -INFINITY ? 0.f : fast_exp2(m_ - mmax);
         lsum += w * l_;
-        const f32x4 x = load_dev4(bo + sp * (128 * D) + i * 4);
+        const f32x4 x = load_dev4(bo + sp * so + i * 4);
         acc[0] += w * x[0]; acc[1] += w * x[1]; acc[2] += w * x[2]; acc[3] += w * x[3];
       }
       finish_row(mrow, c, mmax, lsum, acc);
@@ -473,12 +469,12 @@ void fwd_kernel(const KArgs a) {
   // done with the last tile first; a halved tile's writers use the part of LDS they have just read their partner's state from)
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if (!halved) __syncthreads();
-  if (row >= 0 && writer && g == 0) lsep[row] = l_tot > 0.f ? m_ref + fast_log2(l_tot) : -INFINITY;
+  if (row >= 0 && writer && g == 0) lsep[int64_t(qc.hg) * a.M + row] = l_tot > 0.f ? m_ref + fast_log2(l_tot) : -INFINITY;
   if (writer) {
     char* patch = smem + (halved ? qc.rb * ((2 + 16 * DBN) * 64 * 4) : wave * row_patch_bytes<D>());
     store_rows_through_lds<E, D, DBN>(patch, o, inv, [&](const int r) -> T* {
-      const int rr = __shfl(row, r);
-      return rr >= 0 ? op + int64_t(rr) * a.o_rs : nullptr;
+      const int rr = __shfl(row, r), hh = DOC ? 0 : __shfl(qc.hg, r);
+      return rr >= 0 ? op + hh * a.o_hs + int64_t(rr) * a.o_rs : nullptr;
     });
   }
   FA_STAMP(g_trace_fwd, 4, FA_CLOCK());
@@ -486,13 +482,14 @@ void fwd_kernel(const KArgs a) {
 
 template <typename Tag, int D, bool CAUSAL, bool DOC>
 static int launch_one(const KArgs& a, hipStream_t s) {
-  constexpr int BM = 128, BN = 64;
-  const int nQt = (DOC ? a.Pp / BM : (a.M + BM - 1) / BM) + (DOC ? split_extra(a) : 0);
+  constexpr int BN = 64;
+  const int slots = DOC ? a.Pp / 128 + split_extra(a) : dense_slots(a);
+  const int bhs = DOC ? a.B * a.H : (a.qtab != nullptr ? a.nHp : a.B * a.nHp);
   const size_t lds = 4 * BN * (D < 32 ? 32 : D) * 2 + 2 * BN * 4;  // K, V double buffered + key ids
   auto kern = fwd_kernel<Tag, D, CAUSAL, DOC>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  hipLaunchKernelGGL(kern, dim3(grid_blocks(nQt, a.B * a.H)), dim3(256), lds, s, a);
+  hipLaunchKernelGGL(kern, dim3(grid_blocks(slots, bhs)), dim3(256), lds, s, a);
   return (int)hipGetLastError();
 }
 

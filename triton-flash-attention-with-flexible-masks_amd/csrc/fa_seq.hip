@@ -1,0 +1,216 @@
+// Tile tables of a packed batch of sequences (FA_SCORE_MODE3_PACKED), and the arrival counters of the launches that
+// split key ranges without a mask plan.
+//
+// The boundaries of the sequences are known on the device only, so the kernels are launched for as many tiles as the
+// totals can give and look their tile up here: a sequence starts a tile of its own, and its rows and keys are named by
+// pointer and length, so the kernels run the code of the unmasked problem on it -- no ids, no gather, no tile that two
+// sequences share.  One kernel, one workgroup per table; it takes the place of the dozen small kernels (ids, positions,
+// mask plan) that a packed batch needed when it was given to the kernels as a document mask.
+#include "fa_tile.h"
+
+namespace fa {
+namespace {
+
+constexpr int kThreads = 1024;
+constexpr int kBuckets = 128;     // classes of tile lengths the table is sorted by, longest first
+constexpr int kLdsSeqs = 8192;    // sequences whose tile offsets fit LDS (more: they are kept in the table's own memory)
+
+struct SeqPlanArgs {
+  const void* cu_q;
+  const void* cu_k;
+  int i64, nseq, Tq, Tk, pack, bm, bk, causal, win;
+  int spare, min_chunk;           // extra entries a split may use (0: no tile is split), key tiles per chunk at least
+  SeqHdr* hdr;
+  SeqTile* qtab;
+  SeqTile* ktab;
+  int nQ, nK;                     // capacities
+  int* cnt;
+  int n_cnt;
+};
+
+struct Seq { int q0, M, k0, N, gap; };
+
+FA_DEV int cu_at(const void* p, int i64, int i, int total) {
+  const long long v = i64 ? reinterpret_cast<const long long*>(p)[i] : (long long)reinterpret_cast<const int*>(p)[i];
+  return v < 0 ? 0 : (v > total ? total : (int)v);
+}
+// sequence s of nseq; number nseq is what lies behind the last boundary
+FA_DEV Seq seq_at(const SeqPlanArgs& p, int s) {
+  Seq r;
+  r.q0 = s == 0 ? 0 : cu_at(p.cu_q, p.i64, s, p.Tq);
+  r.k0 = s == 0 ? 0 : cu_at(p.cu_k, p.i64, s, p.Tk);
+  r.M = max(0, (s < p.nseq ? cu_at(p.cu_q, p.i64, s + 1, p.Tq) : p.Tq) - r.q0);
+  r.N = max(0, (s < p.nseq ? cu_at(p.cu_k, p.i64, s + 1, p.Tk) : p.Tk) - r.k0);
+  r.gap = s < p.nseq ? r.N - r.M : 0;
+  return r;
+}
+
+FA_DEV int wave_scan(int v) {   // inclusive sum over the lanes of a wave
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(v, off);
+    if (lane >= off) v += u;
+  }
+  return v;
+}
+
+// Block 0 writes the query tiles, block 1 the key tiles.
+__global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p, int* __restrict__ spill) {
+  __shared__ int s_off[kLdsSeqs + 1];
+  __shared__ int s_wave[kThreads / 64];
+  __shared__ float s_work[kThreads / 64];
+  __shared__ int s_bucket[kBuckets];
+  __shared__ int s_tot, s_max, s_cnt, s_part;
+  const bool keys = blockIdx.x == 1;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ns = p.nseq + 1;
+  int* off = ns <= kLdsSeqs ? s_off : spill + (keys ? ns + 1 : 0);
+  if (!keys)
+    for (int i = tid; i < p.n_cnt; i += kThreads) p.cnt[i] = 0;
+  if (tid == 0) { s_tot = 0; s_max = 1; s_cnt = 0; s_part = 0; }
+  for (int i = tid; i < kBuckets; i += kThreads) s_bucket[i] = 0;
+  __syncthreads();
+
+  auto tiles_of = [&](const Seq& q) { return keys ? (q.N + p.bk - 1) / p.bk : int((int64_t(q.M) * p.pack + p.bm - 1) / p.bm); };
+  // length of a tile: 64-key tiles its rows see, or 64-row tiles that see its keys
+  auto length_of = [&](const Seq& q, int t) {
+    if (keys) {
+      const int n0 = t * p.bk, n1 = min(q.N, n0 + p.bk) - 1;
+      const int lo = p.causal ? max(0, n0 - q.gap) : 0;
+      const int hi = p.causal ? min(q.M - 1, n1 - q.gap + p.win - 1) : q.M - 1;
+      return hi >= lo ? hi / 64 - lo / 64 + 1 : 0;
+    }
+    const int r0 = int(int64_t(t) * p.bm / p.pack), r1 = int(min(int64_t(q.M) * p.pack, int64_t(t + 1) * p.bm) - 1) / p.pack;
+    const int lo = p.causal ? max(0, q.gap + r0 - p.win + 1) : 0;
+    const int hi = p.causal ? min(q.N - 1, q.gap + r1) : q.N - 1;
+    return hi >= lo ? hi / 64 - lo / 64 + 1 : 0;
+  };
+
+  // tile offsets of the sequences
+  int longest = 1;
+  for (int s0 = 0; s0 < ns; s0 += kThreads) {
+    const int s = s0 + tid;
+    int n = 0;
+    if (s < ns) {
+      const Seq q = seq_at(p, s);
+      n = tiles_of(q);
+      longest = max(longest, (keys ? q.M : q.N) / 64 + 2);
+    }
+    const int inc = wave_scan(n);
+    if (lane == 63) s_wave[wave] = inc;
+    __syncthreads();
+    int base = s_tot;
+    for (int w = 0; w < wave; ++w) base += s_wave[w];
+    if (s < ns) off[s] = base + inc - n;
+    __syncthreads();
+    if (tid == kThreads - 1) s_tot = base + inc;
+    __syncthreads();
+  }
+  if (tid == 0) off[ns] = s_tot;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) longest = max(longest, __shfl_xor(longest, o));
+  if (lane == 0) atomicMax(&s_max, longest);
+  __threadfence_block();
+  __syncthreads();
+  const int nt = min(s_tot, keys ? p.nK : p.nQ);
+  auto seq_of = [&](int t) {   // last sequence whose offset is not past t (empty sequences share their offset with the next)
+    int a = 0, b = ns - 1;
+    while (a < b) {
+      const int m = (a + b + 1) / 2;
+      if (off[m] <= t) a = m; else b = m - 1;
+    }
+    return a;
+  };
+
+  // chunks: the work of all tiles over the entries a split launch aims at
+  int chunk = 0x7fffffff;
+  if (!keys && p.spare > 0) {
+    float work = 0.f;
+    for (int t = tid; t < nt; t += kThreads) {
+      const int s = seq_of(t);
+      work += float(length_of(seq_at(p, s), t - off[s]));
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) work += __shfl_xor(work, o);
+    if (lane == 0) s_work[wave] = work;
+    __syncthreads();
+    work = 0.f;
+    for (int w = 0; w < kThreads / 64; ++w) work += s_work[w];
+    chunk = max(p.min_chunk, int(work / p.spare) + 1);
+  }
+  const int longest_all = min(s_max, chunk);
+  auto chunks_of = [&](int len) { return min(kSplitKMaxFew, max(1, (len + chunk - 1) / chunk)); };
+  auto bucket_of = [&](int len, int nc) {   // 0: the longest
+    const int l = (len + nc - 1) / nc;
+    return kBuckets - 1 - min(kBuckets - 1, int(int64_t(l) * kBuckets / (longest_all + 1)));
+  };
+  for (int t = tid; t < nt; t += kThreads) {
+    const int s = seq_of(t), len = length_of(seq_at(p, s), t - off[s]), nc = chunks_of(len);
+    atomicAdd(&s_bucket[bucket_of(len, nc)], nc);
+  }
+  __syncthreads();
+  if (wave == 0) {   // exclusive offsets of the buckets
+    int carry = 0;
+    for (int b0 = 0; b0 < kBuckets; b0 += 64) {
+      const int n = s_bucket[b0 + lane], inc = wave_scan(n);
+      s_bucket[b0 + lane] = carry + inc - n;
+      carry += __shfl(inc, 63);
+    }
+    if (lane == 0) s_tot = carry;
+  }
+  __syncthreads();
+  SeqTile* tab = keys ? p.ktab : p.qtab;
+  const int cap = keys ? p.nK : p.nQ;
+  for (int t = tid; t < nt; t += kThreads) {
+    const int s = seq_of(t);
+    const Seq q = seq_at(p, s);
+    const int len = length_of(q, t - off[s]), nc = chunks_of(len);
+    const int at = atomicAdd(&s_bucket[bucket_of(len, nc)], nc);
+    int cnt = 0, part = 0;
+    if (nc > 1) { cnt = atomicAdd(&s_cnt, 1); part = atomicAdd(&s_part, nc); }
+    for (int c = 0; c < nc && at + c < cap; ++c) {
+      SeqTile e = {};
+      e.q0 = q.q0; e.M = q.M; e.k0 = q.k0; e.N = q.N; e.gap = q.gap; e.tile = t - off[s];
+      e.chunk = c; e.nchunk = nc; e.cnt = cnt; e.part = part;
+      tab[at + c] = e;
+    }
+  }
+  if (tid == 0) {
+    if (keys) p.hdr->nk = min(s_tot, cap);
+    else p.hdr->nq = min(s_tot, cap);
+  }
+}
+
+__global__ __launch_bounds__(256) void zero_kernel(int* __restrict__ p, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+}  // namespace
+
+int launch_zero_counters(int* cnt, int n, hipStream_t s) {
+  hipLaunchKernelGGL(zero_kernel, dim3((n + 255) / 256), dim3(256), 0, s, cnt, n);
+  return (int)hipGetLastError();
+}
+
+int launch_seq_plan(const fa_params* p, const FwdCfg& c, const TabLayout& w, hipStream_t s) {
+  char* ws = reinterpret_cast<char*>(p->workspace);
+  const int nh = p->H / c.pack;
+  SeqPlanArgs a;
+  a.cu_q = p->eq; a.cu_k = p->ek; a.i64 = p->id_dtype == FA_IDTYPE_I64; a.nseq = p->nseq;
+  a.Tq = p->M; a.Tk = p->N; a.pack = c.pack; a.bm = c.bm; a.bk = seq_key_tile(p->D);
+  a.causal = p->causal != 0;
+  a.win = p->window > 0 && p->window < 0x3fffffff ? p->window : 0x3fffffff;
+  a.spare = w.nCnt; a.min_chunk = c.dec ? 4 : 8;
+  a.hdr = reinterpret_cast<SeqHdr*>(ws + w.off_hdr);
+  a.qtab = reinterpret_cast<SeqTile*>(ws + w.off_q);
+  a.ktab = reinterpret_cast<SeqTile*>(ws + w.off_k);
+  a.nQ = w.nQ; a.nK = w.nK;
+  a.cnt = reinterpret_cast<int*>(ws + w.off_cnt);
+  a.n_cnt = w.nCnt * nh;
+  hipLaunchKernelGGL(seq_plan_kernel, dim3(2), dim3(kThreads), 0, s, a, reinterpret_cast<int*>(ws + w.off_spill));
+  return (int)hipGetLastError();
+}
+
+}  // namespace fa

@@ -104,7 +104,7 @@ struct TileLoader {
   // base: first row of the (batch, head) slice; rs: row stride in elements
   FA_DEV void init(const void* base, int64_t rs, int nrows) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const unsigned bytes = (unsigned)((int64_t(nrows - 1) * rs + GD) * 2);
+    const unsigned bytes = nrows > 0 ? (unsigned)((int64_t(nrows - 1) * rs + GD) * 2) : 0u;
     rsrc = make_rsrc(base, bytes);
     row_bytes = int(rs) * 2;
     // The swizzle of a row depends on the row modulo NW * RPI only (see swz), so the lanes of wave
@@ -256,9 +256,58 @@ struct TileIter {
 // row this lane owns, its id, the id / row-index summaries of the wave's 32 rows
 // and of the workgroup's 128 rows, and the mask decisions per key tile.
 // ---------------------------------------------------------------------------
+// Where a workgroup of the forms without ids finds its work: the whole (batch, head group), or one sequence of a
+// packed batch, and which tile and chunk of it.
+struct TileGeo {
+  int M, N, gap;         // query rows, keys and diagonal offset of the batch entry or sequence
+  int b, h0, hk;         // batch, first query head of the tile, key head
+  int tile, chunk, nchunk;
+  int cnt, part, pstride;   // arrival counter; partial result of chunk c: part + c * pstride
+  int64_t q0, k0;        // first query row and first key of the sequence
+};
+FA_DEV TileGeo seq_geo(const KArgs& a, const SeqTile* __restrict__ e, int head) {
+  TileGeo w;
+  w.M = __builtin_amdgcn_readfirstlane(e->M); w.N = __builtin_amdgcn_readfirstlane(e->N);
+  w.gap = __builtin_amdgcn_readfirstlane(e->gap); w.tile = __builtin_amdgcn_readfirstlane(e->tile);
+  w.q0 = __builtin_amdgcn_readfirstlane(e->q0); w.k0 = __builtin_amdgcn_readfirstlane(e->k0);
+  w.chunk = __builtin_amdgcn_readfirstlane(e->chunk); w.nchunk = __builtin_amdgcn_readfirstlane(e->nchunk);
+  w.cnt = __builtin_amdgcn_readfirstlane(e->cnt) * a.nHp + head;
+  w.part = __builtin_amdgcn_readfirstlane(e->part) * a.nHp + head; w.pstride = a.nHp;
+  w.b = 0; w.h0 = head * a.pack; w.hk = w.h0 / a.G;
+  return w;
+}
+// slot: tile and chunk, the last tile (causal: the longest key range) first; bh: batch and head group.
+// M < 0: an unused slot of a packed batch.
+FA_DEV TileGeo dense_geo(const KArgs& a, int slot, int bh) {
+  TileGeo w;
+  if (a.qtab != nullptr) {
+    w = seq_geo(a, a.qtab + slot, bh);
+    if (slot >= __builtin_amdgcn_readfirstlane(a.shdr->nq)) w.M = -1;
+    return w;
+  }
+  w.M = a.M; w.N = a.N; w.gap = a.gap; w.q0 = w.k0 = 0;
+  w.b = bh / a.nHp; w.h0 = (bh - w.b * a.nHp) * a.pack; w.hk = w.h0 / a.G;
+  w.nchunk = a.dsplit;
+  w.tile = slot / a.dsplit; w.chunk = slot - w.tile * a.dsplit;
+  w.tile = a.nTiles - 1 - w.tile;
+  w.cnt = bh * a.nTiles + w.tile; w.part = w.cnt * a.dsplit; w.pstride = 1;
+  return w;
+}
+// The decode form: heads and batches fastest, then tiles, then chunks.
+FA_DEV TileGeo tile_geo(const KArgs& a, int bid) {
+  const int bhs = a.qtab != nullptr ? a.nHp : a.B * a.nHp;
+  const int slot = bid / bhs;
+  return dense_geo(a, slot, bid - slot * bhs);
+}
+// slots per (batch, head group)
+FA_HD int dense_slots(const KArgs& a) { return a.qtab != nullptr ? a.nQent : a.nTiles * a.dsplit; }
+FA_HD int tile_geo_blocks(const KArgs& a) { return dense_slots(a) * (a.qtab != nullptr ? a.nHp : a.B * a.nHp); }
+
 template <bool CAUSAL, bool DOC>
 struct QTileCtx {
-  int row;    // original row index of this lane's query (lanes l and l^32 share it), -1 if none
+  int row;    // row index of this lane's query inside its batch entry or sequence (lanes l and l^32 share it), -1 if none
+  int hg;     // its head among those that share the tile (0 with ids)
+  int N;      // keys
   int rowc;   // row clamped into [0, M) for loads
   int eq_i;
   // Causal terms are written in key positions: the diagonal of row i sits at key gp + r, where without ids
@@ -282,26 +331,35 @@ struct QTileCtx {
   const int* ekp;
   const IdSummary* ksum;
 
-  // tile: index of the 128-row tile (natural order, or permuted order with ids).
+  // ge.tile: index of the tile (natural order of the packed rows, or 128 rows of the permuted order with ids).
   // Returns false when the tile holds no row.
-  // wave: index (0..3) of this wave inside the 128-row tile.
-  FA_DEV bool init(const KArgs& a, int b, int h, int tile, int wave) {
+  // wave: index (0..3) of this wave inside the tile.
+  FA_DEV bool init(const KArgs& a, const TileGeo& ge, int wave) {
+    const int b = ge.b, h = ge.h0, tile = ge.tile;
     const int lane = threadIdx.x & 63;
     const int lq = lane & 31;
     eq_i = 0; ekp = nullptr; ksum = nullptr;
     w_lo = 0; w_hi = -1; w_glob = 1; g_lo = 0; g_hi = -1; g_glob = 1;
     g_kfirst = 0; g_klast = 0x3fffffff;
-    gp = DOC ? 0 : a.gap;
+    gp = DOC ? 0 : ge.gap;
+    hg = 0; N = ge.N;
     int posc;   // r of this lane's row, 0 if none
     rb = wave; sub = 0; halved = false;
     if (!DOC) {
-      const int m0 = tile * 128;
-      if (a.M - m0 <= 64 && a.bmask == nullptr) { halved = true; rb = wave & 1; sub = wave >> 1; }
+      const int m0 = tile * a.bm, Mr = ge.M * a.pack;   // packed rows: row r is query r / pack of head r % pack
+      if ((Mr - m0 <= 64 || a.bm <= 64) && a.bmask == nullptr) { halved = true; rb = wave & 1; sub = wave >> 1; }
       const int mw = m0 + rb * 32;
-      row = mw + lq < a.M ? mw + lq : -1;
-      w_rmin = mw; w_rmax = min(mw + 31, a.M - 1);
+      const int end = min(Mr, m0 + a.bm);   // (tiles of 32 rows: the waves of the second row block have none)
+      row = mw + lq < end ? mw + lq : -1;
+      w_rmin = mw; w_rmax = min(mw + 31, end - 1);
       if (w_rmax < w_rmin) w_rmax = -1;
-      g_rmin = m0; g_rmax = min(m0 + 127, a.M - 1);
+      g_rmin = m0; g_rmax = end - 1;
+      if (a.pack > 1) {
+        const int pr = row;
+        if (pr >= 0) { row = pr / a.pack; hg = pr - row * a.pack; }
+        w_rmin /= a.pack; if (w_rmax >= 0) w_rmax /= a.pack;
+        g_rmin /= a.pack; g_rmax /= a.pack;
+      }
       posc = row >= 0 ? row : 0;
     } else {
       ekp = a.ek32 + b * a.ek_bs + h * a.ek_hs;
@@ -337,8 +395,8 @@ struct QTileCtx {
       w_glob = __builtin_amdgcn_ballot_w64(eq_i >= 0 && row >= 0) != 0;
     }
     rowc = row >= 0 ? row : 0;
-    lim_i = CAUSAL ? min(max(gp + posc, a.pfx_m1), a.N - 1) : a.N - 1;
-    w_limmin = CAUSAL ? min(max(gp + w_rmin, a.pfx_m1), a.N - 1) : a.N - 1;
+    lim_i = CAUSAL ? min(max(gp + posc, a.pfx_m1), N - 1) : N - 1;
+    w_limmin = CAUSAL ? min(max(gp + w_rmin, a.pfx_m1), N - 1) : N - 1;
     low_i = CAUSAL ? gp + posc - a.win + 1 : -0x3fffffff;
     w_lowmin = CAUSAL && w_rmax >= 0 ? gp + w_rmin - a.win + 1 : -0x3fffffff;
     w_lowmax = CAUSAL && w_rmax >= 0 ? gp + w_rmax - a.win + 1 : -0x3fffffff;
@@ -351,7 +409,7 @@ struct QTileCtx {
     return CAUSAL && g_rmax >= 0 ? max(f, max(0, gp + g_rmin - a.win + 1) / 64) : f;   // sliding window
   }
   FA_DEV int last_tile(const KArgs& a) const {
-    const int hi_key = CAUSAL ? min(a.N, max(gp + g_rmax, a.pfx_m1) + 1) : a.N;
+    const int hi_key = CAUSAL ? max(0, min(N, max(gp + g_rmax, a.pfx_m1) + 1)) : N;   // (a sequence with fewer keys than rows: none)
     return min((hi_key + 63) / 64, g_klast + 1);
   }
 
@@ -424,6 +482,55 @@ struct QBlockMask {
   }
 };
 
+// blockIdx -> (tile, batch*head) for grids of `ntile` tiles per (batch, head); grid_blocks() is the
+// matching grid size.  Consecutive workgroup ids land on different XCDs (8 of them, each with its
+// own L2), so the map decides which XCD's L2 sees which head:
+//   BH a multiple of 8 : every XCD is given whole heads (its L2 keeps that head's K/V or Q/dO).
+//        Inside an XCD the order is
+//          head-major (tile_major = false): one head after the other -- best L2 reuse when every
+//               tile streams most of the head (no ids);
+//          tile-major (tile_major = true): tile slot 0 of all the XCD's heads, then slot 1, ... --
+//               with ids the few heavy tiles (global rows) of EVERY head start at once instead of
+//               queueing behind the light tiles of the heads before them.
+//   BH = 1, 2, 4      : a head is shared by 8 / BH XCDs, its tile slots dealt round-robin among them
+//                       (heavy and light slots alternate, so the XCDs stay balanced).
+//   otherwise          : (slot, head) pairs dealt round-robin over the XCDs, slot-major: balanced for
+//                       any BH, at the price of every L2 seeing every head.
+// Returns false for padding ids.
+FA_HD int grid_blocks(int ntile, int BH) {
+  if (BH % 8 == 0) return BH * ntile;
+  if (BH < 8 && 8 % BH == 0) { const int k = 8 / BH; return 8 * ((ntile + k - 1) / k); }
+  return (BH * ntile + 7) / 8 * 8;
+}
+
+// bid: index of the workgroup (blockIdx.x, unless several forms share one grid).
+FA_DEV bool block_to_tile(int ntile, int BH, bool tile_major, int& tile_slot, int& bh, int bid) {
+  const int xcd = bid & 7, idx = bid >> 3;
+  if (BH % 8 == 0) {
+    const int heads = BH / 8;  // heads per XCD
+    if (tile_major) {
+      bh = (idx % heads) * 8 + xcd;
+      tile_slot = idx / heads;
+    } else {
+      bh = (idx / ntile) * 8 + xcd;
+      tile_slot = idx % ntile;
+    }
+    return true;
+  }
+  if (BH < 8 && 8 % BH == 0) {
+    const int k = 8 / BH;
+    bh = xcd / k;
+    tile_slot = idx * k + xcd % k;
+    return tile_slot < ntile;
+  }
+  tile_slot = bid / BH;
+  bh = bid % BH;
+  return tile_slot < ntile;
+}
+FA_DEV bool block_to_tile(int ntile, int BH, bool tile_major, int& tile_slot, int& bh) {
+  return block_to_tile(ntile, BH, tile_major, tile_slot, bh, (int)blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // Work assignment of one workgroup of the forward / dq kernels, including the split of the
 // key range of global-row tiles (SplitCfg, fa_common.h).
@@ -443,9 +550,7 @@ struct QWork {
 // slots [nE, ...), not looked at until q_work_finish: the tile's own summaries and row indices are
 // requested in between, so the two loads overlap instead of forming a dependent chain.
 constexpr int kGtPending = -2;
-template <bool DOC>
 FA_DEV bool q_work(const KArgs& a, const QHeader& hd, int nQt, int slot, QWork& w) {
-  if (!DOC) { w.tile = nQt - 1 - slot; w.gt = -1; w.split = 0; return true; }
   const int nE = split_extra(a);
   if (slot < nE) {
     const int g0 = hd.nLp / 128;   // first global-row tile
@@ -475,6 +580,46 @@ FA_DEV int split_range(const KArgs& a, const QWork& w, int& first, int& last) {
   first = min(last, first + w.split * c);
   last = min(last, first + c);
   return ns;
+}
+
+// The same for the launches without ids (nchunk chunks whatever the tile's range: some may be empty).
+FA_DEV void chunk_range(const TileGeo& ge, int& first, int& last) {
+  if (ge.nchunk == 1) return;
+  const int n = max(0, last - first), c = (n + ge.nchunk - 1) / ge.nchunk;
+  first = min(last, first + ge.chunk * c);
+  last = min(last, first + c);
+}
+
+// Work of one workgroup of the forward / dq kernels, with and without ids: which tile, where its partial result goes
+// when its key range is split, and the key tiles [kt_first, kt_last) to walk.  False: nothing to do.
+template <bool CAUSAL, bool DOC>
+FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, DOC>& qc, int& kt_first, int& kt_last) {
+  int slot, bh;
+  if constexpr (DOC) {
+    const int nQt = a.Pp / 128;
+    if (!block_to_tile(nQt + split_extra(a), a.B * a.H, nQt >= 32, slot, bh)) return false;
+    ge.b = bh / a.H; ge.h0 = bh % a.H; ge.hk = ge.h0 / a.G;
+    ge.M = a.M; ge.N = a.N; ge.gap = a.gap; ge.q0 = ge.k0 = 0;
+    QWork wk;
+    const QHeader hd = a.qhdr[ge.b * a.qh_bs + ge.h0 * a.qh_hs];
+    if (!q_work(a, hd, nQt, slot, wk)) return false;
+    ge.tile = wk.tile;
+    if (!qc.init(a, ge, threadIdx.x >> 6)) return false;
+    q_work_finish(a, hd, wk);
+    kt_first = qc.first_tile(a); kt_last = qc.last_tile(a);
+    ge.chunk = wk.split; ge.nchunk = split_range(a, wk, kt_first, kt_last);
+    ge.cnt = bh * a.split_tiles + wk.gt; ge.part = ge.cnt * a.split_k; ge.pstride = 1;
+    return ge.chunk < ge.nchunk;
+  } else {
+  // the tiles of a packed batch are sorted by their length: longest first over all heads
+  if (!block_to_tile(dense_slots(a), a.qtab != nullptr ? a.nHp : a.B * a.nHp, a.qtab != nullptr, slot, bh)) return false;
+  ge = dense_geo(a, slot, bh);
+  if (ge.M < 0) return false;
+  qc.init(a, ge, threadIdx.x >> 6);
+  kt_first = qc.first_tile(a); kt_last = qc.last_tile(a);
+  chunk_range(ge, kt_first, kt_last);
+  return true;
+  }
 }
 
 // A wave's 32 result rows on their way out.  The accumulators hold a row (or key) per lane and 4 consecutive
@@ -590,55 +735,6 @@ FA_DEV GcolInfo gcol_info(const KArgs& a, int b, int hk) {
   r.ncols = k0 >= a.nKs ? (a.N + 127) / 128 * 128 : (k0 * kSumRows) / 128 * 128;
   if (tiles > kGcolTilesMax) r.ncols = 0;
   return r;
-}
-
-// blockIdx -> (tile, batch*head) for grids of `ntile` tiles per (batch, head); grid_blocks() is the
-// matching grid size.  Consecutive workgroup ids land on different XCDs (8 of them, each with its
-// own L2), so the map decides which XCD's L2 sees which head:
-//   BH a multiple of 8 : every XCD is given whole heads (its L2 keeps that head's K/V or Q/dO).
-//        Inside an XCD the order is
-//          head-major (tile_major = false): one head after the other -- best L2 reuse when every
-//               tile streams most of the head (no ids);
-//          tile-major (tile_major = true): tile slot 0 of all the XCD's heads, then slot 1, ... --
-//               with ids the few heavy tiles (global rows) of EVERY head start at once instead of
-//               queueing behind the light tiles of the heads before them.
-//   BH = 1, 2, 4      : a head is shared by 8 / BH XCDs, its tile slots dealt round-robin among them
-//                       (heavy and light slots alternate, so the XCDs stay balanced).
-//   otherwise          : (slot, head) pairs dealt round-robin over the XCDs, slot-major: balanced for
-//                       any BH, at the price of every L2 seeing every head.
-// Returns false for padding ids.
-FA_HD int grid_blocks(int ntile, int BH) {
-  if (BH % 8 == 0) return BH * ntile;
-  if (BH < 8 && 8 % BH == 0) { const int k = 8 / BH; return 8 * ((ntile + k - 1) / k); }
-  return (BH * ntile + 7) / 8 * 8;
-}
-
-// bid: index of the workgroup (blockIdx.x, unless several forms share one grid).
-FA_DEV bool block_to_tile(int ntile, int BH, bool tile_major, int& tile_slot, int& bh, int bid) {
-  const int xcd = bid & 7, idx = bid >> 3;
-  if (BH % 8 == 0) {
-    const int heads = BH / 8;  // heads per XCD
-    if (tile_major) {
-      bh = (idx % heads) * 8 + xcd;
-      tile_slot = idx / heads;
-    } else {
-      bh = (idx / ntile) * 8 + xcd;
-      tile_slot = idx % ntile;
-    }
-    return true;
-  }
-  if (BH < 8 && 8 % BH == 0) {
-    const int k = 8 / BH;
-    bh = xcd / k;
-    tile_slot = idx * k + xcd % k;
-    return tile_slot < ntile;
-  }
-  tile_slot = bid / BH;
-  bh = bid % BH;
-  return tile_slot < ntile;
-}
-FA_DEV bool block_to_tile(int ntile, int BH, bool tile_major, int& tile_slot, int& bh) {
-  return block_to_tile(ntile, BH, tile_major, tile_slot, bh, (int)blockIdx.x);
 }
 
 }  // namespace fa

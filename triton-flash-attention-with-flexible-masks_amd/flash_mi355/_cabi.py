@@ -11,10 +11,11 @@ from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libflash_mi355.so"
 
-FA_ABI_VERSION = 7
+FA_ABI_VERSION = 8
 FA_SCORE_MODE0_NOPE = 0
 FA_SCORE_MODE1_DOC = 1
 FA_SCORE_MODE2_BLOCK = 2
+FA_SCORE_MODE3_PACKED = 3
 FA_MASK_BLOCK = 64
 FA_DTYPE_BF16 = 0
 FA_DTYPE_FP16 = 1
@@ -22,6 +23,7 @@ FA_DTYPE_FP32 = 2
 FA_IDTYPE_I32 = 0
 FA_IDTYPE_I64 = 1
 FA_FLAG_DQ_DELTA = 1
+FA_FLAG_SPLIT_KEYS = 4
 FA_FLAG_DEBUG_NO_PAIR_WAIT = 0x100
 FA_STATIC_WS_BYTES = 32 << 20
 
@@ -48,6 +50,7 @@ class FaParams(Structure):
         ("sm_scale", c_float), ("flags", c_int32), ("window", c_int32), ("prefix", c_int32),
         ("qpos", c_void_p), ("qpos_stride", c_int64),
         ("split_scratch", c_void_p), ("split_scratch_bytes", c_uint64),
+        ("nseq", c_int32), ("reserved", c_int32),
     ]
 
 

@@ -16,6 +16,7 @@ from . import _cabi
 
 SCORE_FUNC_MODE0_NOPE = 0  # flash_triton.py:20
 SCORE_FUNC_MODE1_DOC = 1   # flash_triton.py:22
+SCORE_FUNC_MODE3_PACKED = 3  # packed sequences: set by attention_varlen(), eq / ek are the cumulative lengths; no counterpart in the reference
 SCORE_FUNC_MODE2_BLOCK = 2  # block mask: set by the block_mask argument of attention(), no counterpart in the reference
 
 _DTYPES = {torch.bfloat16: _cabi.FA_DTYPE_BF16, torch.float16: _cabi.FA_DTYPE_FP16, torch.float32: _cabi.FA_DTYPE_FP32}
@@ -51,7 +52,7 @@ def _stream_ptr(device) -> int:
 class _Plan:
     """fa_params filled in for one problem, plus the tensors that keep its pointers alive."""
 
-    def __init__(self, q, k, v, causal, sm_scale, eq, ek, score_func_mode, window=0, prefix=0, qpos=None):
+    def __init__(self, q, k, v, causal, sm_scale, eq, ek, score_func_mode, window=0, prefix=0, qpos=None, flags=0):
         B, H, M, D = q.shape
         N, Hk = k.shape[2], k.shape[1]
         p = _cabi.FaParams()
@@ -62,13 +63,17 @@ class _Plan:
         p.score_mode = int(score_func_mode)
         p.dtype = _DTYPES[q.dtype]
         p.sm_scale = float(sm_scale)
-        p.flags = 0
+        p.flags = flags
         p.window, p.prefix = int(window), int(prefix)
         self.keep = [q, k, v]
         if score_func_mode == SCORE_FUNC_MODE2_BLOCK:   # eq is the block map [B, H, rows of blocks, columns of blocks], bytes
             p.eq = eq.data_ptr()
             _set3(p.eq_stride, eq)
             self.keep += [eq]
+        elif score_func_mode == SCORE_FUNC_MODE3_PACKED:
+            p.eq, p.ek = eq.data_ptr(), ek.data_ptr()
+            p.id_dtype, p.nseq = _ID_DTYPES[eq.dtype], eq.numel() - 1
+            self.keep += [eq, ek]
         elif score_func_mode != SCORE_FUNC_MODE0_NOPE:
             p.eq, p.ek = eq.data_ptr(), ek.data_ptr()
             _set3(p.eq_stride, eq); _set3(p.ek_stride, ek)
@@ -111,6 +116,11 @@ def _prep_ids(e, name):
     return e
 
 
+def _prep_cu(cu):
+    assert cu.dim() == 1 and not cu.dtype.is_floating_point and cu.dtype != torch.bool, "cu_seqlens must be an integer vector"
+    return (cu if cu.dtype in _ID_DTYPES else cu.to(torch.int64)).contiguous()
+
+
 def _check_same_device(ref, **others):
     """Every tensor whose address is handed to a kernel lives on the device the kernels run on (a host
     or foreign pointer would be a memory fault on the GPU, not an error)."""
@@ -138,7 +148,7 @@ class _Impl:
         assert Hk == Hv, "num of heads in k and v should be equal"
         assert H % Hk == 0, "number of heads in q must be a multiple of that in k & v"
         num_groups = H // Hk
-        assert (N >= M) or (not causal) or (qpos is not None), "KV length should be larger than M length in causal mode!"
+        assert (N >= M) or (not causal) or (qpos is not None) or score_func_mode == SCORE_FUNC_MODE3_PACKED, "KV length should be larger than M length in causal mode!"
         MN_GAP = max(0, N - M)
         if sm_scale is None:
             sm_scale = 1. / math.sqrt(D)
@@ -147,7 +157,7 @@ class _Impl:
         if eq is None:
             assert score_func_mode == SCORE_FUNC_MODE0_NOPE
         # -- checks the reference leaves to the Triton launcher --
-        assert score_func_mode in (SCORE_FUNC_MODE0_NOPE, SCORE_FUNC_MODE1_DOC, SCORE_FUNC_MODE2_BLOCK), "unknown score_func_mode"
+        assert score_func_mode in (SCORE_FUNC_MODE0_NOPE, SCORE_FUNC_MODE1_DOC, SCORE_FUNC_MODE2_BLOCK, SCORE_FUNC_MODE3_PACKED), "unknown score_func_mode"
         window, prefix = int(window or 0), int(prefix or 0)
         assert window >= 0 and prefix >= 0 and not (window and prefix), "window and prefix exclude each other"
         assert causal or not (window or prefix), "window / prefix are causal masks"
@@ -164,6 +174,9 @@ class _Impl:
                 f"block_mask must be [bs|1, H|1, {nbr}, {nbc}] (blocks of 64 x 64)"
             eq = maybe_contiguous((eq != 0).to(torch.uint8).to(q.device)).expand(B, H, nbr, nbc)
             ek = eq
+        elif score_func_mode == SCORE_FUNC_MODE3_PACKED:
+            assert B == 1 and eq.dim() == 1 and eq.shape == ek.shape and eq.dtype == ek.dtype and eq.dtype in _ID_DTYPES and eq.is_contiguous() \
+                and ek.is_contiguous() and q.dtype != torch.float32, "packed sequences: see attention_varlen"
         elif score_func_mode != SCORE_FUNC_MODE0_NOPE:
             eq, ek = _prep_ids(eq, "eq"), _prep_ids(ek, "ek")
             if eq.dtype != ek.dtype:   # one id width per call
@@ -172,14 +185,6 @@ class _Impl:
             assert tuple(ek.shape) == (B, H, N), "ek must be [bs, H, Lk]"
         else:
             eq = ek = None
-            if _short_query_long_key(B, H, M, N, q.dtype):
-                # Few query tiles against a long key range (decoding, the tail of a long prompt): a launch of
-                # B*H*ceil(M/128) workgroups leaves most of the chip idle while each walks every key.  Rows whose
-                # id is >= 0 see every key (flash_triton.py:114), and the kernels cut the key range of such rows
-                # into chunks that separate workgroups process and merge: the same mask, more parallelism.
-                zero = torch.zeros((1, 1, 1), dtype=torch.int32, device=q.device)   # every stride 0: one id for all
-                eq, ek = zero.expand(B, H, M), zero.expand(B, H, N)
-                score_func_mode = SCORE_FUNC_MODE1_DOC
         if qpos is not None:
             assert causal and score_func_mode == SCORE_FUNC_MODE1_DOC and not prefix, \
                 "qpos (per-row causal positions) needs causal=True and eq / ek, and excludes prefix"
@@ -187,6 +192,7 @@ class _Impl:
                 "qpos must be an integer tensor [bs|1, Lq]"
             _check_same_device(q, qpos=qpos)
             qpos = qpos.to(torch.int32).contiguous()
+        flags = _cabi.FA_FLAG_SPLIT_KEYS if score_func_mode == SCORE_FUNC_MODE0_NOPE else 0
         ctx.nothing_to_do = B == 0 or H == 0 or M == 0 or N == 0
         if ctx.nothing_to_do:
             # No rows, or rows without a single key: nothing is launched (the C ABI refuses sizes <= 0).  A row
@@ -199,7 +205,7 @@ class _Impl:
 
         L = _cabi.lib()
         with torch.cuda.device(q.device):
-            plan = _Plan(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos)
+            plan = _Plan(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos, flags)
             Out = torch.empty_like(q)   # q's layout when q is dense (flash_triton.py:539), contiguous otherwise
             lse = torch.empty((B, H, M), device=q.device, dtype=torch.float32)
             p = plan.p
@@ -229,7 +235,8 @@ class _Impl:
         do = _aligned(maybe_contiguous(do))
         _check_same_device(q, do=do, dlse=dlse)
         with torch.cuda.device(q.device):
-            plan = _Plan(q, k, v, ctx.causal, ctx.sm_scale, eq, ek, score_func_mode, window, prefix, qpos)
+            plan = _Plan(q, k, v, ctx.causal, ctx.sm_scale, eq, ek, score_func_mode, window, prefix, qpos,
+                         _cabi.FA_FLAG_SPLIT_KEYS if score_func_mode == SCORE_FUNC_MODE0_NOPE else 0)
             p = plan.p
             if workspace is not None:   # the forward's mask plan is used in place (flash_triton.py:557-562 saves, copies nothing)
                 plan.ensure_workspace(q.device, plan_state=workspace)
@@ -247,7 +254,7 @@ class _Impl:
             if dlse is None:
                 # two launches instead of the reference's three (flash_triton.py:585-634): the dq kernel
                 # forms delta = rowsum(O * dO) from rows it holds anyway and leaves it for the dk/dv kernel
-                p.flags = _cabi.FA_FLAG_DQ_DELTA
+                p.flags |= _cabi.FA_FLAG_DQ_DELTA
                 _cabi.check(L.fa_bwd_dq(ctypes.byref(p), stream), "fa_bwd_dq")
                 _cabi.check(L.fa_bwd_dkdv(ctypes.byref(p), stream), "fa_bwd_dkdv")
             else:
@@ -352,30 +359,33 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k=None, causal=False, sm_
     sequence lengths starting at 0.  Token i of sequence s attends to the keys of sequence s
     only.  Returns [total_q, H, D]; differentiable.
 
-    The packed batch IS the document mask of the operator: one (batch) row of total_* tokens whose
-    ids are the negated sequence numbers, so no padding and no copy -- q, k, v are passed as
-    [1, H, total, D] views, one launch per kernel whatever the number of sequences.  Causal with
-    different boundaries (queries that are the tail of a longer key sequence: chunked prefill,
-    decoding) aligns every sequence bottom-right on its own, which is not one offset of the packed
-    row: the rows then carry their own causal positions (varlen_positions, the qpos argument of the
-    operator).  Nothing is read back to the host.
+    No padding, no copy, one launch per kernel whatever the number of sequences, nothing is read back
+    to the host: q, k, v are passed as [1, H, total, D] views, and the plan kernel turns the boundaries
+    into a table of tiles (every sequence starts its own, so no tile mixes sequences).  Causal with
+    different boundaries (queries that are the tail of a longer key sequence: chunked prefill, decoding)
+    aligns every sequence bottom-right on its own.  fp32 tensors go through the document mask: ids are
+    the negated sequence numbers (varlen_ids), the alignment is one position per row (varlen_positions,
+    the qpos argument of the operator).
     (No counterpart in the reference, which takes eq/ek directly, flash_triton.py:506.)"""
     assert q.dim() == 3 and k.dim() == 3 and v.dim() == 3, "q, k, v must be [total, heads, D]"
     same = cu_seqlens_k is None or cu_seqlens_k is cu_seqlens_q
     Tq, H, _ = q.shape
     Tk = k.shape[0]
-    # the boundaries may live on the host (the ids and positions are built on q's device either way)
+    # the boundaries may live on the host (the tables are built on q's device either way)
     cu_seqlens_q = cu_seqlens_q.to(q.device)
     cu_seqlens_k = cu_seqlens_q if same else cu_seqlens_k.to(q.device)
     assert not same or Tk == Tq, "cu_seqlens_k is needed when k holds a different number of tokens than q"
-    qpos = None
-    if not same:
-        assert cu_seqlens_q.shape == cu_seqlens_k.shape, "cu_seqlens_q and cu_seqlens_k must describe the same sequences"
-        if causal:
-            qpos = varlen_positions(cu_seqlens_q, cu_seqlens_k, Tq).view(1, Tq)
+    assert same or cu_seqlens_q.shape == cu_seqlens_k.shape, "cu_seqlens_q and cu_seqlens_k must describe the same sequences"
+    q4, k4, v4 = (t.transpose(0, 1).unsqueeze(0) for t in (q, k, v))
+    if q.dtype != torch.float32 and cu_seqlens_q.numel() > 1:
+        cq, ck = _prep_cu(cu_seqlens_q), _prep_cu(cu_seqlens_k)
+        if cq.dtype != ck.dtype:   # one id width per call
+            cq, ck = cq.to(torch.int64), ck.to(torch.int64)
+        out = FlashAttention.apply(q4, k4, v4, causal, sm_scale, cq, ck, SCORE_FUNC_MODE3_PACKED, window, 0, None)
+        return out.squeeze(0).transpose(0, 1)
+    qpos = varlen_positions(cu_seqlens_q, cu_seqlens_k, Tq).view(1, Tq) if causal and not same else None
     eq = varlen_ids(cu_seqlens_q, Tq)
     ek = eq if same else varlen_ids(cu_seqlens_k, Tk)
-    q4, k4, v4 = (t.transpose(0, 1).unsqueeze(0) for t in (q, k, v))
     out = attention(q4, k4, v4, causal, sm_scale, eq.view(1, 1, Tq).expand(1, H, Tq), ek.view(1, 1, Tk).expand(1, H, Tk),
                     SCORE_FUNC_MODE1_DOC, window=window, qpos=qpos)
     return out.squeeze(0).transpose(0, 1)
