@@ -1,0 +1,83 @@
+"""The native host path against the Python classes it stands in for: same bits, same autograd behaviour."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(kind, q, k, v, e, bm, cls, use_native):
+    from flash_mi355 import api
+    args = {"plain": (None, None, 0, 0, 0, None), "window": (None, None, 0, 37, 0, None), "doc": (e, e, 1, 0, 0, None),
+            "pos": (e, e, 1, 0, 0, torch.arange(q.shape[2], device="cuda", dtype=torch.int32)[None]), "block": (bm, bm, 2, 0, 0, None)}[kind]
+    want_lse = cls is api.FlashAttentionWithLse
+    if use_native:
+        out = api._host().attention(q, k, v, True, None, *args, want_lse)
+        assert out is not None, "the native path takes the usual calls"
+    else:
+        out = cls.apply(q, k, v, True, None, *args)
+    return out if want_lse else (out,)
+
+
+@pytest.mark.parametrize("layout", ["bhld", "blhd"])
+@pytest.mark.parametrize("lse", [False, True])
+@pytest.mark.parametrize("kind", ["plain", "window", "doc", "pos", "block"])
+def test_native_path_gives_the_bits_of_the_python_path(kind, lse, layout):
+    from flash_mi355 import api, workloads as W
+    B, H, Hk, L, D = 2, 4, 2, 200, 64
+    g = torch.Generator().manual_seed(1)
+    def t(h):
+        x = torch.randn(B, L, h, D, generator=g).bfloat16().cuda()
+        return x.transpose(1, 2) if layout == "blhd" else x.transpose(1, 2).contiguous()
+    q, k, v, do = t(H), t(Hk), t(Hk), t(H)
+    ids = torch.from_numpy(np.stack([W.doc_ids_uniform(np.random.default_rng(2), L, 8, 60, 0.1) for _ in range(B)])).cuda()
+    e = ids[:, None].expand(B, H, L)
+    bm = (torch.rand(B, 1, 4, 4, generator=g) < 0.5).cuda() | torch.eye(4, dtype=torch.bool, device="cuda")
+    cls = api.FlashAttentionWithLse if lse else api.FlashAttention
+    w = torch.randn(B, H, L, generator=g).cuda()
+    got = []
+    for native in (True, False):
+        x = [z.detach().requires_grad_(True) for z in (q, k, v)]
+        out = _call(kind, *x, e, bm, cls, native)
+        grads = torch.autograd.grad(out, x, (do, w)[:len(out)])
+        assert all(z.shape == y.shape and z.stride(-1) == 1 for z, y in zip(grads, x))
+        got.append([*[z.detach() for z in out], *grads])
+    for a, b in zip(*got):
+        assert a.dtype == b.dtype and a.stride() == b.stride() and torch.equal(a, b)
+
+
+def test_autograd_behaviour_of_the_native_node():
+    from flash_mi355 import attention
+    q, k, v = (torch.randn(1, 2, 64, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
+    with torch.no_grad():
+        assert not attention(q, k, v, True).requires_grad
+    out = attention(q, k, v, True)
+    out.sum().backward(retain_graph=True)          # an expanded gradient (stride 0)
+    first = q.grad.clone()
+    out.sum().backward()
+    assert torch.equal(q.grad, 2 * first)
+    with pytest.raises(RuntimeError, match="second time"):
+        out.sum().backward()
+    out = attention(q, k.detach(), v.detach(), True)   # one operand wants a gradient
+    (gq,) = torch.autograd.grad(out.sum(), q)
+    assert torch.equal(gq, first)
+    out = attention(q, k, v, True)
+    with torch.no_grad():
+        k.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+def test_calls_the_native_path_leaves_to_python():
+    """Everything that needs a conversion or an error message comes back as None and then works, or raises, as before."""
+    from flash_mi355 import api, attention
+    q = torch.randn(1, 2, 70, 64, device="cuda", dtype=torch.bfloat16)
+    n = api._host().attention
+    none = [(q, q, q, False, None, None, None, 1, 0, 0, None, False), (q.cpu(), q, q, False, None, None, None, 0, 0, 0, None, False),
+            (q, q[:, :, :10], q[:, :, :10], True, None, None, None, 0, 0, 0, None, False), (q[:, :, :, ::2],) * 3 + (False, None, None, None, 0, 0, 0, None, False),
+            (q, q, q, False, None, None, None, 0, 5, 0, None, False), (q[:, :, :0], q, q, False, None, None, None, 0, 0, 0, None, False)]
+    assert all(n(*a) is None for a in none)
+    odd = torch.randn(1, 2, 70, 72, device="cuda", dtype=torch.bfloat16)[:, :, :, 3:67]   # base not 16-byte aligned
+    assert torch.equal(attention(odd, odd, odd, True), attention(odd.contiguous(), odd.contiguous(), odd.contiguous(), True))
+    ids = torch.zeros(1, 2, 70, dtype=torch.int16, device="cuda") - 1
+    assert torch.equal(attention(q, q, q, True, None, ids, ids, 1), attention(q, q, q, True, None, ids.int(), ids.int(), 1))

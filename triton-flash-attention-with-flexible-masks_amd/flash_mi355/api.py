@@ -4,6 +4,9 @@ Same entry point, argument order, defaults, checks and return values as the
 reference's ``flash_triton.attention`` / ``FlashAttention`` (flash_triton.py:506-641);
 the kernels behind it are the hand-written gfx950 kernels of libflash_mi355.so.
 torch is used for device memory and streams only.
+
+The usual calls go through the native host path (csrc/torch_host.cpp), which returns None for anything it
+would have to convert, copy or refuse; such calls take the classes below, which hold the checks.
 """
 from __future__ import annotations
 
@@ -47,6 +50,22 @@ def _set3(dst, t):
 
 def _stream_ptr(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+_native = None
+
+
+def _host():
+    """The native host path (built next to the library; there is no fallback for a missing one)."""
+    global _native
+    if _native is None:
+        _cabi.lib()   # says how to build when nothing is built
+        try:
+            from . import _native as native
+        except ImportError as e:
+            raise _cabi.FlashMI355Error(f"the native host path does not load ({e}): build it with `python -m flash_mi355.build`") from e
+        _native = native
+    return _native
 
 
 class _Plan:
@@ -317,6 +336,9 @@ def attention(q, k, v, causal=False, sm_scale=None, eq=None, ek=None, score_func
     qpos[i] (it sees keys j <= qpos[i]) instead of max(0, Lk - Lq) + i; needs causal=True and eq / ek
     (the ids confine a row to its sequence, qpos aligns each sequence on its own), excludes prefix."""
     eq, ek, score_func_mode = _block_args(block_mask, eq, ek, score_func_mode)
+    out = (_native or _host()).attention(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos, False)
+    if out is not None:
+        return out
     return FlashAttention.apply(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos)
 
 
@@ -328,6 +350,9 @@ def attention_with_lse(q, k, v, causal=False, sm_scale=None, eq=None, ek=None,
     """(O, LSE) with LSE in natural-log units (-inf for rows without a kept key); differentiable
     through both results."""
     eq, ek, score_func_mode = _block_args(block_mask, eq, ek, score_func_mode)
+    out = (_native or _host()).attention(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos, True)
+    if out is not None:
+        return out
     return FlashAttentionWithLse.apply(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos)
 
 
@@ -367,6 +392,9 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k=None, causal=False, sm_
     the negated sequence numbers (varlen_ids), the alignment is one position per row (varlen_positions,
     the qpos argument of the operator).
     (No counterpart in the reference, which takes eq/ek directly, flash_triton.py:506.)"""
+    out = (_native or _host()).attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, causal, sm_scale, window)
+    if out is not None:
+        return out
     assert q.dim() == 3 and k.dim() == 3 and v.dim() == 3, "q, k, v must be [total, heads, D]"
     same = cu_seqlens_k is None or cu_seqlens_k is cu_seqlens_q
     Tq, H, _ = q.shape

@@ -28,6 +28,10 @@ PROBE_LIB_PATH = PKG_DIR / "libfa_probe.so"
 # workgroup and the extra export fa_trace_read); never loaded by the operator
 TRACE_LIB_PATH = PKG_DIR / "libflash_mi355_trace.so"
 TRACE_OBJ_DIR = PKG_DIR / "_obj_trace"
+# host path of the operator (checks, allocation, launches, autograd node): a Python extension module that links
+# torch and the library next to it
+HOST_SOURCE = "torch_host.cpp"
+HOST_LIB_PATH = PKG_DIR / "_native.so"
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -47,6 +51,22 @@ def _compile(src: Path, obj: Path, extra) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{r.stderr[-4000:]}")
     return r.stderr
+
+
+def _build_host() -> None:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    lib_dir = Path(torch.__file__).resolve().parent / "lib"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *[f"-isystem{p}" for p in cpp_extension.include_paths()], "-isystem/opt/rocm/include", f"-isystem{sysconfig.get_paths()['include']}",
+           str(CSRC / HOST_SOURCE), "-o", str(HOST_LIB_PATH), f"-L{PKG_DIR}", "-lflash_mi355", "-Wl,-rpath,$ORIGIN",
+           f"-L{lib_dir}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-ltorch"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for {HOST_SOURCE}:\n{r.stderr[-4000:]}")
 
 
 def build(force: bool = True, verbose: bool = False, extra_flags=()) -> Path:
@@ -89,6 +109,9 @@ def build(force: bool = True, verbose: bool = False, extra_flags=()) -> Path:
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
+    host_src = CSRC / HOST_SOURCE
+    if force or not HOST_LIB_PATH.exists() or HOST_LIB_PATH.stat().st_mtime < max(host_src.stat().st_mtime, newest_hdr):
+        _build_host()
     return LIB_PATH
 
 
