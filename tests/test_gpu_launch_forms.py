@@ -150,3 +150,19 @@ def test_packed_graph_replay():
             torch.cuda.synchronize()
             got = out.clone()
             assert torch.equal(got, attention_varlen(q, k, v, cq, ck, causal=True)), rep
+
+
+# fp32: launches of few workgroups split a tile of the streamed side over the four waves; the sizes around its edges, and
+# the smallest launch that keeps 128 rows to a workgroup.  B, H, Hk, M, N, D, causal, doc, window
+FP32_CASES = [
+    (1, 2, 2, 1, 1, 64, True, False, 0), (1, 2, 1, 33, 129, 64, True, False, 0), (2, 2, 2, 128, 300, 128, True, True, 0),
+    (1, 4, 2, 257, 257, 64, True, True, 0), (1, 2, 2, 200, 200, 32, False, True, 0), (1, 2, 2, 150, 700, 16, True, True, 90),
+    (1, 2, 2, 97, 500, 64, False, False, 0), (1, 3, 1, 300, 300, 128, True, False, 64), (8, 24, 24, 129, 129, 16, True, False, 0),
+]
+
+
+@pytest.mark.parametrize("case", FP32_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-c%d-d%d-w%d" % c)
+def test_fp32_launch_forms(case):
+    from tests.test_gpu_parity import _run_case
+    B, H, Hk, M, N, D, causal, doc, window = case
+    _run_case(B, H, Hk, M, N, D, torch.float32, causal, doc, seed=3, window=window, tol_o=2e-4, tol_lse=2e-4)

@@ -24,6 +24,12 @@
 // rows first, then global rows: a tile of local rows meets the keys of its own documents only),
 // rows are gathered through the permutation, causal terms use the diagonal positions the plan
 // stored, and tiles that the plan's summaries rule out for the whole workgroup are not loaded.
+//
+// NARROW form, for launches that leave CUs idle: a wave's chain of fp32 MFMAs is what such a launch waits for (a
+// 32 x 32 block costs 64 clocks per MFMA, 4096 of them in the forward at D = 64), so the four waves of a workgroup
+// own the SAME 32 rows (or keys) and each takes a quarter of every streamed tile of 128; their sums are added up
+// once, through LDS.  Four times the workgroups, a quarter of the chain: 2 x 4 heads x 512 rows with documents,
+// D = 64: see kNarrowWgs.
 #include "fa_tile.h"
 
 namespace fa {
@@ -31,15 +37,17 @@ namespace {
 
 FA_DEV f32x16 mfma_f32(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 
-constexpr int kRows = 32;       // rows of a streamed tile
+constexpr int kRows = 32;       // rows of a block: what a wave works on at a time
 constexpr int kThreads = 256;
+template <bool NARROW> constexpr int kTileRows = NARROW ? 128 : kRows;   // rows of a streamed tile
+template <bool NARROW> constexpr int kOwnRows = NARROW ? kRows : 128;    // rows (or keys) of a workgroup
 
-// A [32 x D] tile on its way from global memory to LDS, held in registers in between.
-template <int D>
+// A [R x D] tile on its way from global memory to LDS, held in registers in between.
+template <int D, int R>
 struct TileRegs {
-  static constexpr int C4 = D / 4, N4 = kRows * C4, PER = (N4 + kThreads - 1) / kThreads;
+  static constexpr int C4 = D / 4, N4 = R * C4, PER = (N4 + kThreads - 1) / kThreads;
   f32x4 v[PER];
-  // rows row0 .. row0+31 of a matrix with `nrows` rows; rows past the end read as zero
+  // rows row0 .. row0+R-1 of a matrix with `nrows` rows; rows past the end read as zero
   FA_DEV void load(const float* base, int64_t rs, int row0, int nrows) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -50,7 +58,7 @@ struct TileRegs {
       v[i] = ok ? *reinterpret_cast<const f32x4*>(base + int64_t(row0 + r) * rs + 4 * c4) : z;
     }
   }
-  // the same for a tile whose rows are rows[0..31] of the matrix (-1: no row, reads as zero)
+  // the same for a tile whose rows are rows[0..R-1] of the matrix (-1: no row, reads as zero)
   FA_DEV void load_rows(const float* base, int64_t rs, const int* rows) {
     int ri[PER];
 #pragma unroll
@@ -125,13 +133,22 @@ FA_DEV void wg_reduce3(int& lo, int& hi, int& glob) {
   glob = red[2] | red[5] | red[8] | red[11];
 }
 
-template <int D>
-constexpr size_t lds_bytes() { return size_t(2 * kRows * (D + 1) + 4 * kRows + 64) * 4; }
+template <int D, bool NARROW>
+constexpr size_t lds_bytes() {
+  constexpr size_t tiles = size_t(2 * kTileRows<NARROW> * (D + 1) + 4 * kTileRows<NARROW> + 64) * 4;
+  constexpr size_t sums = NARROW ? size_t(4 * 32 * ((D + 31) / 32) * 64) * 4 : 0;   // the waves' accumulators side by side (dk/dv: the most)
+  return tiles > sums ? tiles : sums;
+}
+
+// NARROW form: the four waves' values of `n` accumulator registers side by side in LDS (which the tile stream no
+// longer needs); wave w then adds up the registers 4 * w .. + 3 of every group of 16.
+FA_DEV void narrow_put(float* lds, int n, int i, float v) { lds[((threadIdx.x >> 6) * n + i) * 64 + (threadIdx.x & 63)] = v; }
+FA_DEV float narrow_get(const float* lds, int n, int w, int i) { return lds[(w * n + i) * 64 + (threadIdx.x & 63)]; }
 
 // Query side of the forward and dq kernels: which row a lane owns, its id, its causal limits, what
 // its wave and its workgroup can see.  Without ids: natural order.  With ids: tile `tile` of the
 // permuted order of the mask plan; the diagonal of a row sits at the position the plan stored.
-template <bool CAUSAL, bool DOC>
+template <bool CAUSAL, bool DOC, bool NARROW>
 struct QSideF32 {
   int row, rowc;        // the lane's row (-1: none), clamped for loads
   bool live;
@@ -142,20 +159,21 @@ struct QSideF32 {
   bool w_any;           // the wave holds a row
   int w_lo, w_hi, w_glob;
   int g_lo, g_hi, g_glob;
-  int kt0, nkt;         // key tiles (of kRows) the workgroup walks: [kt0, nkt)
+  int kt0, nkt;         // key tiles (of kTileRows) the workgroup walks: [kt0, nkt)
   // returns false when the tile holds no row at all (uniform over the workgroup)
   FA_DEV bool init(const KArgs& a, int b, int h, int tile, int wave, int lq) {
+    constexpr int TR = kTileRows<NARROW>, OWN = kOwnRows<NARROW>;
     int posc, g_pmin, g_pmax, kfirst = 0, klast = 0x3fffffff;
     if (!DOC) {
-      const int m0 = tile * 128, mw = m0 + wave * 32;
+      const int m0 = tile * OWN, mw = NARROW ? m0 : m0 + wave * 32;
       row = mw + lq < a.M ? mw + lq : -1;
       posc = a.gap + min(mw + lq, a.M - 1);
       eq_i = 0;
-      g_pmin = a.gap + m0; g_pmax = a.gap + min(m0 + 127, a.M - 1);
+      g_pmin = a.gap + m0; g_pmax = a.gap + min(m0 + OWN - 1, a.M - 1);
     } else {
-      const IdSummary* qs = a.qsum + b * a.qs_bs + h * a.qs_hs + 2 * tile;
-      const IdSummary s0 = qs[0], s1 = qs[1];
-      const int64_t pi = b * a.pm_bs + h * a.pm_hs + tile * 128 + wave * 32 + lq;
+      const IdSummary* qs = a.qsum + b * a.qs_bs + h * a.qs_hs + (NARROW ? tile / 2 : 2 * tile);
+      const IdSummary s0 = qs[0], s1 = qs[NARROW ? 0 : 1];   // (32 rows: the summary of the 64 they are part of)
+      const int64_t pi = b * a.pm_bs + h * a.pm_hs + tile * OWN + (NARROW ? 0 : wave * 32) + lq;
       row = a.perm[pi];
       eq_i = a.peq[pi];
       posc = a.ppos[pi];
@@ -170,6 +188,7 @@ struct QSideF32 {
     lim_i = CAUSAL ? min(max(posc, a.pfx_m1), a.N - 1) : a.N - 1;
     low_i = CAUSAL ? posc - a.win + 1 : -0x3fffffff;
     w_any = __builtin_amdgcn_ballot_w64(live) != 0;
+    if (NARROW && !w_any) return false;
     w_lim = half_max(live ? lim_i : -1);
     w_low = half_min(live ? low_i : 0x7fffffff);
     w_lo = 0x7fffffff; w_hi = (int)0x80000000; w_glob = 0;
@@ -181,13 +200,13 @@ struct QSideF32 {
     g_lo = w_lo; g_hi = w_hi; g_glob = w_glob;
     if (DOC) wg_reduce3(g_lo, g_hi, g_glob);
     const int n_end = CAUSAL ? min(a.N, max(g_pmax, a.pfx_m1) + 1) : a.N;
-    kt0 = CAUSAL ? max(0, g_pmin - a.win + 1) / kRows : 0;   // sliding window: first tile any row sees
-    nkt = (n_end + kRows - 1) / kRows;                       // the same for all waves: the tile stream has barriers
+    kt0 = CAUSAL ? max(0, g_pmin - a.win + 1) / TR : 0;   // sliding window: first tile any row sees
+    nkt = (n_end + TR - 1) / TR;                       // the same for all waves: the tile stream has barriers
     if (DOC) {                                               // the plan's key range of these rows (tiles of kSumRows keys)
       if (klast < kfirst) nkt = 0;
       else {
-        kt0 = max(kt0, kfirst * (kSumRows / kRows));
-        nkt = min(nkt, (klast + 1) * (kSumRows / kRows));
+        kt0 = max(kt0, kfirst * kSumRows / TR);
+        nkt = min(nkt, ((klast + 1) * kSumRows + TR - 1) / TR);
       }
     }
     return true;
@@ -196,22 +215,22 @@ struct QSideF32 {
 };
 
 // ---------------------------------------------------------------------------------------------
-template <int D, bool CAUSAL, bool DOC>
+template <int D, bool CAUSAL, bool DOC, bool NARROW>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void fwd_f32_kernel(const KArgs a) {
-  constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32;
+  constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32, TR = kTileRows<NARROW>, OWN = kOwnRows<NARROW>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* lk = reinterpret_cast<float*>(smem);
-  float* lv = lk + kRows * RS;
-  int* lid = reinterpret_cast<int*>(lv + kRows * RS);
+  float* lv = lk + TR * RS;
+  int* lid = reinterpret_cast<int*>(lv + TR * RS);
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = lane & 31, g = lane >> 5;
   const int BH = a.B * a.H;
-  const int nQt = DOC ? a.Pp / 128 : (a.M + 127) / 128;
+  const int nQt = DOC ? a.Pp / OWN : (a.M + OWN - 1) / OWN;
   const int tile = nQt - 1 - blockIdx.x / BH;   // the last rows see the most keys (with ids: the global rows): first
   const int bh = blockIdx.x % BH, b = bh / a.H, h = bh % a.H, hk = h / a.G;
-  QSideF32<CAUSAL, DOC> qc;
+  QSideF32<CAUSAL, DOC, NARROW> qc;
   if (!qc.init(a, b, h, tile, wave, lq)) return;
   const int row = qc.row, rowc = qc.rowc;
 
@@ -242,7 +261,11 @@ void fwd_f32_kernel(const KArgs a) {
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;   // running reference point (scaled) and this lane's partial row sum
 
-  TileRegs<D> rk, rv;
+  // this wave's part of a tile: all of it, or (NARROW) its 32 rows
+  const float* lkw = lk + (NARROW ? wave * kRows * RS : 0);
+  const float* lvw = lv + (NARROW ? wave * kRows * RS : 0);
+  const int* lidw = lid + (NARROW ? wave * kRows : 0);
+  TileRegs<D, TR> rk, rv;
   int rid = 0;
   // With ids, key tiles that no row of the workgroup can see (by the 64-key summaries of the mask
   // plan) are not even loaded: a packed batch costs its block diagonal, not the whole triangle.
@@ -251,7 +274,7 @@ void fwd_f32_kernel(const KArgs a) {
   // block mask: the byte rows of the workgroup's two 64-row halves (the second one may lie past the last row)
   const unsigned char* bm0 = nullptr;
   const unsigned char* bm1 = nullptr;
-  if (!DOC && a.bmask != nullptr) {
+  if (!DOC && !NARROW && a.bmask != nullptr) {
     const unsigned char* base = a.bmask + b * a.bm_bs + h * a.bm_hs;
     bm0 = base + int64_t(2 * tile) * a.bm_rs;
     if (2 * tile + 1 < a.nBr) bm1 = base + int64_t(2 * tile + 1) * a.bm_rs;
@@ -259,13 +282,18 @@ void fwd_f32_kernel(const KArgs a) {
   auto next_kt = [&](int kt) {
     if (DOC)
       while (kt < nkt) {
-        const IdSummary ks = ksum[(kt * kRows) / kSumRows];
+        const int j = (kt * TR) / kSumRows;
+        const IdSummary ks = ksum[j];
         if (doc_may_keep(g_lo, g_hi, g_glob, ks.lo, ks.hi)) break;
+        if (TR > kSumRows && j + 1 < a.nKs) {
+          const IdSummary k2 = ksum[j + 1];
+          if (doc_may_keep(g_lo, g_hi, g_glob, k2.lo, k2.hi)) break;
+        }
         ++kt;
       }
     if (!DOC && bm0 != nullptr)
       while (kt < nkt) {   // tiles whose block is off for both halves are not even loaded
-        const int col = (kt * kRows) / FA_MASK_BLOCK;
+        const int col = (kt * TR) / FA_MASK_BLOCK;
         if ((bm0[col] | (bm1 != nullptr ? bm1[col] : 0)) != 0) break;
         ++kt;
       }
@@ -273,23 +301,23 @@ void fwd_f32_kernel(const KArgs a) {
   };
   int kt = next_kt(kt0);
   if (kt < nkt) {
-    rk.load(kp, a.k_rs, kt * kRows, a.N);
-    rv.load(vp, a.v_rs, kt * kRows, a.N);
-    if (DOC && threadIdx.x < kRows) rid = ekp[min(kt * kRows + (int)threadIdx.x, a.N - 1)];
+    rk.load(kp, a.k_rs, kt * TR, a.N);
+    rv.load(vp, a.v_rs, kt * TR, a.N);
+    if (DOC && threadIdx.x < TR) rid = ekp[min(kt * TR + (int)threadIdx.x, a.N - 1)];
   }
 
   while (kt < nkt) {
-    const int n0 = kt * kRows;
+    const int n0 = kt * TR + (NARROW ? wave * kRows : 0);   // first key of this wave's part
     const int kt_next = next_kt(kt + 1);
     __syncthreads();   // the previous tile is no longer read
     rk.store(lk);
     rv.store(lv);
-    if (DOC && threadIdx.x < kRows) lid[threadIdx.x] = rid;
+    if (DOC && threadIdx.x < TR) lid[threadIdx.x] = rid;
     __syncthreads();
     if (kt_next < nkt) {   // the next tile travels while this one is used
-      rk.load(kp, a.k_rs, kt_next * kRows, a.N);
-      rv.load(vp, a.v_rs, kt_next * kRows, a.N);
-      if (DOC && threadIdx.x < kRows) rid = ekp[min(kt_next * kRows + (int)threadIdx.x, a.N - 1)];
+      rk.load(kp, a.k_rs, kt_next * TR, a.N);
+      rv.load(vp, a.v_rs, kt_next * TR, a.N);
+      if (DOC && threadIdx.x < TR) rid = ekp[min(kt_next * TR + (int)threadIdx.x, a.N - 1)];
     }
     kt = kt_next;
     bool skip = qc.skips(n0);
@@ -299,7 +327,7 @@ void fwd_f32_kernel(const KArgs a) {
     }
     if (DOC && !skip) {
       const bool kv = n0 + lq < a.N;
-      const int id = lid[lq];
+      const int id = lidw[lq];
       const int k_lo = half_min(kv ? id : 0x7fffffff), k_hi = half_max(kv ? id : (int)0x80000000);
       skip = !doc_may_keep(w_lo, w_hi, w_glob, k_lo, k_hi);
     }
@@ -308,10 +336,10 @@ void fwd_f32_kernel(const KArgs a) {
     f32x16 s;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
-    pipelined<KS2, kChunk>([&](int i) __attribute__((always_inline)) { return lk[lq * RS + 2 * i + g]; },
+    pipelined<KS2, kChunk>([&](int i) __attribute__((always_inline)) { return lkw[lq * RS + 2 * i + g]; },
                            [&](int i, float x) __attribute__((always_inline)) { s = mfma_f32(x, qreg[i], s); });
     mask_lim(s, lim_i - n0 - 4 * g, low_i - n0 - 4 * g, -INFINITY);
-    if (DOC) mask_doc(s, reinterpret_cast<const char*>(lid) + g * 16, eq_i, glob_i, -INFINITY);
+    if (DOC) mask_doc(s, reinterpret_cast<const char*>(lidw) + g * 16, eq_i, glob_i, -INFINITY);
 
     float mx = s[0];
 #pragma unroll
@@ -336,12 +364,50 @@ void fwd_f32_kernel(const KArgs a) {
     pipelined<16 * DBN, kChunk>(
         [&](int i) __attribute__((always_inline)) {
           const int r = i % 16, key = 8 * (r >> 2) + 4 * g + (r & 3);
-          return lv[key * RS + 32 * (i / 16) + lq];
+          return lvw[key * RS + 32 * (i / 16) + lq];
         },
         [&](int i, float x) __attribute__((always_inline)) { o[i / 16] = mfma_f32(x, s[i % 16], o[i / 16]); });
   }
 
-  const float l_tot = xhalf_sum(l_run);
+  float l_tot = xhalf_sum(l_run);
+  if (NARROW) {   // the four waves saw a quarter of the keys each: one state out of four
+    constexpr int NV = 16 * DBN;
+    float* mb = reinterpret_cast<float*>(smem);
+    __syncthreads();   // nobody reads tiles any more
+    narrow_put(mb, 2, 0, m_run);
+    narrow_put(mb, 2, 1, l_tot);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) narrow_put(mb + 512, NV, i, o[i / 16][i % 16]);
+    __syncthreads();
+    float w_[4];
+    l_tot = 0.f;
+    m_run = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m_run = fmaxf(m_run, narrow_get(mb, 2, w, 0));
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float mw = narrow_get(mb, 2, w, 0);
+      w_[w] = mw == -INFINITY ? 0.f : fast_exp2(mw - m_run);
+      l_tot += w_[w] * narrow_get(mb, 2, w, 1);
+    }
+    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    if (row >= 0) {
+      float* op = reinterpret_cast<float*>(a.o) + b * a.o_bs + h * a.o_hs + int64_t(row) * a.o_rs;
+#pragma unroll
+      for (int db = 0; db < DBN; ++db) {
+        const int d0 = 32 * db + 8 * wave + 4 * g;
+        if (d0 >= D) continue;
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) x[t] += w_[w] * narrow_get(mb + 512, NV, w, 16 * db + 4 * wave + t);
+        *reinterpret_cast<f32x4*>(op + d0) = f32x4{x[0] * inv, x[1] * inv, x[2] * inv, x[3] * inv};
+      }
+      if (g == 0 && wave == 0) a.lse[(int64_t(b) * a.H + h) * a.M + row] = l_tot > 0.f ? m_run + fast_log2(l_tot) : -INFINITY;
+    }
+    return;
+  }
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if (row >= 0) {
     float* op = reinterpret_cast<float*>(a.o) + b * a.o_bs + h * a.o_hs + int64_t(row) * a.o_rs;
@@ -359,22 +425,22 @@ void fwd_f32_kernel(const KArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-template <int D, bool CAUSAL, bool DOC>
+template <int D, bool CAUSAL, bool DOC, bool NARROW>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void dq_f32_kernel(const KArgs a) {
-  constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32;
+  constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32, TR = kTileRows<NARROW>, OWN = kOwnRows<NARROW>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* lk = reinterpret_cast<float*>(smem);
-  float* lv = lk + kRows * RS;
-  int* lid = reinterpret_cast<int*>(lv + kRows * RS);
+  float* lv = lk + TR * RS;
+  int* lid = reinterpret_cast<int*>(lv + TR * RS);
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = lane & 31, g = lane >> 5;
   const int BH = a.B * a.H;
-  const int nQt = DOC ? a.Pp / 128 : (a.M + 127) / 128;
+  const int nQt = DOC ? a.Pp / OWN : (a.M + OWN - 1) / OWN;
   const int tile = nQt - 1 - blockIdx.x / BH;
   const int bh = blockIdx.x % BH, b = bh / a.H, h = bh % a.H, hk = h / a.G;
-  QSideF32<CAUSAL, DOC> qc;
+  QSideF32<CAUSAL, DOC, NARROW> qc;
   if (!qc.init(a, b, h, tile, wave, lq)) return;
   const int row = qc.row, rowc = qc.rowc;
 
@@ -397,7 +463,7 @@ void dq_f32_kernel(const KArgs a) {
 #pragma unroll
     for (int s = 0; s < KS2; ++s) part += op[2 * s + g] * doreg[s];
     delta_i = xhalf_sum(part);
-    if (row >= 0 && g == 0) a.delta[(int64_t(b) * a.H + h) * a.M + row] = delta_i;
+    if (row >= 0 && g == 0 && (!NARROW || wave == 0)) a.delta[(int64_t(b) * a.H + h) * a.M + row] = delta_i;
   } else {
     delta_i = a.delta[(int64_t(b) * a.H + h) * a.M + rowc];
   }
@@ -413,7 +479,11 @@ void dq_f32_kernel(const KArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
 
-  TileRegs<D> rk, rv;
+  // this wave's part of a tile: all of it, or (NARROW) its 32 rows
+  const float* lkw = lk + (NARROW ? wave * kRows * RS : 0);
+  const float* lvw = lv + (NARROW ? wave * kRows * RS : 0);
+  const int* lidw = lid + (NARROW ? wave * kRows : 0);
+  TileRegs<D, TR> rk, rv;
   int rid = 0;
   // With ids, key tiles that no row of the workgroup can see (by the 64-key summaries of the mask
   // plan) are not even loaded: a packed batch costs its block diagonal, not the whole triangle.
@@ -422,7 +492,7 @@ void dq_f32_kernel(const KArgs a) {
   // block mask: the byte rows of the workgroup's two 64-row halves (the second one may lie past the last row)
   const unsigned char* bm0 = nullptr;
   const unsigned char* bm1 = nullptr;
-  if (!DOC && a.bmask != nullptr) {
+  if (!DOC && !NARROW && a.bmask != nullptr) {
     const unsigned char* base = a.bmask + b * a.bm_bs + h * a.bm_hs;
     bm0 = base + int64_t(2 * tile) * a.bm_rs;
     if (2 * tile + 1 < a.nBr) bm1 = base + int64_t(2 * tile + 1) * a.bm_rs;
@@ -430,13 +500,18 @@ void dq_f32_kernel(const KArgs a) {
   auto next_kt = [&](int kt) {
     if (DOC)
       while (kt < nkt) {
-        const IdSummary ks = ksum[(kt * kRows) / kSumRows];
+        const int j = (kt * TR) / kSumRows;
+        const IdSummary ks = ksum[j];
         if (doc_may_keep(g_lo, g_hi, g_glob, ks.lo, ks.hi)) break;
+        if (TR > kSumRows && j + 1 < a.nKs) {
+          const IdSummary k2 = ksum[j + 1];
+          if (doc_may_keep(g_lo, g_hi, g_glob, k2.lo, k2.hi)) break;
+        }
         ++kt;
       }
     if (!DOC && bm0 != nullptr)
       while (kt < nkt) {   // tiles whose block is off for both halves are not even loaded
-        const int col = (kt * kRows) / FA_MASK_BLOCK;
+        const int col = (kt * TR) / FA_MASK_BLOCK;
         if ((bm0[col] | (bm1 != nullptr ? bm1[col] : 0)) != 0) break;
         ++kt;
       }
@@ -444,23 +519,23 @@ void dq_f32_kernel(const KArgs a) {
   };
   int kt = next_kt(kt0);
   if (kt < nkt) {
-    rk.load(kp, a.k_rs, kt * kRows, a.N);
-    rv.load(vp, a.v_rs, kt * kRows, a.N);
-    if (DOC && threadIdx.x < kRows) rid = ekp[min(kt * kRows + (int)threadIdx.x, a.N - 1)];
+    rk.load(kp, a.k_rs, kt * TR, a.N);
+    rv.load(vp, a.v_rs, kt * TR, a.N);
+    if (DOC && threadIdx.x < TR) rid = ekp[min(kt * TR + (int)threadIdx.x, a.N - 1)];
   }
 
   while (kt < nkt) {
-    const int n0 = kt * kRows;
+    const int n0 = kt * TR + (NARROW ? wave * kRows : 0);   // first key of this wave's part
     const int kt_next = next_kt(kt + 1);
     __syncthreads();
     rk.store(lk);
     rv.store(lv);
-    if (DOC && threadIdx.x < kRows) lid[threadIdx.x] = rid;
+    if (DOC && threadIdx.x < TR) lid[threadIdx.x] = rid;
     __syncthreads();
     if (kt_next < nkt) {
-      rk.load(kp, a.k_rs, kt_next * kRows, a.N);
-      rv.load(vp, a.v_rs, kt_next * kRows, a.N);
-      if (DOC && threadIdx.x < kRows) rid = ekp[min(kt_next * kRows + (int)threadIdx.x, a.N - 1)];
+      rk.load(kp, a.k_rs, kt_next * TR, a.N);
+      rv.load(vp, a.v_rs, kt_next * TR, a.N);
+      if (DOC && threadIdx.x < TR) rid = ekp[min(kt_next * TR + (int)threadIdx.x, a.N - 1)];
     }
     kt = kt_next;
     bool skip = qc.skips(n0);
@@ -470,7 +545,7 @@ void dq_f32_kernel(const KArgs a) {
     }
     if (DOC && !skip) {
       const bool kv = n0 + lq < a.N;
-      const int id = lid[lq];
+      const int id = lidw[lq];
       const int k_lo = half_min(kv ? id : 0x7fffffff), k_hi = half_max(kv ? id : (int)0x80000000);
       skip = !doc_may_keep(w_lo, w_hi, w_glob, k_lo, k_hi);
     }
@@ -480,7 +555,7 @@ void dq_f32_kernel(const KArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
     pipelined<2 * KS2, kChunk>(
-        [&](int i) __attribute__((always_inline)) { return ((i & 1) ? lv : lk)[lq * RS + 2 * (i / 2) + g]; },
+        [&](int i) __attribute__((always_inline)) { return ((i & 1) ? lvw : lkw)[lq * RS + 2 * (i / 2) + g]; },
         [&](int i, float x) __attribute__((always_inline)) {
           if (i & 1) dp = mfma_f32(x, doreg[i / 2], dp);
           else s = mfma_f32(x, qreg[i / 2], s);
@@ -489,16 +564,39 @@ void dq_f32_kernel(const KArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = fast_exp2(__builtin_fmaf(s[r], c, -L_i)) * (dp[r] - delta_i);
     mask_lim(s, lim_i - n0 - 4 * g, low_i - n0 - 4 * g, 0.f);
-    if (DOC) mask_doc(s, reinterpret_cast<const char*>(lid) + g * 16, eq_i, glob_i, 0.f);
+    if (DOC) mask_doc(s, reinterpret_cast<const char*>(lidw) + g * 16, eq_i, glob_i, 0.f);
     // dQ^T += K^T dS^T
     pipelined<16 * DBN, kChunk>(
         [&](int i) __attribute__((always_inline)) {
           const int r = i % 16, key = 8 * (r >> 2) + 4 * g + (r & 3);
-          return lk[key * RS + 32 * (i / 16) + lq];
+          return lkw[key * RS + 32 * (i / 16) + lq];
         },
         [&](int i, float x) __attribute__((always_inline)) { acc[i / 16] = mfma_f32(x, s[i % 16], acc[i / 16]); });
   }
 
+  if (NARROW) {
+    constexpr int NV = 16 * DBN;
+    float* mb = reinterpret_cast<float*>(smem);
+    __syncthreads();   // nobody reads tiles any more
+#pragma unroll
+    for (int i = 0; i < NV; ++i) narrow_put(mb, NV, i, acc[i / 16][i % 16]);
+    __syncthreads();
+    if (row >= 0) {
+      float* dqp = reinterpret_cast<float*>(a.dq) + b * a.dq_bs + h * a.dq_hs + int64_t(row) * a.dq_rs;
+#pragma unroll
+      for (int db = 0; db < DBN; ++db) {
+        const int d0 = 32 * db + 8 * wave + 4 * g;
+        if (d0 >= D) continue;
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) x[t] += narrow_get(mb, NV, w, 16 * db + 4 * wave + t);
+        *reinterpret_cast<f32x4*>(dqp + d0) = f32x4{x[0] * a.scale, x[1] * a.scale, x[2] * a.scale, x[3] * a.scale};
+      }
+    }
+    return;
+  }
   if (row >= 0) {
     float* dqp = reinterpret_cast<float*>(a.dq) + b * a.dq_bs + h * a.dq_hs + int64_t(row) * a.dq_rs;
 #pragma unroll
@@ -515,23 +613,29 @@ void dq_f32_kernel(const KArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-template <int D, bool CAUSAL, bool DOC>
+template <int D, bool CAUSAL, bool DOC, bool NARROW>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void dkdv_f32_kernel(const KArgs a) {
-  constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32;
+  constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32, TR = kTileRows<NARROW>, OWN = kOwnRows<NARROW>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* lqt = reinterpret_cast<float*>(smem);
-  float* ldo = lqt + kRows * RS;
-  float* laux = ldo + kRows * RS;               // [LSE | delta | eq | row name] x 32
-  const int* leq = reinterpret_cast<const int*>(laux + 2 * kRows);
-  const int* lnm = reinterpret_cast<const int*>(laux + 3 * kRows);
+  float* ldo = lqt + TR * RS;
+  float* laux = ldo + TR * RS;                  // [LSE | delta | eq | row name] x TR
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = lane & 31, g = lane >> 5;
   const int BHk = a.B * a.Hk;
   const int kt = blockIdx.x / BHk;               // causal: the first keys are seen by the most rows: first
   const int bhk = blockIdx.x % BHk, b = bhk / a.Hk, hk = bhk % a.Hk;
-  const int n0 = kt * 128, nw = n0 + wave * 32;
+  const int n0 = kt * OWN, nw = NARROW ? n0 : n0 + wave * 32;
+  // this wave's part of a query tile: all of it, or (NARROW) its 32 rows
+  const int part = NARROW ? wave * kRows : 0;
+  const float* lqtw = lqt + part * RS;
+  const float* ldow = ldo + part * RS;
+  const float* llse = laux + part;
+  const float* ldel = laux + TR + part;
+  const int* leq = reinterpret_cast<const int*>(laux + 2 * TR) + part;
+  const int* lnm = reinterpret_cast<const int*>(laux + 3 * TR) + part;
   const int key = nw + lq, keyc = min(key, a.N - 1);
 
   const float* kp = reinterpret_cast<const float*>(a.k) + b * a.k_bs + hk * a.k_hs + int64_t(keyc) * a.k_rs;
@@ -549,10 +653,10 @@ void dkdv_f32_kernel(const KArgs a) {
   const int row_lo = CAUSAL ? (key <= a.pfx_m1 ? 0 : max(0, key - gk)) : 0;
   const int row_hi = CAUSAL ? min(rcap, key - gk + a.win - 1) : rcap;
   const unsigned row_span = (key < a.N && row_hi >= row_lo) ? (unsigned)(row_hi - row_lo + 1) : 0u;
-  const int wg_rhi = CAUSAL ? min(rcap, n0 + 127 - gk + a.win - 1) : rcap;   // last name that sees a key of the workgroup
-  // query tiles of 32 rows: natural order from the diagonal on, or every tile of the permuted order
-  const int mt0 = DOC ? 0 : (CAUSAL ? (n0 <= a.pfx_m1 ? 0 : max(0, n0 - gk) / kRows) : 0);
-  const int nMt = DOC ? a.Pp / kRows : max(0, wg_rhi + kRows) / kRows;
+  const int wg_rhi = CAUSAL ? min(rcap, n0 + OWN - 1 - gk + a.win - 1) : rcap;   // last name that sees a key of the workgroup
+  // query tiles of TR rows: natural order from the diagonal on, or every tile of the permuted order
+  const int mt0 = DOC ? 0 : (CAUSAL ? (n0 <= a.pfx_m1 ? 0 : max(0, n0 - gk) / TR) : 0);
+  const int nMt = DOC ? a.Pp / TR : max(0, wg_rhi + TR) / TR;
 
   f32x16 dv[DBN], dk[DBN];
 #pragma unroll
@@ -575,18 +679,18 @@ void dkdv_f32_kernel(const KArgs a) {
       wk_lo = half_min(key < a.N ? ek_j : 0x7fffffff);
       wk_hi = half_max(key < a.N ? ek_j : (int)0x80000000);
     }
-    // one auxiliary value per thread of the first four groups of 32: LSE, delta, id, name of a tile row
-    auto aux_load = [&](int mt) -> float {
-      const int t = threadIdx.x & 31, which = threadIdx.x >> 5;
+    // the auxiliary values of a tile (LSE, delta, id, name of every row): number i of 4 * TR
+    auto aux_load = [&](int mt, int i) -> float {
+      const int t = i % TR, which = i / TR;
       if (!DOC) {
-        const int r = mt * kRows + t, rc = min(r, a.M - 1);
+        const int r = mt * TR + t, rc = min(r, a.M - 1);
         if (which == 0) return lsep[rc];
         if (which == 1) return delp[rc];
         return 0.f;
       }
-      if (which == 2) return __int_as_float(pqp[mt * kRows + t]);
-      if (which == 3) return __int_as_float(ppp[mt * kRows + t]);
-      const int r = max(pmp[mt * kRows + t], 0);
+      if (which == 2) return __int_as_float(pqp[mt * TR + t]);
+      if (which == 3) return __int_as_float(ppp[mt * TR + t]);
+      const int r = max(pmp[mt * TR + t], 0);
       return which == 0 ? lsep[r] : delp[r];
     };
     // With ids: query tiles whose 64-entry summary of the plan excludes every key of the workgroup
@@ -598,36 +702,42 @@ void dkdv_f32_kernel(const KArgs a) {
       qsum = a.qsum + b * a.qs_bs + h * a.qs_hs;
     }
     // block mask: the one or two byte columns of the workgroup's 128 keys
-    const unsigned char* bmc = (!DOC && a.bmask != nullptr) ? a.bmask + b * a.bm_bs + h * a.bm_hs + n0 / FA_MASK_BLOCK : nullptr;
+    const unsigned char* bmc = (!DOC && !NARROW && a.bmask != nullptr) ? a.bmask + b * a.bm_bs + h * a.bm_hs + n0 / FA_MASK_BLOCK : nullptr;
     const bool bm_two = n0 / FA_MASK_BLOCK + 1 < a.nBc;
     auto next_mt = [&](int mt) {
       if (DOC)
         while (mt < nMt) {
-          const IdSummary qs = qsum[(mt * kRows) / kSumRows];
-          const bool out = qs.nvalid == 0 || !doc_may_keep(qs.lo, qs.hi, qs.glob, gk_lo, gk_hi) ||
-                           (CAUSAL && ((qs.rmax < n0 && n0 > a.pfx_m1) || qs.rmin > wg_rhi));
-          if (!out) break;
+          auto out = [&](const IdSummary& qs) {
+            return qs.nvalid == 0 || !doc_may_keep(qs.lo, qs.hi, qs.glob, gk_lo, gk_hi) ||
+                   (CAUSAL && ((qs.rmax < n0 && n0 > a.pfx_m1) || qs.rmin > wg_rhi));
+          };
+          const int j = (mt * TR) / kSumRows;
+          if (!out(qsum[j])) break;
+          if (TR > kSumRows && !out(qsum[j + 1])) break;   // (the permuted order is a multiple of 256 entries)
           ++mt;
         }
       if (bmc != nullptr)
         while (mt < nMt) {   // tiles whose block is off for both key columns are not even loaded
-          const unsigned char* r = bmc + int64_t((mt * kRows) / FA_MASK_BLOCK) * a.bm_rs;
+          const unsigned char* r = bmc + int64_t((mt * TR) / FA_MASK_BLOCK) * a.bm_rs;
           if ((r[0] | (bm_two ? r[1] : 0)) != 0) break;
           ++mt;
         }
       return mt;
     };
-    TileRegs<D> rq, rdo;
-    float raux = 0.f;
+    TileRegs<D, TR> rq, rdo;
+    constexpr int NAUX = (4 * TR + kThreads - 1) / kThreads;
+    float raux[NAUX] = {};
     auto load_tile = [&](int mt) {
       if (DOC) {
-        rq.load_rows(qp, a.q_rs, pmp + mt * kRows);
-        rdo.load_rows(dop, a.do_rs, pmp + mt * kRows);
+        rq.load_rows(qp, a.q_rs, pmp + mt * TR);
+        rdo.load_rows(dop, a.do_rs, pmp + mt * TR);
       } else {
-        rq.load(qp, a.q_rs, mt * kRows, a.M);
-        rdo.load(dop, a.do_rs, mt * kRows, a.M);
+        rq.load(qp, a.q_rs, mt * TR, a.M);
+        rdo.load(dop, a.do_rs, mt * TR, a.M);
       }
-      if (threadIdx.x < 4 * kRows) raux = aux_load(mt);
+#pragma unroll
+      for (int j = 0; j < NAUX; ++j)
+        if (j * kThreads + threadIdx.x < 4 * TR) raux[j] = aux_load(mt, j * kThreads + threadIdx.x);
     };
     int mt = next_mt(mt0);
     if (mt < nMt) load_tile(mt);
@@ -636,10 +746,12 @@ void dkdv_f32_kernel(const KArgs a) {
       __syncthreads();
       rq.store(lqt);
       rdo.store(ldo);
-      if (threadIdx.x < 4 * kRows) laux[threadIdx.x] = raux;
+#pragma unroll
+      for (int j = 0; j < NAUX; ++j)
+        if (j * kThreads + threadIdx.x < 4 * TR) laux[j * kThreads + threadIdx.x] = raux[j];
       __syncthreads();
       if (mt_next < nMt) load_tile(mt_next);
-      const int m0 = mt * kRows;   // natural order only
+      const int m0 = mt * TR + part;   // natural order only
       mt = mt_next;
       // names of the tile's rows (-1: none): smallest / largest among the 32
       const int nm = DOC ? lnm[lq] : (m0 + lq < a.M ? m0 + lq : -1);
@@ -663,7 +775,7 @@ void dkdv_f32_kernel(const KArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) { x[r] = 0.f; dp[r] = 0.f; }
       pipelined<2 * KS2, kChunk>(
-          [&](int i) __attribute__((always_inline)) { return ((i & 1) ? ldo : lqt)[lq * RS + 2 * (i / 2) + g]; },
+          [&](int i) __attribute__((always_inline)) { return ((i & 1) ? ldow : lqtw)[lq * RS + 2 * (i / 2) + g]; },
           [&](int i, float v_) __attribute__((always_inline)) {
             if (i & 1) dp = mfma_f32(v_, vreg[i / 2], dp);
             else x = mfma_f32(v_, kreg[i / 2], x);
@@ -672,8 +784,8 @@ void dkdv_f32_kernel(const KArgs a) {
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
         const int i0 = 8 * q4 + 4 * g;
-        const f32x4 Lv = *reinterpret_cast<const f32x4*>(laux + i0);
-        const f32x4 dl = *reinterpret_cast<const f32x4*>(laux + kRows + i0);
+        const f32x4 Lv = *reinterpret_cast<const f32x4*>(llse + i0);
+        const f32x4 dl = *reinterpret_cast<const f32x4*>(ldel + i0);
         const i32x4 eqv = *reinterpret_cast<const i32x4*>(leq + i0);
         i32x4 nmv = {m0 + i0, m0 + i0 + 1, m0 + i0 + 2, m0 + i0 + 3};   // rows past the end lie beyond every span
         if (DOC) nmv = *reinterpret_cast<const i32x4*>(lnm + i0);
@@ -690,7 +802,7 @@ void dkdv_f32_kernel(const KArgs a) {
       pipelined<32 * DBN, kChunk>(
           [&](int i) __attribute__((always_inline)) {
             const int r = (i / 2) % 16, qr = 8 * (r >> 2) + 4 * g + (r & 3);
-            return ((i & 1) ? lqt : ldo)[qr * RS + 32 * (i / 32) + lq];
+            return ((i & 1) ? lqtw : ldow)[qr * RS + 32 * (i / 32) + lq];
           },
           [&](int i, float v_) __attribute__((always_inline)) {
             const int r = (i / 2) % 16, db = i / 32;
@@ -700,6 +812,31 @@ void dkdv_f32_kernel(const KArgs a) {
     }
   }
 
+  if (NARROW) {
+    constexpr int NV = 32 * DBN;
+    float* mb = reinterpret_cast<float*>(smem);
+    __syncthreads();   // nobody reads tiles any more
+#pragma unroll
+    for (int i = 0; i < NV; ++i) narrow_put(mb, NV, i, i < NV / 2 ? dv[(i / 16) % DBN][i % 16] : dk[(i / 16) % DBN][i % 16]);
+    __syncthreads();
+    if (key < a.N) {
+#pragma unroll
+      for (int i = 0; i < 2 * DBN; ++i) {   // dV's groups of 16 registers, then dK's
+        const int d0 = 32 * (i % DBN) + 8 * wave + 4 * g;
+        if (d0 >= D) continue;
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) x[t] += narrow_get(mb, NV, w, 16 * i + 4 * wave + t);
+        float* p = i < DBN ? reinterpret_cast<float*>(a.dv) + b * a.dv_bs + hk * a.dv_hs + int64_t(key) * a.dv_rs
+                           : reinterpret_cast<float*>(a.dk) + b * a.dk_bs + hk * a.dk_hs + int64_t(key) * a.dk_rs;
+        const float sc = i < DBN ? 1.f : a.scale;
+        *reinterpret_cast<f32x4*>(p + d0) = f32x4{x[0] * sc, x[1] * sc, x[2] * sc, x[3] * sc};
+      }
+    }
+    return;
+  }
   if (key < a.N) {
     float* dvp = reinterpret_cast<float*>(a.dv) + b * a.dv_bs + hk * a.dv_hs + int64_t(key) * a.dv_rs;
     float* dkp = reinterpret_cast<float*>(a.dk) + b * a.dk_bs + hk * a.dk_hs + int64_t(key) * a.dk_rs;
@@ -743,16 +880,31 @@ __global__ __launch_bounds__(kThreads) void delta_f32_kernel(const KArgs a) {
 
 enum { kFwd, kDq, kDkdv };
 
+// Workgroups of 128 rows (keys) below which the NARROW form is launched: with one workgroup to a CU, it takes four
+// rounds of a quarter of the chain where the other form takes one of all of it.  (Not under a block mask, whose
+// 64 x 64 blocks the tile stream of this form does not follow.)
+constexpr int kNarrowWgs = 192;
+
+template <int WHICH, int D, bool CAUSAL, bool DOC, bool NARROW>
+int launch_form(const KArgs& a, hipStream_t s) {
+  constexpr int OWN = kOwnRows<NARROW>;
+  auto kern = WHICH == kFwd ? fwd_f32_kernel<D, CAUSAL, DOC, NARROW> : WHICH == kDq ? dq_f32_kernel<D, CAUSAL, DOC, NARROW>
+                                                                                    : dkdv_f32_kernel<D, CAUSAL, DOC, NARROW>;
+  // query tiles: of the natural order, or of the mask plan's permuted order with ids
+  const int blocks = WHICH == kDkdv ? ((a.N + OWN - 1) / OWN) * a.B * a.Hk : (DOC ? a.Pp / OWN : (a.M + OWN - 1) / OWN) * a.B * a.H;
+  static bool lds_allowed[64] = {};   // per kernel instantiation and device
+  if (int e = allow_lds(kern, lds_bytes<D, NARROW>(), lds_allowed)) return e;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), (lds_bytes<D, NARROW>()), s, a);
+  return (int)hipGetLastError();
+}
 template <int WHICH, int D, bool CAUSAL, bool DOC>
 int launch_one(const KArgs& a, hipStream_t s) {
-  auto kern = WHICH == kFwd ? fwd_f32_kernel<D, CAUSAL, DOC> : WHICH == kDq ? dq_f32_kernel<D, CAUSAL, DOC>
-                                                                            : dkdv_f32_kernel<D, CAUSAL, DOC>;
-  // query tiles: of the natural order, or of the mask plan's permuted order with ids
-  const int blocks = WHICH == kDkdv ? ((a.N + 127) / 128) * a.B * a.Hk : (DOC ? a.Pp / 128 : (a.M + 127) / 128) * a.B * a.H;
-  static bool lds_allowed[64] = {};   // per kernel instantiation and device
-  if (int e = allow_lds(kern, lds_bytes<D>(), lds_allowed)) return e;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), lds_bytes<D>(), s, a);
-  return (int)hipGetLastError();
+  const int64_t wgs = WHICH == kDkdv ? int64_t((a.N + 127) / 128) * a.B * a.Hk : int64_t((a.M + 127) / 128) * a.B * a.H;
+  // (dk/dv at D = 128: a 128-row tile on its way through registers does not fit next to the operands and sums)
+  if constexpr (WHICH != kDkdv || D <= 64) {
+    if (wgs < kNarrowWgs && a.bmask == nullptr) return launch_form<WHICH, D, CAUSAL, DOC, true>(a, s);
+  }
+  return launch_form<WHICH, D, CAUSAL, DOC, false>(a, s);
 }
 
 template <int WHICH, int D>
