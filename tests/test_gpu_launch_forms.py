@@ -166,3 +166,12 @@ def test_fp32_launch_forms(case):
     from tests.test_gpu_parity import _run_case
     B, H, Hk, M, N, D, causal, doc, window = case
     _run_case(B, H, Hk, M, N, D, torch.float32, causal, doc, seed=3, window=window, tol_o=2e-4, tol_lse=2e-4)
+
+
+@pytest.mark.parametrize("M,N,per_head,id_dtype,qpos", [(1, 1, False, torch.int32, None), (64, 2048, True, torch.int64, None), (1025, 1025, False, torch.int64, None),
+                                                        (2048, 2048, True, torch.int32, None), (2048, 2049, False, torch.int32, None),
+                                                        (333, 1999, False, torch.int32, "random"), (1984, 640, False, torch.int64, "steps")])
+def test_mask_plan_forms(M, N, per_head, id_dtype, qpos):
+    """The one-workgroup plan and the three-launch plan on both sides of the size where one takes over from the other."""
+    from tests.test_gpu_parity import _run_case
+    _run_case(1, 2, 2, M, N, 32, torch.bfloat16, True, True, seed=8, per_head_ids=per_head, id_dtype=id_dtype, qpos=qpos)

@@ -218,6 +218,113 @@ __global__ __launch_bounds__(256) void plan_qsum_kernel(int Pp, int nQs, int nKs
   }
 }
 
+// The whole plan of one (batch, stored head) by one workgroup, for sizes that fit its LDS: the three kernels above in one
+// launch, with barriers in the place of kernel boundaries.  512 rows: 6 us instead of 13 of kernels, and two launches
+// less for the host (4 us each).  From a few thousand rows or keys on, one CU walking the ids takes longer than
+// the boundaries cost (measured with 16 waves: 18 against 15 us at 4096 rows, 53 against 17 at 16384).
+constexpr int kPlanOneMax = 2048;        // rows and keys
+constexpr int kPlanOneThreads = 1024;
+template <bool I64>
+__global__ __launch_bounds__(kPlanOneThreads) void plan_one_kernel(PlanSide k, int nKs, int* __restrict__ ek32, IdSummary* __restrict__ ksum,
+                                                                   PlanSide q, int Pp, int nQs, int* __restrict__ eq32, int* __restrict__ perm,
+                                                                   int* __restrict__ peq, int* __restrict__ ppos, const int* __restrict__ qpos,
+                                                                   int64_t qp_bs, int gap, int causal, int kend_min, QHeader* __restrict__ hdr,
+                                                                   IdSummary* __restrict__ qsum, int* __restrict__ sk_cnt, int n_sk) {
+  constexpr int kMaxPp = kPlanOneMax + kPermAlign, NW = kPlanOneThreads / 64;
+  __shared__ int s_perm[kMaxPp], s_eq[kMaxPp], s_pos[kMaxPp];
+  __shared__ int s_lo[kPlanOneMax / kSumRows], s_hi[kPlanOneMax / kSumRows], s_cnt[kPlanOneMax / 64];
+  __shared__ int s_k0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int h = blockIdx.x, b = blockIdx.y;
+  if (h == 0 && b == 0)   // the arrival counters of the split-key merge start every forward at zero
+    for (int i = tid; i < n_sk; i += kPlanOneThreads) sk_cnt[i] = 0;
+  if (h < k.H1) {
+    const int64_t bh = int64_t(b) * k.H1 + h;
+    for (int t = wave; t < nKs; t += NW) {
+      const int r = t * kSumRows + lane;
+      const bool valid = r < k.L;
+      const int v = valid ? load_id<I64>(k.ids, b * k.s_b + h * k.s_h + int64_t(r) * k.s_r) : 0;
+      ek32[bh * k.Lp + r] = v;
+      const int lo = wave_min(valid ? v : 0x7fffffff), hi = wave_max(valid ? v : (int)0x80000000);
+      if (lane == 0) {
+        IdSummary x;
+        x.lo = lo; x.hi = hi; x.glob = 0; x.rmin = t * kSumRows; x.rmax = min(k.L, (t + 1) * kSumRows) - 1;
+        x.nvalid = x.rmax - x.rmin + 1; x.kfirst = 0; x.klast = 0;
+        ksum[bh * nKs + t] = x;
+        s_lo[t] = lo; s_hi[t] = hi;
+      }
+    }
+  }
+  if (h >= q.H1) return;   // (uniform over the workgroup)
+  const int64_t bh = int64_t(b) * q.H1 + h;
+  const int M = q.L, Mp = q.Lp, nBlk = Mp / 64;
+  for (int i = tid; i < Pp; i += kPlanOneThreads) { s_perm[i] = -1; s_eq[i] = 0; s_pos[i] = -1; }
+  constexpr int PER = kPlanOneMax / kPlanOneThreads;
+  int id[PER];
+  unsigned long long loc[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int r = j * kPlanOneThreads + tid;
+    id[j] = r < M ? load_id<I64>(q.ids, b * q.s_b + h * q.s_h + int64_t(r) * q.s_r) : 0;
+    loc[j] = __builtin_amdgcn_ballot_w64(r < M && id[j] < 0);
+    if (r < Mp) {
+      eq32[bh * Mp + r] = id[j];
+      if (lane == 0) s_cnt[r / 64] = __builtin_popcountll(loc[j]);
+    }
+  }
+  if (tid == 0) s_k0 = 0x7fffffff;
+  __syncthreads();
+  int nL = 0;
+  for (int i = 0; i < nBlk; ++i) nL += s_cnt[i];
+  const int nG = M - nL, nLp = (nL + kPermAlign - 1) / kPermAlign * kPermAlign;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int r = j * kPlanOneThreads + tid;
+    if (r < M) {
+      int before = __builtin_popcountll(loc[j] & ((1ull << lane) - 1ull));   // local rows before this one
+      for (int i = 0; i < r / 64; ++i) before += s_cnt[i];
+      const int pos = id[j] < 0 ? before : nLp + (r - before);
+      s_perm[pos] = r; s_eq[pos] = id[j];
+      s_pos[pos] = qpos != nullptr ? clamp_pos(qpos[b * qp_bs + r]) : gap + r;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < Pp; i += kPlanOneThreads) { perm[bh * Pp + i] = s_perm[i]; peq[bh * Pp + i] = s_eq[i]; ppos[bh * Pp + i] = s_pos[i]; }
+  for (int t = wave; t < nQs; t += NW) {
+    const int i = t * kSumRows + lane;
+    const int v = s_eq[i], ps = s_pos[i];
+    const bool valid = s_perm[i] >= 0, local = valid && v < 0;
+    IdSummary x;
+    x.lo = wave_min(local ? v : 0x7fffffff);
+    x.hi = wave_max(local ? v : (int)0x80000000);
+    x.rmin = wave_min(valid ? ps : 0x7fffffff);
+    x.rmax = wave_max(valid ? ps : -1);
+    x.glob = __builtin_amdgcn_ballot_w64(valid && v >= 0) != 0 ? 1 : 0;
+    x.nvalid = __builtin_popcountll(__builtin_amdgcn_ballot_w64(valid));
+    int kfirst = 0, klast = nKs - 1;
+    if (q.H1 == k.H1) {   // ids of both sides stored per the same heads: narrow the key range
+      const int kend = causal ? min(nKs, max(x.rmax / kSumRows + 1, kend_min)) : nKs;
+      const bool cand = lane < kend && doc_may_keep(x.lo, x.hi, x.glob, s_lo[min(lane, nKs - 1)], s_hi[min(lane, nKs - 1)]);
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(cand);   // (at most 64 key tiles at these sizes)
+      kfirst = m != 0 ? __builtin_ctzll(m) : 0x7fffffff;
+      klast = m != 0 ? 63 - __builtin_clzll(m) : -1;
+    }
+    x.kfirst = x.nvalid > 0 ? kfirst : 0x7fffffff;
+    x.klast = x.nvalid > 0 ? klast : -1;
+    if (lane == 0) {
+      qsum[bh * nQs + t] = x;
+      if (x.nvalid > 0 && x.glob == 0 && x.klast >= x.kfirst) atomicMin(&s_k0, x.kfirst);
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    QHeader o;
+    o.nL = nL; o.nG = nG; o.nLp = nLp; o.nT128 = (nLp + (nG + 127) / 128 * 128) / 128;
+    o.k0 = s_k0; o.pad[0] = o.pad[1] = o.pad[2] = 0;
+    hdr[bh] = o;
+  }
+}
+
 int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s) {
   char* ws = reinterpret_cast<char*>(p->workspace);
   const bool i64 = p->id_dtype == FA_IDTYPE_I64;
@@ -236,6 +343,21 @@ int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s) {
     const int64_t* sq = p->eq_stride;
     const PlanSide ks = {p->ek, sk[0], sk[1], sk[2], p->N, w.Np, w.Hk1};
     const PlanSide qs = {p->eq, sq[0], sq[1], sq[2], p->M, w.Mp, w.Hq1};
+    const int gap = p->N > p->M ? p->N - p->M : 0;
+    const int kend_min = p->prefix > 0 ? ((p->prefix < p->N ? p->prefix : p->N) - 1) / kSumRows + 1 : 0;
+    const int* qpos = p->causal ? p->qpos : nullptr;
+    int* sk_cnt = reinterpret_cast<int*>(ws + w.off_sk_cnt);
+    const int n_sk = p->B * p->H * w.split.tiles;
+    if (p->M <= kPlanOneMax && p->N <= kPlanOneMax) {
+      dim3 grid(w.Hk1 > w.Hq1 ? w.Hk1 : w.Hq1, p->B);
+      if (i64)
+        hipLaunchKernelGGL(plan_one_kernel<true>, grid, dim3(kPlanOneThreads), 0, s, ks, w.nKs, ek32, ksum, qs, w.Pp, w.nQs, eq32, perm, peq, ppos,
+                           qpos, p->qpos_stride, gap, p->causal ? 1 : 0, kend_min, hdr, qsum, sk_cnt, n_sk);
+      else
+        hipLaunchKernelGGL(plan_one_kernel<false>, grid, dim3(kPlanOneThreads), 0, s, ks, w.nKs, ek32, ksum, qs, w.Pp, w.nQs, eq32, perm, peq, ppos,
+                           qpos, p->qpos_stride, gap, p->causal ? 1 : 0, kend_min, hdr, qsum, sk_cnt, n_sk);
+      return (int)hipGetLastError();
+    }
     const int nKb = (w.nKs + 3) / 4;
     dim3 grid_kc(nKb + w.nCh, w.Hk1 > w.Hq1 ? w.Hk1 : w.Hq1, p->B);
     if (i64)
@@ -244,13 +366,11 @@ int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s) {
       hipLaunchKernelGGL(plan_kc_kernel<false>, grid_kc, dim3(256), 0, s, ks, w.nKs, nKb, ek32, ksum, qs, w.Pp, w.nCh, eq32, perm, peq, ppos, cnt);
     if ((e = hipGetLastError()) != hipSuccess) return (int)e;
     dim3 grid(w.nCh, w.Hq1, p->B);
-    const int gap = p->N > p->M ? p->N - p->M : 0;
     hipLaunchKernelGGL(plan_scatter_kernel, grid, dim3(256), 0, s, p->M, w.Mp, w.Pp, w.nCh, w.Hq1, eq32, cnt, perm, peq, ppos,
-                       p->causal ? p->qpos : nullptr, p->qpos_stride, gap, hdr);
+                       qpos, p->qpos_stride, gap, hdr);
     if ((e = hipGetLastError()) != hipSuccess) return (int)e;
     hipLaunchKernelGGL(plan_qsum_kernel, dim3((w.nQs + 3) / 4, w.Hq1, p->B), dim3(256), 0, s, w.Pp, w.nQs, w.nKs, w.Hq1, w.Hk1,
-                       p->causal ? 1 : 0, p->prefix > 0 ? ((p->prefix < p->N ? p->prefix : p->N) - 1) / kSumRows + 1 : 0, perm, peq, ppos, ksum, qsum, reinterpret_cast<int*>(ws + w.off_sk_cnt),
-                       p->B * p->H * w.split.tiles, hdr);
+                       p->causal ? 1 : 0, kend_min, perm, peq, ppos, ksum, qsum, sk_cnt, n_sk, hdr);
     if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   }
   return 0;
