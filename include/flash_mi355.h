@@ -240,6 +240,11 @@ int fa_bwd_dkdv(const fa_params* p, void* stream);
 /* dq (needs lse, and delta unless FA_FLAG_DQ_DELTA is set). */
 int fa_bwd_dq(const fa_params* p, void* stream);
 
+/* The whole backward: delta, dq, dk and dv of one forward, in as few launches as the sizes allow (the three calls
+   above, with delta formed inside dq where that is a launch of its own, or dq and dk/dv side by side in one launch
+   when neither fills the chip).  FA_FLAG_DQ_DELTA is implied. */
+int fa_bwd(const fa_params* p, void* stream);
+
 /* Number of wave-level pair waits of fa_bwd_dkdv that expired on the current device since the library
    was loaded (see FA_FLAG_DEBUG_NO_PAIR_WAIT: each one also shows as NaN in 32 rows of dk).  0 in any
    healthy run.  Waits for the device to be idle before it reads the count (a diagnostic, not for hot

@@ -86,6 +86,38 @@ struct TileRegs {
   }
 };
 
+// Tiles of TR rows of the streamed side that may hold a kept pair, by the plan's summaries of 64 rows each: every lane
+// tests one summary, a ballot keeps 64 answers.  (Tested one after the other, each was a round trip to memory in
+// front of its tile: a dozen microseconds of a small launch.)
+template <int TR>
+struct SumScan {
+  unsigned long long mask;
+  int base = -1;   // first summary of the 64 in `mask`
+  // first tile in [t, end) one of whose summaries passes; `n` summaries in all
+  template <class Test>
+  FA_DEV int next(int t, int end, int n, const Test& test) {
+    while (t < end) {
+      const int e = t * TR / kSumRows;
+      if (base < 0 || e - base >= 64) {
+        base = e;
+        const int i = base + (threadIdx.x & 63);
+        bool ok = false;
+        if (i < n) ok = test(i);
+        mask = __builtin_amdgcn_ballot_w64(ok);
+      }
+      const unsigned long long rest = mask >> (e - base);
+      if (rest != 0) {
+        const int hit = e + __builtin_ctzll(rest);
+        const int th = max(t, hit * kSumRows / TR);
+        if (th < end) return th;
+        return end;
+      }
+      t = (base + 64) * kSumRows / TR;
+    }
+    return end;
+  }
+};
+
 // min / max over the 32 lanes of a half wave (both halves hold the same 32 rows)
 FA_DEV int half_min(int x) {
 #pragma unroll
@@ -279,18 +311,9 @@ void fwd_f32_kernel(const KArgs a) {
     bm0 = base + int64_t(2 * tile) * a.bm_rs;
     if (2 * tile + 1 < a.nBr) bm1 = base + int64_t(2 * tile + 1) * a.bm_rs;
   }
+  SumScan<TR> scan;
   auto next_kt = [&](int kt) {
-    if (DOC)
-      while (kt < nkt) {
-        const int j = (kt * TR) / kSumRows;
-        const IdSummary ks = ksum[j];
-        if (doc_may_keep(g_lo, g_hi, g_glob, ks.lo, ks.hi)) break;
-        if (TR > kSumRows && j + 1 < a.nKs) {
-          const IdSummary k2 = ksum[j + 1];
-          if (doc_may_keep(g_lo, g_hi, g_glob, k2.lo, k2.hi)) break;
-        }
-        ++kt;
-      }
+    if (DOC) return scan.next(kt, nkt, a.nKs, [&](int i) { return doc_may_keep(g_lo, g_hi, g_glob, ksum[i].lo, ksum[i].hi); });
     if (!DOC && bm0 != nullptr)
       while (kt < nkt) {   // tiles whose block is off for both halves are not even loaded
         const int col = (kt * TR) / FA_MASK_BLOCK;
@@ -426,10 +449,8 @@ void fwd_f32_kernel(const KArgs a) {
 
 // ---------------------------------------------------------------------------------------------
 template <int D, bool CAUSAL, bool DOC, bool NARROW>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void dq_f32_kernel(const KArgs a) {
+FA_DEV void dq_f32_body(const KArgs& a, const int bid, char* smem) {
   constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32, TR = kTileRows<NARROW>, OWN = kOwnRows<NARROW>;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
   float* lk = reinterpret_cast<float*>(smem);
   float* lv = lk + TR * RS;
   int* lid = reinterpret_cast<int*>(lv + TR * RS);
@@ -438,8 +459,8 @@ void dq_f32_kernel(const KArgs a) {
   const int lq = lane & 31, g = lane >> 5;
   const int BH = a.B * a.H;
   const int nQt = DOC ? a.Pp / OWN : (a.M + OWN - 1) / OWN;
-  const int tile = nQt - 1 - blockIdx.x / BH;
-  const int bh = blockIdx.x % BH, b = bh / a.H, h = bh % a.H, hk = h / a.G;
+  const int tile = nQt - 1 - bid / BH;
+  const int bh = bid % BH, b = bh / a.H, h = bh % a.H, hk = h / a.G;
   QSideF32<CAUSAL, DOC, NARROW> qc;
   if (!qc.init(a, b, h, tile, wave, lq)) return;
   const int row = qc.row, rowc = qc.rowc;
@@ -497,18 +518,9 @@ void dq_f32_kernel(const KArgs a) {
     bm0 = base + int64_t(2 * tile) * a.bm_rs;
     if (2 * tile + 1 < a.nBr) bm1 = base + int64_t(2 * tile + 1) * a.bm_rs;
   }
+  SumScan<TR> scan;
   auto next_kt = [&](int kt) {
-    if (DOC)
-      while (kt < nkt) {
-        const int j = (kt * TR) / kSumRows;
-        const IdSummary ks = ksum[j];
-        if (doc_may_keep(g_lo, g_hi, g_glob, ks.lo, ks.hi)) break;
-        if (TR > kSumRows && j + 1 < a.nKs) {
-          const IdSummary k2 = ksum[j + 1];
-          if (doc_may_keep(g_lo, g_hi, g_glob, k2.lo, k2.hi)) break;
-        }
-        ++kt;
-      }
+    if (DOC) return scan.next(kt, nkt, a.nKs, [&](int i) { return doc_may_keep(g_lo, g_hi, g_glob, ksum[i].lo, ksum[i].hi); });
     if (!DOC && bm0 != nullptr)
       while (kt < nkt) {   // tiles whose block is off for both halves are not even loaded
         const int col = (kt * TR) / FA_MASK_BLOCK;
@@ -614,10 +626,8 @@ void dq_f32_kernel(const KArgs a) {
 
 // ---------------------------------------------------------------------------------------------
 template <int D, bool CAUSAL, bool DOC, bool NARROW>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void dkdv_f32_kernel(const KArgs a) {
+FA_DEV void dkdv_f32_body(const KArgs& a, const int bid, char* smem) {
   constexpr int RS = D + 1, KS2 = D / 2, DBN = (D + 31) / 32, TR = kTileRows<NARROW>, OWN = kOwnRows<NARROW>;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
   float* lqt = reinterpret_cast<float*>(smem);
   float* ldo = lqt + TR * RS;
   float* laux = ldo + TR * RS;                  // [LSE | delta | eq | row name] x TR
@@ -625,8 +635,8 @@ void dkdv_f32_kernel(const KArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = lane & 31, g = lane >> 5;
   const int BHk = a.B * a.Hk;
-  const int kt = blockIdx.x / BHk;               // causal: the first keys are seen by the most rows: first
-  const int bhk = blockIdx.x % BHk, b = bhk / a.Hk, hk = bhk % a.Hk;
+  const int kt = bid / BHk;               // causal: the first keys are seen by the most rows: first
+  const int bhk = bid % BHk, b = bhk / a.Hk, hk = bhk % a.Hk;
   const int n0 = kt * OWN, nw = NARROW ? n0 : n0 + wave * 32;
   // this wave's part of a query tile: all of it, or (NARROW) its 32 rows
   const int part = NARROW ? wave * kRows : 0;
@@ -704,18 +714,14 @@ void dkdv_f32_kernel(const KArgs a) {
     // block mask: the one or two byte columns of the workgroup's 128 keys
     const unsigned char* bmc = (!DOC && !NARROW && a.bmask != nullptr) ? a.bmask + b * a.bm_bs + h * a.bm_hs + n0 / FA_MASK_BLOCK : nullptr;
     const bool bm_two = n0 / FA_MASK_BLOCK + 1 < a.nBc;
+    SumScan<TR> scan;
     auto next_mt = [&](int mt) {
       if (DOC)
-        while (mt < nMt) {
-          auto out = [&](const IdSummary& qs) {
-            return qs.nvalid == 0 || !doc_may_keep(qs.lo, qs.hi, qs.glob, gk_lo, gk_hi) ||
-                   (CAUSAL && ((qs.rmax < n0 && n0 > a.pfx_m1) || qs.rmin > wg_rhi));
-          };
-          const int j = (mt * TR) / kSumRows;
-          if (!out(qsum[j])) break;
-          if (TR > kSumRows && !out(qsum[j + 1])) break;   // (the permuted order is a multiple of 256 entries)
-          ++mt;
-        }
+        return scan.next(mt, nMt, a.nQs, [&](int i) {
+          const IdSummary qs = qsum[i];
+          return qs.nvalid > 0 && doc_may_keep(qs.lo, qs.hi, qs.glob, gk_lo, gk_hi) &&
+                 !(CAUSAL && ((qs.rmax < n0 && n0 > a.pfx_m1) || qs.rmin > wg_rhi));
+        });
       if (bmc != nullptr)
         while (mt < nMt) {   // tiles whose block is off for both key columns are not even loaded
           const unsigned char* r = bmc + int64_t((mt * TR) / FA_MASK_BLOCK) * a.bm_rs;
@@ -855,6 +861,29 @@ void dkdv_f32_kernel(const KArgs a) {
   }
 }
 
+template <int D, bool CAUSAL, bool DOC, bool NARROW>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void dq_f32_kernel(const KArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  dq_f32_body<D, CAUSAL, DOC, NARROW>(a, (int)blockIdx.x, smem);
+}
+template <int D, bool CAUSAL, bool DOC, bool NARROW>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void dkdv_f32_kernel(const KArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  dkdv_f32_body<D, CAUSAL, DOC, NARROW>(a, (int)blockIdx.x, smem);
+}
+// Both in one launch, for problems that leave CUs idle (NARROW): they run side by side instead of one after the other.
+// delta is read by both and comes from a launch of its own.
+template <int D, bool CAUSAL, bool DOC>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void dqkv_f32_kernel(const KArgs a, const int n_dkdv) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int bid = (int)blockIdx.x;
+  if (bid < n_dkdv) dkdv_f32_body<D, CAUSAL, DOC, true>(a, bid, smem);   // the longer ones first
+  else dq_f32_body<D, CAUSAL, DOC, true>(a, bid - n_dkdv, smem);
+}
+
 // delta[b,h,m] = sum_d O[b,h,m,d] * dO[b,h,m,d]; D/4 lanes per row, 16-byte loads.
 template <int D>
 __global__ __launch_bounds__(kThreads) void delta_f32_kernel(const KArgs a) {
@@ -907,6 +936,22 @@ int launch_one(const KArgs& a, hipStream_t s) {
   return launch_form<WHICH, D, CAUSAL, DOC, false>(a, s);
 }
 
+template <int D, bool CAUSAL, bool DOC>
+int launch_both(const KArgs& a, hipStream_t s) {
+  constexpr int OWN = kOwnRows<true>;
+  auto kern = dqkv_f32_kernel<D, CAUSAL, DOC>;
+  const int n_dkdv = ((a.N + OWN - 1) / OWN) * a.B * a.Hk, n_dq = (DOC ? a.Pp / OWN : (a.M + OWN - 1) / OWN) * a.B * a.H;
+  static bool lds_allowed[64] = {};   // per kernel instantiation and device
+  if (int e = allow_lds(kern, lds_bytes<D, true>(), lds_allowed)) return e;
+  hipLaunchKernelGGL(kern, dim3(n_dkdv + n_dq), dim3(kThreads), (lds_bytes<D, true>()), s, a, n_dkdv);
+  return (int)hipGetLastError();
+}
+template <int D>
+int launch_both_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) {
+  if (causal) return doc ? launch_both<D, true, true>(a, s) : launch_both<D, true, false>(a, s);
+  return doc ? launch_both<D, false, true>(a, s) : launch_both<D, false, false>(a, s);
+}
+
 template <int WHICH, int D>
 int launch_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) {
   if (causal) return doc ? launch_one<WHICH, D, true, true>(a, s) : launch_one<WHICH, D, true, false>(a, s);
@@ -929,6 +974,21 @@ int launch_d(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) {
 int launch_fwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kFwd>(a, D, causal, doc, s); }
 int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kDq>(a, D, causal, doc, s); }
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kDkdv>(a, D, causal, doc, s); }
+
+// dq and dk/dv in one launch, delta in one before it: whether these sizes take that form, and the launch
+bool bwd_f32_in_one(const KArgs& a, int D) {
+  // the two forms have to fit side by side, or nearly: one workgroup to a CU
+  const int64_t wgs = int64_t((a.M + 31) / 32) * a.B * a.H + int64_t((a.N + 31) / 32) * a.B * a.Hk;
+  return D <= 64 && a.bmask == nullptr && wgs <= 2 * kCUs;
+}
+int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) {
+  switch (D) {
+    case 64: return launch_both_cd<64>(a, causal, doc, s);
+    case 32: return launch_both_cd<32>(a, causal, doc, s);
+    case 16: return launch_both_cd<16>(a, causal, doc, s);
+    default: return -1;
+  }
+}
 
 int launch_bwd_delta_f32(const KArgs& a, int D, hipStream_t s) {
   const int BH = a.B * a.H < 65535 ? a.B * a.H : 65535;

@@ -137,10 +137,7 @@ variable_list backward(const Problem& x, const Tensor& o, const Tensor& lse, Ten
   set_strides(p.o_stride, o); set_strides(p.do_stride, dout);
   set_strides(p.dq_stride, dq); set_strides(p.dk_stride, dk); set_strides(p.dv_stride, dv);
   if (!dlse.defined()) {
-    // the dq kernel forms delta = rowsum(O * dO) from rows it holds anyway and leaves it for the dk/dv kernel
-    p.flags |= FA_FLAG_DQ_DELTA;
-    check(fa_bwd_dq(&p, stream), "fa_bwd_dq");
-    check(fa_bwd_dkdv(&p, stream), "fa_bwd_dkdv");
+    check(fa_bwd(&p, stream), "fa_bwd");
   } else {
     check(fa_bwd_delta(&p, stream), "fa_bwd_delta");
     // dS = P * (dP - delta) + dLSE * P: a gradient arriving at LSE only shifts delta

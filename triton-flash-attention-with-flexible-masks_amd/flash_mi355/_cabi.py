@@ -30,7 +30,7 @@ FA_STATIC_WS_BYTES = 32 << 20
 # every symbol include/flash_mi355.h declares
 EXPORTS = (
     "fa_version", "fa_params_size", "fa_error_string", "fa_last_hip_error", "fa_validate",
-    "fa_workspace_bytes", "fa_workspace_plan_bytes", "fa_mask_plan", "fa_fwd", "fa_bwd_delta", "fa_bwd_dkdv", "fa_bwd_dq",
+    "fa_workspace_bytes", "fa_workspace_plan_bytes", "fa_mask_plan", "fa_fwd", "fa_bwd_delta", "fa_bwd_dkdv", "fa_bwd_dq", "fa_bwd",
     "fa_mask_dump", "fa_fwd_static", "fa_workspace_scratch_bytes", "fa_pair_wait_expired",
 )
 
@@ -86,7 +86,7 @@ def lib() -> ctypes.CDLL:
     L.fa_workspace_scratch_bytes.argtypes = [POINTER(FaParams)]
     L.fa_pair_wait_expired.restype = c_int
     L.fa_pair_wait_expired.argtypes = [POINTER(c_uint64)]
-    for name in ("fa_mask_plan", "fa_fwd", "fa_fwd_static", "fa_bwd_delta", "fa_bwd_dkdv", "fa_bwd_dq"):
+    for name in ("fa_mask_plan", "fa_fwd", "fa_fwd_static", "fa_bwd_delta", "fa_bwd_dkdv", "fa_bwd_dq", "fa_bwd"):
         fn = getattr(L, name)
         fn.restype = c_int
         fn.argtypes = [POINTER(FaParams), c_void_p]

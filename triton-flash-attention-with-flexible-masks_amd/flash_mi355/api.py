@@ -271,11 +271,8 @@ class _Impl:
             _set4(p.dq_stride, dq); _set4(p.dk_stride, dk); _set4(p.dv_stride, dv)
             stream = _stream_ptr(q.device)
             if dlse is None:
-                # two launches instead of the reference's three (flash_triton.py:585-634): the dq kernel
-                # forms delta = rowsum(O * dO) from rows it holds anyway and leaves it for the dk/dv kernel
-                p.flags |= _cabi.FA_FLAG_DQ_DELTA
-                _cabi.check(L.fa_bwd_dq(ctypes.byref(p), stream), "fa_bwd_dq")
-                _cabi.check(L.fa_bwd_dkdv(ctypes.byref(p), stream), "fa_bwd_dkdv")
+                # two launches instead of the reference's three (flash_triton.py:585-634)
+                _cabi.check(L.fa_bwd(ctypes.byref(p), stream), "fa_bwd")
             else:
                 _cabi.check(L.fa_bwd_delta(ctypes.byref(p), stream), "fa_bwd_delta")
                 if dlse is not None:
