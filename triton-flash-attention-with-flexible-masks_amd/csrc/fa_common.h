@@ -455,7 +455,12 @@ struct TabLayout {
 // Keys per entry of the key-tile table: the 64-key role-split form at D = 128 (sequences are short), 128 keys below.
 constexpr int kSeqKeyTile = 64;
 FA_HD int seq_key_tile(int D) { return D > 64 ? kSeqKeyTile : 128; }
-constexpr int kSeqTargetWgs = 3 * kCUs;   // workgroups a split launch of packed sequences aims at
+// Workgroups the split key ranges of a packed batch aim at.  A split tile pays for its partial results (64 KB per chunk
+// of 128 rows at D = 128, written and read again), so they are cut to fill the chip (two workgroups to a CU) and,
+// once there are tiles enough for that, only where one is several times as long as the rest.  Swept over 64 .. 2048:
+// 32 sequences of up to 128 queries on 500 - 3500 keys (720 tiles) 105 / 107 / 118 / 130 / 163 us at 64 / 128 / 448 /
+// 768 / 1536, one of 256 queries on 8000 keys (64 tiles) 105 / 68 / 59 / 78 / 137.
+constexpr int kSeqTargetWgs = 448, kSeqFullWgs = 400, kSeqTargetFull = 128;
 inline TabLayout tab_layout(const fa_params* p, const FwdCfg& c) {
   TabLayout w = {};
   uint64_t o = 0;

@@ -14,12 +14,13 @@ namespace {
 constexpr int kThreads = 1024;
 constexpr int kBuckets = 128;     // classes of tile lengths the table is sorted by, longest first
 constexpr int kLdsSeqs = 8192;    // sequences whose tile offsets fit LDS (more: they are kept in the table's own memory)
+constexpr int kLdsCu = 2048;      // sequences whose boundaries are kept in LDS too (more: read again where they are needed)
 
 struct SeqPlanArgs {
   const void* cu_q;
   const void* cu_k;
   int i64, nseq, Tq, Tk, pack, bm, bk, causal, win;
-  int spare, min_chunk;           // extra entries a split may use (0: no tile is split), key tiles per chunk at least
+  int spare, min_chunk, heads;    // extra entries a split may use, key tiles per chunk at least, head groups of the launch
   SeqHdr* hdr;
   SeqTile* qtab;
   SeqTile* ktab;
@@ -35,13 +36,11 @@ FA_DEV int cu_at(const void* p, int i64, int i, int total) {
   return v < 0 ? 0 : (v > total ? total : (int)v);
 }
 // sequence s of nseq; number nseq is what lies behind the last boundary
-FA_DEV Seq seq_at(const SeqPlanArgs& p, int s) {
+FA_DEV int bound_at(const void* cu, int i64, int nseq, int total, int s) { return s == 0 ? 0 : (s > nseq ? total : cu_at(cu, i64, s, total)); }
+FA_DEV Seq seq_of_bounds(int nseq, int s, int q0, int q1, int k0, int k1) {
   Seq r;
-  r.q0 = s == 0 ? 0 : cu_at(p.cu_q, p.i64, s, p.Tq);
-  r.k0 = s == 0 ? 0 : cu_at(p.cu_k, p.i64, s, p.Tk);
-  r.M = max(0, (s < p.nseq ? cu_at(p.cu_q, p.i64, s + 1, p.Tq) : p.Tq) - r.q0);
-  r.N = max(0, (s < p.nseq ? cu_at(p.cu_k, p.i64, s + 1, p.Tk) : p.Tk) - r.k0);
-  r.gap = s < p.nseq ? r.N - r.M : 0;
+  r.q0 = q0; r.k0 = k0; r.M = max(0, q1 - q0); r.N = max(0, k1 - k0);
+  r.gap = s < nseq ? r.N - r.M : 0;
   return r;
 }
 
@@ -58,6 +57,7 @@ FA_DEV int wave_scan(int v) {   // inclusive sum over the lanes of a wave
 // Block 0 writes the query tiles, block 1 the key tiles.
 __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p, int* __restrict__ spill) {
   __shared__ int s_off[kLdsSeqs + 1];
+  __shared__ int s_cuq[kLdsCu + 2], s_cuk[kLdsCu + 2];
   __shared__ int s_wave[kThreads / 64];
   __shared__ float s_work[kThreads / 64];
   __shared__ int s_bucket[kBuckets];
@@ -68,6 +68,17 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
   int* off = ns <= kLdsSeqs ? s_off : spill + (keys ? ns + 1 : 0);
   if (!keys)
     for (int i = tid; i < p.n_cnt; i += kThreads) p.cnt[i] = 0;
+  const bool in_lds = ns <= kLdsCu;
+  if (in_lds)
+    for (int i = tid; i <= ns; i += kThreads) {
+      s_cuq[i] = bound_at(p.cu_q, p.i64, p.nseq, p.Tq, i);
+      s_cuk[i] = bound_at(p.cu_k, p.i64, p.nseq, p.Tk, i);
+    }
+  auto seq_at = [&](int s) {
+    if (in_lds) return seq_of_bounds(p.nseq, s, s_cuq[s], s_cuq[s + 1], s_cuk[s], s_cuk[s + 1]);
+    return seq_of_bounds(p.nseq, s, bound_at(p.cu_q, p.i64, p.nseq, p.Tq, s), bound_at(p.cu_q, p.i64, p.nseq, p.Tq, s + 1),
+                         bound_at(p.cu_k, p.i64, p.nseq, p.Tk, s), bound_at(p.cu_k, p.i64, p.nseq, p.Tk, s + 1));
+  };
   if (tid == 0) { s_tot = 0; s_max = 1; s_cnt = 0; s_part = 0; }
   for (int i = tid; i < kBuckets; i += kThreads) s_bucket[i] = 0;
   __syncthreads();
@@ -93,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
     const int s = s0 + tid;
     int n = 0;
     if (s < ns) {
-      const Seq q = seq_at(p, s);
+      const Seq q = seq_at(s);
       n = tiles_of(q);
       longest = max(longest, (keys ? q.M : q.N) / 64 + 2);
     }
@@ -123,13 +134,24 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
     return a;
   };
 
+  // sequence and length of tile t; the thread's first one is looked up once for the three passes below
+  int my_seq = -1, my_len = 0;
+  if (tid < nt) { my_seq = seq_of(tid); my_len = length_of(seq_at(my_seq), tid - off[my_seq]); }
+  auto look = [&](int t, int& s, int& len) {
+    if (t == tid) { s = my_seq; len = my_len; return; }
+    s = seq_of(t);
+    len = length_of(seq_at(s), t - off[s]);
+  };
+
   // chunks: the work of all tiles over the entries a split launch aims at
   int chunk = 0x7fffffff;
-  if (!keys && p.spare > 0) {
+  if (!keys) {
+    const int spare = int64_t(nt) * p.heads >= kSeqFullWgs ? min(p.spare, kSeqTargetFull / p.heads + 1) : p.spare;
     float work = 0.f;
     for (int t = tid; t < nt; t += kThreads) {
-      const int s = seq_of(t);
-      work += float(length_of(seq_at(p, s), t - off[s]));
+      int s, len;
+      look(t, s, len);
+      work += float(len);
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) work += __shfl_xor(work, o);
@@ -137,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
     __syncthreads();
     work = 0.f;
     for (int w = 0; w < kThreads / 64; ++w) work += s_work[w];
-    chunk = max(p.min_chunk, int(work / p.spare) + 1);
+    chunk = max(p.min_chunk, int(work / spare) + 1);
   }
   const int longest_all = min(s_max, chunk);
   auto chunks_of = [&](int len) { return min(kSplitKMaxFew, max(1, (len + chunk - 1) / chunk)); };
@@ -146,7 +168,9 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
     return kBuckets - 1 - min(kBuckets - 1, int(int64_t(l) * kBuckets / (longest_all + 1)));
   };
   for (int t = tid; t < nt; t += kThreads) {
-    const int s = seq_of(t), len = length_of(seq_at(p, s), t - off[s]), nc = chunks_of(len);
+    int s, len;
+    look(t, s, len);
+    const int nc = chunks_of(len);
     atomicAdd(&s_bucket[bucket_of(len, nc)], nc);
   }
   __syncthreads();
@@ -163,9 +187,10 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
   SeqTile* tab = keys ? p.ktab : p.qtab;
   const int cap = keys ? p.nK : p.nQ;
   for (int t = tid; t < nt; t += kThreads) {
-    const int s = seq_of(t);
-    const Seq q = seq_at(p, s);
-    const int len = length_of(q, t - off[s]), nc = chunks_of(len);
+    int s, len;
+    look(t, s, len);
+    const Seq q = seq_at(s);
+    const int nc = chunks_of(len);
     const int at = atomicAdd(&s_bucket[bucket_of(len, nc)], nc);
     int cnt = 0, part = 0;
     if (nc > 1) { cnt = atomicAdd(&s_cnt, 1); part = atomicAdd(&s_part, nc); }
@@ -202,7 +227,7 @@ int launch_seq_plan(const fa_params* p, const FwdCfg& c, const TabLayout& w, hip
   a.Tq = p->M; a.Tk = p->N; a.pack = c.pack; a.bm = c.bm; a.bk = seq_key_tile(p->D);
   a.causal = p->causal != 0;
   a.win = p->window > 0 && p->window < 0x3fffffff ? p->window : 0x3fffffff;
-  a.spare = w.nCnt; a.min_chunk = c.dec ? 4 : 8;
+  a.spare = w.nCnt; a.min_chunk = c.dec ? 4 : 8; a.heads = nh;
   a.hdr = reinterpret_cast<SeqHdr*>(ws + w.off_hdr);
   a.qtab = reinterpret_cast<SeqTile*>(ws + w.off_q);
   a.ktab = reinterpret_cast<SeqTile*>(ws + w.off_k);
