@@ -83,7 +83,10 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
   for (int i = tid; i < kBuckets; i += kThreads) s_bucket[i] = 0;
   __syncthreads();
 
-  auto tiles_of = [&](const Seq& q) { return keys ? (q.N + p.bk - 1) / p.bk : int((int64_t(q.M) * p.pack + p.bm - 1) / p.bm); };
+  // (packed rows stay below 2^31; tile heights are powers of two: no 64-bit or general division by them)
+  const int sh = __builtin_ctz(keys ? p.bk : p.bm);
+  const unsigned pack = p.pack, bm = p.bm;
+  auto tiles_of = [&](const Seq& q) { return keys ? (q.N + p.bk - 1) >> sh : int((unsigned(q.M) * pack + bm - 1) >> sh); };
   // length of a tile: 64-key tiles its rows see, or 64-row tiles that see its keys
   auto length_of = [&](const Seq& q, int t) {
     if (keys) {
@@ -92,7 +95,7 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
       const int hi = p.causal ? min(q.M - 1, n1 - q.gap + p.win - 1) : q.M - 1;
       return hi >= lo ? hi / 64 - lo / 64 + 1 : 0;
     }
-    const int r0 = int(int64_t(t) * p.bm / p.pack), r1 = int(min(int64_t(q.M) * p.pack, int64_t(t + 1) * p.bm) - 1) / p.pack;
+    const int r0 = int((unsigned(t) << sh) / pack), r1 = int((min(unsigned(q.M) * pack, unsigned(t + 1) << sh) - 1) / pack);
     const int lo = p.causal ? max(0, q.gap + r0 - p.win + 1) : 0;
     const int hi = p.causal ? min(q.N - 1, q.gap + r1) : q.N - 1;
     return hi >= lo ? hi / 64 - lo / 64 + 1 : 0;
@@ -162,10 +165,11 @@ __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p,
     chunk = max(p.min_chunk, int(work / spare) + 1);
   }
   const int longest_all = min(s_max, chunk);
-  auto chunks_of = [&](int len) { return min(kSplitKMaxFew, max(1, (len + chunk - 1) / chunk)); };
+  const float to_bucket = float(kBuckets) / float(longest_all + 1);
+  auto chunks_of = [&](int len) { return len <= chunk ? 1 : min(kSplitKMaxFew, (len + chunk - 1) / chunk); };
   auto bucket_of = [&](int len, int nc) {   // 0: the longest
-    const int l = (len + nc - 1) / nc;
-    return kBuckets - 1 - min(kBuckets - 1, int(int64_t(l) * kBuckets / (longest_all + 1)));
+    const int l = nc == 1 ? len : (len + nc - 1) / nc;
+    return kBuckets - 1 - min(kBuckets - 1, int(float(l) * to_bucket));
   };
   for (int t = tid; t < nt; t += kThreads) {
     int s, len;
