@@ -165,13 +165,11 @@ void bwd_dkdv_kernel(const KArgs a) {
   const unsigned row_span = (key < N && row_hi >= row_lo) ? (unsigned)(row_hi - row_lo + 1) : 0u;
 
   // per query head state (set at the top of the head loop)
-  const float* lsep = nullptr;
-  const float* delp = nullptr;
+  // what this wave loads of a tile's row values: LSE, delta, ids (in row order) or diagonal positions (in the permuted order)
+  const int* auxp = nullptr;
   int ek_j = 0;
   int wk_lo = 0, wk_hi = 0;   // id interval of this wave's 32 keys
-  const int* eqp = nullptr;
   const int* pmp = nullptr;
-  const int* ppp = nullptr;   // diagonal positions in the permuted order
   const IdSummary* qsum = nullptr;
 
   Loader ldQ, ldO;
@@ -209,8 +207,7 @@ void bwd_dkdv_kernel(const KArgs a) {
       ldQ.issue(m0, smem + bufi * TILE_BYTES);
       ldO.issue(m0, smem + (2 + bufi) * TILE_BYTES);
       const int r = m0 + lane < M ? m0 + lane : M - 1;
-      if (wave == 0) glb_load_lds4(lsep + r, aux);
-      if (wave == 1) glb_load_lds4(delp + r, aux + 256);
+      if (wave < 2) glb_load_lds4(auxp + r, aux + wave * 256);
     } else {
       // The row indices were fetched a tile ago and have arrived (the caller waited for every
       // outstanding load before the barrier).  Tell the compiler so here: the wait it would place
@@ -228,10 +225,7 @@ void bwd_dkdv_kernel(const KArgs a) {
         }
       }
       const int r = ri_aux >= 0 ? ri_aux : 0;
-      if (wave == 0) glb_load_lds4(lsep + r, aux);
-      if (wave == 1) glb_load_lds4(delp + r, aux + 256);
-      if (wave == 2) glb_load_lds4(eqp + r, aux + 512);
-      if (wave == 3) glb_load_lds4(ppp + tile * BQ + lane, aux + 768);
+      if (wave < 4) glb_load_lds4(auxp + (wave == 3 ? tile * BQ + lane : r), aux + wave * 256);
     }
   };
 
@@ -528,27 +522,27 @@ void bwd_dkdv_kernel(const KArgs a) {
   };
 
   for (int gi = 0; gi < a.G; ++gi) {
-    const int h = hk * a.G + gi;
-    lsep = a.lse + (int64_t(b) * a.H + h) * a.M + q0;
-    delp = a.delta + (int64_t(b) * a.H + h) * a.M + q0;
-    ldQ.init(reinterpret_cast<const T*>(a.q) + b * a.q_bs + h * a.q_hs + q0 * a.q_rs, a.q_rs, M);
-    ldO.init(reinterpret_cast<const T*>(a.dout) + b * a.do_bs + h * a.do_hs + q0 * a.do_rs, a.do_rs, M);
+    LateArgs& ga = late_args();   // (the head loop encloses the tile loop: what its set-up reads would stay in registers)
+    const int h = hk * ga.G + gi;
+    auxp = reinterpret_cast<const int*>(wave == 0 ? ga.lse : ga.delta) + (int64_t(b) * ga.H + h) * ga.M + q0;
+    ldQ.init(reinterpret_cast<const T*>(ga.q) + b * ga.q_bs + h * ga.q_hs + q0 * ga.q_rs, ga.q_rs, M);
+    ldO.init(reinterpret_cast<const T*>(ga.dout) + b * ga.do_bs + h * ga.do_hs + q0 * ga.do_rs, ga.do_rs, M);
     int gk_lo = 0, gk_hi = 0;   // id interval of the workgroup's 128 keys
     int nQtiles = (M + BQ - 1) / BQ;
-    int first = CAUSAL ? (n0 <= a.pfx_m1 ? 0 : max(0, n0 - gk) / BQ) : 0;
+    int first = CAUSAL ? (n0 <= ga.pfx_m1 ? 0 : max(0, n0 - gk) / BQ) : 0;
     // sliding window: the last row that sees a key of this workgroup
-    const int wg_rhi = CAUSAL ? min(rcap, n0 + BK - 1 - gk + a.win - 1) : rcap;
+    const int wg_rhi = CAUSAL ? min(rcap, n0 + BK - 1 - gk + ga.win - 1) : rcap;
     if (CAUSAL && !DOC) nQtiles = min(nQtiles, max(0, wg_rhi + 1 + BQ - 1) / BQ);
     if (DOC) {
-      ek_j = a.ek32[b * a.ek_bs + h * a.ek_hs + keyc];
-      eqp = a.eq32 + b * a.eq_bs + h * a.eq_hs;
-      pmp = a.perm + b * a.pm_bs + h * a.pm_hs;
-      ppp = a.ppos + b * a.pm_bs + h * a.pm_hs;
-      qsum = a.qsum + b * a.qs_bs + h * a.qs_hs;
-      const IdSummary* ks = a.ksum + b * a.ks_bs + h * a.ks_hs;
+      ek_j = ga.ek32[b * ga.ek_bs + h * ga.ek_hs + keyc];
+      pmp = ga.perm + b * ga.pm_bs + h * ga.pm_hs;
+      if (wave == 2) auxp = ga.eq32 + b * ga.eq_bs + h * ga.eq_hs;
+      if (wave == 3) auxp = ga.ppos + b * ga.pm_bs + h * ga.pm_hs;
+      qsum = ga.qsum + b * ga.qs_bs + h * ga.qs_hs;
+      const IdSummary* ks = ga.ksum + b * ga.ks_bs + h * ga.ks_hs;
       const IdSummary s0 = ks[n0 / kSumRows];
       gk_lo = s0.lo; gk_hi = s0.hi;
-      if (BK > kSumRows && n0 / kSumRows + 1 < a.nKs) {
+      if (BK > kSumRows && n0 / kSumRows + 1 < ga.nKs) {
         const IdSummary s1 = ks[n0 / kSumRows + 1];
         gk_lo = min(gk_lo, s1.lo); gk_hi = max(gk_hi, s1.hi);
       }
@@ -560,35 +554,35 @@ void bwd_dkdv_kernel(const KArgs a) {
         hi_ = max(hi_, __shfl_xor(hi_, off));
       }
       wk_lo = lo_; wk_hi = hi_;
-      nQtiles = a.nQs;
+      nQtiles = ga.nQs;
       first = 0;
     }
     // decisions of this wave pair (keys nw .. nw+31) for query tile t, evaluated by the lane that tests the tile
     // block mask: the byte column(s) of the workgroup's one or two 64-key blocks; a query tile is one
     // row of blocks, a wave's 32 keys lie inside one block (no element mask needed)
-    const unsigned char* bmk = (!DOC && a.bmask != nullptr) ? a.bmask + b * a.bm_bs + h * a.bm_hs + n0 / 64 : nullptr;
+    const unsigned char* bmk = (!DOC && ga.bmask != nullptr) ? ga.bmask + b * ga.bm_bs + h * ga.bm_hs + n0 / 64 : nullptr;
     auto dec = [&](int t, const IdSummary& qs) {
       bool skip, lim, doc = false, glob = false, col = false, none = false;
       if (!DOC) {
         const int m0 = t * BQ;
         const int rmin = m0, rmax = min(m0 + BQ - 1, M - 1);
-        skip = (nw >= N) || (CAUSAL && ((gap + rmax < nw && nw > a.pfx_m1) || gap + rmin - a.win + 1 > nw + 31));
+        skip = (nw >= N) || (CAUSAL && ((gap + rmax < nw && nw > ga.pfx_m1) || gap + rmin - ga.win + 1 > nw + 31));
         lim = (m0 + BQ > M) || (nw + 32 > N) ||
-              (CAUSAL && ((gap + rmin < nw + 31 && nw + 31 > a.pfx_m1) || gap + rmax - a.win + 1 > nw));
+              (CAUSAL && ((gap + rmin < nw + 31 && nw + 31 > ga.pfx_m1) || gap + rmax - ga.win + 1 > nw));
         if (bmk != nullptr) {
-          const bool in = t < a.nBr;
-          const unsigned char* r = bmk + int64_t(t) * a.bm_rs;
+          const bool in = t < ga.nBr;
+          const unsigned char* r = bmk + int64_t(t) * ga.bm_rs;
           const unsigned b0 = in ? r[0] : 0u;
-          const unsigned b1 = (in && BK > 64 && n0 / 64 + 1 < a.nBc) ? r[1] : 0u;
+          const unsigned b1 = (in && BK > 64 && n0 / 64 + 1 < ga.nBc) ? r[1] : 0u;
           const unsigned mine = (BK > 64 && kb >= 2) ? b1 : b0;
           skip = skip || mine == 0;
           none = (b0 | b1) == 0;
         }
       } else {
-        skip = (nw >= N) || (CAUSAL && ((qs.rmax < nw && nw > a.pfx_m1) || qs.rmin - a.win + 1 > nw + 31)) ||
+        skip = (nw >= N) || (CAUSAL && ((qs.rmax < nw && nw > ga.pfx_m1) || qs.rmin - ga.win + 1 > nw + 31)) ||
                !doc_may_keep(qs.lo, qs.hi, qs.glob, wk_lo, wk_hi);
         lim = (qs.nvalid < BQ) || (nw + 32 > N) ||
-              (CAUSAL && ((qs.rmin < nw + 31 && nw + 31 > a.pfx_m1) || qs.rmax - a.win + 1 > nw));
+              (CAUSAL && ((qs.rmin < nw + 31 && nw + 31 > ga.pfx_m1) || qs.rmax - ga.win + 1 > nw));
         doc = !doc_all_keep(qs.lo, qs.hi, wk_lo, wk_hi);
         glob = qs.glob != 0;
         // one local id for the whole tile (padding rows aside, which the row-range mask drops):
@@ -600,7 +594,7 @@ void bwd_dkdv_kernel(const KArgs a) {
                         (none ? TF_NONE : 0), qs.lo);
     };
     TileIter it;
-    it.init_queries(first, nQtiles, qsum, gk_lo, gk_hi, CAUSAL && n0 > a.pfx_m1 ? n0 - gk : (int)0x80000000,
+    it.init_queries(first, nQtiles, qsum, gk_lo, gk_hi, CAUSAL && n0 > ga.pfx_m1 ? n0 - gk : (int)0x80000000,
                     CAUSAL ? wg_rhi : 0x7fffffff, dec);
     if (gi > 0) __syncthreads();  // the previous head's last tile may still be read from LDS
 
@@ -650,8 +644,9 @@ void bwd_dkdv_kernel(const KArgs a) {
   FA_TRACE_ONLY(if (SPLIT && threadIdx.x == 64 * NKB && blockIdx.x < fa::kTraceWgs) g_trace_dkdv[blockIdx.x * 8 + 1] = tr_wait;)
   {
     // dK / dV rows leave through LDS (store_rows_through_lds), once every wave is done with the last query tile
-    T* dvp = reinterpret_cast<T*>(a.dv) + b * a.dv_bs + hk * a.dv_hs + k0 * a.dv_rs;
-    T* dkp = reinterpret_cast<T*>(a.dk) + b * a.dk_bs + hk * a.dk_hs + k0 * a.dk_rs;
+    LateArgs& la = late_args();
+    T* dvp = reinterpret_cast<T*>(la.dv) + b * la.dv_bs + hk * la.dv_hs + k0 * la.dv_rs;
+    T* dkp = reinterpret_cast<T*>(la.dk) + b * la.dk_bs + hk * la.dk_hs + k0 * la.dk_rs;
     __syncthreads();
     char* patch = smem + wave * row_patch_bytes<D>();
     auto store = [&](T* base, const int64_t rs, const f32x16 (&v)[DBN], const float sc) __attribute__((always_inline)) {
@@ -667,10 +662,10 @@ void bwd_dkdv_kernel(const KArgs a) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[db][r] = __builtin_nanf("");
       }
-      if (role == 0) store(dvp, a.dv_rs, acc, 1.0f); else store(dkp, a.dk_rs, acc, a.scale);
+      if (role == 0) store(dvp, la.dv_rs, acc, 1.0f); else store(dkp, la.dk_rs, acc, la.scale);
     } else {
-      store(dvp, a.dv_rs, acc, 1.0f);
-      store(dkp, a.dk_rs, acc2, a.scale);
+      store(dvp, la.dv_rs, acc, 1.0f);
+      store(dkp, la.dk_rs, acc2, la.scale);
     }
   }
   }   // run of key tiles

@@ -23,12 +23,13 @@ constexpr int kDqPre2 = 3;
 FA_TRACE_ARRAY(g_trace_dq);
 #endif
 
-template <typename Tag, int D, bool CAUSAL, bool DOC>
+template <typename Tag, int D, bool CAUSAL, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2, D <= 64 ? 3 : 2)))
 void bwd_dq_kernel(const KArgs a) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
+  constexpr bool DOC = MODE == GEO_DOC, GEN = MODE == GEO_GENERAL;
   constexpr int BN = 64, KS = D / 16;
   constexpr int DL = D < 32 ? 32 : D;  // LDS row width: D = 16 is staged as 32 columns, the upper 16 zero
   constexpr int DBN = DL / 32;
@@ -41,7 +42,7 @@ void bwd_dq_kernel(const KArgs a) {
   FA_TRACE_ONLY(int tr_tiles = 0;)
 
   TileGeo ge;
-  QTileCtx<CAUSAL, DOC> qc;
+  QTileCtx<CAUSAL, MODE> qc;
   int kt_first, kt_last;
   if (!tile_work(a, ge, qc, kt_first, kt_last)) return;
   const int b = ge.b, h = ge.h0, hk = ge.hk, nsplit = ge.nchunk;
@@ -53,7 +54,6 @@ void bwd_dq_kernel(const KArgs a) {
   const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + ge.k0 * a.k_rs;
   const T* vp = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + ge.k0 * a.v_rs;
   const T* dop = reinterpret_cast<const T*>(a.dout) + b * a.do_bs + (h + qc.hg) * a.do_hs + ge.q0 * a.do_rs;
-  T* dqp = reinterpret_cast<T*>(a.dq) + b * a.dq_bs + h * a.dq_hs + ge.q0 * a.dq_rs;
   const int64_t row_l = (int64_t(b) * a.H + h + qc.hg) * a.M + ge.q0 + rowc;   // of LSE and delta
   const T* op = reinterpret_cast<const T*>(a.o) + b * a.o_bs + (h + qc.hg) * a.o_hs + ge.q0 * a.o_rs;
   const bool own_delta = a.dq_delta != 0;   // delta = rowsum(O * dO) is computed here instead of being read
@@ -255,12 +255,17 @@ void bwd_dq_kernel(const KArgs a) {
         for (int r = 0; r < 16; ++r) dq[db][r] += mb[(16 * db + r) * 64];
     }
   }
+  // (where scalar registers run out; the other forms keep what the end needs, and do not wait for it here)
+  decltype(auto) la = [&]() -> decltype(auto) { if constexpr (MODE == GEO_PLAIN) return (a); else return late_args(); }();
+  T* dqp = reinterpret_cast<T*>(la.dq) + b * la.dq_bs + h * la.dq_hs + ge.q0 * la.dq_rs;
   const bool writer = !halved || sub == 0;   // the wave that holds the rows' result
-  if (nsplit > 1) {
+  if (MODE != GEO_PLAIN && nsplit > 1) {
     // This workgroup saw one chunk of the keys: store the partial sum; the last chunk to arrive
     // adds them up in a fixed order and writes dQ.
-    const int rows = DOC ? 128 : a.bm;   // rows of a partial result
-    float* po = a.sk_o + (ge.part + int64_t(ge.chunk) * ge.pstride) * (rows * D);
+    split_home<MODE>(la, ge);
+    const int rows = DOC ? 128 : la.bm;   // rows of a partial result
+    const int pstride = DOC ? 1 : ge.pstride;
+    float* po = la.sk_o + (ge.part + int64_t(ge.chunk) * pstride) * (rows * D);
 #pragma unroll
     for (int db = 0; db < DBN; ++db)
 #pragma unroll
@@ -269,24 +274,24 @@ void bwd_dq_kernel(const KArgs a) {
         f32x4 x = {dq[db][4 * q4 + 0], dq[db][4 * q4 + 1], dq[db][4 * q4 + 2], dq[db][4 * q4 + 3]};
         store_dev(po + part_index<D>(qc.rb, 4 * db + q4, lane) * 4, x);
       }
-    if (!split_arrive(a.sk_cnt + ge.cnt, nsplit)) { FA_STAMP(g_trace_dq, 4, FA_CLOCK()); return; }
+    if (!split_arrive(la.sk_cnt + ge.cnt, nsplit)) { FA_STAMP(g_trace_dq, 4, FA_CLOCK()); return; }
     FA_STAMP(g_trace_dq, 6, FA_CLOCK());
     // (up to eight chunks are requested together, four or two steps of them: every device-scope load is a
     // round trip of its own, so they are put in flight side by side instead of one after the other)
     constexpr int C4 = D / 4;
-    const float* bo = a.sk_o + int64_t(ge.part) * (rows * D);
-    const int64_t so = int64_t(ge.pstride) * (rows * D);   // from chunk to chunk
-    const int* prm = DOC ? a.perm + b * a.pm_bs + h * a.pm_hs + ge.tile * 128 : nullptr;
+    const float* bo = la.sk_o + int64_t(ge.part) * (rows * D);
+    const int64_t so = int64_t(pstride) * (rows * D);   // from chunk to chunk
+    const int* prm = DOC ? la.perm + b * la.pm_bs + h * la.pm_hs + ge.tile * 128 : nullptr;
     // row of the tile -> row of the operands (with ids), or packed row (without), -1: no such row
     auto row_of = [&](int r) __attribute__((always_inline)) {
-      return DOC ? prm[r] : (ge.tile * a.bm + r < ge.M * a.pack ? ge.tile * a.bm + r : -1);
+      return DOC ? prm[r] : (ge.tile * la.bm + r < ge.M * la.pack ? ge.tile * la.bm + r : -1);
     };
     auto finish_row = [&](int prow, int c, f32x4 acc) __attribute__((always_inline)) {
-      const int mrow = DOC ? prow : prow / a.pack, mh = DOC ? 0 : prow - mrow * a.pack;
-      const typename E::vec2 x0 = E::cvt2(acc[0] * a.scale, acc[1] * a.scale);
-      const typename E::vec2 x1 = E::cvt2(acc[2] * a.scale, acc[3] * a.scale);
+      const int mrow = DOC ? prow : prow / la.pack, mh = DOC ? 0 : prow - mrow * la.pack;
+      const typename E::vec2 x0 = E::cvt2(acc[0] * la.scale, acc[1] * la.scale);
+      const typename E::vec2 x1 = E::cvt2(acc[2] * la.scale, acc[3] * la.scale);
       typename E::vec4 x = {x0[0], x0[1], x1[0], x1[1]};
-      *reinterpret_cast<typename E::vec4*>(dqp + mh * a.dq_hs + int64_t(mrow) * a.dq_rs + 4 * c) = x;
+      *reinterpret_cast<typename E::vec4*>(dqp + mh * la.dq_hs + int64_t(mrow) * la.dq_rs + 4 * c) = x;
     };
     // NS chunk slots of IT steps each: 16 loads in flight per thread whatever the number of chunks
     auto merge_batched = [&](auto it_c, auto ns_c) __attribute__((always_inline)) {
@@ -345,32 +350,31 @@ void bwd_dq_kernel(const KArgs a) {
   if (!halved) __syncthreads();
   if (writer) {
     char* patch = smem + (halved ? qc.rb * (16 * DBN * 64 * 4) : wave * row_patch_bytes<D>());
-    store_rows_through_lds<E, D, DBN>(patch, dq, a.scale, [&](const int r) -> T* {
-      const int rr = __shfl(row, r), hh = DOC ? 0 : __shfl(qc.hg, r);
-      return rr >= 0 ? dqp + hh * a.dq_hs + int64_t(rr) * a.dq_rs : nullptr;
+    store_rows_through_lds<E, D, DBN>(patch, dq, la.scale, [&](const int r) -> T* {
+      const int rr = __shfl(row, r), hh = GEN ? __shfl(qc.hg, r) : 0;
+      return rr >= 0 ? dqp + hh * la.dq_hs + int64_t(rr) * la.dq_rs : nullptr;
     });
   }
   FA_STAMP(g_trace_dq, 4, FA_CLOCK());
 }
 
 
-template <typename Tag, int D, bool CAUSAL, bool DOC>
+template <typename Tag, int D, bool CAUSAL, int MODE>
 static int launch_one(const KArgs& a, hipStream_t s) {
   constexpr int BN = 64;
-  const int slots = DOC ? a.Pp / 128 + split_extra(a) : dense_slots(a);
-  const int bhs = DOC ? a.B * a.H : (a.qtab != nullptr ? a.nHp : a.B * a.nHp);
   const size_t lds = 4 * BN * (D < 32 ? 32 : D) * 2 + 2 * BN * 4;  // K, V double buffered + key ids
-  auto kern = bwd_dq_kernel<Tag, D, CAUSAL, DOC>;
+  auto kern = bwd_dq_kernel<Tag, D, CAUSAL, MODE>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  hipLaunchKernelGGL(kern, dim3(grid_blocks(slots, bhs)), dim3(256), lds, s, a);
+  hipLaunchKernelGGL(kern, dim3(grid_blocks(launch_slots<MODE>(a), launch_groups<MODE>(a))), dim3(256), lds, s, a);
   return (int)hipGetLastError();
 }
 
 template <typename Tag, int D>
 static int launch_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) {
-  if (causal) return doc ? launch_one<Tag, D, true, true>(a, s) : launch_one<Tag, D, true, false>(a, s);
-  return doc ? launch_one<Tag, D, false, true>(a, s) : launch_one<Tag, D, false, false>(a, s);
+  if (doc) return causal ? launch_one<Tag, D, true, GEO_DOC>(a, s) : launch_one<Tag, D, false, GEO_DOC>(a, s);
+  if (geo_general(a)) return causal ? launch_one<Tag, D, true, GEO_GENERAL>(a, s) : launch_one<Tag, D, false, GEO_GENERAL>(a, s);
+  return causal ? launch_one<Tag, D, true, GEO_PLAIN>(a, s) : launch_one<Tag, D, false, GEO_PLAIN>(a, s);
 }
 
 template <typename Tag>

@@ -399,6 +399,16 @@ struct KArgs {
   float scale_log2e;      // sm_scale * log2(e)
 };
 
+// The kernel arguments read again, where they are needed late: left alone, the compiler loads every argument at the
+// top of the kernel, and the ones only the end uses fill scalar registers (and, spilled, vector lanes that the tile loop
+// reads back) all the way through.
+typedef const __attribute__((address_space(4))) KArgs LateArgs;
+FA_DEV LateArgs& late_args() {
+  LateArgs* p = (LateArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+
 // Workspace layout shared by host and device code.
 struct WsLayout {
   int Hq1, Hk1;           // heads stored for eq / ek (1 when the head stride is 0)

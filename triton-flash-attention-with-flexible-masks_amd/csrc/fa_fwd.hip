@@ -35,12 +35,13 @@ constexpr int kFwdPre2 = 4;
 FA_TRACE_ARRAY(g_trace_fwd);
 #endif
 
-template <typename Tag, int D, bool CAUSAL, bool DOC>
+template <typename Tag, int D, bool CAUSAL, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2, D <= 64 ? 3 : 2)))
 void fwd_kernel(const KArgs a) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
+  constexpr bool DOC = MODE == GEO_DOC, GEN = MODE == GEO_GENERAL;
   constexpr int BN = 64, KS = D / 16;
   constexpr int DL = D < 32 ? 32 : D;  // LDS row width: D = 16 is staged as 32 columns, the upper 16 zero
   constexpr int DBN = DL / 32;
@@ -55,7 +56,7 @@ void fwd_kernel(const KArgs a) {
   // heaviest tiles first: with ids the global-row tiles sit at the end of the permuted
   // order and see the longest key ranges; without ids the last rows do
   TileGeo ge;
-  QTileCtx<CAUSAL, DOC> qc;
+  QTileCtx<CAUSAL, MODE> qc;
   int kt_first, kt_last;
   if (!tile_work(a, ge, qc, kt_first, kt_last)) return;
   const int b = ge.b, h = ge.h0, hk = ge.hk, nsplit = ge.nchunk;
@@ -66,9 +67,9 @@ void fwd_kernel(const KArgs a) {
   const T* qp = reinterpret_cast<const T*>(a.q) + b * a.q_bs + (h + qc.hg) * a.q_hs + ge.q0 * a.q_rs;
   const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + ge.k0 * a.k_rs;
   const T* vp = reinterpret_cast<const T*>(a.v) + b * a.v_bs + hk * a.v_hs + ge.k0 * a.v_rs;
-  T* op = reinterpret_cast<T*>(a.o) + b * a.o_bs + h * a.o_hs + ge.q0 * a.o_rs;
-  float* lsep = a.lse + (int64_t(b) * a.H + h) * a.M + ge.q0;
 
+  T* op0 = reinterpret_cast<T*>(a.o) + b * a.o_bs + h * a.o_hs;   // (GEO_PLAIN: formed while the first loads travel)
+  float* lsep0 = a.lse + (int64_t(b) * a.H + h) * a.M;
   // Q^T fragments (B operand): lane holds d = 16*ks + 8*g .. +7 of its query row.
   vec8 qf[KS];
 #pragma unroll
@@ -351,14 +352,26 @@ void fwd_kernel(const KArgs a) {
         for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * ca + mb[(2 + 16 * db + r) * 64] * cb;
     }
   }
+  // (where scalar registers run out; the other forms keep what the end needs, and do not wait for it here)
+  decltype(auto) la = [&]() -> decltype(auto) { if constexpr (MODE == GEO_PLAIN) return (a); else return late_args(); }();
+  T* op;
+  float* lsep;
+  if constexpr (MODE == GEO_PLAIN) {
+    op = op0; lsep = lsep0;
+  } else {
+    op = reinterpret_cast<T*>(la.o) + b * la.o_bs + h * la.o_hs + ge.q0 * la.o_rs;
+    lsep = la.lse + (int64_t(b) * la.H + h) * la.M + ge.q0;
+  }
   const bool writer = !halved || sub == 0;   // the wave that holds the rows' result
   const float l_tot = xhalf_sum(l_run);
-  if (nsplit > 1) {
+  if (MODE != GEO_PLAIN && nsplit > 1) {
     // This workgroup saw one chunk of the keys: store the unnormalised partial result; the last
     // chunk to arrive combines them (log-sum-exp merge) and writes O and LSE.
-    const int rows = DOC ? 128 : a.bm;   // rows of a partial result
-    float* po = a.sk_o + (ge.part + int64_t(ge.chunk) * ge.pstride) * (rows * D);
-    float* pml = a.sk_ml + (ge.part + int64_t(ge.chunk) * ge.pstride) * (rows * 2);
+    split_home<MODE>(la, ge);
+    const int rows = DOC ? 128 : la.bm;   // rows of a partial result
+    const int pstride = DOC ? 1 : ge.pstride;
+    float* po = la.sk_o + (ge.part + int64_t(ge.chunk) * pstride) * (rows * D);
+    float* pml = la.sk_ml + (ge.part + int64_t(ge.chunk) * pstride) * (rows * 2);
     const int rt = qc.rb * 32 + (lane & 31);   // row inside the tile
     if (g == 0 && writer && rt < rows) store_dev(pml + rt * 2, m_ref, l_tot);
 #pragma unroll
@@ -369,28 +382,28 @@ void fwd_kernel(const KArgs a) {
         f32x4 x = {o[db][4 * q4 + 0], o[db][4 * q4 + 1], o[db][4 * q4 + 2], o[db][4 * q4 + 3]};
         store_dev(po + part_index<D>(qc.rb, 4 * db + q4, lane) * 4, x);
       }
-    if (!split_arrive(a.sk_cnt + ge.cnt, nsplit)) { FA_STAMP(g_trace_fwd, 4, FA_CLOCK()); return; }
+    if (!split_arrive(la.sk_cnt + ge.cnt, nsplit)) { FA_STAMP(g_trace_fwd, 4, FA_CLOCK()); return; }
     FA_STAMP(g_trace_fwd, 6, FA_CLOCK());
     // merge: the whole workgroup walks the tile, one float4 of one row per thread and step.  The
     // partial results come through device-scope loads, each a round trip of its own: up to eight chunks are
     // requested together, four or two steps of them (16 + 16 loads in flight per thread), instead of one by one.
     constexpr int C4 = D / 4;
-    const float* bo = a.sk_o + int64_t(ge.part) * (rows * D);
-    const float* bml = a.sk_ml + int64_t(ge.part) * (rows * 2);
-    const int64_t so = int64_t(ge.pstride) * (rows * D), sml = int64_t(ge.pstride) * (rows * 2);   // from chunk to chunk
-    const int* prm = DOC ? a.perm + b * a.pm_bs + h * a.pm_hs + ge.tile * 128 : nullptr;
+    const float* bo = la.sk_o + int64_t(ge.part) * (rows * D);
+    const float* bml = la.sk_ml + int64_t(ge.part) * (rows * 2);
+    const int64_t so = int64_t(pstride) * (rows * D), sml = int64_t(pstride) * (rows * 2);   // from chunk to chunk
+    const int* prm = DOC ? la.perm + b * la.pm_bs + h * la.pm_hs + ge.tile * 128 : nullptr;
     // row of the tile -> row of the operands (with ids), or packed row (without), -1: no such row
     auto row_of = [&](int r) __attribute__((always_inline)) {
-      return DOC ? prm[r] : (ge.tile * a.bm + r < ge.M * a.pack ? ge.tile * a.bm + r : -1);
+      return DOC ? prm[r] : (ge.tile * la.bm + r < ge.M * la.pack ? ge.tile * la.bm + r : -1);
     };
     auto finish_row = [&](int prow, int c, float mmax, float lsum, f32x4 acc) __attribute__((always_inline)) {
       const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
-      const int mrow = DOC ? prow : prow / a.pack, mh = DOC ? 0 : prow - mrow * a.pack;
-      if (c == 0) lsep[int64_t(mh) * a.M + mrow] = lsum > 0.f ? mmax + fast_log2(lsum) : -INFINITY;
+      const int mrow = DOC ? prow : prow / la.pack, mh = DOC ? 0 : prow - mrow * la.pack;
+      if (c == 0) lsep[int64_t(mh) * la.M + mrow] = lsum > 0.f ? mmax + fast_log2(lsum) : -INFINITY;
       const typename E::vec2 x0 = E::cvt2(acc[0] * inv, acc[1] * inv);
       const typename E::vec2 x1 = E::cvt2(acc[2] * inv, acc[3] * inv);
       typename E::vec4 x = {x0[0], x0[1], x1[0], x1[1]};
-      *reinterpret_cast<typename E::vec4*>(op + mh * a.o_hs + int64_t(mrow) * a.o_rs + 4 * c) = x;
+      *reinterpret_cast<typename E::vec4*>(op + mh * la.o_hs + int64_t(mrow) * la.o_rs + 4 * c) = x;
     };
     // NS chunk slots of IT steps each: 16 + 16 loads in flight per thread whatever the number of chunks
     auto merge_batched = [&](auto it_c, auto ns_c) __attribute__((always_inline)) {
@@ -469,34 +482,33 @@ void fwd_kernel(const KArgs a) {
   // done with the last tile first; a halved tile's writers use the part of LDS they have just read their partner's state from)
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if (!halved) __syncthreads();
-  if (row >= 0 && writer && g == 0) lsep[int64_t(qc.hg) * a.M + row] = l_tot > 0.f ? m_ref + fast_log2(l_tot) : -INFINITY;
+  if (row >= 0 && writer && g == 0) lsep[(GEN ? int64_t(qc.hg) * la.M : 0) + row] = l_tot > 0.f ? m_ref + fast_log2(l_tot) : -INFINITY;
   if (writer) {
     char* patch = smem + (halved ? qc.rb * ((2 + 16 * DBN) * 64 * 4) : wave * row_patch_bytes<D>());
     store_rows_through_lds<E, D, DBN>(patch, o, inv, [&](const int r) -> T* {
-      const int rr = __shfl(row, r), hh = DOC ? 0 : __shfl(qc.hg, r);
-      return rr >= 0 ? op + hh * a.o_hs + int64_t(rr) * a.o_rs : nullptr;
+      const int rr = __shfl(row, r), hh = GEN ? __shfl(qc.hg, r) : 0;
+      return rr >= 0 ? op + hh * la.o_hs + int64_t(rr) * la.o_rs : nullptr;
     });
   }
   FA_STAMP(g_trace_fwd, 4, FA_CLOCK());
 }
 
-template <typename Tag, int D, bool CAUSAL, bool DOC>
+template <typename Tag, int D, bool CAUSAL, int MODE>
 static int launch_one(const KArgs& a, hipStream_t s) {
   constexpr int BN = 64;
-  const int slots = DOC ? a.Pp / 128 + split_extra(a) : dense_slots(a);
-  const int bhs = DOC ? a.B * a.H : (a.qtab != nullptr ? a.nHp : a.B * a.nHp);
   const size_t lds = 4 * BN * (D < 32 ? 32 : D) * 2 + 2 * BN * 4;  // K, V double buffered + key ids
-  auto kern = fwd_kernel<Tag, D, CAUSAL, DOC>;
+  auto kern = fwd_kernel<Tag, D, CAUSAL, MODE>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  hipLaunchKernelGGL(kern, dim3(grid_blocks(slots, bhs)), dim3(256), lds, s, a);
+  hipLaunchKernelGGL(kern, dim3(grid_blocks(launch_slots<MODE>(a), launch_groups<MODE>(a))), dim3(256), lds, s, a);
   return (int)hipGetLastError();
 }
 
 template <typename Tag, int D>
 static int launch_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) {
-  if (causal) return doc ? launch_one<Tag, D, true, true>(a, s) : launch_one<Tag, D, true, false>(a, s);
-  return doc ? launch_one<Tag, D, false, true>(a, s) : launch_one<Tag, D, false, false>(a, s);
+  if (doc) return causal ? launch_one<Tag, D, true, GEO_DOC>(a, s) : launch_one<Tag, D, false, GEO_DOC>(a, s);
+  if (geo_general(a)) return causal ? launch_one<Tag, D, true, GEO_GENERAL>(a, s) : launch_one<Tag, D, false, GEO_GENERAL>(a, s);
+  return causal ? launch_one<Tag, D, true, GEO_PLAIN>(a, s) : launch_one<Tag, D, false, GEO_PLAIN>(a, s);
 }
 
 template <typename Tag>

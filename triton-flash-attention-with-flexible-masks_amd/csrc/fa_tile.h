@@ -258,11 +258,16 @@ struct TileIter {
 // ---------------------------------------------------------------------------
 // Where a workgroup of the forms without ids finds its work: the whole (batch, head group), or one sequence of a
 // packed batch, and which tile and chunk of it.
+// What a launch of the forward / dq kernels looks like: rows of one head in natural order, tiles of 128; the mask plan's
+// permuted order; or any of heads that share a tile, tiles of 64 rows, split key ranges, packed sequences (FwdCfg).
+// (Forms of their own because the set-up counts: 37 us is what a workgroup of a doc-masked 16K forward lives, and
+// the general form's divisions and table look-ups made it 2-4 % slower.)
+enum { GEO_PLAIN, GEO_DOC, GEO_GENERAL };
 struct TileGeo {
   int M, N, gap;         // query rows, keys and diagonal offset of the batch entry or sequence
   int b, h0, hk;         // batch, first query head of the tile, key head
   int tile, chunk, nchunk;
-  int cnt, part, pstride;   // arrival counter; partial result of chunk c: part + c * pstride
+  int cnt, part, pstride;   // arrival counter; partial result of chunk c: part + c * pstride (with ids: see split_home)
   int64_t q0, k0;        // first query row and first key of the sequence
 };
 FA_DEV TileGeo seq_geo(const KArgs& a, const SeqTile* __restrict__ e, int head) {
@@ -303,8 +308,9 @@ FA_DEV TileGeo tile_geo(const KArgs& a, int bid) {
 FA_HD int dense_slots(const KArgs& a) { return a.qtab != nullptr ? a.nQent : a.nTiles * a.dsplit; }
 FA_HD int tile_geo_blocks(const KArgs& a) { return dense_slots(a) * (a.qtab != nullptr ? a.nHp : a.B * a.nHp); }
 
-template <bool CAUSAL, bool DOC>
+template <bool CAUSAL, int MODE>
 struct QTileCtx {
+  static constexpr bool DOC = MODE == GEO_DOC, GEN = MODE == GEO_GENERAL;
   int row;    // row index of this lane's query inside its batch entry or sequence (lanes l and l^32 share it), -1 if none
   int hg;     // its head among those that share the tile (0 with ids)
   int N;      // keys
@@ -346,15 +352,16 @@ struct QTileCtx {
     int posc;   // r of this lane's row, 0 if none
     rb = wave; sub = 0; halved = false;
     if (!DOC) {
-      const int m0 = tile * a.bm, Mr = ge.M * a.pack;   // packed rows: row r is query r / pack of head r % pack
-      if ((Mr - m0 <= 64 || a.bm <= 64) && a.bmask == nullptr) { halved = true; rb = wave & 1; sub = wave >> 1; }
+      const int bm = GEN ? a.bm : 128, m0 = tile * bm;
+      const int Mr = GEN ? ge.M * a.pack : ge.M;   // packed rows: row r is query r / pack of head r % pack
+      if ((Mr - m0 <= 64 || bm <= 64) && a.bmask == nullptr) { halved = true; rb = wave & 1; sub = wave >> 1; }
       const int mw = m0 + rb * 32;
-      const int end = min(Mr, m0 + a.bm);   // (tiles of 32 rows: the waves of the second row block have none)
+      const int end = min(Mr, m0 + bm);   // (tiles of 32 rows: the waves of the second row block have none)
       row = mw + lq < end ? mw + lq : -1;
       w_rmin = mw; w_rmax = min(mw + 31, end - 1);
       if (w_rmax < w_rmin) w_rmax = -1;
       g_rmin = m0; g_rmax = end - 1;
-      if (a.pack > 1) {
+      if (GEN && a.pack > 1) {
         const int pr = row;
         if (pr >= 0) { row = pr / a.pack; hg = pr - row * a.pack; }
         w_rmin /= a.pack; if (w_rmax >= 0) w_rmax /= a.pack;
@@ -592,10 +599,10 @@ FA_DEV void chunk_range(const TileGeo& ge, int& first, int& last) {
 
 // Work of one workgroup of the forward / dq kernels, with and without ids: which tile, where its partial result goes
 // when its key range is split, and the key tiles [kt_first, kt_last) to walk.  False: nothing to do.
-template <bool CAUSAL, bool DOC>
-FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, DOC>& qc, int& kt_first, int& kt_last) {
+template <bool CAUSAL, int MODE>
+FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, MODE>& qc, int& kt_first, int& kt_last) {
   int slot, bh;
-  if constexpr (DOC) {
+  if constexpr (MODE == GEO_DOC) {
     const int nQt = a.Pp / 128;
     if (!block_to_tile(nQt + split_extra(a), a.B * a.H, nQt >= 32, slot, bh)) return false;
     ge.b = bh / a.H; ge.h0 = bh % a.H; ge.hk = ge.h0 / a.G;
@@ -608,19 +615,45 @@ FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, DOC>& qc, in
     q_work_finish(a, hd, wk);
     kt_first = qc.first_tile(a); kt_last = qc.last_tile(a);
     ge.chunk = wk.split; ge.nchunk = split_range(a, wk, kt_first, kt_last);
-    ge.cnt = bh * a.split_tiles + wk.gt; ge.part = ge.cnt * a.split_k; ge.pstride = 1;
+    ge.cnt = wk.gt; ge.part = 0; ge.pstride = 1;
     return ge.chunk < ge.nchunk;
+  } else if constexpr (MODE == GEO_PLAIN) {
+    const int nQt = (a.M + 127) / 128;
+    if (!block_to_tile(nQt, a.B * a.H, false, slot, bh)) return false;
+    ge.b = bh / a.H; ge.h0 = bh % a.H; ge.hk = ge.h0 / a.G;
+    ge.M = a.M; ge.N = a.N; ge.gap = a.gap; ge.q0 = ge.k0 = 0;
+    ge.tile = nQt - 1 - slot;
+    ge.chunk = 0; ge.nchunk = 1; ge.cnt = ge.part = 0; ge.pstride = 1;
+    qc.init(a, ge, threadIdx.x >> 6);
+    kt_first = qc.first_tile(a); kt_last = qc.last_tile(a);
+    return true;
   } else {
-  // the tiles of a packed batch are sorted by their length: longest first over all heads
-  if (!block_to_tile(dense_slots(a), a.qtab != nullptr ? a.nHp : a.B * a.nHp, a.qtab != nullptr, slot, bh)) return false;
-  ge = dense_geo(a, slot, bh);
-  if (ge.M < 0) return false;
-  qc.init(a, ge, threadIdx.x >> 6);
-  kt_first = qc.first_tile(a); kt_last = qc.last_tile(a);
-  chunk_range(ge, kt_first, kt_last);
-  return true;
+    // the tiles of a packed batch are sorted by their length: longest first over all heads
+    if (!block_to_tile(dense_slots(a), a.qtab != nullptr ? a.nHp : a.B * a.nHp, a.qtab != nullptr, slot, bh)) return false;
+    ge = dense_geo(a, slot, bh);
+    if (ge.M < 0) return false;
+    qc.init(a, ge, threadIdx.x >> 6);
+    kt_first = qc.first_tile(a); kt_last = qc.last_tile(a);
+    chunk_range(ge, kt_first, kt_last);
+    return true;
   }
 }
+// With ids the home of a split tile's partial results is worked out where it is needed (TileGeo::cnt holds the tile's number
+// among the splittable ones until then).
+template <int MODE, typename A>
+FA_DEV void split_home(const A& a, TileGeo& ge) {
+  if constexpr (MODE == GEO_DOC) {
+    ge.cnt = (ge.b * a.H + ge.h0) * a.split_tiles + ge.cnt;
+    ge.part = ge.cnt * a.split_k;
+    ge.pstride = 1;
+  }
+}
+// slots and (batch, head group) pairs of a launch
+template <int MODE>
+FA_HD int launch_slots(const KArgs& a) { return MODE == GEO_DOC ? a.Pp / 128 + split_extra(a) : MODE == GEO_PLAIN ? (a.M + 127) / 128 : dense_slots(a); }
+template <int MODE>
+FA_HD int launch_groups(const KArgs& a) { return MODE != GEO_GENERAL ? a.B * a.H : a.qtab != nullptr ? a.nHp : a.B * a.nHp; }
+inline bool geo_general(const KArgs& a) { return a.pack > 1 || a.dsplit > 1 || a.bm != 128 || a.qtab != nullptr; }
 
 // A wave's 32 result rows on their way out.  The accumulators hold a row (or key) per lane and 4 consecutive
 // columns per register quad: stored from there, a wave instruction writes 64 pieces of 8 bytes, a row apart, and
