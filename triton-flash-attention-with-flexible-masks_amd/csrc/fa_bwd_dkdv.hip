@@ -300,6 +300,7 @@ void bwd_dkdv_kernel(const KArgs a) {
     ++pair_seq;
     auto first_product = [&](const char* rows, const int qb) __attribute__((always_inline)) {
       f32x16 x = zero;
+      mfma_phase();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -317,11 +318,13 @@ void bwd_dkdv_kernel(const KArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x008, PRE, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
+      vector_phase();
       return x;
     };
     auto second_product = [&](const char* tr, const vec8 (&yf)[2], const int qb) __attribute__((always_inline)) {
       // NM transposed fragments (two LDS reads each), requested PRE fragments ahead of their MFMA
       // in program order
+      mfma_phase();
       constexpr int NM = 2 * DBN, PRE = NM < kKvPre2 ? NM : kKvPre2;
       auto fetch = [&](const int i) __attribute__((always_inline)) {
         const int half = i / DBN, db = i % DBN;
@@ -443,6 +446,7 @@ void bwd_dkdv_kernel(const KArgs a) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       f32x16 x = zero, dp = zero;
+      mfma_phase();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -462,6 +466,7 @@ void bwd_dkdv_kernel(const KArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x008, PRE, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
+      vector_phase();
       // S -> P, masks, dS = P * (dP - delta) for this lane's 16 query rows of the block
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
@@ -482,6 +487,7 @@ void bwd_dkdv_kernel(const KArgs a) {
       // requested PRE MFMAs ahead in program order, P and dS are converted just in time; the
       // scheduling barriers pin that order.
       {
+        mfma_phase();
         constexpr int NM = 4 * DBN, PRE = NM < kKvPre2 + 1 ? NM : kKvPre2 + 1;
         auto fetch = [&](const int i) __attribute__((always_inline)) {
           const int half = i / (2 * DBN), db = (i % (2 * DBN)) / 2;

@@ -134,6 +134,7 @@ void bwd_dq_kernel(const KArgs a) {
     // one 32-key block of the tile (kb a literal on the usual path: every offset an immediate)
     auto block = [&](const int kb) __attribute__((always_inline)) {
       f32x16 s = zero, dp = zero;
+      mfma_phase();
       __builtin_amdgcn_sched_barrier(0);
       // S and dP are accumulated alternately (an MFMA that accumulates onto the result of the MFMA
       // issued right before it waits a full extra MFMA time), operands a few LDS reads ahead.
@@ -155,6 +156,7 @@ void bwd_dq_kernel(const KArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x008, PRE, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
+      vector_phase();
       // P and dS for this lane's 16 keys of the block
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -173,6 +175,7 @@ void bwd_dq_kernel(const KArgs a) {
       // program order, dS is converted just in time; the scheduling barriers pin that order (left
       // to itself the scheduler puts every read right before its MFMA).
       {
+        mfma_phase();
         constexpr int NM = 2 * DBN, PRE = NM < kDqPre2 ? NM : kDqPre2;
         auto fetch = [&](const int i) __attribute__((always_inline)) {
           const int half = i / DBN, db = i % DBN;

@@ -269,6 +269,11 @@ FA_DEV void settle(V& x) {
 FA_DEV void settle(float& x) { asm volatile("" : "+v"(x)); }
 FA_DEV void settle(int& x) { asm volatile("" : "+v"(x)); }
 
+// Issue priority of a wave while it feeds the matrix pipe.  Two waves share a SIMD; the one that has MFMAs to issue goes
+// first, and the other's softmax fills the slots in between: 0.5 - 3 % of the kernels' times.
+FA_DEV void mfma_phase() { __builtin_amdgcn_s_setprio(1); }
+FA_DEV void vector_phase() { __builtin_amdgcn_s_setprio(0); }
+
 FA_DEV float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 FA_DEV float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 

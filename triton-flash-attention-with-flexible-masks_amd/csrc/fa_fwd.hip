@@ -139,6 +139,7 @@ void fwd_kernel(const KArgs a) {
     const bool need_lim = (flags & TF_LIM) != 0, need_doc = (flags & TF_DOC) != 0;
 
     f32x16 s[2];
+    mfma_phase();
     __builtin_amdgcn_sched_barrier(0);
     // Two accumulator chains are fed alternately: an MFMA that accumulates onto the result of the MFMA
     // issued right before it waits a full extra MFMA time, two interleaved chains do not.  With both
@@ -180,6 +181,7 @@ void fwd_kernel(const KArgs a) {
         for (int r = 0; r < 16; ++r) s[0][r] += s[1][r];
       }
     }
+    vector_phase();
     if (need_lim) {
       asm volatile("" ::: "memory");  // keep this a real (wave-uniform) branch: never if-converted
       const int rel = qc.lim_i - n0 - 4 * g;
@@ -263,6 +265,7 @@ void fwd_kernel(const KArgs a) {
     // PRE MFMAs ahead in program order, P is converted just in time; the scheduling barriers pin
     // that order (left to itself the scheduler puts every read right before its MFMA).
     {
+      mfma_phase();
       constexpr int NPV = 2 * NB * DBN, PRE = NPV < kFwdPre2 ? NPV : kFwdPre2;
       auto fetch = [&](const int i) __attribute__((always_inline)) {
         const int c16 = i / DBN, db = i % DBN;
