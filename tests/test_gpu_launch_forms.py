@@ -26,6 +26,9 @@ FORWARD_CASES = [
     (1, 6, 2, 43, 2500, 64, torch.float16, True, 300, 0),
     (1, 2, 2, 129, 20000, 128, torch.bfloat16, False, 0, 0),
     (2, 12, 4, 333, 333, 128, torch.bfloat16, True, 0, 0),     # short prompt, groups of three
+    (1, 8, 2, 200, 200, 64, torch.bfloat16, True, 0, 0),       # the decode form with several tiles, the last one partly filled
+    (1, 3, 3, 95, 700, 128, torch.float16, True, 150, 0),
+    (2, 4, 4, 129, 64, 32, torch.bfloat16, False, 0, 0),       # ... more queries than keys
 ]
 
 

@@ -103,10 +103,16 @@ inline SplitCfg split_config(int B, int H, int M, int N, int D, uint64_t budget 
 //          read the same K / V sit on one XCD, and a short query block fills tiles instead of padding them.
 //   bm   : 128 rows, or 64 when 128-row tiles would leave CUs without a workgroup (the 64-row form splits every key
 //          tile between two waves, see QTileCtx::halved).
-//   dec  : at most 32 packed rows: the form of fa_decode.hip.
+//   dec  : few rows in all: the form of fa_decode.hip, tiles of 32 packed rows.
 //   split: chunks of the key range; only with FA_FLAG_SPLIT_KEYS, which gives the launch a workspace for them.
 // ---------------------------------------------------------------------------
 constexpr int kCUs = 256;
+// The decode form also takes problems of at most this many 32-row tiles (one workgroup to a CU) whose rows see at most
+// kDecKeys keys on average: four waves on different key blocks are a shorter chain than four on the same tile.  1 x 8
+// heads x 1000 rows, causal 17.8 -> 15.3 us, 4 x 2 x 4 heads x 64 rows on 1000 keys 18.3 -> 14.8; with more tiles it takes a
+// second round (336 of them: 11.2 -> 14.9), on longer ranges the 64-row form reads K and V half as often (32 heads x 128
+// rows on 2000 keys 21.7 -> 24.2).
+constexpr int kDecTiles = kCUs, kDecKeys = 1024;
 struct FwdCfg { int pack, bm, tiles, split; bool dec; };
 // Chunks for `wgs` tiles of `steps` steps each: the cheapest total by a model of rounds x (set-up + steps of a chunk)
 // + merging, in units of one step; `slots` workgroups run at a time.  A chunk keeps at least `min_steps` steps.
@@ -137,12 +143,13 @@ inline FwdCfg fwd_config(const fa_params* p) {
   c.pack = p->H / p->Hk;
   const int64_t rows = int64_t(p->M) * c.pack, bh = int64_t(p->B) * p->Hk;
   const int nk = p->window > 0 && p->causal && p->window + p->M < p->N ? p->window + p->M : p->N;   // keys a tile can see
-  if (rows <= 32) {
-    c.dec = true; c.bm = 32; c.tiles = 1;
+  const int seen = p->causal && p->N >= p->M ? nk - (nk == p->N ? p->M / 2 : 0) : nk;   // keys a row sees on average
+  if (rows <= 32 || (bh * ((rows + 31) / 32) <= kDecTiles && seen <= kDecKeys)) {
+    c.dec = true; c.bm = 32; c.tiles = int((rows + 31) / 32);
     // a step: four waves x 32 keys.  64 KB at D = 128 take a CU 3 us at the rate the whole card reads; setting a
     // workgroup up takes about as long, handing the result over and merging one and a half steps
     const float rel = 128.f / p->D;
-    if (p->flags & FA_FLAG_SPLIT_KEYS) c.split = pick_split(bh, (nk + 127) / 128, kCUs, 1.2f * rel, 1.5f * rel, 2);
+    if (p->flags & FA_FLAG_SPLIT_KEYS) c.split = pick_split(bh * c.tiles, (nk + 127) / 128, kCUs, 1.2f * rel, 1.5f * rel, 2);
     return c;
   }
   c.tiles = int((rows + 127) / 128);
