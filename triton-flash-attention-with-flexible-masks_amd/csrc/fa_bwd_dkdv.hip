@@ -200,12 +200,25 @@ void bwd_dkdv_kernel(const KArgs a) {
     for (int i = 0; i < Loader::PER; ++i) ri_t[i] = pmp[tile * BQ + g_rit[i]];
     ri_aux = pmp[tile * BQ + lane];
   };
-  auto load_tile = [&](int tile, int bufi) {
+  // Number j of the 2 * PER row loads of a tile (no ids), Q and dO in turn.
+  constexpr int NPART = 2 * Loader::PER;
+  auto load_part = [&](int tile, int bufi, int j) __attribute__((always_inline)) {
+    const int i = j >> 1;
+    const Loader& ld = (j & 1) ? ldO : ldQ;
+    if (Loader::NI % NW == 0 || i * NW + wave < Loader::NI)
+      buf_load_lds16(ld.rsrc, smem + ((j & 1) ? 2 + bufi : bufi) * TILE_BYTES + (i * NW + wave) * 1024, ld.voff,
+                     (tile * BQ + i * NW * Loader::RPI) * ld.row_bytes);
+  };
+  // A row load holds its wave until the CU's one address unit takes it (16 clocks each, four waves at once): the
+  // role-split form without ids issues two right behind the barrier and the rest between the phases of the tile
+  // (sliding window 16K 659 -> 648 us, block mask 1238 -> 1212; with ids, whose loads are gathered, no gain).
+  constexpr int kHead = (SPLIT && !DOC) ? 2 : NPART;
+  auto load_tile = [&](int tile, int bufi, int parts) __attribute__((always_inline)) {
     const char* aux = smem + AUX_OFF + bufi * AUX_BYTES;
     if (!DOC) {
       const int m0 = tile * BQ;
-      ldQ.issue(m0, smem + bufi * TILE_BYTES);
-      ldO.issue(m0, smem + (2 + bufi) * TILE_BYTES);
+#pragma unroll
+      for (int j = 0; j < parts; ++j) load_part(tile, bufi, j);
       const int r = m0 + lane < M ? m0 + lane : M - 1;
       if (wave < 2) glb_load_lds4(auxp + r, aux + wave * 256);
     } else {
@@ -291,12 +304,17 @@ void bwd_dkdv_kernel(const KArgs a) {
   // (LDS-heavy and MFMA-heavy phases of different waves overlap); the gradient wave computes dP of
   // both blocks before it needs the first P.  The wait is bounded, so every wave reaches the end
   // of the kernel whatever happens.
-  auto compute_flag = [&](const int BUF, const int cur, const int flags, const int tile_id) __attribute__((always_inline)) {
+  auto compute_flag = [&](const int BUF, const int cur, const int flags, const int tile_id, const int next) __attribute__((always_inline)) {
+    auto more = [&](const int k) __attribute__((always_inline)) {   // the k-th third of the next tile's row loads that are still to be issued
+      if (kHead == NPART || next < 0) return;
+#pragma unroll
+      for (int j = kHead + k * (NPART - kHead) / 3; j < kHead + (k + 1) * (NPART - kHead) / 3; ++j) load_part(next, BUF ^ 1, j);
+    };
     const char* lqt = smem + BUF * TILE_BYTES;
     const char* ldo = smem + (2 + BUF) * TILE_BYTES;
     const char* aux = smem + AUX_OFF + BUF * AUX_BYTES;
     const int m0 = cur * BQ;  // natural order only
-    if (flags & TF_SKIP) return;   // decided per wave pair: both roles agree
+    if (flags & TF_SKIP) { more(0); more(1); more(2); return; }   // decided per wave pair: both roles agree
     ++pair_seq;
     auto first_product = [&](const char* rows, const int qb) __attribute__((always_inline)) {
       f32x16 x = zero;
@@ -429,9 +447,37 @@ void bwd_dkdv_kernel(const KArgs a) {
         }
       }
     };
-    lse_load(0); x[0] = first_product(rows, 0); score_part(0);
-    lse_load(1); x[1] = first_product(rows, 1); score_part(1);
-    grad_part(0); second_product(trp, yf[0], 0);
+    // (In the 128-key form the first products of the two blocks are fed alternately: an MFMA that accumulates onto the
+    // one issued right before it waits for it, two chains do not.  Dense 16K 4355 -> 4315 us; the 64-key form, where
+    // another workgroup's waves fill those gaps and the score wave publishes its first P later this way, 0.5 % slower.)
+    if constexpr (NKB == 4) {
+      lse_load(0);
+      mfma_phase();
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int NF = 2 * KS, PF = NF < kKvPre ? NF : kKvPre;
+      auto fetch = [&](const int i) __attribute__((always_inline)) { return lds_row8<E>(rows + lo.row[i / 2] + (i & 1) * 32 * DL * 2); };
+      vec8 rf[NF];
+      x[0] = zero; x[1] = zero;
+#pragma unroll
+      for (int i = 0; i < PF; ++i) rf[i] = fetch(i);
+#pragma unroll
+      for (int i = 0; i < NF; ++i) {
+        if (i + PF < NF) rf[i + PF] = fetch(i + PF);
+        __builtin_amdgcn_sched_barrier(0);
+        x[i & 1] = E::mfma32(rf[i], frag[i / 2], x[i & 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      vector_phase();
+      more(0);
+      lse_load(1);
+      score_part(0);
+      more(1);
+      score_part(1);
+    } else {
+      lse_load(0); x[0] = first_product(rows, 0); more(0); score_part(0);
+      lse_load(1); x[1] = first_product(rows, 1); more(1); score_part(1);
+    }
+    grad_part(0); more(2); second_product(trp, yf[0], 0);
     grad_part(1); second_product(trp, yf[1], 1);
   };
 
@@ -522,8 +568,8 @@ void bwd_dkdv_kernel(const KArgs a) {
       }
     }
   };
-  auto compute = [&](const int BUF, const int cur, const int flags, const int tile_id) __attribute__((always_inline)) {
-    if constexpr (SPLIT) compute_flag(BUF, cur, flags, tile_id);
+  auto compute = [&](const int BUF, const int cur, const int flags, const int tile_id, const int next) __attribute__((always_inline)) {
+    if constexpr (SPLIT) compute_flag(BUF, cur, flags, tile_id, next);
     else compute_both(BUF, cur, flags, tile_id);
   };
 
@@ -612,7 +658,7 @@ void bwd_dkdv_kernel(const KArgs a) {
     FA_TRACE_ONLY(if (gi == 0) FA_STAMP(g_trace_dkdv, 2, FA_CLOCK());)
     if (cur >= 0) {
       if (DOC) fetch_idx(cur);
-      load_tile(cur, 0);
+      load_tile(cur, 0, NPART);
       if (DOC && nxt >= 0) fetch_idx(nxt);
     }
     if (LATE_SETTLE && gi == 0) {
@@ -627,9 +673,9 @@ void bwd_dkdv_kernel(const KArgs a) {
       wait_async_loads();
       __syncthreads();
       FA_TRACE_ONLY(if (!tr_first) { FA_STAMP(g_trace_dkdv, 3, FA_CLOCK()); tr_first = true; })
-      if (nxt >= 0) load_tile(nxt, 1);
+      if (nxt >= 0) load_tile(nxt, 1, kHead);
       if (DOC && nxt2 >= 0) fetch_idx(nxt2);
-      compute(0, cur, cur_fl, cur_id);
+      compute(0, cur, cur_fl, cur_id, nxt);
       FA_TRACE_ONLY(++tr_tiles;)
       cur = nxt; cur_fl = nxt_fl; cur_id = nxt_id; nxt = nxt2; nxt_fl = nxt2_fl; nxt_id = nxt2_id;
       if (cur < 0) break;
@@ -637,9 +683,9 @@ void bwd_dkdv_kernel(const KArgs a) {
       if (nxt >= 0) { nxt2 = it.next(dec); nxt2_fl = it.flags; nxt2_id = it.value; }
       wait_async_loads();
       __syncthreads();
-      if (nxt >= 0) load_tile(nxt, 0);
+      if (nxt >= 0) load_tile(nxt, 0, kHead);
       if (DOC && nxt2 >= 0) fetch_idx(nxt2);
-      compute(1, cur, cur_fl, cur_id);
+      compute(1, cur, cur_fl, cur_id, nxt);
       FA_TRACE_ONLY(++tr_tiles;)
       cur = nxt; cur_fl = nxt_fl; cur_id = nxt_id; nxt = nxt2; nxt_fl = nxt2_fl; nxt_id = nxt2_id;
     }
