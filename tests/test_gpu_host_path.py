@@ -81,3 +81,37 @@ def test_calls_the_native_path_leaves_to_python():
     assert torch.equal(attention(odd, odd, odd, True), attention(odd.contiguous(), odd.contiguous(), odd.contiguous(), True))
     ids = torch.zeros(1, 2, 70, dtype=torch.int16, device="cuda") - 1
     assert torch.equal(attention(q, q, q, True, None, ids, ids, 1), attention(q, q, q, True, None, ids.int(), ids.int(), 1))
+
+
+def test_transforms_tracers_and_subclasses_stay_with_python():
+    """What passes a C++ function by would be lost there: a tangent, a trace, a subclass, a function transform."""
+    import torch.autograd.forward_ad as fwAD
+    from flash_mi355 import attention, attention_varlen
+    q, k, v = (torch.randn(1, 2, 64, 64, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    cu = torch.tensor([0, 20, 64], device="cuda", dtype=torch.int32)
+    packed = [t[0].transpose(0, 1).contiguous() for t in (q, k, v)]
+    want = attention(q, k, v, True)
+    with fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp|forward"):
+        attention(fwAD.make_dual(q, torch.ones_like(q)), k, v, True)
+    with fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp|forward"):
+        attention_varlen(fwAD.make_dual(packed[0], torch.ones_like(packed[0])), *packed[1:], cu, causal=True)
+    for f in (lambda x: torch.func.vmap(lambda y: attention(y[None], k, v, True))(x), lambda x: torch.func.grad(lambda y: attention(y, k, v, True).sum())(x)):
+        with pytest.raises(RuntimeError, match="setup_context|functorch"):
+            f(q)
+
+    class Sub(torch.Tensor):
+        pass
+    assert type(attention(q.as_subclass(Sub), k, v, True)) is Sub
+    with pytest.raises(AssertionError):   # sizes are tensors there, and the feature size is no longer one of the known ones
+        torch.jit.trace(lambda a, b, c: attention(a, b, c, True), (q, k, v), check_trace=False)
+    assert torch.equal(attention(torch.nn.Parameter(q), k, v, True).detach(), want)
+
+
+def test_saved_tensor_hooks_see_what_the_node_keeps():
+    from flash_mi355 import attention
+    q, k, v = (torch.randn(1, 2, 300, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
+    want = torch.autograd.grad(attention(q, k, v, True).sum(), (q, k, v))
+    with torch.autograd.graph.save_on_cpu():
+        out = attention(q, k, v, True)
+    got = torch.autograd.grad(out.sum(), (q, k, v))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

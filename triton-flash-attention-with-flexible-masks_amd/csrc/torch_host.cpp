@@ -11,12 +11,14 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <cmath>
 #include <limits>
@@ -157,7 +159,6 @@ struct AttentionBackward : public torch::autograd::Node {
     Problem y = x;
     y.q = q.unpack(); y.k = k.unpack(); y.v = v.unpack(); y.eq = eq.unpack(); y.ek = ek.unpack(); y.qpos = qpos.unpack();
     const Tensor o_ = o.unpack(self), lse_ = lse.unpack(), plan_ = plan.unpack();
-    if (!grads[0].defined() && !(grads.size() > 1 && grads[1].defined())) return {Tensor(), Tensor(), Tensor()};
     at::NoGradGuard no_grad;
     return backward(y, o_, lse_, plan_, grads[0], grads.size() > 1 ? grads[1] : Tensor());
   }
@@ -201,10 +202,17 @@ std::pair<Tensor, Tensor> run(const Problem& x, fa_params& p, bool want_lse) {
 }
 
 // -- arguments ----------------------------------------------------------------------------------------------------------
+// A tensor the kernels may read as it is.  Subclasses and dual tensors (the node has no forward-mode rule) are for the
+// Python classes, which serve them or refuse them.
 bool tensor_arg(PyObject* a, Tensor& t) {
-  if (!THPVariable_Check(a)) return false;
+  if (!THPVariable_CheckExact(a)) return false;
   t = THPVariable_Unpack(a);
-  return t.defined() && !t.unsafeGetTensorImpl()->is_python_dispatch();
+  return t.defined() && t.has_storage() && !t.unsafeGetTensorImpl()->is_python_dispatch() && !t._fw_grad(0).defined();
+}
+// ... and so is every call under a tracer, which would record the allocations and not the launches, or a function
+// transform (vmap, grad, jvp of torch.func), whose tensors are wrappers without memory.
+bool plain_call() {
+  return !torch::jit::tracer::isTracing() && !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
 bool int_arg(PyObject* a, int& v) {
   if (a == Py_None) { v = 0; return true; }
@@ -256,7 +264,7 @@ PyObject* finish(const Problem& x, bool want_lse) {
 PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Problem x;
-  if (n != 12 || !tensor_arg(a[0], x.q) || !tensor_arg(a[1], x.k) || !tensor_arg(a[2], x.v)) Py_RETURN_NONE;
+  if (n != 12 || !plain_call() || !tensor_arg(a[0], x.q) || !tensor_arg(a[1], x.k) || !tensor_arg(a[2], x.v)) Py_RETURN_NONE;
   if (x.q.dim() != 4 || x.k.dim() != 4 || x.v.dim() != 4) Py_RETURN_NONE;
   const auto qs = x.q.sizes(), ks = x.k.sizes();
   if (ks != x.v.sizes() || qs[3] != ks[3] || qs[0] != ks[0] || !fits(qs[0] * qs[1]) || !fits(qs[2]) || !fits(ks[2])) Py_RETURN_NONE;
@@ -299,7 +307,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* attention_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Problem x;
-  if (n != 8 || !tensor_arg(a[0], x.q) || !tensor_arg(a[1], x.k) || !tensor_arg(a[2], x.v) || !tensor_arg(a[3], x.eq)) Py_RETURN_NONE;
+  if (n != 8 || !plain_call() || !tensor_arg(a[0], x.q) || !tensor_arg(a[1], x.k) || !tensor_arg(a[2], x.v) || !tensor_arg(a[3], x.eq)) Py_RETURN_NONE;
   const bool same = a[4] == Py_None || a[4] == a[3];
   if (same) x.ek = x.eq;
   else if (!tensor_arg(a[4], x.ek)) Py_RETURN_NONE;
