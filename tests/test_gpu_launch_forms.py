@@ -178,3 +178,43 @@ def test_mask_plan_forms(M, N, per_head, id_dtype, qpos):
     """The one-workgroup plan and the three-launch plan on both sides of the size where one takes over from the other."""
     from tests.test_gpu_parity import _run_case
     _run_case(1, 2, 2, M, N, 32, torch.bfloat16, True, True, seed=8, per_head_ids=per_head, id_dtype=id_dtype, qpos=qpos)
+
+
+# B, H, Hk, M, N, D, dtype, causal, kind
+SHARED_CASES = [
+    (1, 2, 2, 1, 1, 128, torch.bfloat16, True, "plain"), (1, 4, 1, 65, 65, 64, torch.float16, True, "plain"),
+    (2, 8, 2, 500, 777, 128, torch.bfloat16, True, "plain"), (1, 8, 8, 1300, 1300, 128, torch.bfloat16, False, "plain"),
+    (1, 2, 2, 129, 5000, 128, torch.bfloat16, True, "plain"), (1, 8, 4, 900, 900, 64, torch.bfloat16, True, "window"),
+    (1, 8, 8, 1000, 1000, 128, torch.bfloat16, True, "prefix"), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, "block"),
+    (2, 4, 4, 333, 333, 64, torch.float16, True, "block"), (1, 4, 4, 700, 900, 128, torch.bfloat16, True, "doc"),
+    (2, 4, 2, 257, 257, 64, torch.bfloat16, True, "doc"), (1, 2, 2, 3000, 3000, 128, torch.bfloat16, True, "doc"),
+]
+
+
+@pytest.mark.parametrize("case", SHARED_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-%s-c%d-%s" % (*c[:6], str(c[6])[6:], *c[7:]))
+def test_backward_in_one_launch(case):
+    """dq and dk/dv side by side in one launch give the bits of the separate launches (which a gradient of LSE, here of zeros, takes)."""
+    from flash_mi355 import attention, attention_with_lse, workloads as W
+    B, H, Hk, M, N, D, dtype, causal, kind = case
+    print("case", case, flush=True)
+    q, k, v, do = (t.cuda() for t in _tensors(B, H, Hk, M, N, D, dtype, 11))
+    args, kw = (), {}
+    if kind == "doc":
+        ids = np.stack([W.doc_ids_uniform(np.random.default_rng(4), N, 16, 200, 0.05) for _ in range(B)])
+        ek = torch.from_numpy(ids).cuda()[:, None]
+        args = (None, ek[:, :, N - M:].expand(B, H, M), ek.expand(B, H, N), 1)
+    elif kind == "block":
+        n = -(-M // 64)
+        kw = {"block_mask": (torch.rand(1, 1, n, n, generator=torch.Generator().manual_seed(3)) < 0.4).cuda() | torch.eye(n, dtype=torch.bool, device="cuda")}
+    elif kind != "plain":
+        kw = {kind: 170}
+    grads = []
+    for f in (attention, attention_with_lse):
+        x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        out = f(*x, causal, *args, **kw)
+        if f is attention:
+            grads.append(torch.autograd.grad(out, x, do))
+        else:
+            grads.append(torch.autograd.grad(out, x, (do, torch.zeros(B, H, M, device="cuda"))))
+    for a, b in zip(*grads):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)

@@ -335,6 +335,11 @@ extern "C" int fa_bwd(const fa_params* p, void* stream) {
     if (int e = launch_bwd_dq_f32(a, p->D, causal, doc, s)) return finish(e);
     return finish(launch_bwd_dkdv_f32(a, p->D, causal, doc, s));
   }
+  if (bwd_in_one(a, p->D, causal, doc)) {
+    if (int e = launch_bwd_delta(a, p->dtype, p->D, s)) return finish(e);
+    a.dq_delta = 0;
+    return finish(launch_bwd_both(a, p->dtype, p->D, causal, doc, s));
+  }
   if (int e = launch_bwd_dq(a, p->dtype, p->D, causal, doc, s)) return finish(e);
   return finish(launch_bwd_dkdv(a, p->dtype, p->D, causal, doc, s));
 }

@@ -47,6 +47,10 @@ FA_TRACE_ARRAY(g_trace_dkdv);
 #endif
 
 }  // namespace fa
+#ifdef FA_TRACE
+namespace fa { namespace { FA_TRACE_ARRAY(g_trace_dq); } }   // stamps of dq workgroups that share a launch: not read
+#endif
+#include "fa_dq_body.h"
 #include "fa_dkdv_cols.h"   // the column form; its workgroups stamp the same array: 0 start, 3 tiles resident, 4 after the key loop, 5 end, 6 key blocks of wave 0, 7 chunk | 1 << 40
 namespace fa {
 
@@ -54,10 +58,9 @@ namespace fa {
 //                (fa_dkdv_cols.h) for the leading key columns that only a few global rows see; the workgroups
 //                of this form whose keys lie there leave at once.  One launch, so the column form's memory
 //                traffic overlaps the set-up latencies of this one.
+// bid: index of the workgroup.
 template <typename Tag, int D, bool CAUSAL, bool DOC, bool SPLIT, int NKB, bool COLS>
-__global__ __launch_bounds__(SPLIT ? 128 * NKB : 64 * NKB)
-__attribute__((amdgpu_waves_per_eu((D <= 32 && !COLS) ? 3 : 2, (D <= 32 && !COLS) ? 3 : 2)))
-void bwd_dkdv_kernel(const KArgs a) {
+FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
@@ -78,7 +81,6 @@ void bwd_dkdv_kernel(const KArgs a) {
   constexpr int NW = SPLIT ? 2 * NKB : NKB;
   static_assert(NW >= 4, "the four auxiliary arrays of a tile are loaded by waves 0..3");
   using Loader = TileLoader<DL, BQ, D, NW>;
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int nKt = (a.N + BK - 1) / BK;
   // With the column form in the launch, most key tiles of this form may have nothing to do here (their keys
   // belong to the column form): a workgroup then takes kColsRun key tiles, nSlots tiles apart, and steps over
@@ -86,13 +88,12 @@ void bwd_dkdv_kernel(const KArgs a) {
   // useful one (8192 of them: 50 us), a skipped tile of a run costs a comparison.
   const bool packed = !DOC && a.ktab != nullptr;   // packed sequences: the slots are the plan's key tiles, longest first
   const int nSlots = COLS ? (nKt + kColsRun - 1) / kColsRun : (packed ? a.nKent : nKt);
-  int bid = (int)blockIdx.x;   // index of the workgroup among those of its form
   if constexpr (COLS) {
     static_assert(DOC && (SPLIT ? 128 * NKB : 64 * NKB) == 256, "the column form runs with ids, 4 waves per workgroup");
     // the column form's workgroups come first: few, long, one round of them
     const int nC = dkdv_cols_blocks(a);
     const bool cols = bid < nC;
-    if (!cols) bid -= nC;
+    if (!cols) bid -= nC;   // among those of its form
     if (cols) { dkdv_cols_body<Tag, D, CAUSAL>(a, bid, smem); return; }
   }
 
@@ -724,14 +725,36 @@ void bwd_dkdv_kernel(const KArgs a) {
   FA_STAMP(g_trace_dkdv, 5, FA_CLOCK());
 }
 
+template <typename Tag, int D, bool CAUSAL, bool DOC, bool SPLIT, int NKB, bool COLS>
+__global__ __launch_bounds__(SPLIT ? 128 * NKB : 64 * NKB)
+__attribute__((amdgpu_waves_per_eu((D <= 32 && !COLS) ? 3 : 2, (D <= 32 && !COLS) ? 3 : 2)))
+void bwd_dkdv_kernel(const KArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  dkdv_body<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS>(a, (int)blockIdx.x, smem);
+}
+
+// dk/dv and dq in one launch, for problems of so few workgroups that either leaves CUs idle: they run side by side instead
+// of one after the other.  Both read delta, which a launch before this one has formed (FA_FLAG_DQ_DELTA's way would
+// make dk/dv wait for dq).  dk/dv always in workgroups of 256 threads (64 keys at D = 128), two to a CU, as dq's are.
+template <typename Tag, int D, bool CAUSAL, int MODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void bwd_both_kernel(const KArgs a, const int n_dkdv) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int bid = (int)blockIdx.x;
+  if (bid < n_dkdv) dkdv_body<Tag, D, CAUSAL, MODE == GEO_DOC, (D > 64), (D > 64 ? 2 : 4), false>(a, bid, smem);   // the longer ones first
+  else dq_body<Tag, D, CAUSAL, MODE>(a, bid - n_dkdv, smem);
+}
+
 // Query tiles per workgroup (no ids) below which the 64-key role-split form is launched.
 constexpr int kKvShortTiles = 32;
+template <int D, int NKB>
+constexpr size_t dkdv_lds() { return 4 * 64 * (D < 32 ? 32 : D) * 2 + 2 * 1024 + (D > 64 ? 2 * NKB * 2048 + 64 : 0); }
 template <typename Tag, int D, bool CAUSAL, bool DOC, int NKB, bool COLS = false>
 static int launch_nkb(const KArgs& a, hipStream_t s) {
   constexpr bool SPLIT = D > 64;
-  constexpr int BK = 32 * NKB, BQ = 64;
+  constexpr int BK = 32 * NKB;
   const int nKt = (a.N + BK - 1) / BK;
-  size_t lds = 4 * BQ * (D < 32 ? 32 : D) * 2 + 2 * 1024 + (SPLIT ? 2 * NKB * 2048 + 64 : 0);
+  size_t lds = dkdv_lds<D, NKB>();
   if (COLS && dkdv_cols_lds(D) > lds) lds = dkdv_cols_lds(D);
   auto kern = bwd_dkdv_kernel<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
@@ -786,6 +809,42 @@ static int launch_d(const KArgs& a, int D, bool causal, bool doc, hipStream_t s)
     case 16: return launch_cd<Tag, 16>(a, causal, doc, s);
     default: return -1;
   }
+}
+
+template <typename Tag, int D, bool CAUSAL, int MODE>
+static int launch_both(const KArgs& a, hipStream_t s) {
+  constexpr int NKB = D > 64 ? 2 : 4;
+  constexpr size_t lds = dkdv_lds<D, NKB>() > dq_lds<D>() ? dkdv_lds<D, NKB>() : dq_lds<D>();
+  auto kern = bwd_both_kernel<Tag, D, CAUSAL, MODE>;
+  static bool lds_allowed[64] = {};   // per kernel instantiation and device
+  if (int e = allow_lds(kern, lds, lds_allowed)) return e;
+  const int slots = MODE != GEO_DOC && a.ktab != nullptr ? a.nKent : (a.N + 32 * NKB - 1) / (32 * NKB);
+  const int n_dkdv = grid_blocks(slots, a.B * a.Hk), n_dq = grid_blocks(launch_slots<MODE>(a), launch_groups<MODE>(a));
+  hipLaunchKernelGGL(kern, dim3(n_dkdv + n_dq), dim3(256), lds, s, a, n_dkdv);
+  return (int)hipGetLastError();
+}
+template <typename Tag, int D>
+static int launch_both_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) {
+  if (doc) return causal ? launch_both<Tag, D, true, GEO_DOC>(a, s) : launch_both<Tag, D, false, GEO_DOC>(a, s);
+  if (geo_general(a)) return causal ? launch_both<Tag, D, true, GEO_GENERAL>(a, s) : launch_both<Tag, D, false, GEO_GENERAL>(a, s);
+  return causal ? launch_both<Tag, D, true, GEO_PLAIN>(a, s) : launch_both<Tag, D, false, GEO_PLAIN>(a, s);
+}
+
+// Whether a backward of these sizes takes the shared launch: all its workgroups fit the chip at once, two to a CU.
+bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
+  if (D < 64) return false;
+  if (doc && (a.gap >= kGcolMinGap || a.qpos != nullptr || !causal)) return false;   // dk/dv with its column form
+  const int BK = D > 64 ? 64 : 128;
+  const int64_t kv = int64_t(!doc && a.ktab != nullptr ? a.nKent : (a.N + BK - 1) / BK) * a.B * a.Hk;
+  const int64_t dq = doc ? int64_t(launch_slots<GEO_DOC>(a)) * launch_groups<GEO_DOC>(a)
+                         : geo_general(a) ? int64_t(launch_slots<GEO_GENERAL>(a)) * launch_groups<GEO_GENERAL>(a)
+                                          : int64_t(launch_slots<GEO_PLAIN>(a)) * launch_groups<GEO_PLAIN>(a);
+  return kv + dq <= 2 * kCUs;
+}
+int launch_bwd_both(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s) {
+  if (D == 128) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 128>(a, causal, doc, s) : launch_both_cd<fp16_t, 128>(a, causal, doc, s);
+  if (D == 64) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 64>(a, causal, doc, s) : launch_both_cd<fp16_t, 64>(a, causal, doc, s);
+  return -1;
 }
 
 #ifdef FA_TRACE

@@ -533,6 +533,8 @@ int launch_seq_plan(const fa_params* p, const FwdCfg& c, const TabLayout& w, hip
 int launch_bwd_delta(const KArgs& a, int dtype, int D, hipStream_t s);
 int launch_bwd_dq(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);
 int launch_bwd_dkdv(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);
+bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc);
+int launch_bwd_both(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);   // dq and dk/dv, delta read by both
 int read_pair_wait_expired(unsigned long long* n);   // expired pair waits of the dk/dv kernel on the current device (synchronises)
 #ifdef FA_TRACE
 int trace_read_fwd(long long* host, int n);

@@ -58,7 +58,7 @@ void fwd_kernel(const KArgs a) {
   TileGeo ge;
   QTileCtx<CAUSAL, MODE> qc;
   int kt_first, kt_last;
-  if (!tile_work(a, ge, qc, kt_first, kt_last)) return;
+  if (!tile_work(a, ge, qc, kt_first, kt_last, (int)blockIdx.x)) return;
   const int b = ge.b, h = ge.h0, hk = ge.hk, nsplit = ge.nchunk;
   FA_STAMP(g_trace_fwd, 1, FA_CLOCK()); FA_STAMP(g_trace_fwd, 7, (long long)ge.tile | ((long long)ge.chunk << 16) | ((long long)nsplit << 24));
   const int row = qc.row, rowc = qc.rowc, eq_i = qc.eq_i;

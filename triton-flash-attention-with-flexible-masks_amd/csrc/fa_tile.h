@@ -534,9 +534,6 @@ FA_DEV bool block_to_tile(int ntile, int BH, bool tile_major, int& tile_slot, in
   bh = bid % BH;
   return tile_slot < ntile;
 }
-FA_DEV bool block_to_tile(int ntile, int BH, bool tile_major, int& tile_slot, int& bh) {
-  return block_to_tile(ntile, BH, tile_major, tile_slot, bh, (int)blockIdx.x);
-}
 
 // ---------------------------------------------------------------------------
 // Work assignment of one workgroup of the forward / dq kernels, including the split of the
@@ -600,11 +597,11 @@ FA_DEV void chunk_range(const TileGeo& ge, int& first, int& last) {
 // Work of one workgroup of the forward / dq kernels, with and without ids: which tile, where its partial result goes
 // when its key range is split, and the key tiles [kt_first, kt_last) to walk.  False: nothing to do.
 template <bool CAUSAL, int MODE>
-FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, MODE>& qc, int& kt_first, int& kt_last) {
+FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, MODE>& qc, int& kt_first, int& kt_last, const int bid) {
   int slot, bh;
   if constexpr (MODE == GEO_DOC) {
     const int nQt = a.Pp / 128;
-    if (!block_to_tile(nQt + split_extra(a), a.B * a.H, nQt >= 32, slot, bh)) return false;
+    if (!block_to_tile(nQt + split_extra(a), a.B * a.H, nQt >= 32, slot, bh, bid)) return false;
     ge.b = bh / a.H; ge.h0 = bh % a.H; ge.hk = ge.h0 / a.G;
     ge.M = a.M; ge.N = a.N; ge.gap = a.gap; ge.q0 = ge.k0 = 0;
     QWork wk;
@@ -619,7 +616,7 @@ FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, MODE>& qc, i
     return ge.chunk < ge.nchunk;
   } else if constexpr (MODE == GEO_PLAIN) {
     const int nQt = (a.M + 127) / 128;
-    if (!block_to_tile(nQt, a.B * a.H, false, slot, bh)) return false;
+    if (!block_to_tile(nQt, a.B * a.H, false, slot, bh, bid)) return false;
     ge.b = bh / a.H; ge.h0 = bh % a.H; ge.hk = ge.h0 / a.G;
     ge.M = a.M; ge.N = a.N; ge.gap = a.gap; ge.q0 = ge.k0 = 0;
     ge.tile = nQt - 1 - slot;
@@ -629,7 +626,7 @@ FA_DEV bool tile_work(const KArgs& a, TileGeo& ge, QTileCtx<CAUSAL, MODE>& qc, i
     return true;
   } else {
     // the tiles of a packed batch are sorted by their length: longest first over all heads
-    if (!block_to_tile(dense_slots(a), a.qtab != nullptr ? a.nHp : a.B * a.nHp, a.qtab != nullptr, slot, bh)) return false;
+    if (!block_to_tile(dense_slots(a), a.qtab != nullptr ? a.nHp : a.B * a.nHp, a.qtab != nullptr, slot, bh, bid)) return false;
     ge = dense_geo(a, slot, bh);
     if (ge.M < 0) return false;
     qc.init(a, ge, threadIdx.x >> 6);
