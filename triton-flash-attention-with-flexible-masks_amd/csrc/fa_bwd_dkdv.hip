@@ -830,7 +830,13 @@ static int launch_both_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) 
   return causal ? launch_both<Tag, D, true, GEO_PLAIN>(a, s) : launch_both<Tag, D, false, GEO_PLAIN>(a, s);
 }
 
-// Whether a backward of these sizes takes the shared launch: all its workgroups fit the chip at once, two to a CU.
+// Whether a backward of these sizes takes the shared launch: with at most four workgroups to a CU in all (two run at a time),
+// where the drain of one launch and the start of the next weigh most.  Forward + backward, separate -> shared, D = 128: 8 heads
+// on 2 key heads, causal, 2000 / 3000 / 5000 rows (316 - 790 workgroups) 306 -> 226, 443 -> 327, 783 -> 567 us; 8 heads,
+// 2000 / 3000 / 4000 / 5000 rows (384 - 952) 116 -> 92, 166 -> 132, 283 -> 205, 361 -> 310; with documents 2000 / 3000 /
+// 4000 rows 115 -> 102, 130 -> 113, no change at 4000 (past the line).  The exception: without a causal mask all
+// workgroups of dk/dv are as long, and when its 128-key form fills its rounds by itself there is nothing to
+// share (8 heads x 4000 rows, 252 of 256 CUs: 301 -> 325; 5000 rows, 320 workgroups in two rounds: 612 -> 482).
 bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
   if (D < 64) return false;
   if (doc && (a.gap >= kGcolMinGap || a.qpos != nullptr || !causal)) return false;   // dk/dv with its column form
@@ -839,7 +845,12 @@ bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
   const int64_t dq = doc ? int64_t(launch_slots<GEO_DOC>(a)) * launch_groups<GEO_DOC>(a)
                          : geo_general(a) ? int64_t(launch_slots<GEO_GENERAL>(a)) * launch_groups<GEO_GENERAL>(a)
                                           : int64_t(launch_slots<GEO_PLAIN>(a)) * launch_groups<GEO_PLAIN>(a);
-  return kv + dq <= 2 * kCUs;
+  if (kv + dq > 4 * kCUs) return false;
+  if (D > 64 && !doc && !causal && a.ktab == nullptr && a.bmask == nullptr && (a.M + 63) / 64 * a.G >= kKvShortTiles) {
+    const int64_t last = (int64_t(a.N + 127) / 128 * a.B * a.Hk - 1) % kCUs + 1;   // workgroups of its last round
+    if (last >= kCUs * 7 / 8) return false;
+  }
+  return true;
 }
 int launch_bwd_both(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s) {
   if (D == 128) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 128>(a, causal, doc, s) : launch_both_cd<fp16_t, 128>(a, causal, doc, s);
