@@ -188,7 +188,8 @@ SHARED_CASES = [
     (1, 8, 8, 1000, 1000, 128, torch.bfloat16, True, "prefix"), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, "block"),
     (2, 4, 4, 333, 333, 64, torch.float16, True, "block"), (1, 4, 4, 700, 900, 128, torch.bfloat16, True, "doc"),
     (2, 4, 2, 257, 257, 64, torch.bfloat16, True, "doc"), (1, 2, 2, 3000, 3000, 128, torch.bfloat16, True, "doc"),    (1, 8, 2, 1500, 1500, 128, torch.bfloat16, True, "plain"),   # (the separate dk/dv takes 128 keys to a workgroup)
-    (1, 8, 8, 4200, 4200, 128, torch.bfloat16, False, "plain"),
+    (1, 8, 8, 4200, 4200, 128, torch.bfloat16, False, "plain"), (1, 8, 8, 6000, 6000, 128, torch.bfloat16, True, "plain"),
+    (2, 8, 8, 2500, 2500, 64, torch.bfloat16, True, "doc"),
 ]
 
 

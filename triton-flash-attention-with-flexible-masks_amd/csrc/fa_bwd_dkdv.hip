@@ -20,6 +20,8 @@
 // one tile ahead), and only tiles whose id interval and row range can meet this workgroup's keys
 // are visited.  The query heads of a grouped-query group are walked inside the kernel, so dK, dV
 // are written once, already summed (the reference sums afterwards, flash_triton.py:635-637).
+#include <algorithm>
+
 #include "fa_tile.h"
 
 namespace fa {
@@ -747,6 +749,11 @@ void bwd_both_kernel(const KArgs a, const int n_dkdv) {
 
 // Query tiles per workgroup (no ids) below which the 64-key role-split form is launched.
 constexpr int kKvShortTiles = 32;
+static int dkdv_tiles(const KArgs& a, bool causal) {
+  int tiles = (a.M + 63) / 64;
+  if (causal) tiles = a.win < 0x3fffffff ? std::min(tiles, a.win / 64 + 3) : (tiles + 1) / 2;
+  return tiles * a.G;
+}
 template <int D, int NKB>
 constexpr size_t dkdv_lds() { return 4 * 64 * (D < 32 ? 32 : D) * 2 + 2 * 1024 + (D > 64 ? 2 * NKB * 2048 + 64 : 0); }
 template <typename Tag, int D, bool CAUSAL, bool DOC, int NKB, bool COLS = false>
@@ -785,10 +792,7 @@ static int launch_one(const KArgs& a, hipStream_t s) {
   if constexpr (D > 64) {
     if (DOC || a.bmask != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s);
     if (a.ktab != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, kSeqKeyTile / 32>(a, s);
-    int tiles = (a.M + 63) / 64;
-    if (CAUSAL) tiles = a.win < 0x3fffffff ? min(tiles, a.win / 64 + 3) : (tiles + 1) / 2;
-    tiles *= a.G;
-    return tiles < kKvShortTiles ? launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s) : launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
+    return dkdv_tiles(a, CAUSAL) < kKvShortTiles ? launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s) : launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
   } else {
     return launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
   }
@@ -830,13 +834,18 @@ static int launch_both_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) 
   return causal ? launch_both<Tag, D, true, GEO_PLAIN>(a, s) : launch_both<Tag, D, false, GEO_PLAIN>(a, s);
 }
 
-// Whether a backward of these sizes takes the shared launch: with at most four workgroups to a CU in all (two run at a time),
-// where the drain of one launch and the start of the next weigh most.  Forward + backward, separate -> shared, D = 128: 8 heads
-// on 2 key heads, causal, 2000 / 3000 / 5000 rows (316 - 790 workgroups) 306 -> 226, 443 -> 327, 783 -> 567 us; 8 heads,
-// 2000 / 3000 / 4000 / 5000 rows (384 - 952) 116 -> 92, 166 -> 132, 283 -> 205, 361 -> 310; with documents 2000 / 3000 /
-// 4000 rows 115 -> 102, 130 -> 113, no change at 4000 (past the line).  The exception: without a causal mask all
-// workgroups of dk/dv are as long, and when its 128-key form fills its rounds by itself there is nothing to
-// share (8 heads x 4000 rows, 252 of 256 CUs: 301 -> 325; 5000 rows, 320 workgroups in two rounds: 612 -> 482).
+// Whether a backward of these sizes takes the shared launch: with at most eight workgroups to a CU in all (two run at a time),
+// where the drain of one launch and the start of the next weigh most; beyond that, forming delta in a launch of its own
+// reads more than is gained.  Forward + backward, separate -> shared,
+// D = 128: 8 heads on 2 key heads, causal, 2000 / 3000 / 5000 rows (316 - 790 workgroups) 306 -> 226, 443 -> 327, 783 -> 567
+// us; 8 heads, 2000 / 3000 / 4000 / 6000 / 10000 rows (384 - 1888) 116 -> 92, 166 -> 132, 283 -> 205, 441 -> 401, 964 -> 943;
+// with documents 2000 / 3000 / 5000 rows 115 -> 102, 130 -> 113, 158 -> 146; 16 / 24 packed sequences of 500 106 -> 97,
+// 133 -> 114; D = 64, 10000 rows 593 -> 514.
+// The exception: the 128-key form of dk/dv (long streams) reads less than the 64-key form that shares a launch, and where
+// it fills its rounds of one workgroup to a CU by itself there is nothing to share (8 heads x 4000 rows without a causal
+// mask, 252 of 256 CUs: 301 -> 325; 7000 rows 899 -> 909; causal 8000 637 -> 645) -- except in a single causal round, whose
+// workgroups are anything but equally long (the 4000 rows above).  D = 64 likewise, two workgroups to a CU (64 heads x 2048
+// rows without a causal mask, two full rounds: 328 both ways).
 bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
   if (D < 64) return false;
   if (doc && (a.gap >= kGcolMinGap || a.qpos != nullptr || !causal)) return false;   // dk/dv with its column form
@@ -845,10 +854,11 @@ bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
   const int64_t dq = doc ? int64_t(launch_slots<GEO_DOC>(a)) * launch_groups<GEO_DOC>(a)
                          : geo_general(a) ? int64_t(launch_slots<GEO_GENERAL>(a)) * launch_groups<GEO_GENERAL>(a)
                                           : int64_t(launch_slots<GEO_PLAIN>(a)) * launch_groups<GEO_PLAIN>(a);
-  if (kv + dq > 4 * kCUs) return false;
-  if (D > 64 && !doc && !causal && a.ktab == nullptr && a.bmask == nullptr && (a.M + 63) / 64 * a.G >= kKvShortTiles) {
-    const int64_t last = (int64_t(a.N + 127) / 128 * a.B * a.Hk - 1) % kCUs + 1;   // workgroups of its last round
-    if (last >= kCUs * 7 / 8) return false;
+  if (kv + dq > 8 * kCUs) return false;
+  if (!doc && a.ktab == nullptr && a.bmask == nullptr && (D <= 64 || dkdv_tiles(a, causal) >= kKvShortTiles)) {
+    const int64_t slots = D > 64 ? kCUs : 2 * kCUs;   // 128 keys to a workgroup either way
+    const int64_t wgs = int64_t(a.N + 127) / 128 * a.B * a.Hk, rounds = (wgs + slots - 1) / slots;
+    if (wgs * 100 >= rounds * slots * 85 && (!causal || rounds > 1)) return false;
   }
   return true;
 }
