@@ -227,7 +227,8 @@ int fa_fwd(const fa_params* p, void* stream);
    split scratch).  Every call on a GPU uses that GPU's one array, which keeps the last call's
    contents: calls that overlap on one GPU (different streams, different threads) race and must be
    ordered by the caller; a backward needs its own fa_mask_plan into a caller's workspace.
-   With score_mode 0 or 2 there is no workspace and the call is fa_fwd. */
+   With score_mode 0 or 2 there is no workspace and the call is fa_fwd without FA_FLAG_SPLIT_KEYS (which is
+   ignored).  Packed sequences (score_mode 3) are refused with FA_ERR_MODE: their tile tables need fa_mask_plan. */
 #define FA_STATIC_WS_BYTES (32u << 20)
 int fa_fwd_static(const fa_params* p, void* stream);
 

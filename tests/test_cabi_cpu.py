@@ -144,6 +144,25 @@ def test_workspace_size():
     assert L.fa_workspace_plan_bytes(ctypes.byref(p)) == want - scratch
 
 
+def test_static_forward_never_takes_a_workspace_that_nobody_planned():
+    """fa_fwd_static ignores p->workspace: what would read tables or counters out of it is refused (packed sequences) or
+    left out (split key ranges).  No operand is set, so the call ends at the checks, with a GPU or without."""
+    L = _cabi.lib()
+    buf = ctypes.create_string_buffer(4096)
+    p = _good_params(buf)
+    p.q = None
+    p.workspace, p.workspace_bytes = 256 * 1024, 1 << 40    # a filled struct that was used before
+    assert L.fa_fwd_static(ctypes.byref(p), None) == -1
+    p.score_mode, p.nseq, p.eq, p.ek, p.B = _cabi.FA_SCORE_MODE3_PACKED, 2, p.k, p.k, 1
+    assert L.fa_fwd_static(ctypes.byref(p), None) == -7
+    # one row against a long key range is split when the flag is set and a workspace is there
+    p = _good_params(buf)
+    p.q, p.M, p.N = None, 1, 16384
+    p.flags = _cabi.FA_FLAG_SPLIT_KEYS
+    assert L.fa_workspace_bytes(ctypes.byref(p)) > 0 and L.fa_validate(ctypes.byref(p), 0) == -8
+    assert L.fa_fwd_static(ctypes.byref(p), None) == -1     # no workspace asked for: the flag is left out
+
+
 def test_python_layer_asserts_like_the_reference():
     q = torch.zeros(1, 4, 8, 64, dtype=torch.bfloat16)
     k = torch.zeros(1, 2, 16, 64, dtype=torch.bfloat16)

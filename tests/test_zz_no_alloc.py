@@ -155,3 +155,29 @@ def test_static_scratch_refuses_what_does_not_fit():
     assert rc == -8, rc   # FA_ERR_WORKSPACE
     with pytest.raises(_cabi.FlashMI355Error, match="workspace"):
         _cabi.check(rc, "fa_fwd_static")
+
+
+def test_static_forward_without_ids_does_not_split_key_ranges():
+    """One query row against a key range that fa_fwd would split: the static call leaves FA_FLAG_SPLIT_KEYS out and the
+    workspace of a struct used before alone, and gives the bits of fa_fwd without the flag."""
+    from flash_mi355 import _cabi
+    from flash_mi355.api import _Plan, _set4, _stream_ptr
+    L = _cabi.lib()
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(1, h, n, 64, generator=g).to(torch.bfloat16).to(dev) for h, n in ((4, 1), (2, 9000), (2, 9000)))
+    plan = _Plan(q, k, v, True, 0.125, None, None, 0, flags=_cabi.FA_FLAG_SPLIT_KEYS)
+    p = plan.p
+    o, lse = torch.full_like(q, float("nan")), torch.full((1, 4, 1), float("nan"), device=dev)
+    p.o, p.lse = o.data_ptr(), lse.data_ptr()
+    _set4(p.o_stride, o)
+    assert L.fa_workspace_bytes(ctypes.byref(p)) > 0
+    print("case static forward with FA_FLAG_SPLIT_KEYS", flush=True)
+    _cabi.check(L.fa_fwd_static(ctypes.byref(p), _stream_ptr(dev)), "fa_fwd_static")
+    torch.cuda.synchronize()
+    got = o.clone(), lse.clone()
+    o.fill_(float("nan")); lse.fill_(float("nan"))
+    p.flags = 0
+    _cabi.check(L.fa_fwd(ctypes.byref(p), _stream_ptr(dev)), "fa_fwd")
+    torch.cuda.synchronize()
+    assert torch.isfinite(o.float()).all() and torch.equal(got[0], o) and torch.equal(got[1], lse)

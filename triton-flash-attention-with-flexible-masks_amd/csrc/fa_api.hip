@@ -264,8 +264,12 @@ static int static_scratch(void** out) {
 
 extern "C" int fa_fwd_static(const fa_params* p, void* stream) {
   if (p == nullptr) return FA_ERR_NULLPTR;
-  if (p->score_mode != FA_SCORE_MODE1_DOC) return fa_fwd(p, stream);   // no workspace in these modes
+  // Packed sequences need tile tables and split key ranges arrival counters, both written by fa_mask_plan into a caller's
+  // workspace, and p->workspace is nobody's here (not even cleared): the first are refused, the second left out.
+  if (p->score_mode == FA_SCORE_MODE3_PACKED) return FA_ERR_MODE;
   fa_params q = *p;
+  q.flags &= ~FA_FLAG_SPLIT_KEYS;
+  if (q.score_mode != FA_SCORE_MODE1_DOC) return fa_fwd(&q, stream);   // no workspace in these modes
   q.workspace = reinterpret_cast<void*>(uintptr_t(256));   // placeholder for the checks below; replaced before any launch
   q.workspace_bytes = ~uint64_t(0);
   int rc = fa_validate(&q, 0);
