@@ -217,8 +217,8 @@ int fa_fwd(const fa_params* p, void* stream);
 
 /* fa_fwd for callers that cannot allocate device memory and hold no workspace (code under HIP graph
    capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
-   Same operands and results as fa_mask_plan + fa_fwd, but p->workspace / p->workspace_bytes are
-   ignored: the mask plan and the scratch of the split key ranges live in a static device array of
+   Same operands and results as fa_mask_plan + fa_fwd, but p->workspace, p->split_scratch and their
+   sizes are ignored: the mask plan and the scratch of the split key ranges live in a static device array of
    FA_STATIC_WS_BYTES inside the library (held by every GPU the library runs on until the process
    ends).  The call enqueues the plan kernels and the forward on `stream` and allocates nothing, on
    the host or the device.  Problems whose plan does not fit the array are refused with

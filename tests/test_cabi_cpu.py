@@ -163,6 +163,18 @@ def test_static_forward_never_takes_a_workspace_that_nobody_planned():
     assert L.fa_fwd_static(ctypes.byref(p), None) == -1     # no workspace asked for: the flag is left out
 
 
+def test_static_forward_leaves_the_callers_split_scratch_alone():
+    """The scratch of the split key ranges lies in the library's array: a split_scratch left over in the struct (here a
+    misaligned one) is neither used nor looked at.  No operand is set, so the call ends at the checks."""
+    L = _cabi.lib()
+    buf = ctypes.create_string_buffer(4096)
+    p = _good_params(buf)
+    p.score_mode, p.eq, p.ek, p.N, p.q = 1, p.k, p.k, 4096, None
+    p.split_scratch, p.split_scratch_bytes = 256 * 1024 + 64, 64
+    assert L.fa_workspace_scratch_bytes(ctypes.byref(p)) > 64
+    assert L.fa_fwd_static(ctypes.byref(p), None) == -1
+
+
 def test_python_layer_asserts_like_the_reference():
     q = torch.zeros(1, 4, 8, 64, dtype=torch.bfloat16)
     k = torch.zeros(1, 2, 16, 64, dtype=torch.bfloat16)

@@ -272,6 +272,8 @@ extern "C" int fa_fwd_static(const fa_params* p, void* stream) {
   if (q.score_mode != FA_SCORE_MODE1_DOC) return fa_fwd(&q, stream);   // no workspace in these modes
   q.workspace = reinterpret_cast<void*>(uintptr_t(256));   // placeholder for the checks below; replaced before any launch
   q.workspace_bytes = ~uint64_t(0);
+  q.split_scratch = nullptr;   // the scratch lies in the static array too, whatever the struct was used for before
+  q.split_scratch_bytes = 0;
   int rc = fa_validate(&q, 0);
   if (rc != FA_OK) return rc;
   const WsLayout w = ws_layout(&q, kStaticSplitBudget);
