@@ -197,6 +197,25 @@ def test_python_layer_asserts_like_the_reference():
         attention(q, k, k)                                                          # CPU tensors: no CPU fallback
 
 
+def test_the_packed_mode_is_not_a_score_func_mode():
+    """Mode 3 is how attention_varlen hands packed sequences on; given as score_func_mode (with vectors that would pass
+    for cumulative lengths) it is refused like any unknown mode, before the device of the operands is looked at."""
+    from flash_mi355 import api
+    q = torch.zeros(1, 4, 8, 64, dtype=torch.bfloat16)
+    cu = torch.tensor([0, 3, 8], dtype=torch.int32)
+    for f in (attention, api.attention_with_lse):
+        for mode in (3, 4, -1):
+            with pytest.raises(AssertionError, match="unknown score_func_mode"):
+                f(q, q, q, True, None, cu, cu, mode)
+    for cls in (api.FlashAttention, api.FlashAttentionWithLse):
+        with pytest.raises(AssertionError, match="unknown score_func_mode"):
+            cls.apply(q, q, q, True, None, cu, cu, 3)
+    with pytest.raises(AssertionError, match="KV length"):   # ... and does not lift the rule on lengths
+        attention(q, q[:, :, :4], q[:, :, :4], True, None, cu, cu, 3)
+    with pytest.raises(AssertionError, match="GPU only"):    # the packed path's own calls pass the check
+        api.attention_varlen(q[0], q[0], q[0], cu)
+
+
 def test_operands_on_another_device_are_refused():
     """Ids, k, v or dO that do not live on q's device are refused with an AssertionError before any
     pointer reaches a kernel (checked on the helper itself: no GPU is needed to compare devices)."""

@@ -19,8 +19,8 @@ from . import _cabi
 
 SCORE_FUNC_MODE0_NOPE = 0  # flash_triton.py:20
 SCORE_FUNC_MODE1_DOC = 1   # flash_triton.py:22
-SCORE_FUNC_MODE3_PACKED = 3  # packed sequences: set by attention_varlen(), eq / ek are the cumulative lengths; no counterpart in the reference
 SCORE_FUNC_MODE2_BLOCK = 2  # block mask: set by the block_mask argument of attention(), no counterpart in the reference
+SCORE_FUNC_MODE3_PACKED = 3  # packed sequences: attention_varlen() alone, eq / ek are the cumulative lengths; no counterpart in the reference
 
 _DTYPES = {torch.bfloat16: _cabi.FA_DTYPE_BF16, torch.float16: _cabi.FA_DTYPE_FP16, torch.float32: _cabi.FA_DTYPE_FP32}
 _ID_DTYPES = {torch.int32: _cabi.FA_IDTYPE_I32, torch.int64: _cabi.FA_IDTYPE_I64}
@@ -156,7 +156,7 @@ class _Impl:
     """Forward and backward shared by the two autograd functions below."""
 
     @staticmethod
-    def forward(ctx, q, k, v, causal, sm_scale, eq, ek, score_func_mode, window=0, prefix=0, qpos=None):
+    def forward(ctx, q, k, v, causal, sm_scale, eq, ek, score_func_mode, window=0, prefix=0, qpos=None, packed=False):
         # -- checks of flash_triton.py:510-530, same order and messages --
         Dq, Dk, Dv = q.shape[-1], k.shape[-1], v.shape[-1]
         assert Dq == Dk and Dk == Dv, "feature size of q, k, v should be equal"
@@ -167,7 +167,7 @@ class _Impl:
         assert Hk == Hv, "num of heads in k and v should be equal"
         assert H % Hk == 0, "number of heads in q must be a multiple of that in k & v"
         num_groups = H // Hk
-        assert (N >= M) or (not causal) or (qpos is not None) or score_func_mode == SCORE_FUNC_MODE3_PACKED, "KV length should be larger than M length in causal mode!"
+        assert (N >= M) or (not causal) or (qpos is not None) or packed, "KV length should be larger than M length in causal mode!"
         MN_GAP = max(0, N - M)
         if sm_scale is None:
             sm_scale = 1. / math.sqrt(D)
@@ -176,7 +176,8 @@ class _Impl:
         if eq is None:
             assert score_func_mode == SCORE_FUNC_MODE0_NOPE
         # -- checks the reference leaves to the Triton launcher --
-        assert score_func_mode in (SCORE_FUNC_MODE0_NOPE, SCORE_FUNC_MODE1_DOC, SCORE_FUNC_MODE2_BLOCK, SCORE_FUNC_MODE3_PACKED), "unknown score_func_mode"
+        assert score_func_mode in ((SCORE_FUNC_MODE3_PACKED,) if packed else (SCORE_FUNC_MODE0_NOPE, SCORE_FUNC_MODE1_DOC, SCORE_FUNC_MODE2_BLOCK)), \
+            "unknown score_func_mode"
         window, prefix = int(window or 0), int(prefix or 0)
         assert window >= 0 and prefix >= 0 and not (window and prefix), "window and prefix exclude each other"
         assert causal or not (window or prefix), "window / prefix are causal masks"
@@ -193,7 +194,7 @@ class _Impl:
                 f"block_mask must be [bs|1, H|1, {nbr}, {nbc}] (blocks of 64 x 64)"
             eq = maybe_contiguous((eq != 0).to(torch.uint8).to(q.device)).expand(B, H, nbr, nbc)
             ek = eq
-        elif score_func_mode == SCORE_FUNC_MODE3_PACKED:
+        elif packed:
             assert B == 1 and eq.dim() == 1 and eq.shape == ek.shape and eq.dtype == ek.dtype and eq.dtype in _ID_DTYPES and eq.is_contiguous() \
                 and ek.is_contiguous() and q.dtype != torch.float32, "packed sequences: see attention_varlen"
         elif score_func_mode != SCORE_FUNC_MODE0_NOPE:
@@ -314,6 +315,18 @@ class FlashAttentionWithLse(torch.autograd.Function):
         return _backward(ctx, do, dlse)
 
 
+class _PackedAttention(torch.autograd.Function):
+    """attention_varlen's own: the one place where eq / ek are the boundaries of packed sequences."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, causal, sm_scale, cu_q, cu_k, window):
+        return _forward(ctx, q, k, v, causal, sm_scale, cu_q, cu_k, SCORE_FUNC_MODE3_PACKED, window, packed=True)[0]
+
+    @staticmethod
+    def backward(ctx, do):
+        return _backward(ctx, do, None)[:3] + (None,) * 5
+
+
 def _block_args(block_mask, eq, ek, score_func_mode):
     if block_mask is None:
         return eq, ek, score_func_mode
@@ -406,7 +419,7 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k=None, causal=False, sm_
         cq, ck = _prep_cu(cu_seqlens_q), _prep_cu(cu_seqlens_k)
         if cq.dtype != ck.dtype:   # one id width per call
             cq, ck = cq.to(torch.int64), ck.to(torch.int64)
-        out = FlashAttention.apply(q4, k4, v4, causal, sm_scale, cq, ck, SCORE_FUNC_MODE3_PACKED, window, 0, None)
+        out = _PackedAttention.apply(q4, k4, v4, causal, sm_scale, cq, ck, window)
         return out.squeeze(0).transpose(0, 1)
     qpos = varlen_positions(cu_seqlens_q, cu_seqlens_k, Tq).view(1, Tq) if causal and not same else None
     eq = varlen_ids(cu_seqlens_q, Tq)
