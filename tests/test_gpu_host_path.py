@@ -115,3 +115,25 @@ def test_saved_tensor_hooks_see_what_the_node_keeps():
         out = attention(q, k, v, True)
     got = torch.autograd.grad(out.sum(), (q, k, v))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_boundaries_may_be_refilled_before_the_backward(native):
+    """One buffer of cumulative lengths for every micro-batch: it is read by the forward, not by the backward."""
+    from flash_mi355 import attention_varlen
+    scale = 0.125 if native else 2   # (a scale that is no float takes the Python path)
+    q, k, v, do = (torch.randn(300, h, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True) for h in (4, 2, 2, 4))
+    lens = torch.tensor([[0, 100, 164, 300], [0, 7, 70, 290]], device="cuda", dtype=torch.int32)
+    def step(cu_q, cu_k):
+        out = attention_varlen(q, k, v, cu_q, cu_k, causal=True, sm_scale=scale)
+        assert (out.grad_fn.name() == "FlashAttentionBackward") == native
+        return out
+    want = [torch.autograd.grad(step(c, c.clone()), (q, k, v), do) for c in lens]
+    cu_q, cu_k = lens[0].clone(), lens[0].clone()
+    first = step(cu_q, cu_k)
+    cu_q.copy_(lens[1]); cu_k.copy_(lens[1])
+    second = step(cu_q, cu_k)
+    cu_q.zero_(); cu_k.fill_(300)
+    got = [torch.autograd.grad(o, (q, k, v), do) for o in (first, second)]
+    for a, b in zip(got, want):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))

@@ -40,7 +40,7 @@ void check(int rc, const char* what) {
 // One call's problem: everything fa_params needs besides the results.
 struct Problem {
   Tensor q, k, v, eq, ek, qpos;   // [B, H, M, D] ..., or [tokens, heads, D] when packed
-  int mode = 0, window = 0, prefix = 0;
+  int mode = 0, window = 0, prefix = 0, nseq = 0;
   bool causal = false, packed = false;
   double scale = 0;
   int B, H, Hk, M, N, D;
@@ -92,9 +92,11 @@ fa_params params_of(const Problem& x) {
     p.eq_stride[1] = x.eq.size(1) == 1 ? 0 : x.eq.stride(1);
     p.eq_stride[2] = x.eq.size(2) == 1 ? x.eq.size(3) : x.eq.stride(2);
   } else if (x.mode == FA_SCORE_MODE3_PACKED) {
-    p.eq = x.eq.data_ptr(); p.ek = x.ek.data_ptr();
-    p.id_dtype = x.eq.scalar_type() == at::kInt ? FA_IDTYPE_I32 : FA_IDTYPE_I64;
-    p.nseq = (int)x.eq.numel() - 1;
+    p.nseq = x.nseq;
+    if (x.eq.defined()) {   // the forward (see backward())
+      p.eq = x.eq.data_ptr(); p.ek = x.ek.data_ptr();
+      p.id_dtype = x.eq.scalar_type() == at::kInt ? FA_IDTYPE_I32 : FA_IDTYPE_I64;
+    }
   }
   if (x.qpos.defined()) {
     p.qpos = x.qpos.const_data_ptr<int32_t>();
@@ -131,6 +133,9 @@ variable_list backward(const Problem& x, const Tensor& o, const Tensor& lse, Ten
   dout = laid_out_or_copy(dout);
   TORCH_CHECK(dout.device() == x.q.device() && dout.scalar_type() == x.q.scalar_type(), "the gradient must share q's device and type");
   fa_params p = params_of(x);
+  // The boundaries of packed sequences are read by the plan kernel alone and not kept (a caller may refill their buffer
+  // while the backward is outstanding); the plan stands in for the pointers that the C ABI wants set.
+  if (x.packed) p.eq = p.ek = plan.data_ptr();
   Tensor scratch;
   if (plan.defined()) scratch = set_workspace(p, x.q, plan);
   Tensor delta = at::empty_like(lse), dq = at::empty_like(x.q), dk = grad_like(x.k, x.packed), dv = grad_like(x.v, x.packed);
@@ -192,7 +197,8 @@ std::pair<Tensor, Tensor> run(const Problem& x, fa_params& p, bool want_lse) {
     node->x = x;
     for (Tensor* t : {&node->x.q, &node->x.k, &node->x.v, &node->x.eq, &node->x.ek, &node->x.qpos}) *t = Tensor();
     node->q = SavedVariable(x.q, false); node->k = SavedVariable(x.k, false); node->v = SavedVariable(x.v, false);
-    node->eq = SavedVariable(x.eq, false); node->ek = SavedVariable(x.ek, false); node->qpos = SavedVariable(x.qpos, false);
+    if (!x.packed) { node->eq = SavedVariable(x.eq, false); node->ek = SavedVariable(x.ek, false); }
+    node->qpos = SavedVariable(x.qpos, false);
     node->lse = SavedVariable(lse, false); node->plan = SavedVariable(plan, false);
     torch::autograd::set_history(o, node);
     if (want_lse) torch::autograd::set_history(lse_e, node);
@@ -324,6 +330,7 @@ PyObject* attention_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
   x.causal = causal != 0;
   x.mode = FA_SCORE_MODE3_PACKED;
   x.packed = true;
+  x.nseq = (int)x.eq.numel() - 1;
   return finish(x, false);
   END_HANDLE_TH_ERRORS
 }

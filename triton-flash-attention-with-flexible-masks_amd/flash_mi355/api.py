@@ -71,7 +71,7 @@ def _host():
 class _Plan:
     """fa_params filled in for one problem, plus the tensors that keep its pointers alive."""
 
-    def __init__(self, q, k, v, causal, sm_scale, eq, ek, score_func_mode, window=0, prefix=0, qpos=None, flags=0):
+    def __init__(self, q, k, v, causal, sm_scale, eq, ek, score_func_mode, window=0, prefix=0, qpos=None, flags=0, nseq=0):
         B, H, M, D = q.shape
         N, Hk = k.shape[2], k.shape[1]
         p = _cabi.FaParams()
@@ -91,7 +91,7 @@ class _Plan:
             self.keep += [eq]
         elif score_func_mode == SCORE_FUNC_MODE3_PACKED:
             p.eq, p.ek = eq.data_ptr(), ek.data_ptr()
-            p.id_dtype, p.nseq = _ID_DTYPES[eq.dtype], eq.numel() - 1
+            p.id_dtype, p.nseq = _ID_DTYPES.get(eq.dtype, 0), nseq   # (the backward's stand-in is no id vector and not read)
             self.keep += [eq, ek]
         elif score_func_mode != SCORE_FUNC_MODE0_NOPE:
             p.eq, p.ek = eq.data_ptr(), ek.data_ptr()
@@ -225,7 +225,7 @@ class _Impl:
 
         L = _cabi.lib()
         with torch.cuda.device(q.device):
-            plan = _Plan(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos, flags)
+            plan = _Plan(q, k, v, causal, sm_scale, eq, ek, score_func_mode, window, prefix, qpos, flags, eq.numel() - 1 if packed else 0)
             Out = torch.empty_like(q)   # q's layout when q is dense (flash_triton.py:539), contiguous otherwise
             lse = torch.empty((B, H, M), device=q.device, dtype=torch.float32)
             p = plan.p
@@ -233,6 +233,9 @@ class _Impl:
             _set4(p.o_stride, Out)
             plan.ensure_workspace(q.device)
             _cabi.check(L.fa_fwd(ctypes.byref(p), _stream_ptr(q.device)), "fa_fwd")
+        ctx.nseq = plan.p.nseq
+        if packed:   # the backward reads the plan's tables alone: the caller may refill the boundaries' buffer meanwhile
+            eq = ek = None
         ctx.save_for_backward(q, k, v, Out, lse, eq, ek, plan.workspace, qpos)
         ctx.sm_scale = sm_scale
         ctx.causal = causal
@@ -249,6 +252,8 @@ class _Impl:
         q, k, v, o, lse, eq, ek, workspace, qpos = ctx.saved_tensors
         B, H, M, D, N, Hk, num_groups, MN_GAP = ctx.shapes
         score_func_mode, window, prefix = ctx.score_func_info
+        if score_func_mode == SCORE_FUNC_MODE3_PACKED:
+            eq = ek = workspace   # stands in for the boundaries, which the C ABI wants set and this stage does not read
         L = _cabi.lib()
         if do is None:   # only LSE was used
             do = torch.zeros_like(o)
@@ -256,7 +261,7 @@ class _Impl:
         _check_same_device(q, do=do, dlse=dlse)
         with torch.cuda.device(q.device):
             plan = _Plan(q, k, v, ctx.causal, ctx.sm_scale, eq, ek, score_func_mode, window, prefix, qpos,
-                         _cabi.FA_FLAG_SPLIT_KEYS if score_func_mode == SCORE_FUNC_MODE0_NOPE else 0)
+                         _cabi.FA_FLAG_SPLIT_KEYS if score_func_mode == SCORE_FUNC_MODE0_NOPE else 0, ctx.nseq)
             p = plan.p
             if workspace is not None:   # the forward's mask plan is used in place (flash_triton.py:557-562 saves, copies nothing)
                 plan.ensure_workspace(q.device, plan_state=workspace)
