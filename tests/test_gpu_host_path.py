@@ -137,3 +137,26 @@ def test_boundaries_may_be_refilled_before_the_backward(native):
     got = [torch.autograd.grad(o, (q, k, v), do) for o in (first, second)]
     for a, b in zip(got, want):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (2, 1), (1, 4), (2, 4)])
+def test_a_block_map_may_be_refilled_before_the_backward(shape):
+    """One mask buffer for all layers: each call's backward belongs to the map its forward saw, and a map of any layout
+    whose columns lie side by side gives the bits of a dense one."""
+    from flash_mi355 import attention
+    q, k, v, do = (torch.randn(2, h, 200, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True) for h in (4, 2, 2, 4))
+    maps = [(torch.rand(*shape, 4, 4, device="cuda") < 0.5) | torch.eye(4, dtype=torch.bool, device="cuda") for _ in range(2)]
+    run = lambda m: attention(q, k, v, True, block_mask=m)
+    want = [torch.autograd.grad(run(m), (q, k, v), do) for m in maps]
+    wide = torch.zeros(4, *shape, 9, dtype=torch.uint8, device="cuda")
+    views = [maps[0].clone(), maps[0].to(torch.uint8) * 7, wide.permute(1, 2, 0, 3)[..., 2:6], wide.permute(1, 2, 0, 3)[..., 3:7]]
+    for buf in views:
+        buf.copy_(maps[0])
+        first = run(buf)
+        assert first.grad_fn.name() == "FlashAttentionBackward"
+        buf.copy_(maps[1])
+        second = run(buf)
+        buf.zero_()
+        got = [torch.autograd.grad(o, (q, k, v), do) for o in (first, second)]
+        for a, b in zip(got, want):
+            assert all(torch.equal(x, y) for x, y in zip(a, b))

@@ -74,6 +74,13 @@ void set_strides(int64_t (&dst)[4], const Tensor& t) {
   }
 }
 
+void set_block_map(fa_params& p, const Tensor& map) {
+  p.eq = map.data_ptr();
+  p.eq_stride[0] = map.size(0) == 1 ? 0 : map.stride(0);
+  p.eq_stride[1] = map.size(1) == 1 ? 0 : map.stride(1);
+  p.eq_stride[2] = map.size(2) == 1 ? map.size(3) : map.stride(2);
+}
+
 fa_params params_of(const Problem& x) {
   fa_params p = {};
   p.q = x.q.data_ptr(); p.k = x.k.data_ptr(); p.v = x.v.data_ptr();
@@ -87,10 +94,7 @@ fa_params params_of(const Problem& x) {
     for (int i = 0; i < 3; ++i) { p.eq_stride[i] = x.eq.stride(i); p.ek_stride[i] = x.ek.stride(i); }
     p.id_dtype = x.eq.scalar_type() == at::kInt ? FA_IDTYPE_I32 : FA_IDTYPE_I64;
   } else if (x.mode == FA_SCORE_MODE2_BLOCK) {
-    p.eq = x.eq.data_ptr();
-    p.eq_stride[0] = x.eq.size(0) == 1 ? 0 : x.eq.stride(0);
-    p.eq_stride[1] = x.eq.size(1) == 1 ? 0 : x.eq.stride(1);
-    p.eq_stride[2] = x.eq.size(2) == 1 ? x.eq.size(3) : x.eq.stride(2);
+    set_block_map(p, x.eq);
   } else if (x.mode == FA_SCORE_MODE3_PACKED) {
     p.nseq = x.nseq;
     if (x.eq.defined()) {   // the forward (see backward())
@@ -177,11 +181,15 @@ struct AttentionBackward : public torch::autograd::Node {
 // O and, when want_lse, LSE in natural-log units
 std::pair<Tensor, Tensor> run(const Problem& x, fa_params& p, bool want_lse) {
   const bool grad = at::GradMode::is_enabled() && (x.q.requires_grad() || x.k.requires_grad() || x.v.requires_grad());
-  Tensor o, lse, lse_e, plan;
+  Tensor o, lse, lse_e, plan, eq = x.eq;
   {
     const at::NoGradGuard no_grad;
     const c10::DeviceGuard guard(x.q.device());
     void* stream = c10::hip::getCurrentHIPStream(x.q.device().index()).stream();
+    if (grad && x.mode == FA_SCORE_MODE2_BLOCK) {   // the backward reads the map again: it keeps one that nobody else writes
+      eq = at::ne(x.eq, 0).contiguous();
+      set_block_map(p, eq);
+    }
     o = at::empty_like(x.q);
     lse = at::empty({x.B, x.H, x.M}, x.q.options().dtype(at::kFloat));
     p.o = o.data_ptr(); p.lse = lse.data_ptr<float>();
@@ -197,7 +205,7 @@ std::pair<Tensor, Tensor> run(const Problem& x, fa_params& p, bool want_lse) {
     node->x = x;
     for (Tensor* t : {&node->x.q, &node->x.k, &node->x.v, &node->x.eq, &node->x.ek, &node->x.qpos}) *t = Tensor();
     node->q = SavedVariable(x.q, false); node->k = SavedVariable(x.k, false); node->v = SavedVariable(x.v, false);
-    if (!x.packed) { node->eq = SavedVariable(x.eq, false); node->ek = SavedVariable(x.ek, false); }
+    if (!x.packed) { node->eq = SavedVariable(eq, false); node->ek = SavedVariable(x.ek, false); }
     node->qpos = SavedVariable(x.qpos, false);
     node->lse = SavedVariable(lse, false); node->plan = SavedVariable(plan, false);
     torch::autograd::set_history(o, node);
@@ -296,7 +304,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (x.eq.device() != x.q.device() || x.ek.device() != x.q.device()) Py_RETURN_NONE;
     if (x.eq.sizes() != at::IntArrayRef({x.B, x.H, x.M}) || x.ek.sizes() != at::IntArrayRef({x.B, x.H, x.N})) Py_RETURN_NONE;
   } else if (x.mode == FA_SCORE_MODE2_BLOCK) {
-    // bytes that are zero or not are what the kernels read: a bool map is used as it is
+    // bytes that are zero or not are what the kernels read: a bool map is used as it is (a copy of it with a gradient, see run())
     if (!tensor_arg(a[5], x.eq) || x.eq.dim() != 4 || x.eq.device() != x.q.device()) Py_RETURN_NONE;
     if (x.eq.scalar_type() != at::kBool && x.eq.scalar_type() != at::kByte) Py_RETURN_NONE;
     const auto es = x.eq.sizes();
