@@ -144,6 +144,38 @@ def test_workspace_size():
     assert L.fa_workspace_plan_bytes(ctypes.byref(p)) == want - scratch
 
 
+def _packed_params(buf, nseq, M, N, H, Hk, D):
+    p = _good_params(buf)
+    p.score_mode, p.nseq, p.eq, p.ek = _cabi.FA_SCORE_MODE3_PACKED, nseq, p.k, p.k
+    p.B, p.M, p.N, p.H, p.Hk, p.D = 1, M, N, H, Hk, D
+    return p
+
+
+@pytest.mark.parametrize("nseq,M,N,H,Hk,D,bm", [
+    (600, 15000, 15000, 8, 8, 128, 64),      # many short sequences: not the form with one workgroup to a CU
+    (600, 15000, 15000, 32, 32, 64, 64),
+    (1001, 5096, 350000, 32, 8, 128, 64),    # 1000 decoding sequences and a prompt
+    (64, 512, 64 * 500, 32, 8, 128, 64),
+    (64, 512, 64 * 1024, 32, 8, 128, 32),     # long key ranges
+    (64, 512, 64 * 2048, 16, 16, 64, 64),
+    (64, 512, 64 * 4096, 16, 16, 64, 32),
+    (16, 256, 16 * 100, 8, 8, 128, 32),      # few tiles
+    (17, 512, 17 * 100, 8, 8, 128, 64),
+    (24, 15000, 15000, 32, 8, 128, 128),
+])
+def test_tile_height_of_packed_sequences(nseq, M, N, H, Hk, D, bm):
+    """The tables are laid out for the tile height the totals ask for; the decode form (32 rows) is for few tiles or
+    long key ranges."""
+    L = _cabi.lib()
+    buf = ctypes.create_string_buffer(4096)
+    p = _packed_params(buf, nseq, M, N, H, Hk, D)
+    r256 = lambda x: (x + 255) // 256 * 256
+    spare = 448 // Hk + 1
+    plan = lambda b: (256 + r256((M * (H // Hk) // b + nseq + 1 + spare) * 64) + r256((N // (64 if D > 64 else 128) + nseq + 1) * 64)
+                      + r256(spare * Hk * 4))
+    assert [b for b in (32, 64, 128) if plan(b) == L.fa_workspace_plan_bytes(ctypes.byref(p))] == [bm]
+
+
 def test_static_forward_never_takes_a_workspace_that_nobody_planned():
     """fa_fwd_static ignores p->workspace: what would read tables or counters out of it is refused (packed sequences) or
     left out (split key ranges).  No operand is set, so the call ends at the checks, with a GPU or without."""

@@ -86,6 +86,8 @@ PACKED_CASES = [
     ([40, 90, 12], [20, 300, 0], 5, 4, 4, 128, True, 0),                                                    # fewer keys than queries, none
     ([40, 9, 12], [20, 300, 50], 0, 4, 2, 32, False, 0),                                                    # cross attention
     ([100, 60], [400, 200], 0, 4, 2, 128, True, 128),
+    ([int(x) for x in np.random.default_rng(1).integers(0, 9, 150)], [int(x) for x in np.random.default_rng(2).integers(0, 70, 150)], 0, 8, 4, 64, True, 0),
+    ([1] * 70 + [300] + [2] * 70, [40] * 70 + [500] + [30] * 70, 3, 4, 2, 128, True, 0),                      # short ones and one long
 ]
 
 

@@ -103,7 +103,7 @@ inline SplitCfg split_config(int B, int H, int M, int N, int D, uint64_t budget 
 //          read the same K / V sit on one XCD, and a short query block fills tiles instead of padding them.
 //   bm   : 128 rows, or 64 when 128-row tiles would leave CUs without a workgroup (the 64-row form splits every key
 //          tile between two waves, see QTileCtx::halved).
-//   dec  : few rows in all: the form of fa_decode.hip, tiles of 32 packed rows.
+//   dec  : few rows in all (packed sequences: in an average one): the form of fa_decode.hip, tiles of 32 packed rows.
 //   split: chunks of the key range; only with FA_FLAG_SPLIT_KEYS, which gives the launch a workspace for them.
 // ---------------------------------------------------------------------------
 constexpr int kCUs = 256;
@@ -113,6 +113,13 @@ constexpr int kCUs = 256;
 // second round (336 of them: 11.2 -> 14.9), on longer ranges the 64-row form reads K and V half as often (32 heads x 128
 // rows on 2000 keys 21.7 -> 24.2).
 constexpr int kDecTiles = kCUs, kDecKeys = 1024;
+// With packed sequences of at most 32 rows on average the decode form, one workgroup to a CU, is the better one for few
+// tiles (a split key range adds to them) and, whatever their number, for long key ranges: 4 sequences x 8 key heads on 8192
+// keys 44 us against 70 of 64-row tiles; 64 on 1100 keys 63 : 68, on 2048 112 : 122, on 8192 434 : 471, 256 on 2048 423 : 420
+// (D = 64: 64 on 2048 129 : 124, 16 on 2048 44 : 37, on 8192 128 : 135).  Many short ranges want several workgroups to a CU:
+// 64 on 512 keys 36 : 33, 4 key heads 37 : 27, 256 on 128 62 : 45, 1024 on 128 236 : 163; 600 sequences of 3 - 48 tokens, 8
+// heads 165 : 69, 32 heads of D = 64 460 : 126.
+constexpr int kDecSeqTiles = kCUs / 2, kDecSeqKeys = 1024;   // keys at D = 128; four times as many at 64
 struct FwdCfg { int pack, bm, tiles, split; bool dec; };
 // Chunks for `wgs` tiles of `steps` steps each: the cheapest total by a model of rounds x (set-up + steps of a chunk)
 // + merging, in units of one step; `slots` workgroups run at a time.  A chunk keeps at least `min_steps` steps.
@@ -134,8 +141,8 @@ inline FwdCfg fwd_config(const fa_params* p) {
   if (p->score_mode == FA_SCORE_MODE3_PACKED) {
     // the host knows the totals only: 32-row tiles when an average sequence fills no more
     c.pack = p->H / p->Hk;
-    const int64_t rows = int64_t(p->M) * c.pack, avg = rows / (p->nseq > 0 ? p->nseq : 1);
-    c.dec = avg <= 32;
+    const int64_t nseq = p->nseq > 0 ? p->nseq : 1, rows = int64_t(p->M) * c.pack, avg = rows / nseq;
+    c.dec = avg <= 32 && (nseq * (p->H / c.pack) <= kDecSeqTiles || p->N / nseq * p->D * p->D >= int64_t(kDecSeqKeys) * 128 * 128);
     c.bm = c.dec ? 32 : (avg <= 64 || (rows / 128 + p->nseq) * p->Hk < kCUs ? 64 : 128);
     return c;
   }
