@@ -248,6 +248,21 @@ def test_the_packed_mode_is_not_a_score_func_mode():
         api.attention_varlen(q[0], q[0], q[0], cu)
 
 
+def test_which_packed_batches_go_through_the_document_mask():
+    from flash_mi355 import api
+    f = api._host().varlen_as_documents
+    assert f(20000, 20000, 1000, 8, 8, 128, True)          # 20 tokens on average, 8000 tiles
+    assert not f(20000, 20000, 500, 8, 8, 128, True)       # 40 tokens on average
+    assert not f(8000, 8000, 500, 8, 8, 128, True)         # 16, but 4000 tiles only
+    assert f(8000, 8000, 500, 8, 8, 128, True) == f(8000, 8000, 1000, 8, 8, 64, True) == False
+    assert f(8000, 8000, 512, 8, 8, 128, True) and f(8000, 8000, 1024, 8, 8, 64, True)
+    assert f(20000, 20000, 1200, 32, 8, 128, True) and not f(20000, 20000, 1000, 32, 8, 128, True)   # groups of four fill tiles sooner
+    assert not f(20000, 20000, 1000, 8, 8, 128, False) and f(20000, 20000, 3000, 8, 8, 128, False)   # positions cost more
+    assert not f(3000, 90000, 3000, 32, 8, 128, False)     # queries on a cache of keys
+    assert not f(3000, 3000, 3000, 8, 0, 128, True)        # (no key heads: refused later)
+    assert not f(1 << 31, 1 << 31, 1 << 24, 8, 8, 128, True) and f(1 << 31, 1 << 31, 1 << 28, 8, 8, 128, True)
+
+
 def test_operands_on_another_device_are_refused():
     """Ids, k, v or dO that do not live on q's device are refused with an AssertionError before any
     pointer reaches a kernel (checked on the helper itself: no GPU is needed to compare devices)."""

@@ -132,6 +132,36 @@ def test_packed_sequences(i, grad):
                 check_close(f"{name} {a}:{b}", sl(got.float().cpu()), ref, quiet=True)
 
 
+@pytest.mark.parametrize("same,causal,window,H,Hk,D,dtype,kind", [
+    (True, True, 0, 4, 4, 128, torch.bfloat16, torch.int32), (True, False, 0, 8, 4, 128, torch.float16, torch.int64),
+    (True, True, 3, 8, 8, 64, torch.bfloat16, torch.int32), (False, True, 0, 8, 8, 128, torch.bfloat16, torch.int64),
+    (False, False, 0, 8, 8, 128, torch.bfloat16, torch.int32), (False, True, 2, 16, 16, 64, torch.float16, torch.int32)])
+def test_short_sequences_as_a_document_mask(same, causal, window, H, Hk, D, dtype, kind):
+    """A batch that attention_varlen hands to the kernels as a document mask, against the tile tables of the same call: the
+    boundaries given once or twice (with other lengths on the key side), empty sequences, rows behind the last boundary."""
+    from flash_mi355 import api
+    n = 1100
+    rng = np.random.default_rng(12)
+    lq = rng.integers(0, 9, n)
+    lk = lq if same else rng.permutation(lq)
+    tail = 5
+    T = int(lq.sum()) + tail
+    print("case", same, causal, window, H, Hk, D, dtype, T, flush=True)
+    assert api._host().varlen_as_documents(T, T, n, H, Hk, D, same)
+    cq, ck = (torch.from_numpy(np.concatenate([[0], np.cumsum(x)])).to(kind).cuda() for x in (lq, lk))
+    g = torch.Generator().manual_seed(13)
+    q, k, v, do = (torch.randn(T, h, D, generator=g).to(dtype).cuda() for h in (H, Hk, Hk, H))
+    res = []
+    for f in (lambda a, b, c: api.attention_varlen(a, b, c, cq, None if same else ck, causal=causal, window=window),
+              lambda a, b, c: api._PackedAttention.apply(*(t.transpose(0, 1).unsqueeze(0) for t in (a, b, c)), causal, None, cq, ck, window).squeeze(0).transpose(0, 1)):
+        x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        out = f(*x)
+        res.append([out.detach(), *torch.autograd.grad(out, x, do)])
+    for name, a, b in zip(("o", "dq", "dk", "dv"), *res):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        check_close(name, a, b.float())
+
+
 def test_packed_graph_replay():
     """A captured packed call is replayed with other boundaries in the same buffer: the tile tables are rebuilt on the device."""
     from flash_mi355 import attention_varlen

@@ -317,6 +317,35 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Whether a packed batch goes to the kernels as a document mask.  With tile tables every sequence has tiles of its own,
+// which very short ones leave nearly empty, while the tiles of a document mask hold many of them; the ids (and, with two
+// vectors of boundaries, the positions) take some kernels and 30 (100) us on the host, which only a launch of many tiles
+// is worth.  Below 112 / (G + 2) tokens on average (G heads to a key head), forward and backward, tables : mask, us:
+//   20000 tokens, D = 128: G = 1, 8 heads, average 8 701 : 202, 24 264 : 205, 32 212 : 202, 44 179 : 204; G = 4, 32 heads, 8 1184 :
+//   567, 16 773 : 568, 24 493 : 567; G = 8, 8 1021 : 584, 12 656 : 588, 16 557 : 589; D = 64, G = 1, 32 heads, 16 963 : 421, 32 543 : 422,
+//   44 452 : 428.  From 4096 sequences x key heads (D = 128), more of the shorter tiles of a smaller D: 5000 tokens, G = 1, 8
+//   heads, average 4 (9900) 351 : 196, 8 (4980) 186 : 163, 12 (3340) 135 : 162; D = 64, 32 heads, 12 (13300) 300 : 172, 24 (6660) 169 : 189.
+// Two vectors: 20000 tokens, G = 1, average 4 1355 : 292, 16 372 : 289, 32 213 : 288.  (Different totals: queries on a cache of
+// keys, where the tables are 3 - 20 times faster.)
+bool as_documents(int64_t Tq, int64_t Tk, int64_t nseq, int64_t H, int64_t Hk, int64_t D, bool same) {
+  if (Tq != Tk || Hk <= 0) return false;
+  const int64_t more = same ? 1 : 2;
+  return Tq * (H / Hk + 2) * more < 112 * nseq && nseq * Hk * D >= 4096 * 128 * more;
+}
+// varlen_as_documents(Tq, Tk, nseq, H, Hk, D, same): the rule, for the Python path
+PyObject* varlen_as_documents(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 7, "varlen_as_documents takes seven numbers");
+  int64_t v[7];
+  for (int i = 0; i < 7; ++i) {
+    v[i] = PyLong_AsLongLong(a[i]);
+    if (v[i] == -1 && PyErr_Occurred()) return nullptr;
+  }
+  if (as_documents(v[0], v[1], v[2], v[3], v[4], v[5], v[6] != 0)) Py_RETURN_TRUE;
+  Py_RETURN_FALSE;
+  END_HANDLE_TH_ERRORS
+}
+
 // attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, causal, sm_scale, window)
 PyObject* attention_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -332,6 +361,7 @@ PyObject* attention_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!operands_ok(x) || x.H % x.Hk != 0 || x.q.scalar_type() == at::kFloat) Py_RETURN_NONE;
   if (!id_type(x.eq) || x.ek.scalar_type() != x.eq.scalar_type() || x.eq.device() != x.q.device() || x.ek.device() != x.q.device() ||
       !x.eq.is_contiguous() || !x.ek.is_contiguous() || x.eq.numel() < 2) Py_RETURN_NONE;
+  if (as_documents(x.M, x.N, x.eq.numel() - 1, x.H, x.Hk, x.D, same)) Py_RETURN_NONE;
   const int causal = PyObject_IsTrue(a[5]);
   if (causal < 0) { PyErr_Clear(); Py_RETURN_NONE; }
   if (!scale_arg(a[6], x.D, x.scale) || !int_arg(a[7], x.window)) Py_RETURN_NONE;
@@ -346,6 +376,7 @@ PyObject* attention_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&attention)), METH_FASTCALL, nullptr},
     {"attention_varlen", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&attention_varlen)), METH_FASTCALL, nullptr},
+    {"varlen_as_documents", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&varlen_as_documents)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -403,9 +403,10 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k=None, causal=False, sm_
     to the host: q, k, v are passed as [1, H, total, D] views, and the plan kernel turns the boundaries
     into a table of tiles (every sequence starts its own, so no tile mixes sequences).  Causal with
     different boundaries (queries that are the tail of a longer key sequence: chunked prefill, decoding)
-    aligns every sequence bottom-right on its own.  fp32 tensors go through the document mask: ids are
-    the negated sequence numbers (varlen_ids), the alignment is one position per row (varlen_positions,
-    the qpos argument of the operator).
+    aligns every sequence bottom-right on its own.  fp32 tensors, and batches of very many very short
+    sequences (the rule is in csrc/torch_host.cpp), go through the document mask: ids are the negated
+    sequence numbers (varlen_ids), the alignment is one position per row (varlen_positions, the qpos
+    argument of the operator).
     (No counterpart in the reference, which takes eq/ek directly, flash_triton.py:506.)"""
     out = (_native or _host()).attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, causal, sm_scale, window)
     if out is not None:
@@ -420,7 +421,8 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k=None, causal=False, sm_
     assert not same or Tk == Tq, "cu_seqlens_k is needed when k holds a different number of tokens than q"
     assert same or cu_seqlens_q.shape == cu_seqlens_k.shape, "cu_seqlens_q and cu_seqlens_k must describe the same sequences"
     q4, k4, v4 = (t.transpose(0, 1).unsqueeze(0) for t in (q, k, v))
-    if q.dtype != torch.float32 and cu_seqlens_q.numel() > 1:
+    nseq = cu_seqlens_q.numel() - 1
+    if q.dtype != torch.float32 and nseq > 0 and not _host().varlen_as_documents(Tq, Tk, nseq, H, k.shape[1], q.shape[2], same):
         cq, ck = _prep_cu(cu_seqlens_q), _prep_cu(cu_seqlens_k)
         if cq.dtype != ck.dtype:   # one id width per call
             cq, ck = cq.to(torch.int64), ck.to(torch.int64)
