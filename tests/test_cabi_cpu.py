@@ -144,6 +144,23 @@ def test_workspace_size():
     assert L.fa_workspace_plan_bytes(ctypes.byref(p)) == want - scratch
 
 
+@pytest.mark.parametrize("M,N", [(1, 16384), (100, 9000), (3, 300), (2000, 16384), (4096, 4096)])
+def test_a_window_past_every_key_is_no_window(M, N):
+    """Window sizes up to the largest int (callers that mean "none") shape the launch like window = 0: the form and the
+    chunks of the key range, seen in the workspace they ask for."""
+    L = _cabi.lib()
+    buf = ctypes.create_string_buffer(4096)
+    p = _good_params(buf)
+    p.M, p.N, p.flags = M, N, _cabi.FA_FLAG_SPLIT_KEYS
+    want = L.fa_workspace_bytes(ctypes.byref(p))
+    assert (want > 0) == (N > 8000)
+    for window in (N, N + M, (1 << 30) - 1, 1 << 30, (1 << 31) - 1 - M, (1 << 31) - M, (1 << 31) - 1):
+        p.window = window
+        assert L.fa_workspace_bytes(ctypes.byref(p)) == want, window
+    p.window = 64   # a real one leaves short ranges, which are not cut
+    assert M != 1 or L.fa_workspace_bytes(ctypes.byref(p)) == 0
+
+
 def _packed_params(buf, nseq, M, N, H, Hk, D):
     p = _good_params(buf)
     p.score_mode, p.nseq, p.eq, p.ek = _cabi.FA_SCORE_MODE3_PACKED, nseq, p.k, p.k

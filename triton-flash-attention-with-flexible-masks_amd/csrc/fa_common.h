@@ -149,7 +149,7 @@ inline FwdCfg fwd_config(const fa_params* p) {
   if (p->score_mode != FA_SCORE_MODE0_NOPE || p->dtype == FA_DTYPE_FP32) { c.tiles = (p->M + 127) / 128; return c; }
   c.pack = p->H / p->Hk;
   const int64_t rows = int64_t(p->M) * c.pack, bh = int64_t(p->B) * p->Hk;
-  const int nk = p->window > 0 && p->causal && p->window + p->M < p->N ? p->window + p->M : p->N;   // keys a tile can see
+  const int nk = p->window > 0 && p->causal && p->window < p->N - p->M ? p->window + p->M : p->N;   // keys a tile can see
   const int seen = p->causal && p->N >= p->M ? nk - (nk == p->N ? p->M / 2 : 0) : nk;   // keys a row sees on average
   if (rows <= 32 || (bh * ((rows + 31) / 32) <= kDecTiles && seen <= kDecKeys)) {
     c.dec = true; c.bm = 32; c.tiles = int((rows + 31) / 32);
