@@ -168,6 +168,38 @@ def _packed_params(buf, nseq, M, N, H, Hk, D):
     return p
 
 
+def test_packed_rows_stay_inside_an_int(tmp_path):
+    """Heads share tiles only while the packed rows, up to the end of the last tile, can be counted in int; the launch shape
+    is compiled for the host from the header the launches use."""
+    import os
+    import subprocess
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    csrc = ROOT / "triton-flash-attention-with-flexible-masks_amd" / "csrc"
+    src = tmp_path / "shape.hip"
+    src.write_text(r'''
+#include <cstdio>
+#include "fa_common.h"
+int main() {
+  const int rows[][3] = {{1 << 26, 32, 1}, {1 << 26, 31, 1}, {1 << 26, 64, 2}, {(1 << 26) - 9, 32, 1}, {(1 << 26) - 4, 32, 1}, {1 << 26, 128, 8}, {333, 32, 8}, {1 << 26, 16, 16}};
+  for (const auto& r : rows)
+    for (int mode : {FA_SCORE_MODE0_NOPE, FA_SCORE_MODE3_PACKED}) {
+      fa_params p = {};
+      p.B = 1; p.M = r[0]; p.N = 1 << 20; p.H = r[1]; p.Hk = r[2]; p.D = 16; p.causal = 0; p.dtype = FA_DTYPE_BF16; p.score_mode = mode; p.nseq = 3;
+      const fa::FwdCfg c = fa::fwd_config(&p);
+      const long long last = ((long long)r[0] * c.pack + c.bm - 1) / c.bm * c.bm;
+      printf("%d %d %d\n", r[1] / r[2], c.pack, last <= 0x7fffffffLL && (mode == FA_SCORE_MODE3_PACKED || (long long)c.tiles * c.bm == last));
+    }
+}
+''')
+    exe = tmp_path / "shape"
+    subprocess.run([hipcc, "--offload-host-only", "-std=c++17", "-O1", f"-I{csrc}", str(src), "-o", str(exe)], check=True, capture_output=True)
+    out = [tuple(map(int, l.split())) for l in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines()]
+    assert len(out) == 16 and all(ok for _, _, ok in out), out
+    assert [pack for _, pack, _ in out[::2]] == [1, 31, 1, 32, 1, 16, 4, 1] == [pack for _, pack, _ in out[1::2]], out
+
+
 @pytest.mark.parametrize("nseq,M,N,H,Hk,D,bm", [
     (600, 15000, 15000, 8, 8, 128, 64),      # many short sequences: not the form with one workgroup to a CU
     (600, 15000, 15000, 32, 32, 64, 64),

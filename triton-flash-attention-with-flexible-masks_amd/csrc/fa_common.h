@@ -136,19 +136,25 @@ inline int pick_split(int64_t wgs, int steps, int slots, float setup, float merg
   }
   return best;
 }
+// Query heads that share a tile.  The kernels count packed rows in int, up to the end of the last tile: none share where
+// that would not hold (M = 2^26 rows of 32 heads to a key head fit the card).
+inline int shared_heads(const fa_params* p) {
+  const int G = p->H / p->Hk;
+  return int64_t(p->M) * G <= 0x7fffffff - 256 ? G : 1;
+}
 inline FwdCfg fwd_config(const fa_params* p) {
   FwdCfg c = {1, 128, 0, 1, false};
   if (p->score_mode == FA_SCORE_MODE3_PACKED) {
     // the host knows the totals only: 32-row tiles when an average sequence fills no more
-    c.pack = p->H / p->Hk;
+    c.pack = shared_heads(p);
     const int64_t nseq = p->nseq > 0 ? p->nseq : 1, rows = int64_t(p->M) * c.pack, avg = rows / nseq;
     c.dec = avg <= 32 && (nseq * (p->H / c.pack) <= kDecSeqTiles || p->N / nseq * p->D * p->D >= int64_t(kDecSeqKeys) * 128 * 128);
-    c.bm = c.dec ? 32 : (avg <= 64 || (rows / 128 + p->nseq) * p->Hk < kCUs ? 64 : 128);
+    c.bm = c.dec ? 32 : (avg <= 64 || (rows / 128 + p->nseq) * (p->H / c.pack) < kCUs ? 64 : 128);
     return c;
   }
   if (p->score_mode != FA_SCORE_MODE0_NOPE || p->dtype == FA_DTYPE_FP32) { c.tiles = (p->M + 127) / 128; return c; }
-  c.pack = p->H / p->Hk;
-  const int64_t rows = int64_t(p->M) * c.pack, bh = int64_t(p->B) * p->Hk;
+  c.pack = shared_heads(p);
+  const int64_t rows = int64_t(p->M) * c.pack, bh = int64_t(p->B) * (p->H / c.pack);
   const int nk = p->window > 0 && p->causal && p->window < p->N - p->M ? p->window + p->M : p->N;   // keys a tile can see
   const int seen = p->causal && p->N >= p->M ? nk - (nk == p->N ? p->M / 2 : 0) : nk;   // keys a row sees on average
   if (rows <= 32 || (bh * ((rows + 31) / 32) <= kDecTiles && seen <= kDecKeys)) {
