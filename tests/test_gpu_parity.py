@@ -263,10 +263,13 @@ def test_long_key_ranges_of_global_rows():
 
 
 def test_short_query_long_key_without_ids():
-    """Few query rows against a long key range and no ids: the operator hands the call to the kernels as
-    all-global rows, whose key range is cut into chunks for separate workgroups (up to 16 here)."""
-    from flash_mi355 import api
-    assert api._short_query_long_key(1, 2, 100, 8300, torch.bfloat16) and not api._short_query_long_key(1, 2, 100, 8300, torch.float32)
+    """Few query rows against a long key range and no ids: the key range of every tile is cut into chunks for
+    separate workgroups (FA_FLAG_SPLIT_KEYS; seen in the partial results the call asks a workspace for)."""
+    import ctypes
+    from flash_mi355 import _cabi
+    for B, H, Hk, M, N, D, causal, window in ((1, 2, 1, 100, 8300, 128, 1, 0), (1, 4, 2, 1, 9000, 64, 0, 0), (2, 2, 2, 300, 16500, 32, 1, 5000)):
+        p = _cabi.FaParams(B=B, H=H, Hk=Hk, M=M, N=N, D=D, causal=causal, window=window, flags=_cabi.FA_FLAG_SPLIT_KEYS)
+        assert _cabi.lib().fa_workspace_scratch_bytes(ctypes.byref(p)) > 0
     _run_case(1, 2, 1, 100, 8300, 128, torch.bfloat16, True, False, seed=61)
     _run_case(1, 4, 2, 1, 9000, 64, torch.float16, False, False, seed=62)
     _run_case(2, 2, 2, 300, 16500, 32, torch.bfloat16, True, False, seed=63, window=5000)

@@ -147,11 +147,6 @@ def _check_same_device(ref, **others):
         assert t is None or t.device == ref.device, f"{name} is on {t.device}, q is on {ref.device}: all operands must share q's device"
 
 
-def _short_query_long_key(B, H, M, N, dtype):
-    """No ids, fewer query tiles than half the chip has CUs, and a key range long enough to be cut (16-bit types)."""
-    return dtype != torch.float32 and B * H * ((M + 127) // 128) <= 128 and N >= 8192
-
-
 class _Impl:
     """Forward and backward shared by the two autograd functions below."""
 
