@@ -160,3 +160,29 @@ def test_a_block_map_may_be_refilled_before_the_backward(shape):
         got = [torch.autograd.grad(o, (q, k, v), do) for o in (first, second)]
         for a, b in zip(got, want):
             assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("kind", ["plain", "window", "doc", "pos", "block", "packed"])
+def test_saved_tensor_hooks_with_every_mask(kind, native):
+    """What the node keeps (operands, ids, the copy of a block map, positions, the plan) may be moved away and come back
+    with other strides: ids that all heads share come back head by head."""
+    from flash_mi355 import api, workloads as W
+    B, H, Hk, L, D = 1, 4, 2, 300, 64
+    q, k, v = (torch.randn(B, h, L, D, device="cuda", dtype=torch.bfloat16, requires_grad=True) for h in (H, Hk, Hk))
+    ids = torch.from_numpy(W.doc_ids_uniform(np.random.default_rng(3), L, 8, 60, 0.1)).cuda()
+    e = ids[None, None].expand(B, H, L)
+    bm = (torch.rand(B, 1, 5, 5, device="cuda") < 0.5) | torch.eye(5, dtype=torch.bool, device="cuda")
+    cu = torch.tensor([0, 100, 101, 290], device="cuda", dtype=torch.int32)
+
+    def call():
+        if kind == "packed":
+            return api.attention_varlen(*(t[0].transpose(0, 1) for t in (q, k, v)), cu, causal=True, sm_scale=0.125 if native else 1)
+        return _call(kind, q, k, v, e, bm, api.FlashAttentionWithLse, native)[0]
+    want = torch.autograd.grad(call().square().sum(), (q, k, v))
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.dtype), t.cpu())[1], lambda t: t.cuda()):
+        out = call()
+    assert len(seen) >= (6 if kind in ("doc", "pos", "block", "packed") else 5)
+    got = torch.autograd.grad(out.square().sum(), (q, k, v))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -44,6 +44,7 @@ struct Problem {
   bool causal = false, packed = false;
   double scale = 0;
   int B, H, Hk, M, N, D;
+  int64_t id_strides[2][3] = {};   // of eq, ek: the plan's layout follows them, and what saved-tensor hooks hand back may lie otherwise
 };
 
 int elem_type(const Tensor& t) {
@@ -91,7 +92,7 @@ fa_params params_of(const Problem& x) {
   p.flags = x.mode == FA_SCORE_MODE0_NOPE ? FA_FLAG_SPLIT_KEYS : 0;
   if (x.mode == FA_SCORE_MODE1_DOC) {
     p.eq = x.eq.data_ptr(); p.ek = x.ek.data_ptr();
-    for (int i = 0; i < 3; ++i) { p.eq_stride[i] = x.eq.stride(i); p.ek_stride[i] = x.ek.stride(i); }
+    for (int i = 0; i < 3; ++i) { p.eq_stride[i] = x.id_strides[0][i]; p.ek_stride[i] = x.id_strides[1][i]; }
     p.id_dtype = x.eq.scalar_type() == at::kInt ? FA_IDTYPE_I32 : FA_IDTYPE_I64;
   } else if (x.mode == FA_SCORE_MODE2_BLOCK) {
     set_block_map(p, x.eq);
@@ -303,6 +304,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!tensor_arg(a[5], x.eq) || !tensor_arg(a[6], x.ek) || !id_type(x.eq) || x.ek.scalar_type() != x.eq.scalar_type()) Py_RETURN_NONE;
     if (x.eq.device() != x.q.device() || x.ek.device() != x.q.device()) Py_RETURN_NONE;
     if (x.eq.sizes() != at::IntArrayRef({x.B, x.H, x.M}) || x.ek.sizes() != at::IntArrayRef({x.B, x.H, x.N})) Py_RETURN_NONE;
+    for (int i = 0; i < 3; ++i) { x.id_strides[0][i] = x.eq.stride(i); x.id_strides[1][i] = x.ek.stride(i); }
   } else if (x.mode == FA_SCORE_MODE2_BLOCK) {
     // bytes that are zero or not are what the kernels read: a bool map is used as it is (a copy of it with a gradient, see run())
     if (!tensor_arg(a[5], x.eq) || x.eq.dim() != 4 || x.eq.device() != x.q.device()) Py_RETURN_NONE;

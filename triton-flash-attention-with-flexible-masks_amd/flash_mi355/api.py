@@ -229,6 +229,7 @@ class _Impl:
             plan.ensure_workspace(q.device)
             _cabi.check(L.fa_fwd(ctypes.byref(p), _stream_ptr(q.device)), "fa_fwd")
         ctx.nseq = plan.p.nseq
+        ctx.id_strides = plan.p.eq_stride[:], plan.p.ek_stride[:]   # the plan's layout follows them
         if packed:   # the backward reads the plan's tables alone: the caller may refill the boundaries' buffer meanwhile
             eq = ek = None
         ctx.save_for_backward(q, k, v, Out, lse, eq, ek, plan.workspace, qpos)
@@ -258,6 +259,8 @@ class _Impl:
             plan = _Plan(q, k, v, ctx.causal, ctx.sm_scale, eq, ek, score_func_mode, window, prefix, qpos,
                          _cabi.FA_FLAG_SPLIT_KEYS if score_func_mode == SCORE_FUNC_MODE0_NOPE else 0, ctx.nseq)
             p = plan.p
+            if score_func_mode == SCORE_FUNC_MODE1_DOC:   # (saved-tensor hooks may hand ids back that lie otherwise; they are not read here)
+                p.eq_stride[:], p.ek_stride[:] = ctx.id_strides
             if workspace is not None:   # the forward's mask plan is used in place (flash_triton.py:557-562 saves, copies nothing)
                 plan.ensure_workspace(q.device, plan_state=workspace)
             delta = torch.empty_like(lse)
