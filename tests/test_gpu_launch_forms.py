@@ -132,6 +132,34 @@ def test_packed_sequences(i, grad):
                 check_close(f"{name} {a}:{b}", sl(got.float().cpu()), ref, quiet=True)
 
 
+@pytest.mark.parametrize("nseq", [2047, 2048, 8191, 8192, 12345])
+def test_very_many_packed_sequences(nseq):
+    """Where the plan kernel's copies of the boundaries and the tile offsets stop fitting LDS (2048 and 8192 sequences, one
+    more for the rows behind the last boundary): the tables against the same batch as a document mask."""
+    from flash_mi355 import api
+    rng = np.random.default_rng(nseq)
+    H, Hk, D = 2, 1, 64
+    lq = rng.integers(0, 4, nseq)
+    lk = lq + rng.integers(0, 4, nseq)
+    lq[7], lk[7], lq[-1], lk[-1] = 150, 400, 90, 90       # a few that fill tiles
+    Tq, Tk = int(lq.sum()) + 3, int(lk.sum()) + 3
+    print("case", nseq, Tq, Tk, flush=True)
+    assert not api._host().varlen_as_documents(Tq, Tk, nseq, H, Hk, D, False)
+    cq, ck = (torch.from_numpy(np.concatenate([[0], np.cumsum(x)])).to(torch.int32).cuda() for x in (lq, lk))
+    g = torch.Generator().manual_seed(nseq)
+    q, k, v, do = (torch.randn(t, h, D, generator=g).to(torch.bfloat16).cuda() for t, h in ((Tq, H), (Tk, Hk), (Tk, Hk), (Tq, H)))
+    x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    out = api.attention_varlen(*x, cq, ck, causal=True)
+    got = [out.detach(), *torch.autograd.grad(out, x, do)]
+    y = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    eq, ek = api.varlen_ids(cq, Tq).view(1, 1, Tq).expand(1, H, Tq), api.varlen_ids(ck, Tk).view(1, 1, Tk).expand(1, H, Tk)
+    out = api.attention(*(t.transpose(0, 1).unsqueeze(0) for t in y), True, None, eq, ek, 1, qpos=api.varlen_positions(cq, ck, Tq).view(1, Tq))
+    out = out.squeeze(0).transpose(0, 1)
+    want = [out.detach(), *torch.autograd.grad(out, y, do)]
+    for name, a, b in zip(("o", "dq", "dk", "dv"), got, want):
+        check_close(name, a, b.float())
+
+
 @pytest.mark.parametrize("same,causal,window,H,Hk,D,dtype,kind", [
     (True, True, 0, 4, 4, 128, torch.bfloat16, torch.int32), (True, False, 0, 8, 4, 128, torch.float16, torch.int64),
     (True, True, 3, 8, 8, 64, torch.bfloat16, torch.int32), (False, True, 0, 8, 8, 128, torch.bfloat16, torch.int64),
