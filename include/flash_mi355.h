@@ -64,7 +64,8 @@ extern "C" {
    are the same); the strides of ids are not used.  A row sees the keys of its own sequence only; with `causal` every
    sequence is aligned at its end: row i of a sequence of m rows and n keys has its diagonal at its key n - m + i (a
    row before the first key sees nothing).  Rows and keys behind the last boundary form one more sequence, aligned
-   at its start.  window is allowed, prefix and qpos are not; 16-bit types; fa_mask_plan writes the tile tables. */
+   at its start.  window is allowed, prefix and qpos are not; 16-bit types; fa_mask_plan writes the tile tables and is
+   the only call that reads the boundaries (the others want the pointers to be non-NULL). */
 #define FA_SCORE_MODE3_PACKED 3
 
 /* element types */
@@ -204,8 +205,9 @@ uint64_t fa_workspace_plan_bytes(const fa_params* p);
 uint64_t fa_workspace_scratch_bytes(const fa_params* p);
 
 /* Mask engine: normalise eq/ek to int32 and build per-tile id summaries
-   into p->workspace.  Must be enqueued before fa_fwd / fa_bwd_* on the same
-   stream whenever score_mode != 0.  The same workspace serves forward and backward.
+   into p->workspace (packed sequences: the tile tables; FA_FLAG_SPLIT_KEYS: the cleared arrival
+   counters).  Must be enqueued before fa_fwd / fa_bwd_* on the same
+   stream whenever fa_workspace_bytes is not 0.  The same workspace serves forward and backward.
    The plan depends on the ids, the sizes AND on `causal` and `prefix` (key ranges are narrowed with
    the causal bound): plan again when any of them changes.  The workspace also holds the scratch
    of the tiles whose key range is split over several workgroups, so two launches that share a

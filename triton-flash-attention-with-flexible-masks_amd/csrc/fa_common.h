@@ -100,7 +100,10 @@ inline SplitCfg split_config(int B, int H, int M, int N, int D, uint64_t budget 
 // tile has, whether the key range of a tile is cut.
 //   pack : the G query heads of one key head share their tiles: packed row r is query r / G of head r % G.  A tile
 //          then meets the diagonal with 128 / G queries instead of 128 (less of it is masked), all the heads that
-//          read the same K / V sit on one XCD, and a short query block fills tiles instead of padding them.
+//          read the same K / V sit on one XCD, and a short query block fills tiles instead of padding them.  For long
+//          blocks too, although the general set-up costs more: causal, 32 heads of D = 128, G = 4, forward and backward
+//          273 -> 268 us at 2K rows, 9427 -> 9292 at 16K, forward alone 2029 -> 1978; window of 1024 1399 -> 1364;
+//          4 x 16 heads of D = 64, G = 2, 2K rows, forward 60 -> 53, 4K rows without a mask 1253 -> 1251.
 //   bm   : 128 rows, or 64 when 128-row tiles would leave CUs without a workgroup (the 64-row form splits every key
 //          tile between two waves, see QTileCtx::halved).
 //   dec  : few rows in all (packed sequences: in an average one): the form of fa_decode.hip, tiles of 32 packed rows.
@@ -111,7 +114,10 @@ constexpr int kCUs = 256;
 // kDecKeys keys on average: four waves on different key blocks are a shorter chain than four on the same tile.  1 x 8
 // heads x 1000 rows, causal 17.8 -> 15.3 us, 4 x 2 x 4 heads x 64 rows on 1000 keys 18.3 -> 14.8; with more tiles it takes a
 // second round (336 of them: 11.2 -> 14.9), on longer ranges the 64-row form reads K and V half as often (32 heads x 128
-// rows on 2000 keys 21.7 -> 24.2).
+// rows on 2000 keys 21.7 -> 24.2).  The backward's dq takes the same tiles, half of its waves without rows: a little slower
+// where they are many, faster where they are few, and the sum of the kernels gains (64-row tiles : these, us: 8 heads x 1000
+// rows 52.8 : 52.4, the backward of it 30.2 : 32.3; 8 heads x 512 33.3 : 31.2; 16 x 500 34.8 : 35.0; 64 rows on 1000 keys
+// 44.3 : 40.0; 40 rows on 900 39.7 : 32.0).
 constexpr int kDecTiles = kCUs, kDecKeys = 1024;
 // With packed sequences of at most 32 rows on average the decode form, one workgroup to a CU, is the better one for few
 // tiles (a split key range adds to them) and, whatever their number, for long key ranges: 4 sequences x 8 key heads on 8192
