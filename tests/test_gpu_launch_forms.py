@@ -132,6 +132,34 @@ def test_packed_sequences(i, grad):
                 check_close(f"{name} {a}:{b}", sl(got.float().cpu()), ref, quiet=True)
 
 
+def test_short_sequences_graph_replay():
+    """A captured packed call that goes through the document mask follows the boundaries in their buffer."""
+    from flash_mi355 import api
+    n, H, Hk, D = 1100, 4, 4, 128
+    rng = np.random.default_rng(31)
+    lens = [rng.permutation(np.arange(n) % 9) for _ in range(2)]
+    T = int(lens[0].sum())
+    assert api._host().varlen_as_documents(T, T, n, H, Hk, D, True)
+    cus = [torch.from_numpy(np.concatenate([[0], np.cumsum(x)])).to(torch.int32).cuda() for x in lens]
+    g = torch.Generator().manual_seed(32)
+    q, k, v = (torch.randn(T, h, D, generator=g).bfloat16().cuda() for h in (H, Hk, Hk))
+    cu = cus[0].clone()
+    print("case", T, flush=True)
+    with torch.no_grad():
+        api.attention_varlen(q, k, v, cu, causal=True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = api.attention_varlen(q, k, v, cu, causal=True)
+        for rep in range(4):
+            cu.copy_(cus[rep % 2])
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            got = out.clone()
+            assert torch.equal(got, api.attention_varlen(q, k, v, cu, causal=True)), rep
+
+
 @pytest.mark.parametrize("nseq", [2047, 2048, 8191, 8192, 12345])
 def test_very_many_packed_sequences(nseq):
     """Where the plan kernel's copies of the boundaries and the tile offsets stop fitting LDS (2048 and 8192 sequences, one
@@ -188,6 +216,51 @@ def test_short_sequences_as_a_document_mask(same, causal, window, H, Hk, D, dtyp
     for name, a, b in zip(("o", "dq", "dk", "dv"), *res):
         assert a.shape == b.shape and a.dtype == b.dtype
         check_close(name, a, b.float())
+
+
+# bf16 has 8 significant bits: a value rounded to it is off by 2^-9 / sqrt(3) = 1.1e-3 of itself on average (2-norm), fp16 by
+# 1.4e-4.  A result carries that once for itself and once for its weights (O) or, with a weight and a dS of each term and the O in
+# delta, three times (gradients): 1.6e-3 and 2.3e-3 as independent errors.  Twice that is what a lost bit would show.
+@pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 1.13e-3), (torch.float16, 1.41e-4)], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("form", ["decode", "split", "tiles", "packed", "packed_split"])
+def test_error_against_64_bits(form, dtype, bound):
+    """O (and the gradients where there are any) of the forms that merge softmax states, against the same sums in 64 bits."""
+    from flash_mi355 import attention, attention_varlen
+    H, Hk, D = 8, 2, 128
+    lens = {"decode": [(1, 5000)], "split": [(90, 9000)], "tiles": [(700, 700)], "packed": [(64, 64), (200, 200), (1, 1), (35, 35)],
+            "packed_split": [(1, 7000), (3, 900), (17, 300)]}[form]
+    fb = form in ("tiles", "packed")
+    g = torch.Generator().manual_seed(21)
+    Tq, Tk = sum(m for m, _ in lens), sum(n for _, n in lens)
+    q, k, v, do = (torch.randn(t, h, D, generator=g).to(dtype) for t, h in ((Tq, H), (Tk, Hk), (Tk, Hk), (Tq, H)))
+    print("case", form, dtype, flush=True)
+    x = [t.cuda().requires_grad_(fb) for t in (q, k, v)]
+    if form.startswith("packed"):
+        cu = [torch.tensor([0, *np.cumsum([p[i] for p in lens])], dtype=torch.int32, device="cuda") for i in (0, 1)]
+        out = attention_varlen(*x, cu[0], cu[1], causal=True)
+    else:
+        out = attention(*(t.transpose(0, 1)[None] for t in x), True)[0].transpose(0, 1)
+    got = {"o": out.detach()}
+    if fb:
+        got.update(zip(("dq", "dk", "dv"), torch.autograd.grad(out, x, do.cuda())))
+    y = [t.double().requires_grad_(fb) for t in (q, k, v)]
+    rows, a, b = [], 0, 0
+    for m, n in lens:
+        keep = torch.arange(m)[:, None] + n - m >= torch.arange(n)[None]
+        heads = []
+        for h in range(H):
+            s = y[0][a:a + m, h] @ y[1][b:b + n, h * Hk // H].t() / math.sqrt(D)
+            heads.append(torch.softmax(s.masked_fill(~keep, -math.inf), -1) @ y[2][b:b + n, h * Hk // H])
+        rows.append(torch.stack(heads, 1))
+        a, b = a + m, b + n
+    ref = torch.cat(rows)
+    want = {"o": ref.detach()}
+    if fb:
+        want.update(zip(("dq", "dk", "dv"), torch.autograd.grad(ref, y, do.double())))
+    for name in got:
+        rel = ((got[name].cpu().double() - want[name]).norm() / want[name].norm()).item()
+        print(f"  {name}: {rel:.3g}", flush=True)
+        assert rel <= 2 * bound * math.sqrt(2 if name == "o" else 4), (name, rel)
 
 
 def test_packed_graph_replay():

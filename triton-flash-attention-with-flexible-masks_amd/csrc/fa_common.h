@@ -143,7 +143,7 @@ inline int pick_split(int64_t wgs, int steps, int slots, float setup, float merg
   return best;
 }
 // Query heads that share a tile.  The kernels count packed rows in int, up to the end of the last tile: none share where
-// that would not hold (M = 2^26 rows of 32 heads to a key head fit the card).
+// that would not hold.  (A little further, at 2^31 rows of all heads, a launch has more work-items than a grid can: an error.)
 inline int shared_heads(const fa_params* p) {
   const int G = p->H / p->Hk;
   return int64_t(p->M) * G <= 0x7fffffff - 256 ? G : 1;
