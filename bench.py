@@ -22,7 +22,7 @@ on the launch stream, against the 2.5 PFLOP/s bf16 MFMA peak -- a fraction of wh
 the matrix pipes can do, never above 1.  The mask plan lets the kernels skip most
 canonical tiles, so the tile-effective rate of the same launch (what ``value``
 counts) is higher and is reported beside it.  ``pct_of_mfma_peak`` is the executed
-rate of the whole step; ``pct_of_mfma_peak_tile_effective`` the north-star figure.
+rate of the whole step; ``pct_of_mfma_peak_tile_effective`` that of ``value``.
 ``roofline.sustained_mfma_probe`` is what a bare MFMA loop on random bf16 operands sustains on the same box
 right after the timed region (``frac_of_sustained`` = achieved over that): context only, ``frac`` is what counts.
 ``cpu_baseline`` times the reference's eager mask-materialising path on the host
@@ -419,7 +419,7 @@ def main():
     # waves do not skip, from a host emulation of the kernels' tile decisions (it reproduces the hardware
     # counter SQ_INSTS_VALU_MFMA_MOPS_BF16 x 512 of the committed profile), so `frac` is the share of the
     # matrix pipes' peak that was really used.  The mask plan lets the kernels skip most of the canonical
-    # 128 x 128 tiles: the tile-effective rate (north-star accounting) of the same launch is given next to it.
+    # 128 x 128 tiles: the tile-effective rate (the accounting of value) of the same launch is given next to it.
     gemm_units = {"fa_fwd": 1.0, "fa_bwd_dkdv": 2.0, "fa_bwd_dq": 1.5}
     ex = W.executed_flops(w)
     executed = {"fa_fwd": ex["fwd"], "fa_bwd_dkdv": ex["dkdv"], "fa_bwd_dq": ex["dq"]}
