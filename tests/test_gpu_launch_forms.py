@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests._tol import check_close
+from tests._tol import TOL_ABS, check_close
 
 pytestmark = pytest.mark.gpu
 
@@ -353,3 +353,50 @@ def test_backward_in_one_launch(case):
             grads.append(torch.autograd.grad(out, x, (do, torch.zeros(B, H, M, device="cuda"))))
     for a, b in zip(*grads):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+# the pipelined dk/dv form (D = 128, at least 32 query tiles over the heads of a group): tiles and key blocks that are partly
+# filled, one key, heads of a group in one stream, a window, a prefix, more keys than queries and fewer
+PIPE_CASES = [
+    (1, 8, 1, 520, 520, torch.bfloat16, True, 0, 0),
+    (1, 8, 1, 260, 333, torch.bfloat16, False, 0, 0),
+    (2, 16, 1, 129, 65, torch.float16, False, 0, 0),
+    (1, 8, 1, 577, 1000, torch.float16, True, 0, 0),
+    (1, 32, 2, 520, 520, torch.bfloat16, True, 100, 0),
+    (1, 16, 1, 520, 520, torch.bfloat16, True, 0, 300),
+    (1, 1, 1, 2049, 100, torch.bfloat16, False, 0, 0),
+    (1, 32, 1, 64, 1, torch.bfloat16, False, 0, 0),
+    (1, 2, 2, 4100, 4100, torch.bfloat16, True, 0, 0),
+]
+
+
+@pytest.mark.parametrize("case", PIPE_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-%s-c%d-w%d-p%d" % (*c[:5], str(c[5])[6:], *c[6:]))
+def test_pipelined_dkdv(case):
+    import ctypes
+    from flash_mi355 import _cabi
+    from flash_mi355.api import _Plan, _set4, _stream_ptr
+    from oracle import attention_oracle as O
+    B, H, Hk, M, N, dtype, causal, window, prefix = case
+    print("case", case, flush=True)
+    D = 128
+    q, k, v, do = _tensors(B, H, Hk, M, N, D, dtype, 9)
+    qd, kd, vd, dod = (t.cuda() for t in (q, k, v, do))
+    o, dq, dk, dv = torch.empty_like(qd), torch.empty_like(qd), torch.full_like(kd, float("nan")), torch.full_like(vd, float("nan"))
+    lse = torch.empty(B, H, M, device="cuda")
+    delta = torch.empty_like(lse)
+    plan = _Plan(qd, kd, vd, causal, 1.0 / math.sqrt(D), None, None, 0, window, prefix)
+    p = plan.p
+    p.o, p.lse, p.dout, p.delta, p.dq, p.dk, p.dv = (t.data_ptr() for t in (o, lse, dod, delta, dq, dk, dv))
+    for f, t in (("o_stride", o), ("do_stride", dod), ("dq_stride", dq), ("dk_stride", dk), ("dv_stride", dv)):
+        _set4(getattr(p, f), t)
+    plan.ensure_workspace(qd.device)
+    ref, s = ctypes.byref(p), _stream_ptr(qd.device)
+    for name in ("fa_fwd", "fa_bwd_delta", "fa_bwd_dkdv"):
+        _cabi.check(getattr(_cabi.lib(), name)(ref, s), name)
+    torch.cuda.synchronize()
+    _, _, _, rdk, rdv = O.attention_autograd(q, k, v, do, causal, None, None, None, 0, window=window, prefix=prefix)
+    # the bound of check_close is one head's: P and dS are rounded per (row, head), independently, and a sum over the G heads of a
+    # group carries sqrt(G) times that error
+    tol = TOL_ABS * math.sqrt(H // Hk)
+    check_close("dk", dk, rdk, tol)
+    check_close("dv", dv, rdv, tol)

@@ -1,8 +1,8 @@
 // dK/dV kernel of the split backward.  Replaces _bwd_kv_kernel of the reference
 // (flash_triton.py:175-321).
 //
-// One workgroup = 128 keys (64 in the role-split form with document ids, two workgroups per CU).
-// D = 128: two waves per 32 keys; they share a SIMD, own the SAME 32 keys and split the work by role, so that each needs only one operand fragment set and one accumulator
+// One workgroup = 128 keys (64 in the role-split form, two workgroups per CU; long streams without ids at D = 128 have a
+// form of their own, fa_dkdv_pipe.hip).  D = 128: two waves per 32 keys; they share a SIMD, own the SAME 32 keys and split the work by role, so that each needs only one operand fragment set and one accumulator
 // set (two waves per SIMD fit in the register file, and one role's vector work overlaps the
 // other role's matrix work):
 //   role 0 ("score" wave)                       role 1 ("gradient" wave)
@@ -146,10 +146,9 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   }
   // Where to wait for these fragments.  The 64-key role-split form serves short tile streams: only
   // right before the tile loop, so that the set-up below overlaps their flight (3 % of the kernel at
-  // 16 query tiles per workgroup, under 1 % at a dozen).  The other forms wait here: for the
-  // 128-key form, which serves long streams, that gave the faster loop (4.24 against 4.39 ms, plain
-  // causal 16K); at D <= 64 the difference stayed inside the run-to-run spread.
-  constexpr bool LATE_SETTLE = SPLIT && NKB == 2;
+  // 16 query tiles per workgroup, under 1 % at a dozen).  The forms of D <= 64 wait here: the
+  // difference stayed inside the run-to-run spread.
+  constexpr bool LATE_SETTLE = SPLIT;
   FA_STAMP(g_trace_dkdv, 1, 0); FA_STAMP(g_trace_dkdv, 7, (long long)kt | ((long long)bhk << 16));
   if (!LATE_SETTLE) {
 #pragma unroll
@@ -453,36 +452,8 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
         }
       }
     };
-    // (In the 128-key form the first products of the two blocks are fed alternately: an MFMA that accumulates onto the
-    // one issued right before it waits for it, two chains do not.  Dense 16K 4355 -> 4315 us; the 64-key form, where
-    // another workgroup's waves fill those gaps and the score wave publishes its first P later this way, 0.5 % slower.)
-    if constexpr (NKB == 4) {
-      lse_load(0);
-      mfma_phase();
-      __builtin_amdgcn_sched_barrier(0);
-      constexpr int NF = 2 * KS, PF = NF < kKvPre ? NF : kKvPre;
-      auto fetch = [&](const int i) __attribute__((always_inline)) { return lds_row8<E>(rows + lo.row[i / 2] + (i & 1) * 32 * DL * 2); };
-      vec8 rf[NF];
-      x[0] = zero; x[1] = zero;
-#pragma unroll
-      for (int i = 0; i < PF; ++i) rf[i] = fetch(i);
-#pragma unroll
-      for (int i = 0; i < NF; ++i) {
-        if (i + PF < NF) rf[i + PF] = fetch(i + PF);
-        __builtin_amdgcn_sched_barrier(0);
-        x[i & 1] = E::mfma32(rf[i], frag[i / 2], x[i & 1]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      vector_phase();
-      more(0);
-      lse_load(1);
-      score_part(0);
-      more(1);
-      score_part(1);
-    } else {
-      lse_load(0); x[0] = first_product(rows, 0); more(0); score_part(0);
-      lse_load(1); x[1] = first_product(rows, 1); more(1); score_part(1);
-    }
+    lse_load(0); x[0] = first_product(rows, 0); more(0); score_part(0);
+    lse_load(1); x[1] = first_product(rows, 1); more(1); score_part(1);
     grad_part(0); more(2); second_product(trp, yf[0], 0);
     grad_part(1); second_product(trp, yf[1], 1);
   };
@@ -750,7 +721,7 @@ void bwd_both_kernel(const KArgs a, const int n_dkdv) {
   else dq_body<Tag, D, CAUSAL, MODE>(a, bid - n_dkdv, smem);
 }
 
-// Query tiles per workgroup (no ids) below which the 64-key role-split form is launched.
+// Query tiles per workgroup (no ids) from which the pipelined form with 128 keys is launched (fa_dkdv_pipe.hip).
 constexpr int kKvShortTiles = 32;
 static int dkdv_tiles(const KArgs& a, bool causal) {
   int tiles = (a.M + 63) / 64;
@@ -795,7 +766,7 @@ static int launch_one(const KArgs& a, hipStream_t s) {
   if constexpr (D > 64) {
     if (DOC || a.bmask != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s);
     if (a.ktab != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, kSeqKeyTile / 32>(a, s);
-    return dkdv_tiles(a, CAUSAL) < kKvShortTiles ? launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s) : launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
+    return dkdv_tiles(a, CAUSAL) < kKvShortTiles ? launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s) : launch_dkdv_pipe(a, __is_same(Tag, bf16_t) ? FA_DTYPE_BF16 : FA_DTYPE_FP16, CAUSAL, s);
   } else {
     return launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
   }
