@@ -6,9 +6,9 @@
 // set (two waves per SIMD fit in the register file, and one role's vector work overlaps the
 // other role's matrix work):
 //   role 0 ("score" wave)                       role 1 ("gradient" wave)
-//   S  = Q K^T      A = Q rows, B = K^T (regs)  dP = dO V^T     A = dO rows, B = V^T (regs)
-//   P  = exp2(S*c - L), masked -> 0             ---------------- barrier ----------------
-//   P (rounded) -> LDS                          dS = P * (dP - delta)      (P read from LDS)
+//   S  = Q K^T      A = Q rows, B = K^T (regs)  delta - dP      A = dO rows, B = -V^T (regs), starting from delta
+//   P  = exp2(S*c - L), masked -> 0             ------------- waits for P --------------
+//   P (rounded) -> LDS                          -dS = P * (delta - dP)     (P read from LDS)
 //   dV^T += dO^T P  A = dO^T (transposed read)  dK^T += Q^T dS  A = Q^T (transposed read)
 // (flash_triton.py:265-308; dK is scaled by sm_scale at the end, :313).  In the accumulator
 // layout each lane owns ONE key column and 16 query rows of every 32-row block, so LSE / delta /
@@ -149,10 +149,25 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   // 16 query tiles per workgroup, under 1 % at a dozen).  The forms of D <= 64 wait here: the
   // difference stayed inside the run-to-run spread.
   constexpr bool LATE_SETTLE = SPLIT;
+  // The gradient's first product starts from delta and runs on -V: its accumulators then hold delta - dP, dS comes out with
+  // the sign turned (put right by the scale at the end), and the subtraction costs no instruction of its own; in the role-split
+  // form the product with the fp16 P converts it on the way.  Together with a copy of the tile loop per role (no branches
+  // on it inside): sliding window 16K 675 -> 641 us, block mask 1155 -> 1089, documents 16K 681 -> 640, 4K 290 -> 281,
+  // packed sequences 285 -> 264, plain 2K at D = 64 167 -> 157.
+  auto negate_v = [&]() __attribute__((always_inline)) {
+    if (!SPLIT) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) frag2[ks] = neg8<E>(frag2[ks]);
+    } else if (role == 1) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) frag[ks] = neg8<E>(frag[ks]);
+    }
+  };
   FA_STAMP(g_trace_dkdv, 1, 0); FA_STAMP(g_trace_dkdv, 7, (long long)kt | ((long long)bhk << 16));
   if (!LATE_SETTLE) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) { settle(frag[ks]); if (!SPLIT) settle(frag2[ks]); }
+    negate_v();
   }
   const float c = a.scale_log2e;
   // rows that may see this lane's key: [row_lo, row_lo + row_span)
@@ -306,7 +321,8 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   // (LDS-heavy and MFMA-heavy phases of different waves overlap); the gradient wave computes dP of
   // both blocks before it needs the first P.  The wait is bounded, so every wave reaches the end
   // of the kernel whatever happens.
-  auto compute_flag = [&](const int BUF, const int cur, const int flags, const int tile_id, const int next) __attribute__((always_inline)) {
+  auto compute_flag = [&](auto role_c, const int BUF, const int cur, const int flags, const int tile_id, const int next) __attribute__((always_inline)) {
+    constexpr int ROLE = decltype(role_c)::value;
     auto more = [&](const int k) __attribute__((always_inline)) {   // the k-th third of the next tile's row loads that are still to be issued
       if (kHead == NPART || next < 0) return;
 #pragma unroll
@@ -318,8 +334,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
     const int m0 = cur * BQ;  // natural order only
     if (flags & TF_SKIP) { more(0); more(1); more(2); return; }   // decided per wave pair: both roles agree
     ++pair_seq;
-    auto first_product = [&](const char* rows, const int qb) __attribute__((always_inline)) {
-      f32x16 x = zero;
+    auto first_product = [&](const char* rows, const int qb, f32x16 x) __attribute__((always_inline)) {
       mfma_phase();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -368,20 +383,28 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
     // so the gradient wave's first product of block 1 falls into the score wave's exponentials and
     // the score wave's second products into the gradient wave's waits.  (Running dV0 before exp1 in
     // the score wave, or dS1 before dK0 in the gradient wave, measured the same or slightly worse.)
-    const char* rows = role == 0 ? lqt : ldo;   // rows operand of the first product
-    const char* trp = role == 0 ? ldo : lqt;    // transposed operand of the second product
+    const char* rows = ROLE == 0 ? lqt : ldo;   // rows operand of the first product
+    const char* trp = ROLE == 0 ? ldo : lqt;    // transposed operand of the second product
     f32x16 x[2];
     vec8 yf[2][2];   // P (score wave) or dS (gradient wave) per block, rounded to the element type
     f32x4 Lv[2][4];  // LSE of this lane's 16 query rows of a block (row 8*q4 + 4*g + t)
     // requested ahead of the product so that the LDS round trip is hidden
-    auto lse_load = [&](const int qb) __attribute__((always_inline)) {
-      if (role == 0) {
+    auto row_load = [&](const int qb) __attribute__((always_inline)) {
+      if constexpr (ROLE == 0) {
+        x[qb] = zero;
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) Lv[qb][q4] = *reinterpret_cast<const f32x4*>(aux + (32 * qb + 8 * q4 + 4 * g) * 4);
+      } else {   // delta, where the gradient's first product starts
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const f32x4 dl = *reinterpret_cast<const f32x4*>(aux + 256 + (32 * qb + 8 * q4 + 4 * g) * 4);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) x[qb][4 * q4 + t] = dl[t];
+        }
       }
     };
     auto score_part = [&](const int qb) __attribute__((always_inline)) {   // S -> P, published
-      if (role != 0) return;
+      if constexpr (ROLE != 0) return;
       char* pbuf = smem + P_OFF + (qb * NKB + kb) * P_BYTES + lane * 16;
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
@@ -415,14 +438,9 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       }
       lds_flag_store(smem + FLAG_OFF + (qb * NKB + kb) * 4, pair_seq);
     };
-    auto grad_part = [&](const int qb) __attribute__((always_inline)) {    // dS = P * (dP - delta)
-      if (role != 1) return;
+    auto grad_part = [&](const int qb) __attribute__((always_inline)) {    // -dS = P * (delta - dP)
+      if constexpr (ROLE != 1) return;
       const char* pbuf = smem + P_OFF + (qb * NKB + kb) * P_BYTES + lane * 16;
-      // LDS round trips are long under load: delta is requested before the wait, both halves of
-      // P together after it
-      f32x4 dl[4];
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) dl[q4] = *reinterpret_cast<const f32x4*>(aux + 256 + (32 * qb + 8 * q4 + 4 * g) * 4);
       const char* fl = smem + FLAG_OFF + (qb * NKB + kb) * 4;
       // (the score wave it waits for shares its SIMD and must not stand behind the polls; in block 1 the second product of
       // block 0 has raised the priority.  Training steps: dense 16K 8989 -> 8960 us, doc-masked 4K 630 -> 631: no cost)
@@ -439,21 +457,17 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
 #pragma unroll
       for (int half = 0; half < 2; ++half) pr8[half] = *reinterpret_cast<const f16x8*>(pbuf + half * 1024);
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const f32x8 pv = __builtin_convertvector(pr8[half], f32x8);
+      for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int q2 = 0; q2 < 2; ++q2) {
-#pragma unroll
-          for (int t = 0; t < 4; t += 2) {
-            const int e = 4 * q2 + t;
-            const typename E::vec2 pr = E::cvt2(pv[e] * (x[qb][8 * half + e] - dl[2 * half + q2][t]), pv[e + 1] * (x[qb][8 * half + e + 1] - dl[2 * half + q2][t + 1]));
-            yf[qb][half][e] = pr[0]; yf[qb][half][e + 1] = pr[1];
-          }
+        for (int e = 0; e < 8; e += 2) {
+          float s0, s1;
+          mul_f16_f32(pr8[half], e, x[qb][8 * half + e], x[qb][8 * half + e + 1], s0, s1);
+          const typename E::vec2 pr = E::cvt2(s0, s1);
+          yf[qb][half][e] = pr[0]; yf[qb][half][e + 1] = pr[1];
         }
-      }
     };
-    lse_load(0); x[0] = first_product(rows, 0); more(0); score_part(0);
-    lse_load(1); x[1] = first_product(rows, 1); more(1); score_part(1);
+    row_load(0); x[0] = first_product(rows, 0, x[0]); more(0); score_part(0);
+    row_load(1); x[1] = first_product(rows, 1, x[1]); more(1); score_part(1);
     grad_part(0); more(2); second_product(trp, yf[0], 0);
     grad_part(1); second_product(trp, yf[1], 1);
   };
@@ -468,7 +482,13 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
     if (flags & TF_SKIP) return;
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      f32x16 x = zero, dp = zero;
+      f32x16 x = zero, dp;
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {   // (delta - dP: see negate_v)
+        const f32x4 dl = *reinterpret_cast<const f32x4*>(aux + 256 + (32 * qb + 8 * q4 + 4 * g) * 4);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) dp[4 * q4 + t] = dl[t];
+      }
       mfma_phase();
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -490,7 +510,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       }
       __builtin_amdgcn_sched_barrier(0);
       vector_phase();
-      // S -> P, masks, dS = P * (dP - delta) for this lane's 16 query rows of the block
+      // S -> P, masks, -dS = P * (delta - dP) for this lane's 16 query rows of the block
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {
         const int i0 = 32 * qb + 8 * q4 + 4 * g;  // row inside the tile
@@ -500,12 +520,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       }
       mask_p(x, qb, flags, tile_id, m0, aux);
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const int i0 = 32 * qb + 8 * q4 + 4 * g;
-        const f32x4 dl = *reinterpret_cast<const f32x4*>(aux + 256 + i0 * 4);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) dp[4 * q4 + t] = x[4 * q4 + t] * (dp[4 * q4 + t] - dl[t]);
-      }
+      for (int r = 0; r < 16; ++r) dp[r] = x[r] * dp[r];
       // dV^T += dO^T P and dK^T += Q^T dS alternately: transposed fragments (two LDS reads each) are
       // requested PRE MFMAs ahead in program order, P and dS are converted just in time; the
       // scheduling barriers pin that order.
@@ -545,11 +560,12 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       }
     }
   };
-  auto compute = [&](const int BUF, const int cur, const int flags, const int tile_id, const int next) __attribute__((always_inline)) {
-    if constexpr (SPLIT) compute_flag(BUF, cur, flags, tile_id, next);
+  auto compute = [&](auto role_c, const int BUF, const int cur, const int flags, const int tile_id, const int next) __attribute__((always_inline)) {
+    if constexpr (SPLIT) compute_flag(role_c, BUF, cur, flags, tile_id, next);
     else compute_both(BUF, cur, flags, tile_id);
   };
 
+  auto walk = [&](auto role_c) __attribute__((always_inline)) {   // (one copy per role)
   for (int gi = 0; gi < a.G; ++gi) {
     LateArgs& ga = late_args();   // (the head loop encloses the tile loop: what its set-up reads would stay in registers)
     const int h = hk * ga.G + gi;
@@ -643,6 +659,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       // first use inside it)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) settle(frag[ks]);
+      negate_v();
     }
     while (cur >= 0) {
       int nxt2 = -1, nxt2_fl = 0, nxt2_id = 0;
@@ -652,7 +669,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       FA_TRACE_ONLY(if (!tr_first) { FA_STAMP(g_trace_dkdv, 3, FA_CLOCK()); tr_first = true; })
       if (nxt >= 0) load_tile(nxt, 1, kHead);
       if (DOC && nxt2 >= 0) fetch_idx(nxt2);
-      compute(0, cur, cur_fl, cur_id, nxt);
+      compute(role_c, 0, cur, cur_fl, cur_id, nxt);
       FA_TRACE_ONLY(++tr_tiles;)
       cur = nxt; cur_fl = nxt_fl; cur_id = nxt_id; nxt = nxt2; nxt_fl = nxt2_fl; nxt_id = nxt2_id;
       if (cur < 0) break;
@@ -662,10 +679,17 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
       __syncthreads();
       if (nxt >= 0) load_tile(nxt, 0, kHead);
       if (DOC && nxt2 >= 0) fetch_idx(nxt2);
-      compute(1, cur, cur_fl, cur_id, nxt);
+      compute(role_c, 1, cur, cur_fl, cur_id, nxt);
       FA_TRACE_ONLY(++tr_tiles;)
       cur = nxt; cur_fl = nxt_fl; cur_id = nxt_id; nxt = nxt2; nxt_fl = nxt2_fl; nxt_id = nxt2_id;
     }
+  }
+
+  };
+  if constexpr (SPLIT) {
+    if (role == 0) walk(IntC<0>{}); else walk(IntC<1>{});
+  } else {
+    walk(IntC<0>{});
   }
 
   FA_STAMP(g_trace_dkdv, 4, FA_CLOCK()); FA_STAMP(g_trace_dkdv, 6, tr_tiles);
@@ -691,10 +715,10 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[db][r] = __builtin_nanf("");
       }
-      if (role == 0) store(dvp, la.dv_rs, acc, 1.0f); else store(dkp, la.dk_rs, acc, la.scale);
+      if (role == 0) store(dvp, la.dv_rs, acc, 1.0f); else store(dkp, la.dk_rs, acc, -la.scale);
     } else {
       store(dvp, la.dv_rs, acc, 1.0f);
-      store(dkp, la.dk_rs, acc2, la.scale);
+      store(dkp, la.dk_rs, acc2, -la.scale);
     }
   }
   }   // run of key tiles

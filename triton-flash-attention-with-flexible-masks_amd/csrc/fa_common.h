@@ -282,6 +282,13 @@ FA_DEV float xhalf_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Elements e, e + 1 of packed fp16 values times fp32 ones, as two instructions that convert on the way.
+FA_DEV void mul_f16_f32(f16x8 p, const int e, float x0, float x1, float& y0, float& y1) {
+  const f16x2 pp = {p[e], p[e + 1]};
+  asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(y0) : "v"(pp), "v"(x0));
+  asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y1) : "v"(pp), "v"(x1));
+}
+
 // Make a 16-byte value loaded from global memory "used" right here.  The compiler waits for a
 // load at the first use of its result; for operands that are loaded once and first used inside
 // the tile loop that wait (s_waitcnt vmcnt) would sit in the loop, where it also waits for the

@@ -5,15 +5,16 @@
 // Query tiles (Q, dO, LSE, delta; 64 rows) are streamed through three stages of LDS, and the gradient wave runs behind:
 // between two barriers
 //   score wave     S(t) = Q K^T  |  P(t) -> LDS (fp16)         |  dV += dO(t)^T P(t)
-//   gradient wave  dS(t-1) = P(t-1) * (dP(t-1) - delta)        |  dK += Q(t-1)^T dS(t-1),  dP(t) = dO(t) V^T
+//   gradient wave  -dS(t-1) = P(t-1) * (delta - dP(t-1))       |  -dK += Q(t-1)^T -dS(t-1),  delta - dP(t) (from delta, with -V)
 // Neither waits for what the other does in the same step (P crosses behind the barrier of the tile stream: no flag, no polling),
 // and the stream goes on through the query heads of a group without draining.
 //
 // What bounds it: the power limit.  On random operands the clock settles at 1.9 GHz with the matrix pipes 48 % busy (3 stages x
 // 32 KB, 32 KB of P: one workgroup to a CU); on zeros the same launch takes 3.4 ms instead of 4.2.  Causal, 32 heads x 16384
 // rows, against the form in which the gradient wave polls for the P of its own tile: 4.51 -> 4.26, 4.42 -> 4.20, 4.84 -> 4.60 ms
-// on three cards.  Steps of 32 rows (four stages) in workgroups of 128 or 64 keys: 4.60 ms against 4.26, and slower than the
-// polling form with 64 keys on short streams too (window of 1024 717 : 692 us, documents 702 : 689, packed sequences 293 : 288).
+// on three cards; with the subtraction of delta in the accumulators (see fa_bwd_dkdv.hip) another 4.20 -> 3.95.
+// Steps of 32 rows (four stages) in workgroups of 128 or 64 keys: 4.60 ms against 4.26, and slower than the polling form with 64
+// keys on short streams too (window of 1024 717 : 692 us, documents 702 : 689, packed sequences 293 : 288).
 #include "fa_tile.h"
 
 namespace fa {
@@ -55,6 +56,12 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
   for (int ks = 0; ks < KS; ++ks) frag[ks] = *reinterpret_cast<const vec8*>(srcp + ks * 16 + g * 8);
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) settle(frag[ks]);
+  // (the gradient's first product starts from delta and runs on -V: its accumulators hold delta - dP, dS comes out with the sign
+  // turned, put right by the scale at the end, and the subtraction costs no instruction of its own)
+  if (role == 1) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) frag[ks] = neg8<E>(frag[ks]);
+  }
   const float c = a.scale_log2e;
   // rows that may see this lane's key: [row_lo, row_lo + row_span)
   const int row_lo = CAUSAL ? (key <= pfx_m1 ? 0 : max(0, key - gap)) : 0;
@@ -110,7 +117,6 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
     constexpr int NF = 2 * KS, PF = kPipePre;
     auto fetch = [&](const int i) __attribute__((always_inline)) { return lds_row8<E>(rows + lo.row[i / 2] + (i & 1) * 32 * D * 2); };
     vec8 rf[NF];
-    x[0] = zero; x[1] = zero;
 #pragma unroll
     for (int i = 0; i < PF; ++i) rf[i] = fetch(i);
 #pragma unroll
@@ -145,7 +151,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
 
   auto stream = [&](auto role_c) __attribute__((always_inline)) {
     constexpr int ROLE = decltype(role_c)::value;
-    f32x16 x[2];   // gradient wave: dP of the tile before, kept from step to step
+    f32x16 x[2];   // gradient wave: delta - dP of the tile before, kept from step to step
     int prev_fl = TF_SKIP;
     int t = first, stage = 0, par = 0;
     bool more = first < last, prev = false;
@@ -188,6 +194,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
           f32x4 Lv[2][4];
 #pragma unroll
           for (int q4 = 0; q4 < 4; ++q4) Lv[0][q4] = *reinterpret_cast<const f32x4*>(aux + (8 * q4 + 4 * g) * 4);
+          x[0] = zero; x[1] = zero;
           first_products(lqt, x);
           load_rest();
 #pragma unroll
@@ -230,33 +237,35 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
         }
       } else {
         if (!(prev_fl & TF_SKIP)) {
-          const char* aux = smem + AUX_OFF + pst * AUX_BYTES + 256;
           const char* pbuf = smem + P_OFF + ((par ^ 1) * NKB + kb) * P_BYTES + lane * 16;
           vec8 yf[4];
-          f32x4 dl[2][4];
           f16x8 ph[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            ph[i] = *reinterpret_cast<const f16x8*>(pbuf + i * 1024);
-            dl[0][i] = *reinterpret_cast<const f32x4*>(aux + (8 * i + 4 * g) * 4);
-          }
+          for (int i = 0; i < 4; ++i) ph[i] = *reinterpret_cast<const f16x8*>(pbuf + i * 1024);
 #pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) dl[1][q4] = *reinterpret_cast<const f32x4*>(aux + (32 + 8 * q4 + 4 * g) * 4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int qb = i >> 1, half = i & 1;
-            const f32x8 pv = __builtin_convertvector(ph[i], f32x8);
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int e = 0; e < 8; e += 2) {
-              const typename E::vec2 pr = E::cvt2(pv[e] * (x[qb][8 * half + e] - dl[qb][2 * half + (e >> 2)][e & 3]),
-                                                  pv[e + 1] * (x[qb][8 * half + e + 1] - dl[qb][2 * half + (e >> 2)][(e & 3) + 1]));
+              float s0, s1;
+              mul_f16_f32(ph[i], e, x[i >> 1][8 * (i & 1) + e], x[i >> 1][8 * (i & 1) + e + 1], s0, s1);
+              const typename E::vec2 pr = E::cvt2(s0, s1);
               yf[i][e] = pr[0]; yf[i][e + 1] = pr[1];
             }
-          }
           load_rest();
           second_products(smem + pst * STAGE, yf);
         } else load_rest();
-        if (!(cur_fl & TF_SKIP)) first_products(ldo, x);
+        if (!(cur_fl & TF_SKIP)) {
+          const char* aux = smem + AUX_OFF + stage * AUX_BYTES + 256;
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const f32x4 dl = *reinterpret_cast<const f32x4*>(aux + (32 * qb + 8 * q4 + 4 * g) * 4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) x[qb][4 * q4 + e] = dl[e];
+            }
+          first_products(ldo, x);
+        }
       }
       prev = more; prev_fl = cur_fl; more = nmore;
       stage = nst; par ^= 1;
@@ -270,7 +279,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
   char* patch = smem + wave * row_patch_bytes<D>();
   T* base = role == 0 ? reinterpret_cast<T*>(la.dv) + b * la.dv_bs + hk * la.dv_hs : reinterpret_cast<T*>(la.dk) + b * la.dk_bs + hk * la.dk_hs;
   const int64_t rs = role == 0 ? la.dv_rs : la.dk_rs;
-  store_rows_through_lds<E, D, DBN>(patch, acc, role == 0 ? 1.0f : la.scale, [&](const int r) -> T* {
+  store_rows_through_lds<E, D, DBN>(patch, acc, role == 0 ? 1.0f : -la.scale, [&](const int r) -> T* {
     return nw + r < N ? base + int64_t(nw + r) * rs : nullptr;
   });
 }
