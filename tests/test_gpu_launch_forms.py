@@ -74,6 +74,27 @@ def test_heads_that_share_a_tile_backward(case):
         check_close(name, got, ref)
 
 
+# the decode form with two workgroups to a CU: more 32-row tiles than CUs on short ranges, and a single tile per head for many heads
+TWO_PER_CU_CASES = [
+    (1, 32, 8, 333, 333, 128, torch.bfloat16, True, 0, 0),
+    (2, 16, 16, 400, 410, 64, torch.float16, False, 0, 0),
+    (1, 33, 33, 300, 300, 32, torch.bfloat16, True, 70, 0),
+    (3, 32, 16, 160, 500, 16, torch.float16, True, 0, 300),
+    (40, 16, 8, 3, 100, 128, torch.bfloat16, True, 0, 0),
+    (300, 2, 1, 1, 65, 64, torch.float16, False, 0, 0),
+]
+
+
+@pytest.mark.parametrize("case", TWO_PER_CU_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-%s-c%d-w%d-p%d" % (
+    *c[:6], str(c[6])[6:], *c[7:]))
+def test_decode_form_two_to_a_cu(case):
+    test_forward_only_forms(case)
+
+
+def test_decode_form_two_to_a_cu_backward():
+    test_heads_that_share_a_tile_backward((1, 32, 8, 333, 333, 128, True))
+
+
 # query lengths, key lengths (None: the queries'), tokens behind the last boundary, H, Hk, D, causal, window
 PACKED_CASES = [
     ([64, 128, 1, 0, 65, 300], None, 0, 4, 2, 128, True, 0),

@@ -121,11 +121,11 @@ extern "C" uint64_t fa_workspace_scratch_bytes(const fa_params* p) {
   return w.total - w.plan;
 }
 
-static KArgs make_args(const fa_params* p, uint64_t split_budget = kSplitScratchBudget) {
+static KArgs make_args(const fa_params* p, bool fwd, uint64_t split_budget = kSplitScratchBudget) {
   KArgs a;
-  const FwdCfg fc = fwd_config(p);
+  const FwdCfg fc = fwd_config(p, fwd);
   a.pack = fc.pack; a.nHp = p->H / fc.pack;
-  a.bm = fc.bm; a.nTiles = fc.tiles; a.dsplit = fc.split;
+  a.bm = fc.bm; a.nTiles = fc.tiles; a.dsplit = fc.split; a.wpc = fc.wpc;
   a.shdr = nullptr; a.qtab = a.ktab = nullptr; a.nQent = a.nKent = 0;
   a.q = p->q; a.k = p->k; a.v = p->v; a.o = p->o; a.lse = p->lse;
   a.dout = p->dout; a.dq = p->dq; a.dk = p->dk; a.dv = p->dv; a.delta = p->delta;
@@ -230,9 +230,9 @@ extern "C" int fa_fwd(const fa_params* p, void* stream) {
   if (rc != FA_OK) return rc;
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (p->dtype == FA_DTYPE_FP32) return finish(launch_fwd_f32(make_args(p), p->D, causal, doc, s));
-  if (fwd_config(p).dec) return finish(launch_decode(make_args(p), p->dtype, p->D, causal, s));
-  return finish(launch_fwd(make_args(p), p->dtype, p->D, causal, doc, s));
+  if (p->dtype == FA_DTYPE_FP32) return finish(launch_fwd_f32(make_args(p, true), p->D, causal, doc, s));
+  if (fwd_config(p).dec) return finish(launch_decode(make_args(p, true), p->dtype, p->D, causal, s));
+  return finish(launch_fwd(make_args(p, true), p->dtype, p->D, causal, doc, s));
 }
 
 // ---------------------------------------------------------------------------
@@ -287,16 +287,16 @@ extern "C" int fa_fwd_static(const fa_params* p, void* stream) {
   // counters with a kernel, so nothing of an earlier call's contents is ever looked at
   if (int e = launch_mask_plan(&q, w, s)) return finish(e);
   const bool causal = q.causal != 0;
-  if (q.dtype == FA_DTYPE_FP32) return finish(launch_fwd_f32(make_args(&q, kStaticSplitBudget), q.D, causal, true, s));
-  return finish(launch_fwd(make_args(&q, kStaticSplitBudget), q.dtype, q.D, causal, true, s));
+  if (q.dtype == FA_DTYPE_FP32) return finish(launch_fwd_f32(make_args(&q, true, kStaticSplitBudget), q.D, causal, true, s));
+  return finish(launch_fwd(make_args(&q, true, kStaticSplitBudget), q.dtype, q.D, causal, true, s));
 }
 
 extern "C" int fa_bwd_delta(const fa_params* p, void* stream) {
   int rc = fa_validate(p, 1);
   if (rc != FA_OK) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_delta_f32(make_args(p), p->D, s));
-  return finish(launch_bwd_delta(make_args(p), p->dtype, p->D, s));
+  if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_delta_f32(make_args(p, false), p->D, s));
+  return finish(launch_bwd_delta(make_args(p, false), p->dtype, p->D, s));
 }
 
 extern "C" int fa_pair_wait_expired(uint64_t* count) {
@@ -312,8 +312,8 @@ extern "C" int fa_bwd_dkdv(const fa_params* p, void* stream) {
   if (rc != FA_OK) return rc;
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dkdv_f32(make_args(p), p->D, causal, doc, s));
-  return finish(launch_bwd_dkdv(make_args(p), p->dtype, p->D, causal, doc, s));
+  if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dkdv_f32(make_args(p, false), p->D, causal, doc, s));
+  return finish(launch_bwd_dkdv(make_args(p, false), p->dtype, p->D, causal, doc, s));
 }
 
 extern "C" int fa_bwd_dq(const fa_params* p, void* stream) {
@@ -321,8 +321,8 @@ extern "C" int fa_bwd_dq(const fa_params* p, void* stream) {
   if (rc != FA_OK) return rc;
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dq_f32(make_args(p), p->D, causal, doc, s));
-  return finish(launch_bwd_dq(make_args(p), p->dtype, p->D, causal, doc, s));
+  if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dq_f32(make_args(p, false), p->D, causal, doc, s));
+  return finish(launch_bwd_dq(make_args(p, false), p->dtype, p->D, causal, doc, s));
 }
 
 extern "C" int fa_bwd(const fa_params* p, void* stream) {
@@ -330,7 +330,7 @@ extern "C" int fa_bwd(const fa_params* p, void* stream) {
   if (rc != FA_OK) return rc;
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  KArgs a = make_args(p);
+  KArgs a = make_args(p, false);
   if (p->dtype == FA_DTYPE_FP32 && bwd_f32_in_one(a, p->D)) {
     if (int e = launch_bwd_delta_f32(a, p->D, s)) return finish(e);
     a.dq_delta = 0;
@@ -355,7 +355,7 @@ extern "C" int fa_mask_dump(const fa_params* p, uint8_t* out, void* stream) {
   if (rc != FA_OK) return rc;
   if (out == nullptr) return FA_ERR_NULLPTR;
   if (p->score_mode == FA_SCORE_MODE3_PACKED) return FA_ERR_NOT_IMPLEMENTED;
-  return finish(launch_mask_dump(make_args(p), p->causal != 0, p->score_mode == FA_SCORE_MODE1_DOC, out,
+  return finish(launch_mask_dump(make_args(p, false), p->causal != 0, p->score_mode == FA_SCORE_MODE1_DOC, out,
                                  reinterpret_cast<hipStream_t>(stream)));
 }
 

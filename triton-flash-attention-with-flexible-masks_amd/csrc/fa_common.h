@@ -118,7 +118,16 @@ constexpr int kCUs = 256;
 // where they are many, faster where they are few, and the sum of the kernels gains (64-row tiles : these, us: 8 heads x 1000
 // rows 52.8 : 52.4, the backward of it 30.2 : 32.3; 8 heads x 512 33.3 : 31.2; 16 x 500 34.8 : 35.0; 64 rows on 1000 keys
 // 44.3 : 40.0; 40 rows on 900 39.7 : 32.0).
-constexpr int kDecTiles = kCUs, kDecKeys = 1024;
+// From there to two such tiles to a CU the forward takes the decode form with two workgroups to a CU, half the stages each,
+// and the backward the tiles it would have without (us, 64-row form : this one): 32 heads on 8 x 333 rows 10.9 : 9.3, x 512
+// 12.9 : 11.2, without a causal mask 11.0 : 10.4; 32 heads x 500 12.4 : 10.8; 16 x 1000 18.7 : 16.8, without a causal mask 20.6 :
+// 21.2 (hence kDecKeys2); D = 64: 16 on 4 heads x 900 12.9 : 9.6, 4 x 16 x 256 7.0 : 6.6.  With more tiles a second round begins:
+// 32 on 8 x 700 (704 tiles) 16.4 : 19.2.
+constexpr int kDecTiles = kCUs, kDecTiles2 = 2 * kCUs, kDecKeys = 1024, kDecKeys2 = 768;
+// A single tile to a head and more heads than CUs: two workgroups to a CU up to this many keys x D (us, one : two to a CU; 512
+// tiles on 100 keys 12.0 : 7.2, 400 24.8 : 20.0, 900 41.6 : 37.9, D = 64 on 1000 28.5 : 24.4, 2048 tiles on 700 136 : 128; on 3000
+// 136 : 139).  Packed sequences take the 64-row form there (256 on 128 keys 37 : 53).
+constexpr int kDecShort = 1536 * 128;
 // With packed sequences of at most 32 rows on average the decode form, one workgroup to a CU, is the better one for few
 // tiles (a split key range adds to them) and, whatever their number, for long key ranges: 4 sequences x 8 key heads on 8192
 // keys 44 us against 70 of 64-row tiles; 64 on 1100 keys 63 : 68, on 2048 112 : 122, on 8192 434 : 471, 256 on 2048 423 : 420
@@ -126,7 +135,7 @@ constexpr int kDecTiles = kCUs, kDecKeys = 1024;
 // 64 on 512 keys 36 : 33, 4 key heads 37 : 27, 256 on 128 62 : 45, 1024 on 128 236 : 163; 600 sequences of 3 - 48 tokens, 8
 // heads 165 : 69, 32 heads of D = 64 460 : 126.
 constexpr int kDecSeqTiles = kCUs / 2, kDecSeqKeys = 1024;   // keys at D = 128; four times as many at 64
-struct FwdCfg { int pack, bm, tiles, split; bool dec; };
+struct FwdCfg { int pack, bm, tiles, split; bool dec; int wpc; };
 // Chunks for `wgs` tiles of `steps` steps each: the cheapest total by a model of rounds x (set-up + steps of a chunk)
 // + merging, in units of one step; `slots` workgroups run at a time.  A chunk keeps at least `min_steps` steps.
 inline int pick_split(int64_t wgs, int steps, int slots, float setup, float merge, int min_steps) {
@@ -148,8 +157,8 @@ inline int shared_heads(const fa_params* p) {
   const int G = p->H / p->Hk;
   return int64_t(p->M) * G <= 0x7fffffff - 256 ? G : 1;
 }
-inline FwdCfg fwd_config(const fa_params* p) {
-  FwdCfg c = {1, 128, 0, 1, false};
+inline FwdCfg fwd_config(const fa_params* p, bool fwd = true) {   // fwd: for the forward (the backward may take other tiles)
+  FwdCfg c = {1, 128, 0, 1, false, 1};
   if (p->score_mode == FA_SCORE_MODE3_PACKED) {
     // the host knows the totals only: 32-row tiles when an average sequence fills no more
     c.pack = shared_heads(p);
@@ -169,6 +178,7 @@ inline FwdCfg fwd_config(const fa_params* p) {
     // workgroup up takes about as long, handing the result over and merging one and a half steps
     const float rel = 128.f / p->D;
     if (p->flags & FA_FLAG_SPLIT_KEYS) c.split = pick_split(bh * c.tiles, (nk + 127) / 128, kCUs, 1.2f * rel, 1.5f * rel, 2);
+    if (c.split == 1 && bh * c.tiles > kCUs && int64_t(nk) * p->D <= kDecShort) c.wpc = 2;
     return c;
   }
   c.tiles = int((rows + 127) / 128);
@@ -176,6 +186,7 @@ inline FwdCfg fwd_config(const fa_params* p) {
   // a step: one 64-key tile; two workgroups to a CU
   if ((p->flags & FA_FLAG_SPLIT_KEYS) && c.tiles * bh < 2 * kCUs)
     c.split = pick_split(c.tiles * bh, (nk + 63) / 64, 2 * kCUs, 3.f, 4.f, 8);
+  if (fwd && c.split == 1 && bh * ((rows + 31) / 32) <= kDecTiles2 && seen <= kDecKeys2) { c.dec = true; c.bm = 32; c.tiles = int((rows + 31) / 32); c.wpc = 2; }
   return c;
 }
 
@@ -422,6 +433,7 @@ struct KArgs {
   int pack, nHp;          // query heads per tile, H / pack
   int bm, nTiles;         // rows per query tile, tiles per (batch, head group)
   int dsplit;             // chunks of the key range of every tile
+  int wpc;                // the decode form: workgroups to a CU
   // packed sequences: tables of the plan (null otherwise) and their capacities
   const SeqHdr* shdr;
   const SeqTile* qtab;

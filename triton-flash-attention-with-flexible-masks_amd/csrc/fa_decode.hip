@@ -10,13 +10,19 @@
 //   * the key range is cut into chunks until the chip is full (pick_split, fa_common.h); the last chunk to arrive
 //     merges the partial results, rows x D fp32 each.
 // Measured (16 sequences x 8 key heads x 6001 keys, G = 4, D = 128, bf16, 394 MB): 228 us in the 128-row form, 77 here, 5.1 TB/s
-// with launch and merge.  Starting the workgroups at different places of their ranges changed nothing (77.3).
+// with launch and merge.  Where short ranges leave more workgroups than CUs, two of them share one (half the LDS, the register file
+// halved too): see kDecTiles2 and kDecShort in fa_common.h.  Starting the workgroups at different places of their ranges changed nothing (77.3).
 #include "fa_tile.h"
 
 namespace fa {
 namespace {
 
-constexpr int kDecStageBytes = 32 * 1024;   // LDS of a wave: stages x (K + V) x 32 keys x D x 2 bytes
+// LDS of a wave: stages x (K + V) x 32 keys x D x 2 bytes.  One workgroup to a CU, or two (short ranges, see kDecTiles).
+template <int WPC> constexpr int dec_stage_bytes() { return 32 * 1024 / WPC; }
+template <int WPC, int D> constexpr size_t dec_lds() {
+  const size_t merge = (512 + 4 * ((D + 31) / 32) * 16 * 64) * 4, tiles = 4 * dec_stage_bytes<WPC>();
+  return merge > tiles ? merge : tiles;
+}
 
 // One wave's tile stream: 32 rows of D elements, global -> LDS, in the swizzled layout of fa_tile.h.
 template <int DL, int GD>
@@ -43,15 +49,15 @@ struct WaveLoader {
 
 template <int N> FA_DEV void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
 
-template <typename Tag, int D, bool CAUSAL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <typename Tag, int D, bool CAUSAL, int WPC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPC, WPC)))
 void decode_kernel(const KArgs a) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
   constexpr int KS = D / 16, DL = D < 32 ? 32 : D, DBN = DL / 32;
   constexpr int TB = 32 * DL * 2;                          // bytes of a 32-key tile
-  constexpr int NST = kDecStageBytes / (2 * TB);           // stages per wave: 2 at D = 128, 4 at 64, 8 below
+  constexpr int NST = dec_stage_bytes<WPC>() / (2 * TB);   // stages per wave: 2 (1) at D = 128, 4 (2) at 64, 8 (4) below
   using Loader = WaveLoader<DL, D>;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -81,7 +87,7 @@ void decode_kernel(const KArgs a) {
   Loader ldK, ldV;
   ldK.init(kp, a.k_rs, ge.N);
   ldV.init(vp, a.v_rs, ge.N);
-  char* my = smem + wave * kDecStageBytes;
+  char* my = smem + wave * dec_stage_bytes<WPC>();
   vec8 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const vec8*>(qp + ks * 16 + g * 8);
@@ -278,14 +284,18 @@ void decode_kernel(const KArgs a) {
   }
 }
 
+template <typename Tag, int D, bool CAUSAL, int WPC>
+int launch_wpc(const KArgs& a, hipStream_t s) {
+  auto kern = decode_kernel<Tag, D, CAUSAL, WPC>;
+  static bool lds_allowed[64] = {};   // per kernel instantiation and device
+  if (int e = allow_lds(kern, dec_lds<WPC, D>(), lds_allowed)) return e;
+  hipLaunchKernelGGL(kern, dim3(tile_geo_blocks(a)), dim3(256), (dec_lds<WPC, D>()), s, a);
+  return (int)hipGetLastError();
+}
 template <typename Tag, int D, bool CAUSAL>
 int launch_one(const KArgs& a, hipStream_t s) {
-  const size_t lds = 4 * kDecStageBytes;
-  auto kern = decode_kernel<Tag, D, CAUSAL>;
-  static bool lds_allowed[64] = {};   // per kernel instantiation and device
-  if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  hipLaunchKernelGGL(kern, dim3(tile_geo_blocks(a)), dim3(256), lds, s, a);
-  return (int)hipGetLastError();
+  if (a.wpc > 1) return launch_wpc<Tag, D, CAUSAL, 2>(a, s);
+  return launch_wpc<Tag, D, CAUSAL, 1>(a, s);
 }
 template <typename Tag>
 int launch_d(const KArgs& a, int D, bool causal, hipStream_t s) {
