@@ -309,8 +309,7 @@ def test_packed_graph_replay():
             assert torch.equal(got, attention_varlen(q, k, v, cq, ck, causal=True)), rep
 
 
-# fp32: launches of few workgroups split a tile of the streamed side over the four waves; the sizes around its edges, and
-# the smallest launch that keeps 128 rows to a workgroup.  B, H, Hk, M, N, D, causal, doc, window
+# fp32: sizes around the edges of blocks of rows and keys.  B, H, Hk, M, N, D, causal, doc, window
 FP32_CASES = [
     (1, 2, 2, 1, 1, 64, True, False, 0), (1, 2, 1, 33, 129, 64, True, False, 0), (2, 2, 2, 128, 300, 128, True, True, 0),
     (1, 4, 2, 257, 257, 64, True, True, 0), (1, 2, 2, 200, 200, 32, False, True, 0), (1, 2, 2, 150, 700, 16, True, True, 90),
@@ -323,6 +322,53 @@ def test_fp32_launch_forms(case):
     from tests.test_gpu_parity import _run_case
     B, H, Hk, M, N, D, causal, doc, window = case
     _run_case(B, H, Hk, M, N, D, torch.float32, causal, doc, seed=3, window=window, tol_o=2e-4, tol_lse=2e-4)
+
+
+# fp32: 16 or 32 rows (keys) to a workgroup and two, four or eight waves to share the other side, by the number of blocks of 16:
+# up to 768 (rows with ids: 2048), up to 4096 (16384), above.  B, H, Hk, M, N, D, causal, kind
+FP32_SHAPE_CASES = [
+    (2, 16, 16, 330, 330, 64, True, "plain"), (2, 16, 8, 384, 400, 32, True, "window"),      # the first shape, dq and dk/dv in launches of their own
+    (2, 16, 16, 500, 501, 64, True, "plain"), (4, 16, 8, 545, 545, 64, True, "doc"), (1, 64, 64, 210, 270, 128, True, "prefix"),   # the second
+    (4, 16, 4, 530, 530, 16, False, "heads"), (2, 16, 16, 600, 333, 32, True, "qpos"), (2, 16, 16, 450, 450, 128, True, "block"),
+    (64, 64, 64, 49, 33, 16, False, "plain"), (32, 128, 64, 50, 65, 64, True, "plain"), (16, 64, 64, 257, 257, 16, True, "doc"),   # the third
+    (8, 32, 32, 260, 260, 128, True, "doc"), (16, 32, 16, 130, 140, 128, True, "block"), (64, 64, 64, 63, 64, 32, True, "window"),
+]
+
+
+@pytest.mark.parametrize("case", FP32_SHAPE_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-c%d-%s" % c)
+def test_fp32_workgroup_shapes(case):
+    B, H, Hk, M, N, D, causal, kind = case
+    if kind == "block":
+        from tests.test_gpu_parity import test_block_mask_parity
+        test_block_mask_parity((B, H, Hk, M, N, D, torch.float32, causal, 0, 0.6, False))
+        return
+    from tests.test_gpu_parity import _run_case
+    _run_case(B, H, Hk, M, N, D, torch.float32, causal, kind in ("doc", "heads", "qpos"), seed=6, window=37 if kind == "window" else 0,
+              prefix=21 if kind == "prefix" else 0, per_head_ids=kind == "heads", qpos="random" if kind == "qpos" else None, tol_o=2e-4, tol_lse=2e-4)
+
+
+@pytest.mark.parametrize("L,heads", [(37, 2), (69, 2), (101, 800)])
+@pytest.mark.parametrize("D", [16, 64, 128])
+def test_fp32_infinities_stay_with_their_documents(L, heads, D):
+    """An infinity reaches the rows (keys) that see it and no others of other blocks, also where a block has fewer than 16 rows or keys: the
+    missing ones are read from some row that is there, and count as zero.  Two documents, the first of 32 rows, whole blocks."""
+    from flash_mi355 import attention, SCORE_FUNC_MODE1_DOC
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v, do = (torch.randn(1, heads, L, D, generator=g).cuda() for _ in range(4))
+    ids = (-1 - (torch.arange(L) >= 32).int()).cuda().view(1, 1, L).expand(1, heads, L)
+    for kept in ("last", "first"):   # the last key and row (which stand in for the ones past the end), the first (for empty places of the order)
+        i = -1 if kept == "last" else 0
+        vi, doi = v.clone(), do.clone()
+        vi[:, :, i, 0] = math.inf
+        doi[:, :, i, 0] = math.inf
+        sees = slice(32, L) if kept == "last" else slice(0, 32)
+        other = slice(0, 32) if kept == "last" else slice(32, L)
+        with torch.no_grad():
+            out = attention(q, k, vi, False, None, ids, ids, SCORE_FUNC_MODE1_DOC)
+        assert torch.isposinf(out[:, :, sees, 0]).all() and torch.isfinite(out[:, :, other]).all() and torch.isfinite(out[..., 1:]).all()
+        qd, kd, vd = (t.clone().requires_grad_(True) for t in (q, k, v))
+        dv, = torch.autograd.grad(attention(qd, kd, vd, False, None, ids, ids, SCORE_FUNC_MODE1_DOC), (vd,), doi)
+        assert torch.isposinf(dv[:, :, sees, 0]).all() and torch.isfinite(dv[:, :, other]).all() and torch.isfinite(dv[..., 1:]).all()
 
 
 @pytest.mark.parametrize("M,N,per_head,id_dtype,qpos", [(1, 1, False, torch.int32, None), (64, 2048, True, torch.int64, None), (1025, 1025, False, torch.int64, None),

@@ -331,13 +331,9 @@ extern "C" int fa_bwd(const fa_params* p, void* stream) {
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   KArgs a = make_args(p, false);
-  if (p->dtype == FA_DTYPE_FP32 && bwd_f32_in_one(a, p->D)) {
-    if (int e = launch_bwd_delta_f32(a, p->D, s)) return finish(e);
-    a.dq_delta = 0;
-    return finish(launch_bwd_f32(a, p->D, causal, doc, s));
-  }
   a.dq_delta = 1;
   if (p->dtype == FA_DTYPE_FP32) {
+    if (bwd_f32_in_one(a)) return finish(launch_bwd_f32(a, p->D, causal, doc, s));
     if (int e = launch_bwd_dq_f32(a, p->D, causal, doc, s)) return finish(e);
     return finish(launch_bwd_dkdv_f32(a, p->D, causal, doc, s));
   }

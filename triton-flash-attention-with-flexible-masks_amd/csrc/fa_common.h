@@ -585,7 +585,7 @@ int launch_fwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 int launch_bwd_delta_f32(const KArgs& a, int D, hipStream_t s);
 int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
-bool bwd_f32_in_one(const KArgs& a, int D);
+bool bwd_f32_in_one(const KArgs& a);
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s);
 int launch_mask_dump(const KArgs& a, bool causal, bool doc, uint8_t* out, hipStream_t s);
