@@ -422,6 +422,56 @@ def test_backward_in_one_launch(case):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
 
 
+# dk/dv by workgroups of 32 keys whose waves share the rows: blocks of rows and keys that are partly filled, heads of a group, one key, more
+# keys than rows, waves without a block; next to dq in one launch, and (documents with keys of no local row) by itself up to its line
+# and the column form behind it.  B, H, Hk, M, N, D, dtype, causal, kind
+SMALL_BWD_CASES = [
+    (1, 1, 1, 1, 1, 64, torch.bfloat16, True, "plain"), (1, 8, 2, 33, 31, 128, torch.float16, False, "plain"), (1, 4, 1, 97, 130, 128, torch.bfloat16, True, "window"),
+    (2, 8, 2, 161, 222, 64, torch.float16, True, "prefix"), (1, 4, 2, 190, 190, 64, torch.bfloat16, True, "block"), (1, 2, 2, 500, 333, 128, torch.float16, False, "block"),
+    (1, 4, 4, 300, 300, 128, torch.bfloat16, True, "doc"), (2, 4, 1, 70, 500, 64, torch.bfloat16, True, "doc"), (1, 4, 2, 65, 1000, 128, torch.float16, True, "heads"),
+    (1, 2, 1, 333, 77, 64, torch.float16, True, "qpos"), (1, 3, 1, 40, 800, 128, torch.bfloat16, False, "doc"),
+    (2, 16, 16, 64, 700, 64, torch.bfloat16, True, "doc"), (1, 32, 16, 130, 900, 128, torch.bfloat16, True, "doc"), (1, 16, 16, 97, 800, 128, torch.float16, False, "heads"),
+    (4, 16, 8, 300, 1600, 128, torch.bfloat16, True, "doc"), (8, 16, 16, 40, 801, 64, torch.float16, False, "doc"),   # (the column form)
+]
+
+
+@pytest.mark.parametrize("case", SMALL_BWD_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-%s-c%d-%s" % (*c[:6], str(c[6])[6:], *c[7:]))
+def test_small_backward(case):
+    B, H, Hk, M, N, D, dtype, causal, kind = case
+    if kind == "block":
+        from tests.test_gpu_parity import test_block_mask_parity
+        test_block_mask_parity((B, H, Hk, M, N, D, dtype, causal, 0, 0.6, False))
+        return
+    from tests.test_gpu_parity import _run_case
+    _run_case(B, H, Hk, M, N, D, dtype, causal, kind in ("doc", "heads", "qpos"), seed=9, window=37 if kind == "window" else 0,
+              prefix=21 if kind == "prefix" else 0, per_head_ids=kind == "heads", qpos="random" if kind == "qpos" else None)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("lq,lk", [([1, 40, 0, 77], [5, 40, 33, 130]), ([64], [64]), ([3] * 9, [1, 0, 200, 31, 32, 33, 64, 65, 2])])
+def test_small_backward_packed(D, lq, lk):
+    """Sequences without rows or without keys, and key tiles that are partly filled: dk and dv of the keys, each sequence by itself."""
+    from flash_mi355 import attention_varlen
+    from oracle import attention_oracle as O
+    H, Hk = 4, 2
+    q, k, v, do = _tensors(1, H, Hk, sum(lq), sum(lk), D, torch.bfloat16, 5)
+    t3 = lambda t: t[0].transpose(0, 1).contiguous()
+    cu = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32).cuda()
+    qd, kd, vd = (t3(t).cuda().requires_grad_(True) for t in (q, k, v))
+    out = attention_varlen(qd, kd, vd, cu(lq), cu(lk), causal=False)
+    out.backward(t3(do).cuda())
+    got = [t.grad.float().cpu().transpose(0, 1)[None] for t in (qd, kd, vd)]
+    a = b = 0
+    for m, n in zip(lq, lk):
+        if m and n:
+            ref = O.attention_autograd(q[:, :, a:a + m], k[:, :, b:b + n], v[:, :, b:b + n], do[:, :, a:a + m], False, None, None, None, 0)[2:]
+            for name, g, r, s in (("dq", got[0], ref[0], slice(a, a + m)), ("dk", got[1], ref[1], slice(b, b + n)), ("dv", got[2], ref[2], slice(b, b + n))):
+                check_close(name, g[:, :, s], r)
+        else:
+            assert got[1][:, :, b:b + n].abs().sum() == 0 and got[2][:, :, b:b + n].abs().sum() == 0 and got[0][:, :, a:a + m].abs().sum() == 0
+        a += m; b += n
+
+
 # the pipelined dk/dv form (D = 128, at least 32 query tiles over the heads of a group): tiles and key blocks that are partly
 # filled, one key, heads of a group in one stream, a window, a prefix, more keys than queries and fewer
 PIPE_CASES = [

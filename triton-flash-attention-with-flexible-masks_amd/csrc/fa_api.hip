@@ -313,7 +313,10 @@ extern "C" int fa_bwd_dkdv(const fa_params* p, void* stream) {
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dkdv_f32(make_args(p, false), p->D, causal, doc, s));
-  return finish(launch_bwd_dkdv(make_args(p, false), p->dtype, p->D, causal, doc, s));
+  const KArgs a = make_args(p, false);
+  if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) == 0 && bwd_small_form(a, p->D, causal, doc) != SMALL_NONE)   // (the bits of fa_bwd)
+    return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, false, s));
+  return finish(launch_bwd_dkdv(a, p->dtype, p->D, causal, doc, s));
 }
 
 extern "C" int fa_bwd_dq(const fa_params* p, void* stream) {
@@ -336,6 +339,11 @@ extern "C" int fa_bwd(const fa_params* p, void* stream) {
     if (bwd_f32_in_one(a)) return finish(launch_bwd_f32(a, p->D, causal, doc, s));
     if (int e = launch_bwd_dq_f32(a, p->D, causal, doc, s)) return finish(e);
     return finish(launch_bwd_dkdv_f32(a, p->D, causal, doc, s));
+  }
+  if (const int form = bwd_small_form(a, p->D, causal, doc)) {
+    if (form == SMALL_DKDV)
+      if (int e = launch_bwd_dq(a, p->dtype, p->D, causal, doc, s)) return finish(e);
+    return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, form == SMALL_BOTH, s));
   }
   if (bwd_in_one(a, p->D, causal, doc)) {
     if (int e = launch_bwd_delta(a, p->dtype, p->D, s)) return finish(e);

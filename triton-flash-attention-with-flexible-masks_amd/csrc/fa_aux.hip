@@ -423,8 +423,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const KArgs a) {
       const T* dp = reinterpret_cast<const T*>(a.dout) + b * a.do_bs + h * a.do_hs + int64_t(row) * a.do_rs + c * 8;
       const vec8 x = *reinterpret_cast<const vec8*>(op);
       const vec8 y = *reinterpret_cast<const vec8*>(dp);
-#pragma unroll
-      for (int t = 0; t < 8; ++t) acc += float(x[t]) * float(y[t]);
+      acc = dot8(x, y);
     }
 #pragma unroll
     for (int off = LPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);

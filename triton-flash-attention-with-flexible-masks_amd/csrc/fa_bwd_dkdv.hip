@@ -832,7 +832,7 @@ static int launch_both_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) 
   return causal ? launch_both<Tag, D, true, GEO_PLAIN>(a, s) : launch_both<Tag, D, false, GEO_PLAIN>(a, s);
 }
 
-// Whether a backward of these sizes takes the shared launch: with at most eight workgroups to a CU in all (two run at a time),
+// Whether a backward of these sizes (that fa_bwd_small.hip has not taken) takes the shared launch: with at most eight workgroups to a CU in all (two run at a time),
 // where the drain of one launch and the start of the next weigh most; beyond that, forming delta in a launch of its own
 // reads more than is gained.  Forward + backward, separate -> shared,
 // D = 128: 8 heads on 2 key heads, causal, 2000 / 3000 / 5000 rows (316 - 790 workgroups) 306 -> 226, 443 -> 327, 783 -> 567

@@ -300,6 +300,17 @@ FA_DEV void mul_f16_f32(f16x8 p, const int e, float x0, float x1, float& y0, flo
   asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y1) : "v"(pp), "v"(x1));
 }
 
+// Eight products of 16-bit elements, added up in order.  Not to be contracted: for fp16 the compiler makes two-element dot
+// products of some such sums and not of others, which round differently, and a delta is to have the same bits wherever it is formed.
+template <typename V>
+FA_DEV float dot8(const V& x, const V& y) {
+#pragma clang fp contract(off)
+  float s = 0.f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) s = __builtin_fmaf(float(x[t]), float(y[t]), s);
+  return s;
+}
+
 // Make a 16-byte value loaded from global memory "used" right here.  The compiler waits for a
 // load at the first use of its result; for operands that are loaded once and first used inside
 // the tile loop that wait (s_waitcnt vmcnt) would sit in the loop, where it also waits for the
@@ -587,6 +598,10 @@ int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t 
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 bool bwd_f32_in_one(const KArgs& a);
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
+// dk/dv of problems that leave CUs idle (fa_bwd_small.hip): not of these sizes, next to dq in one launch, by itself
+enum { SMALL_NONE, SMALL_BOTH, SMALL_DKDV };
+int bwd_small_form(const KArgs& a, int D, bool causal, bool doc);
+int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bool both, hipStream_t s);
 int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s);
 int launch_mask_dump(const KArgs& a, bool causal, bool doc, uint8_t* out, hipStream_t s);
 

@@ -88,13 +88,7 @@ FA_DEV void dq_body(const KArgs& a, const int bid, char* smem) {
   settle(L_i);
   settle(delta_i);
   if (own_delta) {
-    // the lane and its partner (lane ^ 32) hold the two halves of every 16 columns of the row
-    float part = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int t = 0; t < 8; ++t) part += float(of[ks][t]) * float(dof[ks][t]);
-    delta_i = xhalf_sum(part);
+    delta_i = row_delta<KS>(of, dof);   // (the lane and its partner, lane ^ 32, hold the two halves of the row)
     if (row >= 0 && g == 0 && ge.chunk == 0 && sub == 0) a.delta[row_l] = delta_i;   // for the dk/dv kernel
   }
   // D = 128: the product dP starts from delta and runs on -dO, its accumulators then hold delta - dP, dS comes out with the sign

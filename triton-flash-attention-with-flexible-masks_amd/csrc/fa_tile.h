@@ -652,6 +652,20 @@ template <int MODE>
 FA_HD int launch_groups(const KArgs& a) { return MODE != GEO_GENERAL ? a.B * a.H : a.qtab != nullptr ? a.nHp : a.B * a.nHp; }
 inline bool geo_general(const KArgs& a) { return a.pack > 1 || a.dsplit > 1 || a.bm != 128 || a.qtab != nullptr; }
 
+// rowsum(O * dO) of row l % 32 by the two lanes that hold its halves (16-byte pieces 2 ks + l / 32), in the order in which
+// delta_kernel adds up, so that a delta has the same bits wherever it is formed
+template <int KS, typename vec8>
+FA_DEV float row_delta(const vec8 (&o)[KS], const vec8 (&d)[KS]) {
+  float part[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) part[ks] = dot8(o[ks], d[ks]);
+#pragma unroll
+  for (int off = KS / 2; off >= 1; off >>= 1)
+#pragma unroll
+    for (int ks = 0; ks < off; ++ks) part[ks] += part[ks + off];
+  return xhalf_sum(part[0]);
+}
+
 // A wave's 32 result rows on their way out.  The accumulators hold a row (or key) per lane and 4 consecutive
 // columns per register quad: stored from there, a wave instruction writes 64 pieces of 8 bytes, a row apart, and
 // every 128-byte line of the result fills up over sixteen instructions -- measured at 5-13 % of the id

@@ -20,7 +20,7 @@ INCLUDE = PKG_DIR.parent.parent / "include"
 LIB_PATH = PKG_DIR / "libflash_mi355.so"
 OBJ_DIR = PKG_DIR / "_obj"
 
-SOURCES = ["fa_api.hip", "fa_aux.hip", "fa_fwd.hip", "fa_decode.hip", "fa_seq.hip", "fa_bwd_dq.hip", "fa_bwd_dkdv.hip", "fa_dkdv_pipe.hip", "fa_f32.hip"]
+SOURCES = ["fa_api.hip", "fa_aux.hip", "fa_fwd.hip", "fa_decode.hip", "fa_seq.hip", "fa_bwd_dq.hip", "fa_bwd_dkdv.hip", "fa_dkdv_pipe.hip", "fa_bwd_small.hip", "fa_f32.hip"]
 # measurement aid of bench.py --mfma-probe (sustained MFMA rate of the chip); a library of its own
 PROBE_SOURCE = "probe_mfma.hip"
 PROBE_LIB_PATH = PKG_DIR / "libfa_probe.so"
