@@ -314,7 +314,7 @@ extern "C" int fa_bwd_dkdv(const fa_params* p, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dkdv_f32(make_args(p, false), p->D, causal, doc, s));
   const KArgs a = make_args(p, false);
-  if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) == 0 && bwd_small_form(a, p->D, causal, doc) != SMALL_NONE)   // (the bits of fa_bwd)
+  if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) == 0 && bwd_small(a, p->D, doc))   // (the bits of fa_bwd)
     return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, false, s));
   return finish(launch_bwd_dkdv(a, p->dtype, p->D, causal, doc, s));
 }
@@ -340,11 +340,7 @@ extern "C" int fa_bwd(const fa_params* p, void* stream) {
     if (int e = launch_bwd_dq_f32(a, p->D, causal, doc, s)) return finish(e);
     return finish(launch_bwd_dkdv_f32(a, p->D, causal, doc, s));
   }
-  if (const int form = bwd_small_form(a, p->D, causal, doc)) {
-    if (form == SMALL_DKDV)
-      if (int e = launch_bwd_dq(a, p->dtype, p->D, causal, doc, s)) return finish(e);
-    return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, form == SMALL_BOTH, s));
-  }
+  if (bwd_small(a, p->D, doc)) return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, true, s));
   if (bwd_in_one(a, p->D, causal, doc)) {
     if (int e = launch_bwd_delta(a, p->dtype, p->D, s)) return finish(e);
     a.dq_delta = 0;

@@ -31,7 +31,22 @@ namespace fa {
 constexpr int kKvPre = 4;
 constexpr int kKvPre2 = 3;
 
-constexpr int kColsRun = 8;   // key tiles per workgroup when the column form shares the launch
+// Key tiles per workgroup when the column form shares the launch: up to eight, so that the many tiles which belong to that form
+// are stepped over by few workgroups -- but no more than leave one workgroup to a CU, two where that form is not to be expected
+// (it takes two tiles of global rows, all heads of a group counted), since then every tile of a run has work to do.  Before,
+// always eight; dk/dv at D = 128, us: 32/8 heads x 2 x 243 rows on 800 keys 265 -> 49, 4 x 990 on 1685 61 -> 20, 48/12 x 909 on 2844
+// 190 -> 65, 8 x 4274 on 7495 65 -> 33, 32 x 564 on 1365 93 -> 41, 64/16 x 2000 on 6000 370 -> 232; D = 64: 16 x 4339 on 7980 146 -> 59,
+// 32/16 x 2598 on 5933 242 -> 109; unchanged 64 x 1024 on 8192 129, 32 x 4000 on 16384 199.  (At most two to a CU everywhere: 16 x 1024 on
+// 8192, where eight tiles of nine belong to the column form, 35 -> 39.  Powers of two: the tiles with work are the last ones, and of
+// 63 tiles in runs of seven some workgroups met two of them and others none, 64 -> 81.)
+constexpr int kColsRun = 8;
+constexpr int kColsFewRows = 2048;   // rows of a group of heads: a twentieth of them global is about two tiles
+FA_HD int cols_run(const KArgs& a, int nKt) {
+  const int64_t per = a.M * int64_t(a.G) <= kColsFewRows ? kCUs : 2 * kCUs, wgs = int64_t(nKt) * a.B * a.Hk;
+  int r = 1;
+  while (r < kColsRun && wgs >= 2 * r * per) r *= 2;
+  return r;
+}
 
 // SPLIT = true : two waves per block of 32 keys, NKB key blocks per workgroup, roles split over the
 //                wave pairs as described above (D = 128: one wave cannot hold both operand sets and
@@ -85,11 +100,12 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   using Loader = TileLoader<DL, BQ, D, NW>;
   const int nKt = (a.N + BK - 1) / BK;
   // With the column form in the launch, most key tiles of this form may have nothing to do here (their keys
-  // belong to the column form): a workgroup then takes kColsRun key tiles, nSlots tiles apart, and steps over
+  // belong to the column form): a workgroup then takes cols_run key tiles, nSlots tiles apart, and steps over
   // those -- a workgroup that only finds out that it is not needed costs the dispatcher as much as a short
   // useful one (8192 of them: 50 us), a skipped tile of a run costs a comparison.
   const bool packed = !DOC && a.ktab != nullptr;   // packed sequences: the slots are the plan's key tiles, longest first
-  const int nSlots = COLS ? (nKt + kColsRun - 1) / kColsRun : (packed ? a.nKent : nKt);
+  const int run = COLS ? cols_run(a, nKt) : 1;
+  const int nSlots = COLS ? (nKt + run - 1) / run : (packed ? a.nKent : nKt);
   if constexpr (COLS) {
     static_assert(DOC && (SPLIT ? 128 * NKB : 64 * NKB) == 256, "the column form runs with ids, 4 waves per workgroup");
     // the column form's workgroups come first: few, long, one round of them
@@ -120,7 +136,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   }
   const int ncols = COLS ? gcol_info(a, b, hk).ncols : 0;   // leading keys that belong to the column form of this launch
   bool ran = false;
-  for (int rr = 0; rr < (COLS ? kColsRun : 1); ++rr) {
+  for (int rr = 0; rr < run; ++rr) {
   const int kt = kt0 + rr * nSlots;
   const int n0 = kt * BK;
   if (COLS && (kt >= nKt || n0 + BK <= ncols)) continue;
@@ -765,7 +781,7 @@ static int launch_nkb(const KArgs& a, hipStream_t s) {
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
   const int slots = !DOC && a.ktab != nullptr ? a.nKent : nKt;
-  const int blocks = COLS ? grid_blocks((nKt + kColsRun - 1) / kColsRun, a.B * a.Hk) + dkdv_cols_blocks(a) : grid_blocks(slots, a.B * a.Hk);
+  const int blocks = COLS ? grid_blocks((nKt + cols_run(a, nKt) - 1) / cols_run(a, nKt), a.B * a.Hk) + dkdv_cols_blocks(a) : grid_blocks(slots, a.B * a.Hk);
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(SPLIT ? 128 * NKB : 64 * NKB), lds, s, a);
   return (int)hipGetLastError();
 }

@@ -6,7 +6,7 @@
 // their order.  (The forms of fa_bwd_dkdv.hip give every wave, or pair of waves, keys of its own and walk all rows with each:
 // 32 on 8 heads x 1339 rows, D = 64: 120 us for one long chain per 128 keys on 88 CUs, 75 here.)  A block of 32 x 32 pairs costs about
 // 1.4 us at D = 128, one wave to a SIMD, against 0.5 of its MFMAs: the reads of both operands from LDS count as much, and at
-// D = 128 a workgroup holds the whole LDS.  Hence for few workgroups only: see bwd_small_form.
+// D = 128 a workgroup holds the whole LDS.  Hence for few workgroups only: see bwd_small.
 #include "fa_tile.h"
 #ifdef FA_TRACE
 namespace fa { namespace { FA_TRACE_ARRAY(g_trace_dq); } }   // stamps of dq workgroups that share a launch: not read
@@ -391,19 +391,13 @@ int launch_cd(const KArgs& a, bool causal, bool doc, bool both, hipStream_t s) {
 //     beyond 31 packed sequences of up to 114 (118) 12.6 -> 17.6, 4 x 1416, packed (180) 41 -> 49; with grouped heads, whose chains
 //     are longer, up to 216 with dq's workgroups, those counted by the group: 8/2 x 3440, packed (146) 68 -> 56, 32/8 x 652 (216) 73 -> 58;
 //     beyond 16/8 x 2889 with a window (228) 36 -> 41, 32/8 x 2055, packed (352) 131 -> 145
-//   where the rows are the last of many more keys (dk/dv would be launched with its column form for the leading ones), which waits for a few long workgroups on a
-//     problem of this size: D = 64 up to 3072, D = 128 up to 1408.  8/2 x 612 rows on 1314 keys (D = 128) 447 -> 70, 4 x 1095 on
-//     3639 (D = 64) 53 -> 20, and with dq in a launch of its own 48/12 x 909 on 2844 (1068) 282 -> 152, 32/16 x 2598 on 5933
-//     (D = 64, 2976) 765 -> 481, 32 x 564 on 1365 (1376) 119 -> 108; beyond (D = 128) 8 x 4274 on 7495 (1880) 118 -> 121.
-int bwd_small_form(const KArgs& a, int D, bool causal, bool doc) {
-  if (D < 64) return SMALL_NONE;
+bool bwd_small(const KArgs& a, int D, bool doc) {
+  if (D < 64) return false;
   const int64_t kv = dkdv_blocks(a, D, doc);
   const int64_t dq = doc ? grid_blocks(launch_slots<GEO_DOC>(a), launch_groups<GEO_DOC>(a))
                          : geo_general(a) ? grid_blocks(launch_slots<GEO_GENERAL>(a), launch_groups<GEO_GENERAL>(a))
                                           : grid_blocks(launch_slots<GEO_PLAIN>(a), launch_groups<GEO_PLAIN>(a));
-  if (D <= 64 ? kv <= 2 * kCUs : a.G > 1 ? kv + dq / a.G <= 216 : kv <= 96) return SMALL_BOTH;
-  const bool cols = doc && causal && a.qpos == nullptr && a.gap >= kGcolMinGap;
-  return cols && kv <= (D > 64 ? 1408 : 3072) ? SMALL_DKDV : SMALL_NONE;
+  return D <= 64 ? kv <= 2 * kCUs : a.G > 1 ? kv + dq / a.G <= 216 : kv <= 96;
 }
 
 int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bool both, hipStream_t s) {

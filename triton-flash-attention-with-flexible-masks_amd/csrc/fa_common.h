@@ -598,9 +598,8 @@ int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t 
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 bool bwd_f32_in_one(const KArgs& a);
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
-// dk/dv of problems that leave CUs idle (fa_bwd_small.hip): not of these sizes, next to dq in one launch, by itself
-enum { SMALL_NONE, SMALL_BOTH, SMALL_DKDV };
-int bwd_small_form(const KArgs& a, int D, bool causal, bool doc);
+// problems that leave CUs idle (fa_bwd_small.hip): whether dk/dv takes its form there, and with dq in one launch or by itself
+bool bwd_small(const KArgs& a, int D, bool doc);
 int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bool both, hipStream_t s);
 int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s);
 int launch_mask_dump(const KArgs& a, bool causal, bool doc, uint8_t* out, hipStream_t s);
