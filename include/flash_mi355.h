@@ -99,7 +99,8 @@ extern "C" {
                                Set it in every call that shares the workspace, or in none. */
 #define FA_FLAG_DEBUG_NO_PAIR_WAIT 0x100
                             /* Diagnostic, for tests of the failure path below; never set it in production.
-                               In fa_bwd_dkdv at D = 128 two waves share each block of 32 keys: one publishes P in
+                               In fa_bwd_dkdv at D = 128 (but for long streams of rows without ids, which are
+                               pipelined) two waves share each block of 32 keys: one publishes P in
                                on-chip memory, the other polls a sequence number for it.  The poll is bounded (about
                                a millisecond) so that every wave ends whatever happens; a wave whose wait expired
                                has used a P it cannot trust and REPORTS it by writing NaN into its 32 rows of dk
