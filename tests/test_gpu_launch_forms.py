@@ -422,6 +422,30 @@ def test_backward_in_one_launch(case):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
 
 
+# dk/dv at D = 64 with two waves to a block of keys, each for half of every tile of rows: tiles of rows and keys that are partly filled (a half without
+# rows, a wave without keys), a window, a prefix, a block mask, heads of a group; in a launch of its own (the last three) and next to dq's.
+# B, H, Hk, M, N, dtype, causal, kind
+ROWS_CASES = [
+    (4, 32, 8, 530, 530, torch.bfloat16, True, "plain"), (3, 32, 8, 545, 1000, torch.float16, True, "plain"), (5, 8, 8, 1025, 1666, torch.bfloat16, False, "plain"),
+    (4, 16, 4, 777, 900, torch.bfloat16, True, "window"), (4, 32, 8, 600, 600, torch.float16, True, "prefix"), (4, 32, 8, 700, 700, torch.bfloat16, True, "block"),
+    (2, 128, 8, 1100, 1090, torch.float16, False, "plain"), (1, 256, 16, 700, 1700, torch.bfloat16, True, "block"), (1, 512, 16, 161, 2100, torch.float16, True, "plain"),
+]
+
+
+@pytest.mark.parametrize("case", ROWS_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-%s-c%d-%s" % (*c[:5], str(c[5])[6:], *c[6:]))
+def test_dkdv_rows_split_over_two_waves(case):
+    B, H, Hk, M, N, dtype, causal, kind = case
+    if kind == "block":
+        from tests.test_gpu_parity import test_block_mask_parity
+        test_block_mask_parity((B, H, Hk, M, N, 64, dtype, causal, 0, 0.6, False))
+        return
+    from tests.test_gpu_parity import _run_case
+    # dk and dv add up the results of G heads, each rounded as one head's are: sqrt(G) of the bound for one
+    g = math.sqrt(H // Hk)
+    _run_case(B, H, Hk, M, N, 64, dtype, causal, False, seed=4, window=500 if kind == "window" else 0, prefix=270 if kind == "prefix" else 0,
+              ceilings={"dk": g, "dv": g})
+
+
 # dk/dv by workgroups of 32 keys whose waves share the rows: blocks of rows and keys that are partly filled, heads of a group, one key, more
 # keys than rows, waves without a block.  Then documents with keys of no local row, in runs of one, two, four and eight key tiles to a
 # workgroup next to the column form.  B, H, Hk, M, N, D, dtype, causal, kind

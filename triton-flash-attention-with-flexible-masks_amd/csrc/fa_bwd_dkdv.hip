@@ -76,12 +76,15 @@ namespace fa {
 //                of this form whose keys lie there leave at once.  One launch, so the column form's memory
 //                traffic overlaps the set-up latencies of this one.
 // bid: index of the workgroup.
-template <typename Tag, int D, bool CAUSAL, bool DOC, bool SPLIT, int NKB, bool COLS>
+// ROWS = true  : (D = 64) two waves to each block of 32 keys, 64 keys to a workgroup of four; one takes the first 32 rows of every
+//                query tile, the other the last, and their sums are added up at the end.
+template <typename Tag, int D, bool CAUSAL, bool DOC, bool SPLIT, int NKB, bool COLS, bool ROWS>
 FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   using E = Elem<Tag>;
   using T = typename E::scalar;
   using vec8 = typename E::vec8;
-  constexpr int BK = 32 * NKB, BQ = 64, KS = D / 16;
+  static_assert(!ROWS || (!SPLIT && !COLS && NKB == 4), "four waves of both roles");
+  constexpr int BK = ROWS ? 64 : 32 * NKB, BQ = 64, KS = D / 16;
   constexpr int DL = D < 32 ? 32 : D;  // LDS row width: D = 16 is staged as 32 columns, the upper 16 zero
   constexpr int DBN = DL / 32;
   constexpr int TILE_BYTES = BQ * DL * 2;
@@ -105,7 +108,8 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   // useful one (8192 of them: 50 us), a skipped tile of a run costs a comparison.
   const bool packed = !DOC && a.ktab != nullptr;   // packed sequences: the slots are the plan's key tiles, longest first
   const int run = COLS ? cols_run(a, nKt) : 1;
-  const int nSlots = COLS ? (nKt + run - 1) / run : (packed ? a.nKent : nKt);
+  constexpr int SUB = ROWS ? 2 : 1;   // workgroups to an entry of the packed plan
+  const int nSlots = COLS ? (nKt + run - 1) / run : (packed ? a.nKent * SUB : nKt);
   if constexpr (COLS) {
     static_assert(DOC && (SPLIT ? 128 * NKB : 64 * NKB) == 256, "the column form runs with ids, 4 waves per workgroup");
     // the column form's workgroups come first: few, long, one round of them
@@ -116,7 +120,7 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   }
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar
-  const int role = SPLIT ? wave / NKB : 0, kb = wave % NKB;
+  const int role = SPLIT ? wave / NKB : 0, kb = ROWS ? wave & 1 : wave % NKB, half = ROWS ? wave >> 1 : 0;
   const int lq = lane & 31, g = lane >> 5;
   FA_STAMP(g_trace_dkdv, 0, FA_CLOCK()); FA_STAMP(g_trace_dkdv, 5, 0); FA_STAMP(g_trace_dkdv, 7, -1);
   FA_TRACE_ONLY(int tr_tiles = 0; bool tr_first = false; long long tr_wait = 0;)
@@ -128,11 +132,12 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   int M = a.M, N = a.N, gap = a.gap;   // of the batch entry, or of the sequence
   int64_t q0 = 0, k0 = 0;
   if (packed) {
-    if (kt0 >= a.shdr->nk) return;
-    const SeqTile* __restrict__ e = a.ktab + kt0;
+    if (kt0 / SUB >= a.shdr->nk) return;
+    const SeqTile* __restrict__ e = a.ktab + kt0 / SUB;
     M = __builtin_amdgcn_readfirstlane(e->M); N = __builtin_amdgcn_readfirstlane(e->N); gap = __builtin_amdgcn_readfirstlane(e->gap);
     q0 = __builtin_amdgcn_readfirstlane(e->q0); k0 = __builtin_amdgcn_readfirstlane(e->k0);
-    kt0 = __builtin_amdgcn_readfirstlane(e->tile);
+    kt0 = __builtin_amdgcn_readfirstlane(e->tile) * SUB + kt0 % SUB;
+    if (ROWS && kt0 * BK >= N) return;
   }
   const int ncols = COLS ? gcol_info(a, b, hk).ncols : 0;   // leading keys that belong to the column form of this launch
   bool ran = false;
@@ -208,6 +213,12 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   Loader ldQ, ldO;
   LdsOffsets<DL> lo;
   lo.init();
+  if (ROWS) {   // this wave's half of every query tile
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) lo.row[ks] += half * (32 * DL * 2);
+#pragma unroll
+    for (int db = 0; db < DBN; ++db) { lo.tr[db][0] += half * (32 * DL * 2); lo.tr[db][1] += half * (32 * DL * 2); }
+  }
   // gathered loads: byte offset of the lane's chunk inside its row, and the tile rows it fetches
   int g_coff[Loader::PER], g_rit[Loader::PER];
 #pragma unroll
@@ -493,11 +504,11 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   auto compute_both = [&](const int BUF, const int cur, const int flags, const int tile_id) __attribute__((always_inline)) {
     const char* lqt = smem + BUF * TILE_BYTES;
     const char* ldo = smem + (2 + BUF) * TILE_BYTES;
-    const char* aux = smem + AUX_OFF + BUF * AUX_BYTES;
-    const int m0 = cur * BQ;  // natural order only
+    const char* aux = smem + AUX_OFF + BUF * AUX_BYTES + half * 128;
+    const int m0 = cur * BQ + half * 32;  // natural order only
     if (flags & TF_SKIP) return;
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < (ROWS ? 1 : 2); ++qb) {
       f32x16 x = zero, dp;
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {   // (delta - dP: see negate_v)
@@ -717,6 +728,24 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
     T* dvp = reinterpret_cast<T*>(la.dv) + b * la.dv_bs + hk * la.dv_hs + k0 * la.dv_rs;
     T* dkp = reinterpret_cast<T*>(la.dk) + b * la.dk_bs + hk * la.dk_hs + k0 * la.dk_rs;
     __syncthreads();
+    if (ROWS) {
+      float* sums = reinterpret_cast<float*>(smem) + kb * (2 * DBN * 16 * 64) + lane;
+      if (half == 1) {
+#pragma unroll
+        for (int db = 0; db < DBN; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) { sums[(db * 16 + r) * 64] = acc[db][r]; sums[((DBN + db) * 16 + r) * 64] = acc2[db][r]; }
+      }
+      __syncthreads();
+      if (half == 0) {
+#pragma unroll
+        for (int db = 0; db < DBN; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) { acc[db][r] += sums[(db * 16 + r) * 64]; acc2[db][r] += sums[((DBN + db) * 16 + r) * 64]; }
+      }
+      __syncthreads();   // the sums have been read
+      if (half == 1) return;
+    }
     char* patch = smem + wave * row_patch_bytes<D>();
     auto store = [&](T* base, const int64_t rs, const f32x16 (&v)[DBN], const float sc) __attribute__((always_inline)) {
       store_rows_through_lds<E, D, DBN>(patch, v, sc, [&](const int r) -> T* {
@@ -741,23 +770,23 @@ FA_DEV void dkdv_body(const KArgs& a, int bid, char* smem) {
   FA_STAMP(g_trace_dkdv, 5, FA_CLOCK());
 }
 
-template <typename Tag, int D, bool CAUSAL, bool DOC, bool SPLIT, int NKB, bool COLS>
+template <typename Tag, int D, bool CAUSAL, bool DOC, bool SPLIT, int NKB, bool COLS, bool ROWS>
 __global__ __launch_bounds__(SPLIT ? 128 * NKB : 64 * NKB)
 __attribute__((amdgpu_waves_per_eu((D <= 32 && !COLS) ? 3 : 2, (D <= 32 && !COLS) ? 3 : 2)))
 void bwd_dkdv_kernel(const KArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  dkdv_body<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS>(a, (int)blockIdx.x, smem);
+  dkdv_body<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS, ROWS>(a, (int)blockIdx.x, smem);
 }
 
 // dk/dv and dq in one launch, for problems of so few workgroups that either leaves CUs idle: they run side by side instead
 // of one after the other.  Both read delta, which a launch before this one has formed (FA_FLAG_DQ_DELTA's way would
 // make dk/dv wait for dq).  dk/dv always in workgroups of 256 threads (64 keys at D = 128), two to a CU, as dq's are.
-template <typename Tag, int D, bool CAUSAL, int MODE>
+template <typename Tag, int D, bool CAUSAL, int MODE, bool ROWS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_both_kernel(const KArgs a, const int n_dkdv) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int bid = (int)blockIdx.x;
-  if (bid < n_dkdv) dkdv_body<Tag, D, CAUSAL, MODE == GEO_DOC, (D > 64), (D > 64 ? 2 : 4), false>(a, bid, smem);   // the longer ones first
+  if (bid < n_dkdv) dkdv_body<Tag, D, CAUSAL, MODE == GEO_DOC, (D > 64), (D > 64 ? 2 : 4), false, ROWS>(a, bid, smem);   // the longer ones first
   else dq_body<Tag, D, CAUSAL, MODE>(a, bid - n_dkdv, smem);
 }
 
@@ -770,17 +799,33 @@ static int dkdv_tiles(const KArgs& a, bool causal) {
 }
 template <int D, int NKB>
 constexpr size_t dkdv_lds() { return 4 * 64 * (D < 32 ? 32 : D) * 2 + 2 * 1024 + (D > 64 ? 2 * NKB * 2048 + 64 : 0); }
-template <typename Tag, int D, bool CAUSAL, bool DOC, int NKB, bool COLS = false>
+// Which launches of D = 64 without ids take two waves to a block of 32 keys (ROWS): those that wait for the chain of a key tile, its
+// query tiles over all heads of the group, on CUs that the others leave early.  dq, delta and dk/dv, us, before -> after (in
+// brackets: workgroups of 128 keys, query tiles to one): 24/12 heads x 1417 (144, 22) 73 -> 52; 32/16 x 1359 (176, 22) 71 -> 53; 32/8 x 5324, prefix
+// (336, 168) 563 -> 496; 32/16 x 2478 (320, 39) 138 -> 126; block masks 16/8 x 3801 (240, 60) 57 -> 48, 64/16 x 4976 (624, 156) 498 -> 403, 64/32 x 3689
+// (928, 58) 226 -> 191, 12 x 9326 (876, 73) 291 -> 279; packed 32/8 x 7 sequences of up to 1051 (304, 18) 96 -> 72, 16/8 x 4 of up to 1029
+// (176, 9) 57 -> 44.  Beyond the lines every tile is loaded for half the keys, and workgroups double: 64/32 x 466 (256, 8) 37 -> 43, 64 x 454
+// (256, 4) 26 -> 34, a window of 67 keys (160, 4) 16 -> 19, of 179 under 128/32 heads (416, 5 to a head) 84 -> 89, 32/8 x 35 packed of up to 754 (1160, 13) 170 -> 206.  With ids the tiles are not known here.
+static bool rows_form(const KArgs& a, int D, bool causal, bool doc) {
+  if (D != 64 || doc) return false;
+  const bool packed = a.ktab != nullptr;
+  const int64_t wgs = int64_t(packed ? a.nKent : (a.N + 127) / 128) * a.B * a.Hk;
+  if (wgs > (a.bmask != nullptr ? 4 : 2) * kCUs) return false;
+  if (!packed) return dkdv_tiles(a, causal) >= std::max(16, 8 * a.G);
+  const int rows = a.M / std::max(1, a.nKent - 1 - a.N / 128);   // of an average sequence (the table has an entry per 128 keys and one per sequence)
+  return (rows / 64 + 1) * a.G >= (causal ? 16 : 8);
+}
+template <typename Tag, int D, bool CAUSAL, bool DOC, int NKB, bool COLS = false, bool ROWS = false>
 static int launch_nkb(const KArgs& a, hipStream_t s) {
   constexpr bool SPLIT = D > 64;
-  constexpr int BK = 32 * NKB;
+  constexpr int BK = ROWS ? 64 : 32 * NKB;
   const int nKt = (a.N + BK - 1) / BK;
   size_t lds = dkdv_lds<D, NKB>();
   if (COLS && dkdv_cols_lds(D) > lds) lds = dkdv_cols_lds(D);
-  auto kern = bwd_dkdv_kernel<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS>;
+  auto kern = bwd_dkdv_kernel<Tag, D, CAUSAL, DOC, SPLIT, NKB, COLS, ROWS>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  const int slots = !DOC && a.ktab != nullptr ? a.nKent : nKt;
+  const int slots = !DOC && a.ktab != nullptr ? a.nKent * (ROWS ? 2 : 1) : nKt;
   const int blocks = COLS ? grid_blocks((nKt + cols_run(a, nKt) - 1) / cols_run(a, nKt), a.B * a.Hk) + dkdv_cols_blocks(a) : grid_blocks(slots, a.B * a.Hk);
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(SPLIT ? 128 * NKB : 64 * NKB), lds, s, a);
   return (int)hipGetLastError();
@@ -808,6 +853,8 @@ static int launch_one(const KArgs& a, hipStream_t s) {
     if (a.ktab != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, kSeqKeyTile / 32>(a, s);
     return dkdv_tiles(a, CAUSAL) < kKvShortTiles ? launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s) : launch_dkdv_pipe(a, __is_same(Tag, bf16_t) ? FA_DTYPE_BF16 : FA_DTYPE_FP16, CAUSAL, s);
   } else {
+    if constexpr (D == 64 && !DOC)
+      if (rows_form(a, D, CAUSAL, DOC)) return launch_nkb<Tag, D, CAUSAL, DOC, 4, false, true>(a, s);
     return launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
   }
 }
@@ -829,23 +876,24 @@ static int launch_d(const KArgs& a, int D, bool causal, bool doc, hipStream_t s)
   }
 }
 
-template <typename Tag, int D, bool CAUSAL, int MODE>
+template <typename Tag, int D, bool CAUSAL, int MODE, bool ROWS>
 static int launch_both(const KArgs& a, hipStream_t s) {
-  constexpr int NKB = D > 64 ? 2 : 4;
+  constexpr int NKB = D > 64 ? 2 : 4, BK = ROWS ? 64 : 32 * NKB;
   constexpr size_t lds = dkdv_lds<D, NKB>() > dq_lds<D>() ? dkdv_lds<D, NKB>() : dq_lds<D>();
-  auto kern = bwd_both_kernel<Tag, D, CAUSAL, MODE>;
+  auto kern = bwd_both_kernel<Tag, D, CAUSAL, MODE, ROWS>;
   static bool lds_allowed[64] = {};   // per kernel instantiation and device
   if (int e = allow_lds(kern, lds, lds_allowed)) return e;
-  const int slots = MODE != GEO_DOC && a.ktab != nullptr ? a.nKent : (a.N + 32 * NKB - 1) / (32 * NKB);
+  const int slots = MODE != GEO_DOC && a.ktab != nullptr ? a.nKent * (ROWS ? 2 : 1) : (a.N + BK - 1) / BK;
   const int n_dkdv = grid_blocks(slots, a.B * a.Hk), n_dq = grid_blocks(launch_slots<MODE>(a), launch_groups<MODE>(a));
   hipLaunchKernelGGL(kern, dim3(n_dkdv + n_dq), dim3(256), lds, s, a, n_dkdv);
   return (int)hipGetLastError();
 }
-template <typename Tag, int D>
+template <typename Tag, int D, bool ROWS>
 static int launch_both_cd(const KArgs& a, bool causal, bool doc, hipStream_t s) {
-  if (doc) return causal ? launch_both<Tag, D, true, GEO_DOC>(a, s) : launch_both<Tag, D, false, GEO_DOC>(a, s);
-  if (geo_general(a)) return causal ? launch_both<Tag, D, true, GEO_GENERAL>(a, s) : launch_both<Tag, D, false, GEO_GENERAL>(a, s);
-  return causal ? launch_both<Tag, D, true, GEO_PLAIN>(a, s) : launch_both<Tag, D, false, GEO_PLAIN>(a, s);
+  if constexpr (!ROWS)
+    if (doc) return causal ? launch_both<Tag, D, true, GEO_DOC, ROWS>(a, s) : launch_both<Tag, D, false, GEO_DOC, ROWS>(a, s);
+  if (geo_general(a)) return causal ? launch_both<Tag, D, true, GEO_GENERAL, ROWS>(a, s) : launch_both<Tag, D, false, GEO_GENERAL, ROWS>(a, s);
+  return causal ? launch_both<Tag, D, true, GEO_PLAIN, ROWS>(a, s) : launch_both<Tag, D, false, GEO_PLAIN, ROWS>(a, s);
 }
 
 // Whether a backward of these sizes (that fa_bwd_small.hip has not taken) takes the shared launch: with at most eight workgroups to a CU in all (two run at a time),
@@ -877,8 +925,10 @@ bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
   return true;
 }
 int launch_bwd_both(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s) {
-  if (D == 128) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 128>(a, causal, doc, s) : launch_both_cd<fp16_t, 128>(a, causal, doc, s);
-  if (D == 64) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 64>(a, causal, doc, s) : launch_both_cd<fp16_t, 64>(a, causal, doc, s);
+  if (D == 128) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 128, false>(a, causal, doc, s) : launch_both_cd<fp16_t, 128, false>(a, causal, doc, s);
+  if (rows_form(a, D, causal, doc))
+    return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 64, true>(a, causal, doc, s) : launch_both_cd<fp16_t, 64, true>(a, causal, doc, s);
+  if (D == 64) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 64, false>(a, causal, doc, s) : launch_both_cd<fp16_t, 64, false>(a, causal, doc, s);
   return -1;
 }
 
