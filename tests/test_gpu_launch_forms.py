@@ -544,3 +544,37 @@ def test_pipelined_dkdv(case):
     tol = TOL_ABS * math.sqrt(H // Hk)
     check_close("dk", dk, rdk, tol)
     check_close("dv", dv, rdv, tol)
+
+
+# D, heads, queries, keys, mask; keys that no row sees and rows that see no key, in each form of the backward: the polled pair and D <= 64 (dk/dv next to dq
+# and by itself), the pipeline, the small form, rows with ids
+UNSEEN_CASES = [(128, 8, 2100, 2100, "block"), (64, 8, 2100, 2100, "block"), (32, 8, 700, 700, "block"), (128, 1, 300, 300, "block"), (64, 1, 300, 300, "block"),
+                (128, 8, 2100, 4400, "window"), (128, 16, 3000, 3000, "qpos"), (64, 16, 3000, 3000, "qpos")]
+
+
+@pytest.mark.parametrize("case", UNSEEN_CASES, ids=lambda c: "D%d-H%d-M%d-N%d-%s" % c)
+def test_a_gradient_of_nothing_is_plus_zero(case):
+    from flash_mi355 import attention, attention_with_lse, SCORE_FUNC_MODE1_DOC
+    D, H, M, N, kind = case
+    print("case", case, flush=True)
+    q, k, v, do = (t.cuda().requires_grad_(True) for t in _tensors(1, H, H, M, N, D, torch.bfloat16, 3))
+    args, kw = (), {}
+    if kind == "block":   # the first block of keys only
+        block = torch.zeros(1, 1, -(-M // 64), -(-N // 64), dtype=torch.bool, device="cuda")
+        block[..., 0] = True
+        kw = {"block_mask": block}
+        unseen_q, unseen_k = slice(0, 0), slice(64, None)
+    elif kind == "window":
+        kw = {"window": 2000}
+        unseen_q, unseen_k = slice(0, 0), slice(0, N - M - 1999)
+    else:                 # the second half of the rows lies before every key
+        ids = torch.full((1, 1, M), -1, dtype=torch.int32, device="cuda").expand(1, H, M)
+        pos = torch.full((1, M), -1, dtype=torch.int32, device="cuda")
+        pos[:, :M // 2] = 5
+        args, kw = (None, ids, ids, SCORE_FUNC_MODE1_DOC), {"qpos": pos}
+        unseen_q, unseen_k = slice(M // 2, None), slice(6, None)
+    for f in (attention, attention_with_lse):   # (a gradient of the LSE takes the backward's launches one by one)
+        out = f(q, k, v, True, *args, **kw)
+        dq, dk, dv = torch.autograd.grad(out, (q, k, v), do if f is attention else (do, torch.zeros(1, H, M, device="cuda")))
+        for name, t in (("dq", dq[:, :, unseen_q]), ("dk", dk[:, :, unseen_k]), ("dv", dv[:, :, unseen_k])):
+            assert (t == 0).all() and not torch.signbit(t).any(), name

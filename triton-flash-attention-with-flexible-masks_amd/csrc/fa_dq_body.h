@@ -295,8 +295,8 @@ FA_DEV void dq_body(const KArgs& a, const int bid, char* smem) {
     };
     auto finish_row = [&](int prow, int c, f32x4 acc) __attribute__((always_inline)) {
       const int mrow = DOC ? prow : prow / la.pack, mh = DOC ? 0 : prow - mrow * la.pack;
-      const typename E::vec2 x0 = E::cvt2(acc[0] * out_scale, acc[1] * out_scale);
-      const typename E::vec2 x1 = E::cvt2(acc[2] * out_scale, acc[3] * out_scale);
+      const typename E::vec2 x0 = E::cvt2(scaled(acc[0], out_scale), scaled(acc[1], out_scale));
+      const typename E::vec2 x1 = E::cvt2(scaled(acc[2], out_scale), scaled(acc[3], out_scale));
       typename E::vec4 x = {x0[0], x0[1], x1[0], x1[1]};
       *reinterpret_cast<typename E::vec4*>(dqp + mh * la.dq_hs + int64_t(mrow) * la.dq_rs + 4 * c) = x;
     };

@@ -666,6 +666,10 @@ FA_DEV float row_delta(const vec8 (&o)[KS], const vec8 (&d)[KS]) {
   return xhalf_sum(part[0]);
 }
 
+// x * sc with a sum of nothing, +0, staying +0 under a negative sc as well (sums whose sign is turned leave with the scale
+// negated; a product alone made every gradient of an unseen key or row -0).
+FA_DEV float scaled(float x, float sc) { return __builtin_fmaf(x, sc, 0.f); }
+
 // A wave's 32 result rows on their way out.  The accumulators hold a row (or key) per lane and 4 consecutive
 // columns per register quad: stored from there, a wave instruction writes 64 pieces of 8 bytes, a row apart, and
 // every 128-byte line of the result fills up over sixteen instructions -- measured at 5-13 % of the id
@@ -686,8 +690,8 @@ FA_DEV void store_rows_through_lds(char* patch, const f32x16 (&v)[DBN], const fl
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
       if (32 * db + 8 * q4 >= D) continue;  // padded columns of the D = 16 layout
-      const typename E::vec2 x0 = E::cvt2(v[db][4 * q4 + 0] * sc, v[db][4 * q4 + 1] * sc);
-      const typename E::vec2 x1 = E::cvt2(v[db][4 * q4 + 2] * sc, v[db][4 * q4 + 3] * sc);
+      const typename E::vec2 x0 = E::cvt2(scaled(v[db][4 * q4 + 0], sc), scaled(v[db][4 * q4 + 1], sc));
+      const typename E::vec2 x1 = E::cvt2(scaled(v[db][4 * q4 + 2], sc), scaled(v[db][4 * q4 + 3], sc));
       typename E::vec4 x = {x0[0], x0[1], x1[0], x1[1]};
       *reinterpret_cast<typename E::vec4*>(patch + lq * PITCH + (32 * db + 8 * q4 + 4 * g) * 2) = x;
     }
