@@ -293,11 +293,12 @@ FA_DEV float xhalf_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Elements e, e + 1 of packed fp16 values times fp32 ones, as two instructions that convert on the way.
+// Elements e, e + 1 of packed fp16 values times fp32 ones: a multiply-add with zero is one instruction that converts on the way
+// (v_fma_mix_f32; a product alone is two).  Left to the compiler, since the fp32 operands are accumulators of a matrix product: it
+// waits until that product can be read, which it does not do for inline assembly.
 FA_DEV void mul_f16_f32(f16x8 p, const int e, float x0, float x1, float& y0, float& y1) {
-  const f16x2 pp = {p[e], p[e + 1]};
-  asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(y0) : "v"(pp), "v"(x0));
-  asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y1) : "v"(pp), "v"(x1));
+  y0 = __builtin_fmaf(float(p[e]), x0, 0.f);
+  y1 = __builtin_fmaf(float(p[e + 1]), x1, 0.f);
 }
 
 // Eight products of 16-bit elements, added up in order.  Not to be contracted: for fp16 the compiler makes two-element dot
