@@ -289,6 +289,7 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
     }
     int nx2 = -1, ek2 = 0, gi2 = 0, idx2 = 0;
     if (nxt >= 0) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads of the block before are done: its buffer is filled again
       load(nxt, gi_n, idx_n, mine + (buf ^ 1) * stage_bytes<D>());
       nx2 = it.next(a.G, wave, head, chunk); ek2 = it.ek; gi2 = it.gi;
       if (DOC && nx2 >= 0) idx2 = place(nx2, gi2);
