@@ -249,6 +249,18 @@ int fa_bwd_dq(const fa_params* p, void* stream);
    when neither fills the chip).  FA_FLAG_DQ_DELTA is implied. */
 int fa_bwd(const fa_params* p, void* stream);
 
+/* Which kernel forms dk and dv of these parameters: in fa_bwd (whole != 0) or in fa_bwd_dkdv (whole == 0).  One of
+   FA_FORM_*, with FA_FORM_WITH_DQ where dq's workgroups are in the same launch, or the (negative) code of fa_validate.
+   A diagnostic: the sizes at which one form follows the other are no part of the interface.  Touches no GPU API. */
+#define FA_FORM_KEYS  1       /* every wave, or pair of waves, owns 32 keys and walks all rows */
+#define FA_FORM_COLS  2       /* the same next to the column form, which takes the leading keys that global rows alone see */
+#define FA_FORM_ROWS  3       /* D = 64: two waves own the same 32 keys, each half of every tile of rows */
+#define FA_FORM_PIPE  4       /* D = 128, long streams without ids: score and gradient waves one tile apart */
+#define FA_FORM_SMALL 5       /* the four waves of a workgroup own the same 32 keys and share the rows */
+#define FA_FORM_FP32  6
+#define FA_FORM_WITH_DQ 0x100
+int fa_bwd_form(const fa_params* p, int whole);
+
 /* Number of wave-level pair waits of fa_bwd_dkdv that expired on the current device since the library
    was loaded (see FA_FLAG_DEBUG_NO_PAIR_WAIT: each one also shows as NaN in 32 rows of dk).  0 in any
    healthy run.  Waits for the device to be idle before it reads the count (a diagnostic, not for hot

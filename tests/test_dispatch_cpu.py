@@ -1,0 +1,30 @@
+"""Which kernel takes dk and dv, by sizes: the tests that run on the GPU name the form that they are written for, and this file
+holds them to it, so that a rule that moves does not leave them green on another kernel."""
+import ctypes
+
+import pytest
+import torch
+
+from flash_mi355 import _cabi
+from tests._forms import dkdv_form
+
+bf16, fp16, f32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def test_invalid_parameters_have_no_form():
+    assert _cabi.lib().fa_bwd_form(None, 1) == -1
+    p = _cabi.FaParams()
+    assert _cabi.lib().fa_bwd_form(ctypes.byref(p), 1) == -2 and _cabi.lib().fa_bwd_form(ctypes.byref(p), 0) == -2
+
+
+@pytest.mark.parametrize("args,kw,form", [
+    ((1, 2, 2, 300, 300, 32, bf16, True), {}, ("keys", False)), ((1, 1, 1, 300, 300, 64, bf16, True), {}, ("small", True)),
+    ((1, 32, 32, 16384, 16384, 128, bf16, True), {}, ("pipe", False)), ((1, 32, 32, 16384, 16384, 128, bf16, True), {"window": 1024}, ("keys", False)),
+    ((1, 32, 32, 16384, 16384, 128, bf16, True), {"kind": "doc"}, ("keys", False)), ((8, 8, 8, 1024, 8192, 128, fp16, True), {"kind": "doc"}, ("cols", False)),
+    ((1, 8, 8, 1088, 1088, 128, bf16, True), {"kind": "block"}, ("keys", True)), ((1, 8, 8, 1088, 1088, 128, bf16, True), {"whole": False}, ("keys", False)),
+    ((2, 32, 8, 1100, 1100, 64, bf16, True), {}, ("rows", True)), ((2, 4, 4, 512, 512, 64, f32, True), {"kind": "doc"}, ("fp32", True)),
+    # (the diagnostic flag of the pair wait keeps fa_bwd_dkdv off the form without pairs)
+    ((1, 8, 1, 520, 520, 128, bf16, True), {"whole": False}, ("small", False)), ((1, 8, 1, 520, 520, 128, bf16, True), {"whole": False, "no_pair_wait": True}, ("pipe", False)),
+])
+def test_forms(args, kw, form):
+    assert dkdv_form(*args, **kw) == form

@@ -307,6 +307,20 @@ extern "C" int fa_pair_wait_expired(uint64_t* count) {
   return FA_OK;
 }
 
+// FA_FORM_* of the backward, or of dk/dv by itself
+static int bwd_form(const fa_params* p, const KArgs& a, bool whole) {
+  const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
+  if (p->dtype == FA_DTYPE_FP32) return FA_FORM_FP32 | (whole && bwd_f32_in_one(a) ? FA_FORM_WITH_DQ : 0);
+  if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) == 0 && bwd_small(a, p->D, doc)) return FA_FORM_SMALL | (whole ? FA_FORM_WITH_DQ : 0);
+  const bool both = whole && bwd_in_one(a, p->D, causal, doc);
+  return dkdv_form(a, p->D, causal, doc, both) | (both ? FA_FORM_WITH_DQ : 0);
+}
+
+extern "C" int fa_bwd_form(const fa_params* p, int whole) {
+  const int rc = fa_validate(p, whole ? 1 : 3);
+  return rc != FA_OK ? rc : bwd_form(p, make_args(p, false), whole != 0);
+}
+
 extern "C" int fa_bwd_dkdv(const fa_params* p, void* stream) {
   int rc = fa_validate(p, 3);
   if (rc != FA_OK) return rc;
@@ -314,7 +328,7 @@ extern "C" int fa_bwd_dkdv(const fa_params* p, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (p->dtype == FA_DTYPE_FP32) return finish(launch_bwd_dkdv_f32(make_args(p, false), p->D, causal, doc, s));
   const KArgs a = make_args(p, false);
-  if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) == 0 && bwd_small(a, p->D, doc))   // (the bits of fa_bwd)
+  if (bwd_form(p, a, false) == FA_FORM_SMALL)   // (the bits of fa_bwd)
     return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, false, s));
   return finish(launch_bwd_dkdv(a, p->dtype, p->D, causal, doc, s));
 }
@@ -335,13 +349,15 @@ extern "C" int fa_bwd(const fa_params* p, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   KArgs a = make_args(p, false);
   a.dq_delta = 1;
+  const int form = bwd_form(p, a, true);
+  const bool one = (form & FA_FORM_WITH_DQ) != 0;
   if (p->dtype == FA_DTYPE_FP32) {
-    if (bwd_f32_in_one(a)) return finish(launch_bwd_f32(a, p->D, causal, doc, s));
+    if (one) return finish(launch_bwd_f32(a, p->D, causal, doc, s));
     if (int e = launch_bwd_dq_f32(a, p->D, causal, doc, s)) return finish(e);
     return finish(launch_bwd_dkdv_f32(a, p->D, causal, doc, s));
   }
-  if (bwd_small(a, p->D, doc)) return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, true, s));
-  if (bwd_in_one(a, p->D, causal, doc)) {
+  if (form == (FA_FORM_SMALL | FA_FORM_WITH_DQ)) return finish(launch_bwd_small(a, p->dtype, p->D, causal, doc, true, s));
+  if (one) {
     if (int e = launch_bwd_delta(a, p->dtype, p->D, s)) return finish(e);
     a.dq_delta = 0;
     return finish(launch_bwd_both(a, p->dtype, p->D, causal, doc, s));

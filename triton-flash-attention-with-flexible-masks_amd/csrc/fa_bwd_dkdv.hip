@@ -831,8 +831,8 @@ static int launch_nkb(const KArgs& a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-template <typename Tag, int D, bool CAUSAL, bool DOC>
-static int launch_one(const KArgs& a, hipStream_t s) {
+// Which form takes dk/dv, in the launch that it shares with dq (both) or in one of its own.
+int dkdv_form(const KArgs& a, int D, bool causal, bool doc, bool both) {
   // Role-split form (D = 128): a workgroup that visits few query tiles spends a sizeable part of its
   // life in set-up and drain, and two 64-key workgroups per CU cover each other's there; a long tile
   // stream is better served by the 128-key form, which reads every query tile half as often.  With
@@ -845,18 +845,22 @@ static int launch_one(const KArgs& a, hipStream_t s) {
   // mask at all: local rows may need none of the leading keys, and the column form takes those (it decides
   // on the device, from the mask plan, how many they are -- possibly none).  Square causal problems with the
   // same ids on both sides always have a local row on the first keys' diagonal: nothing to gain there.
-  if constexpr (DOC) {
-    if (a.gap >= kGcolMinGap || a.qpos != nullptr || !CAUSAL) return launch_nkb<Tag, D, CAUSAL, DOC, (D > 64 ? 2 : 4), true>(a, s);
-  }
-  if constexpr (D > 64) {
-    if (DOC || a.bmask != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s);
-    if (a.ktab != nullptr) return launch_nkb<Tag, D, CAUSAL, DOC, kSeqKeyTile / 32>(a, s);
-    return dkdv_tiles(a, CAUSAL) < kKvShortTiles ? launch_nkb<Tag, D, CAUSAL, DOC, 2>(a, s) : launch_dkdv_pipe(a, __is_same(Tag, bf16_t) ? FA_DTYPE_BF16 : FA_DTYPE_FP16, CAUSAL, s);
-  } else {
-    if constexpr (D == 64 && !DOC)
-      if (rows_form(a, D, CAUSAL, DOC)) return launch_nkb<Tag, D, CAUSAL, DOC, 4, false, true>(a, s);
-    return launch_nkb<Tag, D, CAUSAL, DOC, 4>(a, s);
-  }
+  if (doc && !both && (a.gap >= kGcolMinGap || a.qpos != nullptr || !causal)) return FA_FORM_COLS;
+  if (D > 64) return !doc && !both && a.bmask == nullptr && a.ktab == nullptr && dkdv_tiles(a, causal) >= kKvShortTiles ? FA_FORM_PIPE : FA_FORM_KEYS;
+  return rows_form(a, D, causal, doc) ? FA_FORM_ROWS : FA_FORM_KEYS;
+}
+template <typename Tag, int D, bool CAUSAL, bool DOC>
+static int launch_one(const KArgs& a, hipStream_t s) {
+  constexpr int NKB = D > 64 ? 2 : 4;
+  static_assert(D <= 64 || kSeqKeyTile == 32 * NKB, "the packed plan's key tiles");
+  const int form = dkdv_form(a, D, CAUSAL, DOC, false);
+  if constexpr (DOC)
+    if (form == FA_FORM_COLS) return launch_nkb<Tag, D, CAUSAL, DOC, NKB, true>(a, s);
+  if constexpr (D > 64 && !DOC)
+    if (form == FA_FORM_PIPE) return launch_dkdv_pipe(a, __is_same(Tag, bf16_t) ? FA_DTYPE_BF16 : FA_DTYPE_FP16, CAUSAL, s);
+  if constexpr (D == 64 && !DOC)
+    if (form == FA_FORM_ROWS) return launch_nkb<Tag, D, CAUSAL, DOC, NKB, false, true>(a, s);
+  return launch_nkb<Tag, D, CAUSAL, DOC, NKB>(a, s);
 }
 
 template <typename Tag, int D>
@@ -926,7 +930,7 @@ bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc) {
 }
 int launch_bwd_both(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s) {
   if (D == 128) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 128, false>(a, causal, doc, s) : launch_both_cd<fp16_t, 128, false>(a, causal, doc, s);
-  if (rows_form(a, D, causal, doc))
+  if (dkdv_form(a, D, causal, doc, true) == FA_FORM_ROWS)
     return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 64, true>(a, causal, doc, s) : launch_both_cd<fp16_t, 64, true>(a, causal, doc, s);
   if (D == 64) return dtype == FA_DTYPE_BF16 ? launch_both_cd<bf16_t, 64, false>(a, causal, doc, s) : launch_both_cd<fp16_t, 64, false>(a, causal, doc, s);
   return -1;

@@ -585,6 +585,7 @@ int launch_bwd_dq(const KArgs& a, int dtype, int D, bool causal, bool doc, hipSt
 int launch_bwd_dkdv(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);
 int launch_dkdv_pipe(const KArgs& a, int dtype, bool causal, hipStream_t s);   // long tile streams without ids at D = 128 (fa_dkdv_pipe.hip)
 bool bwd_in_one(const KArgs& a, int D, bool causal, bool doc);
+int dkdv_form(const KArgs& a, int D, bool causal, bool doc, bool both);   // FA_FORM_* of fa_bwd_dkdv.hip (the problems that fa_bwd_small.hip leaves), 16-bit elements
 int launch_bwd_both(const KArgs& a, int dtype, int D, bool causal, bool doc, hipStream_t s);   // dq and dk/dv, delta read by both
 int read_pair_wait_expired(unsigned long long* n);   // expired pair waits of the dk/dv kernel on the current device (synchronises)
 #ifdef FA_TRACE

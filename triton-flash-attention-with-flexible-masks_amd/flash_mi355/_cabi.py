@@ -25,12 +25,14 @@ FA_IDTYPE_I64 = 1
 FA_FLAG_DQ_DELTA = 1
 FA_FLAG_SPLIT_KEYS = 4
 FA_FLAG_DEBUG_NO_PAIR_WAIT = 0x100
+FA_FORM_KEYS, FA_FORM_COLS, FA_FORM_ROWS, FA_FORM_PIPE, FA_FORM_SMALL, FA_FORM_FP32 = range(1, 7)
+FA_FORM_WITH_DQ = 0x100
 FA_STATIC_WS_BYTES = 32 << 20
 
 # every symbol include/flash_mi355.h declares
 EXPORTS = (
     "fa_version", "fa_params_size", "fa_error_string", "fa_last_hip_error", "fa_validate",
-    "fa_workspace_bytes", "fa_workspace_plan_bytes", "fa_mask_plan", "fa_fwd", "fa_bwd_delta", "fa_bwd_dkdv", "fa_bwd_dq", "fa_bwd",
+    "fa_workspace_bytes", "fa_workspace_plan_bytes", "fa_mask_plan", "fa_fwd", "fa_bwd_delta", "fa_bwd_dkdv", "fa_bwd_dq", "fa_bwd", "fa_bwd_form",
     "fa_mask_dump", "fa_fwd_static", "fa_workspace_scratch_bytes", "fa_pair_wait_expired",
 )
 
@@ -78,6 +80,8 @@ def lib() -> ctypes.CDLL:
     L.fa_last_hip_error.restype = c_int
     L.fa_validate.restype = c_int
     L.fa_validate.argtypes = [POINTER(FaParams), c_int]
+    L.fa_bwd_form.restype = c_int
+    L.fa_bwd_form.argtypes = [POINTER(FaParams), c_int]
     L.fa_workspace_bytes.restype = c_uint64
     L.fa_workspace_bytes.argtypes = [POINTER(FaParams)]
     L.fa_workspace_plan_bytes.restype = c_uint64
