@@ -28,3 +28,12 @@ def test_invalid_parameters_have_no_form():
 ])
 def test_forms(args, kw, form):
     assert dkdv_form(*args, **kw) == form
+
+
+@pytest.mark.parametrize("args,kw", [
+    ((4, 8, 8, 115, 429, 64, bf16, False), {}), ((1, 64, 64, 205, 205, 64, fp16, True), {"kind": "doc"}), ((1, 16, 16, 186, 989, 64, bf16, True), {"kind": "block"}),
+    ((1, 2, 2, 5438, 5438, 64, fp16, True), {"window": 74}), ((2, 4, 4, 125, 1871, 64, bf16, True), {"prefix": 535}), ((1, 8, 8, 118, 1892, 64, bf16, True), {}),
+])
+def test_the_small_form_stops_where_its_workgroups_share_cus(args, kw):
+    """D = 64, one query head to a key head, 340 to 496 workgroups of 32 keys: 1.2 to 1.4 times the time of the form with 128 keys to a workgroup."""
+    assert dkdv_form(*args, **kw)[0] != "small"

@@ -384,21 +384,26 @@ int launch_cd(const KArgs& a, bool causal, bool doc, bool both, hipStream_t s) {
 
 }  // namespace
 
-// Which problems: by the workgroups of 32 keys that they have, against the other forms (dq + dk/dv + delta, us, old -> new):
-//   D = 64, in one launch up to two to a CU: 8 heads x 94 rows 11.7 -> 7.3, 2 x 504 19.1 -> 11.8, 16/4 heads x 2 packed sequences of
-//     up to 184 15.8 -> 7.8, 3 x 8/4 x 1417 (540) 73 -> 59, block mask 2 x 6819 (428) 49 -> 43; beyond 2 x 4885, block mask (612)
-//     84 -> 90, 3 x 8 x 853 (648) 31 -> 34
-//   D = 128 (one workgroup to a CU, for its LDS), in one launch up to 96: 8 x 91 12.3 -> 9.8, 8 x 338 with documents (88) 21 -> 19;
-//     beyond 31 packed sequences of up to 114 (118) 12.6 -> 17.6, 4 x 1416, packed (180) 41 -> 49; with grouped heads, whose chains
-//     are longer, up to 216 with dq's workgroups, those counted by the group: 8/2 x 3440, packed (146) 68 -> 56, 32/8 x 652 (216) 73 -> 58;
-//     beyond 16/8 x 2889 with a window (228) 36 -> 41, 32/8 x 2055, packed (352) 131 -> 145
+// Which problems: by the workgroups of 32 keys that they have (kv; packed sequences: as many as the plan's table holds).  The
+// whole backward in this form : in the next best one, geometric mean over random problems with all masks [smallest, largest]:
+//   D = 64, two workgroups to a CU    kv up to 128            to 192            to 256            to 320            to 384
+//     one query head to a key head    0.79 [0.68, 1.03]  0.88 [0.71, 1.07]  0.94 [0.59, 1.09]  1.04 [0.86, 1.33]  1.16 [0.90, 1.71]
+//     several                         0.74 [0.48, 0.96]  0.82 [0.49, 1.02]  0.86 [0.67, 1.13]  0.95 [0.53, 1.31]  1.01 [0.77, 1.47]
+//     packed sequences                0.75 [0.57, 0.98]  0.81 [0.55, 0.96]  0.84 [0.63, 1.00]  0.81 [0.65, 0.97]  0.90 [0.83, 1.08]
+//     With more, the workgroups share CUs and the longer chains of the other forms cost less than the rows that are read again
+//     (the line at two to a CU for all of them lost up to 1.4).
+//   D = 128, one workgroup to a CU, for its LDS.  One query head to a key head: kv to 64 0.91 [0.62, 1.09], to 96 0.95 [0.77, 1.06], to 128
+//     0.96 [0.60, 1.33], to 160 1.10 [0.78, 1.57].  Several, whose chains are longer, and then dq's workgroups of a group count as one:
+//     sum to 128 0.80 [0.49, 1.05], to 216 0.81 [0.55, 1.20], to 256 0.84 [0.70, 1.03], to 300 0.98 [0.65, 1.46].
 bool bwd_small(const KArgs& a, int D, bool doc) {
   if (D < 64) return false;
   const int64_t kv = dkdv_blocks(a, D, doc);
+  if (D <= 64) return kv <= (a.G > 1 || (!doc && a.ktab != nullptr) ? kCUs * 3 / 2 : kCUs);
+  if (a.G == 1) return kv <= 96;
   const int64_t dq = doc ? grid_blocks(launch_slots<GEO_DOC>(a), launch_groups<GEO_DOC>(a))
                          : geo_general(a) ? grid_blocks(launch_slots<GEO_GENERAL>(a), launch_groups<GEO_GENERAL>(a))
                                           : grid_blocks(launch_slots<GEO_PLAIN>(a), launch_groups<GEO_PLAIN>(a));
-  return D <= 64 ? kv <= 2 * kCUs : a.G > 1 ? kv + dq / a.G <= 216 : kv <= 96;
+  return kv + dq / a.G <= 216;
 }
 
 int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bool both, hipStream_t s) {
