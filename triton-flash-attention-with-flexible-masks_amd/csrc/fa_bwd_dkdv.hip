@@ -800,18 +800,31 @@ static int dkdv_tiles(const KArgs& a, bool causal) {
 template <int D, int NKB>
 constexpr size_t dkdv_lds() { return 4 * 64 * (D < 32 ? 32 : D) * 2 + 2 * 1024 + (D > 64 ? 2 * NKB * 2048 + 64 : 0); }
 // Which launches of D = 64 without ids take two waves to a block of 32 keys (ROWS): those that wait for the chain of a key tile, its
-// query tiles over all heads of the group, on CUs that the others leave early.  dq, delta and dk/dv, us, before -> after (in
-// brackets: workgroups of 128 keys, query tiles to one): 24/12 heads x 1417 (144, 22) 73 -> 52; 32/16 x 1359 (176, 22) 71 -> 53; 32/8 x 5324, prefix
-// (336, 168) 563 -> 496; 32/16 x 2478 (320, 39) 138 -> 126; block masks 16/8 x 3801 (240, 60) 57 -> 48, 64/16 x 4976 (624, 156) 498 -> 403, 64/32 x 3689
-// (928, 58) 226 -> 191, 12 x 9326 (876, 73) 291 -> 279; packed 32/8 x 7 sequences of up to 1051 (304, 18) 96 -> 72, 16/8 x 4 of up to 1029
-// (176, 9) 57 -> 44.  Beyond the lines every tile is loaded for half the keys, and workgroups double: 64/32 x 466 (256, 8) 37 -> 43, 64 x 454
-// (256, 4) 26 -> 34, a window of 67 keys (160, 4) 16 -> 19, of 179 under 128/32 heads (416, 5 to a head) 84 -> 89, 32/8 x 35 packed of up to 754 (1160, 13) 170 -> 206.  With ids the tiles are not known here.
+// query tiles over all heads of the group, on CUs that the others leave early.  By the workgroups of 128 keys that the other form
+// has; the whole backward in this form : in that one, geometric mean over random problems [smallest, largest], 16 tiles or
+// more to a workgroup (48 or more where heads share keys):
+//                                       up to 128          192            256            320            384            448            512
+//   one head, causal, prefix   0.69 [0.67, 0.72]  0.69 [.68, .70]  0.76 [.69, 1.01]  1.05 [.91, 1.20]  1.12 [1.05, 1.23]  1.10  1.04
+//   ... no mask                0.70 [0.65, 0.74]  1.10 [.98, 1.17]  1.04 [.96, 1.25]  0.90 [.83, 1.01]  0.98 [.89, 1.09]  1.08  1.05
+//   ... block mask             0.89 [0.74, 1.01]  0.88 [.81, .96]  0.90 [.77, 1.16]  1.06 [.88, 1.27]  1.11 [.97, 1.19]  1.07  1.12
+//   ... packed                 0.73               0.71             0.73 [.69, .78]  0.88 [.78, .99]  0.94 [.86, 1.08]  1.13
+//   several, causal, prefix    0.67 [0.66, 0.70]  0.69 [.66, .74]  0.74 [.68, .83]  0.80 [.74, 1.00]  0.84 [.76, 1.07]  0.89  0.89
+//   ... window                 0.70 [0.66, 0.73]  0.67 [.65, .69]  0.88 [.71, 1.02]  0.95 [.72, 1.02]  0.87 [.82, .93]  1.03  1.04
+//   ... no mask                0.68 [0.64, 0.73]  0.87 [.84, .88]  0.99 [.89, 1.08]  1.03 [.99, 1.05]  1.01 [.90, 1.05]  1.06  1.06
+//   ... block mask             0.53 [0.49, 0.64]  0.56 [.52, .63]  0.66 [.57, .79]  0.69 [.56, .90]  0.75 [.59, .93]  0.83  0.75, to 1024 0.85
+//       16 to 48 tiles                            0.69             0.99 [.91, 1.06] 0.97 [.82, 1.20] 0.94 [.89, 1.00] 0.96  1.00, to 768 1.01
+//   ... packed                 0.71 [0.68, 0.74]  0.68 [.67, .70]  0.70 [.67, .76]  0.73 [.68, .80]  0.80 [.69, .91]  0.79  0.84
+// Beyond the lines every tile is loaded for half the keys, and workgroups double: also with few tiles, 64/32 heads x 466 (256
+// workgroups, 8 tiles) 37 -> 43 us, a window of 67 keys (160, 4) 16 -> 19.  With ids the tiles are not known here.
 static bool rows_form(const KArgs& a, int D, bool causal, bool doc) {
   if (D != 64 || doc) return false;
-  const bool packed = a.ktab != nullptr;
+  const bool packed = a.ktab != nullptr, window = causal && a.win < 0x3fffffff;
   const int64_t wgs = int64_t(packed ? a.nKent : (a.N + 127) / 128) * a.B * a.Hk;
-  if (wgs > (a.bmask != nullptr ? 4 : 2) * kCUs) return false;
-  if (!packed) return dkdv_tiles(a, causal) >= std::max(16, 8 * a.G);
+  const int tiles = dkdv_tiles(a, causal);   // (a sequence's are not known)
+  const int lim = a.G == 1 ? (packed ? kCUs * 3 / 2 : causal || a.bmask != nullptr ? kCUs : kCUs / 2)
+                           : a.bmask != nullptr ? (tiles < 48 ? kCUs : 4 * kCUs) : packed ? 2 * kCUs : !causal ? kCUs * 3 / 4 : window ? kCUs * 5 / 4 : 2 * kCUs;
+  if (wgs > lim) return false;
+  if (!packed) return tiles >= std::max(16, 8 * a.G);
   const int rows = a.M / std::max(1, a.nKent - 1 - a.N / 128);   // of an average sequence (the table has an entry per 128 keys and one per sequence)
   return (rows / 64 + 1) * a.G >= (causal ? 16 : 8);
 }
