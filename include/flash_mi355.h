@@ -257,7 +257,8 @@ int fa_bwd(const fa_params* p, void* stream);
 #define FA_FORM_ROWS  3       /* D = 64: two waves own the same 32 keys, each half of every tile of rows */
 #define FA_FORM_PIPE  4       /* D = 128, long streams without ids: score and gradient waves one tile apart */
 #define FA_FORM_SMALL 5       /* the four waves of a workgroup own the same 32 keys and share the rows */
-#define FA_FORM_FP32  6
+#define FA_FORM_FP32  6       /* plus 0x10 * s + 0x40 * t where dq and dk/dv are launches of their own: the shapes of dq's and of dk/dv's
+                                 workgroups (0: 16 rows or keys, 1: 32 shared by four waves, 2: 32 shared by two) */
 #define FA_FORM_WITH_DQ 0x100
 int fa_bwd_form(const fa_params* p, int whole);
 

@@ -11,7 +11,7 @@ _DTYPES = {torch.bfloat16: _cabi.FA_DTYPE_BF16, torch.float16: _cabi.FA_DTYPE_FP
 
 
 def dkdv_form(B, H, Hk, M, N, D, dtype, causal, kind="plain", window=0, prefix=0, nseq=0, whole=True, no_pair_wait=False):
-    """(name, whether dq shares the launch).  kind: "plain", "doc", "heads" (ids per head), "qpos" (ids and positions), "block", "packed"."""
+    """(name, whether dq shares the launch), for fp32 (name, shape of dq, of dk/dv) where it does not.  kind: "plain", "doc", "heads" (ids per head), "qpos" (ids and positions), "block", "packed"."""
     buf = ctypes.create_string_buffer(4096)
     base = (ctypes.addressof(buf) + 255) & ~255   # never followed: the call looks at sizes, strides and alignment
     p = _cabi.FaParams()
@@ -40,4 +40,6 @@ def dkdv_form(B, H, Hk, M, N, D, dtype, causal, kind="plain", window=0, prefix=0
         p.flags |= _cabi.FA_FLAG_DEBUG_NO_PAIR_WAIT
     form = _cabi.lib().fa_bwd_form(ctypes.byref(p), int(whole))
     assert form > 0, _cabi.lib().fa_error_string(form)
+    if dtype == torch.float32 and not form & _cabi.FA_FORM_WITH_DQ:   # ... and the shapes of dq's and dk/dv's workgroups
+        return "fp32", (form >> 4) & 3, (form >> 6) & 3
     return NAMES[form & ~_cabi.FA_FORM_WITH_DQ], bool(form & _cabi.FA_FORM_WITH_DQ)

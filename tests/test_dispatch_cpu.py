@@ -46,3 +46,13 @@ def test_the_small_form_stops_where_its_workgroups_share_cus(args, kw):
 def test_rows_are_shared_only_where_cus_are_free(args, kw):
     """D = 64, 288 to 480 workgroups of 128 keys: 1.05 to 1.28 times the time of the form whose waves own their keys."""
     assert dkdv_form(*args, **kw)[0] == "keys"
+
+
+@pytest.mark.parametrize("args,kw", [
+    ((8, 32, 32, 32, 32, 64, f32, True), {"kind": "doc"}), ((4, 64, 64, 25, 25, 128, f32, True), {"kind": "doc"}), ((4, 64, 64, 92, 274, 128, f32, True), {"kind": "doc"}),
+    ((8, 32, 32, 98, 98, 128, f32, False), {}), ((2, 64, 64, 209, 209, 128, f32, False), {}),
+])
+def test_short_fp32_rows_are_not_cut_among_eight_waves(args, kw):
+    """Many short rows: 1.2 to 2.5 times the time in dq where eight waves shared 16 rows, most of the workgroups of them empty with ids."""
+    form, dq, _ = dkdv_form(*args, **kw)
+    assert form == "fp32" and dq != 0

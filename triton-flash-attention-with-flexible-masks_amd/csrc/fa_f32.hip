@@ -696,7 +696,8 @@ int launch(const KArgs& a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Which of three shapes a launch takes, by the blocks of 16 rows (keys) that it has.  us (forward, dq, dk/dv):
+// Which of three shapes a launch takes, by the blocks of 16 rows (keys) that it has -- with ids those of the plan's padded order,
+// whose empty ones cost a workgroup each -- and by the blocks of the other side that one of them walks, its chain.  us (forward, dq, dk/dv):
 //                                          RB 1, SW 8 *       RB 2, SW 4         RB 2, SW 2
 //   D = 64  2 x 4 heads x 1024, causal (512)    22.6 35.6 37.2     28.2 36.9 46.1     48.9 63.5 79.8
 //           2 x 4 x 2048, documents  (1024)     33.6 43.4 54.6     61.1 79.0 46.2     108 140 60
@@ -713,19 +714,33 @@ int launch(const KArgs& a, hipStream_t s) {
 //           8 x 16 x 2048, causal    (16384)    1749 2763 3556     1232 2199 2728     1187 2008 2540
 //   * dk/dv at D = 128: SW 4, since one wave to a SIMD is all that its registers allow
 // Few blocks: the chain of one of them counts, so all waves share it.  Many: the work counts, and a block of 32 reads the
-// other side half as often; then also what a workgroup adds up at its end.  (Rows with ids: the global ones among them walk
-// all keys, the others a few blocks: the chain counts longer.)
+// other side half as often; then also what a workgroup adds up at its end -- the more, the shorter the chain.  (Rows with ids:
+// the global ones among them walk all keys, the others a few blocks: the chain counts longer.)  Over 2000 random problems the
+// launches take 1.03, 1.03 and 1.02 times the best shape's time on average; with lines at fixed numbers of blocks (768 and 4096,
+// with ids 2048 and 16384, padding not counted) 1.06, 1.11 and 1.05, and many short rows with ids up to 2.5 times what they
+// took with tiles in LDS (8 x 32 heads x 32: dq 10.6 -> 26.6; 4 x 64 x 92, D = 128: forward 30 -> 59).
 template <int WHICH, int D> constexpr int kFewWaves = D == 128 && (WHICH == kDkdv || WHICH == kBoth) ? 4 : 8;
+inline int64_t clamped(int64_t x, int64_t lo, int64_t hi) { return x < lo ? lo : x > hi ? hi : x; }
+// 0, 1, 2: the columns of the table
+template <int WHICH, int MODE> int shape(const KArgs& a) {
+  static_assert(WHICH != kBoth, "dq and dk/dv in one launch have one shape");
+  constexpr bool IDS = WHICH != kDkdv && MODE == kDoc;
+  const int64_t n = WHICH == kDkdv ? int64_t((a.N + kSB - 1) / kSB) * a.B * a.Hk : int64_t(((IDS ? a.Pp : a.M) + kSB - 1) / kSB) * a.B * a.H;
+  const int other = WHICH == kDkdv ? a.M : a.N;
+  const int64_t chain = int64_t((std::min(other, MODE == kDoc ? other : a.win + kSB) + kSB - 1) / kSB) * (WHICH == kDkdv ? a.G : 1);
+  if (IDS && chain <= 2) return 2;
+  const int64_t few = WHICH == kFwd && !IDS ? 768 : clamped(16 * chain, 256, IDS ? 2048 : 768);
+  const int64_t many = WHICH == kFwd ? 16384 : IDS ? clamped(128 * chain, 2048, 16384) : clamped(64 * chain, 1024, 4096);
+  return n <= few ? 0 : n < many ? 1 : 2;
+}
 template <int WHICH, int D, bool CAUSAL, int MODE>
 int launch_shape(const KArgs& a, hipStream_t s) {
   if constexpr (WHICH == kBoth) {
     return launch<WHICH, D, CAUSAL, MODE, 1, kFewWaves<WHICH, D>>(a, s);
   } else {
-    const int64_t n = WHICH == kDkdv ? int64_t((a.N + kSB - 1) / kSB) * a.B * a.Hk : int64_t((a.M + kSB - 1) / kSB) * a.B * a.H;
-    constexpr int kFew = WHICH != kDkdv && MODE == kDoc ? 2048 : 768;
-    constexpr int kMany = WHICH == kFwd || (WHICH == kDq && MODE == kDoc && D <= 64) ? 16384 : 4096;
-    if (n <= kFew) return launch<WHICH, D, CAUSAL, MODE, 1, kFewWaves<WHICH, D>>(a, s);
-    if (n < kMany) return launch<WHICH, D, CAUSAL, MODE, 2, 4>(a, s);
+    const int sh = shape<WHICH, MODE>(a);
+    if (sh == 0) return launch<WHICH, D, CAUSAL, MODE, 1, kFewWaves<WHICH, D>>(a, s);
+    if (sh == 1) return launch<WHICH, D, CAUSAL, MODE, 2, 4>(a, s);
     return launch<WHICH, D, CAUSAL, MODE, 2, 2>(a, s);
   }
 }
@@ -780,11 +795,14 @@ int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t 
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kDkdv>(a, D, causal, doc, s); }
 
 // dq and dk/dv side by side in one launch, each forming delta itself: where the workgroups of both (32 rows or keys counted as
-// one) are about as many as the CUs can hold.  2 x 4 heads x 512 rows with documents, D = 64, forward and backward: 64.9 us against
+// one, with ids the empty places of the plan's order too) are about as many as the CUs can hold.  2 x 4 heads x 512 rows with documents, D = 64, forward and backward: 64.9 us against
 // 69.0 with two launches.  At the line, 8 x 8 heads x 128, causal: 28.1 us against 26.2 and the gap between two launches.
 bool bwd_f32_in_one(const KArgs& a) {
-  const int64_t wgs = int64_t((a.M + 31) / 32) * a.B * a.H + int64_t((a.N + 31) / 32) * a.B * a.Hk;
+  const int64_t wgs = int64_t(((a.Pp > 0 ? a.Pp : a.M) + 31) / 32) * a.B * a.H + int64_t((a.N + 31) / 32) * a.B * a.Hk;
   return wgs <= 2 * kCUs;
+}
+int bwd_f32_shapes(const KArgs& a, bool doc) {
+  return doc ? 0x10 * shape<kDq, kDoc>(a) + 0x40 * shape<kDkdv, kDoc>(a) : 0x10 * shape<kDq, kPlain>(a) + 0x40 * shape<kDkdv, kPlain>(a);
 }
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kBoth>(a, D, causal, doc, s); }
 
