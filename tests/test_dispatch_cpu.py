@@ -56,3 +56,47 @@ def test_short_fp32_rows_are_not_cut_among_eight_waves(args, kw):
     """Many short rows: 1.2 to 2.5 times the time in dq where eight waves shared 16 rows, most of the workgroups of them empty with ids."""
     form, dq, _ = dkdv_form(*args, **kw)
     assert form == "fp32" and dq != 0
+
+
+def _kind(k):
+    return k if k in ("doc", "heads", "qpos", "block") else "plain"
+
+
+def _form(case, D, window, prefix, **kw):
+    """(B, H, Hk, M, N, dtype, causal, kind) with a window or prefix of the given size where the kind says so"""
+    B, H, Hk, M, N, dtype, causal, kind = case
+    return dkdv_form(B, H, Hk, M, N, D, dtype, causal, _kind(kind), window=window if kind == "window" else 0, prefix=prefix if kind == "prefix" else 0, **kw)
+
+
+def test_gpu_cases_reach_the_form_they_are_written_for():
+    from tests import test_gpu_launch_forms as F, test_gpu_parity as P
+    assert {_form(c, 64, 500, 270)[0] for c in F.ROWS_CASES} == {"rows"}
+    assert {_form(c, 64, 500, 270)[1] for c in F.ROWS_CASES} == {True, False}
+    assert {_form(c, 64, 500, 270)[0] for c in F.ROWS_BEYOND_CASES} == {"keys"}
+    for lens in ([1000, 833, 961, 64, 1, 532, 990], [700, 0, 1211, 130]):
+        assert dkdv_form(1, 32, 8, sum(lens), sum(lens), 64, bf16, True, "packed", nseq=len(lens))[0] == "rows"
+    for B, H, Hk, M, N, D, causal, form in F.LAYOUT_CASES:
+        assert dkdv_form(B, H, Hk, M, N, D, bf16, causal)[0] == form
+    for B, H, Hk, M, N, dtype, causal, window, prefix in F.PIPE_CASES:
+        assert dkdv_form(B, H, Hk, M, N, 128, dtype, causal, window=window, prefix=prefix, whole=False, no_pair_wait=True)[0] == "pipe"
+    for i, (B, H, Hk, M, N, D, dtype, causal, kind) in enumerate(F.SMALL_BWD_CASES):   # (the second half: runs of key tiles next to the column form)
+        assert _form((B, H, Hk, M, N, dtype, causal, kind), D, 37, 21)[0] == ("small" if i < 11 else "cols")
+    alone = [{dkdv_form(B, H, Hk, M, N, D, dtype, causal, _kind(kind), window=170 if kind == "window" else 0, prefix=170 if kind == "prefix" else 0, whole=w)[0]
+              for w in (True, False)} for B, H, Hk, M, N, D, dtype, causal, kind in F.SHARED_CASES]
+    assert {"keys", "pipe"} in alone and {"rows"} in alone and {"keys"} in alone and {"small"} in alone
+    unseen = {dkdv_form(1, H, H, M, N, D, bf16, True, _kind(kind), window=2000 if kind == "window" else 0, whole=w)[0] for D, H, M, N, kind in F.UNSEEN_CASES for w in (True, False)}
+    assert unseen == {"keys", "rows", "small", "pipe", "cols"}
+    for B, H, Hk, M, N, D, dtype, causal, doc in P.KEYS_CASES:
+        assert dkdv_form(B, H, Hk, M, N, D, dtype, causal, "doc" if doc else "plain")[0] == "keys"
+    for B, H, Hk, M, N, D, dtype, causal, window, _, _ in P.KEYS_BLOCK_CASES:
+        assert dkdv_form(B, H, Hk, M, N, D, dtype, causal, "block", window=window)[0] == "keys"
+    for B, H, Hk, M, N, D, dtype, doc, window, prefix in P.KEYS_BAND_CASES:
+        assert dkdv_form(B, H, Hk, M, N, D, dtype, True, "doc" if doc else "plain", window=window, prefix=prefix)[0] == "keys"
+    for B, H, Hk, M, N, D, dtype, causal, _, window in P.COLS_BIG_CASES:
+        assert dkdv_form(B, H, Hk, M, N, D, dtype, causal, "doc", window=window)[0] == "cols"
+    for B, H, Hk, M, N, causal, kw in ((1, 4, 2, 243, 1419, True, {"window": 876}), (2, 2, 1, 651, 617, False, {}), (2, 4, 2, 248, 1297, True, {"prefix": 530})):
+        assert dkdv_form(B, H, Hk, M, N, 128, bf16, causal, "doc", **kw)[0] == "small"
+        assert dkdv_form(6 * B, H, Hk, M, N, 128, bf16, causal, "doc", **kw)[0] in ("keys", "cols")   # (P crosses between the waves of a pair)
+    shapes = [dkdv_form(B, H, Hk, M, N, D, f32, causal, _kind(kind), window=37 if kind == "window" else 0, prefix=21 if kind == "prefix" else 0)[1:]
+              for B, H, Hk, M, N, D, causal, kind in F.FP32_SHAPE_CASES]
+    assert shapes[:3] == [(0, 0)] * 3 and {s[0] for s in shapes} == {s[1] for s in shapes} == {0, 1, 2}

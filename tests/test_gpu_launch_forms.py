@@ -324,12 +324,14 @@ def test_fp32_launch_forms(case):
     _run_case(B, H, Hk, M, N, D, torch.float32, causal, doc, seed=3, window=window, tol_o=2e-4, tol_lse=2e-4)
 
 
-# fp32: 16 or 32 rows (keys) to a workgroup and two, four or eight waves to share the other side, by the number of blocks of 16:
-# up to 768 (rows with ids: 2048), up to 4096 (16384), above.  B, H, Hk, M, N, D, causal, kind
+# fp32: 16 or 32 rows (keys) to a workgroup and two, four or eight waves to share the other side, by the number of blocks of 16 and by
+# how many of them a row walks (the shapes of dq and dk/dv are held in test_dispatch_cpu.py).  B, H, Hk, M, N, D, causal, kind
 FP32_SHAPE_CASES = [
-    (2, 16, 16, 330, 330, 64, True, "plain"), (2, 16, 8, 384, 400, 32, True, "window"),      # the first shape, dq and dk/dv in launches of their own
-    (2, 16, 16, 500, 501, 64, True, "plain"), (4, 16, 8, 545, 545, 64, True, "doc"), (1, 64, 64, 210, 270, 128, True, "prefix"),   # the second
-    (4, 16, 4, 530, 530, 16, False, "heads"), (2, 16, 16, 600, 333, 32, True, "qpos"), (2, 16, 16, 450, 450, 128, True, "block"),
+    (1, 16, 16, 700, 700, 64, True, "plain"), (1, 16, 16, 740, 750, 32, True, "block"), (1, 8, 8, 1500, 1500, 128, True, "doc"),   # the first shape, dq and dk/dv in launches of their own
+    (2, 16, 16, 330, 330, 64, True, "plain"), (2, 16, 8, 384, 400, 32, True, "window"),      # the second (of the forward the first)
+    (2, 16, 16, 500, 501, 64, True, "plain"), (4, 16, 8, 545, 545, 64, True, "doc"), (1, 64, 64, 210, 270, 128, True, "prefix"),   # the second, dk/dv of the last the third
+    (4, 16, 4, 530, 530, 16, False, "heads"), (2, 16, 16, 600, 333, 32, True, "qpos"), (2, 16, 16, 450, 450, 128, True, "block"),   # the second, dk/dv of the first the first
+    (8, 32, 32, 31, 32, 64, True, "doc"), (4, 64, 64, 92, 92, 128, True, "doc"),             # short rows with ids, most of the plan's order empty: the third, the second
     (64, 64, 64, 49, 33, 16, False, "plain"), (32, 128, 64, 50, 65, 64, True, "plain"), (16, 64, 64, 257, 257, 16, True, "doc"),   # the third
     (8, 32, 32, 260, 260, 128, True, "doc"), (16, 32, 16, 130, 140, 128, True, "block"), (64, 64, 64, 63, 64, 32, True, "window"),
 ]
@@ -387,7 +389,11 @@ SHARED_CASES = [
     (1, 2, 2, 129, 5000, 128, torch.bfloat16, True, "plain"), (1, 8, 4, 900, 900, 64, torch.bfloat16, True, "window"),
     (1, 8, 8, 1000, 1000, 128, torch.bfloat16, True, "prefix"), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, "block"),
     (2, 4, 4, 333, 333, 64, torch.float16, True, "block"), (1, 4, 4, 700, 900, 128, torch.bfloat16, True, "doc"),
-    (2, 4, 2, 257, 257, 64, torch.bfloat16, True, "doc"), (1, 2, 2, 3000, 3000, 128, torch.bfloat16, True, "doc"),    (1, 8, 2, 1500, 1500, 128, torch.bfloat16, True, "plain"),   # (the separate dk/dv takes 128 keys to a workgroup)
+    (2, 4, 2, 257, 257, 64, torch.bfloat16, True, "doc"), (1, 2, 2, 3000, 3000, 128, torch.bfloat16, True, "doc"),
+    (1, 8, 2, 1500, 1500, 128, torch.bfloat16, True, "plain"), (1, 8, 8, 1000, 1000, 128, torch.float16, True, "window"),
+    (2, 32, 8, 1100, 1100, 64, torch.bfloat16, True, "plain"), (3, 32, 8, 1100, 1100, 64, torch.float16, True, "block"),   # (waves that share the rows, in both)
+    (2, 8, 8, 900, 900, 64, torch.bfloat16, True, "window"),
+    # (dk/dv by pairs of waves that poll next to dq, by the pipelined form in a launch of its own)
     (1, 8, 8, 4200, 4200, 128, torch.bfloat16, False, "plain"), (1, 8, 8, 6000, 6000, 128, torch.bfloat16, True, "plain"),
     (2, 8, 8, 2500, 2500, 64, torch.bfloat16, True, "doc"),
 ]
@@ -423,16 +429,23 @@ def test_backward_in_one_launch(case):
 
 
 # dk/dv at D = 64 with two waves to a block of keys, each for half of every tile of rows: tiles of rows and keys that are partly filled (a half without
-# rows, a wave without keys), a window, a prefix, a block mask, heads of a group; in a launch of its own (the last three) and next to dq's.
+# rows, a wave without keys), a window, a prefix, a block mask, heads of a group; next to dq's and (the last) in a launch of its own.
 # B, H, Hk, M, N, dtype, causal, kind
 ROWS_CASES = [
+    (2, 32, 8, 1100, 1100, torch.bfloat16, True, "plain"), (2, 32, 8, 1100, 1090, torch.float16, False, "plain"), (2, 32, 8, 1100, 1100, torch.float16, True, "prefix"),
+    (4, 16, 4, 777, 900, torch.bfloat16, True, "window"), (4, 32, 8, 1100, 1100, torch.bfloat16, True, "window"), (3, 32, 8, 1100, 1100, torch.bfloat16, True, "block"),
+    (2, 8, 8, 1999, 2030, torch.bfloat16, True, "plain"), (1, 8, 8, 1999, 1900, torch.bfloat16, False, "plain"),
+    (2, 128, 8, 1100, 1090, torch.float16, False, "plain"),
+]
+# Sizes that stay with the form whose waves own their keys: short chains, or too many workgroups.
+ROWS_BEYOND_CASES = [
     (4, 32, 8, 530, 530, torch.bfloat16, True, "plain"), (3, 32, 8, 545, 1000, torch.float16, True, "plain"), (5, 8, 8, 1025, 1666, torch.bfloat16, False, "plain"),
-    (4, 16, 4, 777, 900, torch.bfloat16, True, "window"), (4, 32, 8, 600, 600, torch.float16, True, "prefix"), (4, 32, 8, 700, 700, torch.bfloat16, True, "block"),
-    (2, 128, 8, 1100, 1090, torch.float16, False, "plain"), (1, 256, 16, 700, 1700, torch.bfloat16, True, "block"), (1, 512, 16, 161, 2100, torch.float16, True, "plain"),
+    (4, 32, 8, 600, 600, torch.float16, True, "prefix"), (4, 32, 8, 700, 700, torch.bfloat16, True, "block"),
+    (1, 256, 16, 700, 1700, torch.bfloat16, True, "block"), (1, 512, 16, 161, 2100, torch.float16, True, "plain"),
 ]
 
 
-@pytest.mark.parametrize("case", ROWS_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-%s-c%d-%s" % (*c[:5], str(c[5])[6:], *c[6:]))
+@pytest.mark.parametrize("case", ROWS_CASES + ROWS_BEYOND_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-%s-c%d-%s" % (*c[:5], str(c[5])[6:], *c[6:]))
 def test_dkdv_rows_split_over_two_waves(case):
     B, H, Hk, M, N, dtype, causal, kind = case
     if kind == "block":
@@ -499,6 +512,60 @@ def test_small_backward_packed(D, lq, lk):
         a += m; b += n
 
 
+@pytest.mark.parametrize("lens", [[1000, 833, 961, 64, 1, 532, 990], [700, 0, 1211, 130]])
+def test_dkdv_rows_split_over_two_waves_packed(lens):
+    """Two workgroups of 64 keys to an entry of the plan's table: sequences whose last entry has keys for one of them only."""
+    from flash_mi355 import attention_varlen
+    from oracle import attention_oracle as O
+    H, Hk = 32, 8
+    q, k, v, do = _tensors(1, H, Hk, sum(lens), sum(lens), 64, torch.bfloat16, 15)
+    t3 = lambda t: t[0].transpose(0, 1).contiguous()
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32).cuda()
+    qd, kd, vd = (t3(t).cuda().requires_grad_(True) for t in (q, k, v))
+    print("case", lens, flush=True)
+    out = attention_varlen(qd, kd, vd, cu, cu, causal=True)
+    out.backward(t3(do).cuda())
+    a = 0
+    for m in lens:
+        if m:
+            x = slice(a, a + m)
+            ref = O.attention_autograd(q[:, :, x], k[:, :, x], v[:, :, x], do[:, :, x], True, None, None, None, 0)[2:]
+            for name, t, r in (("dq", qd, ref[0]), ("dk", kd, ref[1]), ("dv", vd, ref[2])):
+                # (dk, dv: sums over the heads of a group, each rounded by itself)
+                check_close(name, t.grad[x].transpose(0, 1)[None], r, TOL_ABS if name == "dq" else TOL_ABS * math.sqrt(H // Hk))
+        a += m
+
+
+# A row of [B, L, H, D], or of a cache with room behind it, is read and written as one of [B, H, L, D]: the same bits, in every form of the backward.
+# B, H, Hk, M, N, D, causal, kind
+LAYOUT_CASES = [(1, 32, 32, 4100, 4100, 128, True, "pipe"), (2, 32, 8, 1100, 1100, 64, True, "rows"), (1, 8, 8, 1088, 1088, 128, True, "keys"), (2, 8, 8, 700, 700, 64, True, "keys"),
+                (2, 4, 2, 333, 400, 128, True, "small"), (2, 4, 2, 333, 400, 64, False, "small")]
+
+
+@pytest.mark.parametrize("case", LAYOUT_CASES, ids=lambda c: "B%d-H%d_%d-M%d-N%d-D%d-c%d-%s" % c)
+def test_layouts_give_the_same_bits(case):
+    from flash_mi355 import attention
+    B, H, Hk, M, N, D, causal, _ = case
+    print("case", case, flush=True)
+    q, k, v, do = (t.cuda() for t in _tensors(B, H, Hk, M, N, D, torch.bfloat16, 21))
+
+    def blhd(t):
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+    def roomy(t):
+        room = torch.full((*t.shape[:2], t.shape[2] + 37, D + 8), float("nan"), dtype=t.dtype, device="cuda")
+        room[:, :, :t.shape[2], :D] = t
+        return room[:, :, :t.shape[2], :D]
+    results = []
+    for f in (torch.Tensor.contiguous, blhd, roomy):
+        x = [f(t).detach().requires_grad_(True) for t in (q, k, v)]
+        out = attention(*x, causal)
+        results.append((out.detach(), *torch.autograd.grad(out, x, f(do))))
+    for other in results[1:]:
+        for a, b in zip(results[0], other):
+            assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
 # the pipelined dk/dv form (D = 128, at least 32 query tiles over the heads of a group): tiles and key blocks that are partly
 # filled, one key, heads of a group in one stream, a window, a prefix, more keys than queries and fewer
 PIPE_CASES = [
@@ -536,6 +603,9 @@ def test_pipelined_dkdv(case):
     plan.ensure_workspace(qd.device)
     ref, s = ctypes.byref(p), _stream_ptr(qd.device)
     for name in ("fa_fwd", "fa_bwd_delta", "fa_bwd_dkdv"):
+        if name == "fa_bwd_dkdv":   # (no pair polls in this form; the flag keeps these sizes off the one for small problems)
+            p.flags = _cabi.FA_FLAG_DEBUG_NO_PAIR_WAIT
+            assert _cabi.lib().fa_bwd_form(ref, 0) == _cabi.FA_FORM_PIPE
         _cabi.check(getattr(_cabi.lib(), name)(ref, s), name)
     torch.cuda.synchronize()
     _, _, _, rdk, rdv = O.attention_autograd(q, k, v, do, causal, None, None, None, 0, window=window, prefix=prefix)

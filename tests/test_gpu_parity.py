@@ -31,7 +31,8 @@ def _ids(rng, B, H, L, kind):
 
 def _run_case(B, H, Hk, M, N, D, dtype, causal, doc, seed, ids_kind="uniform", per_head_ids=False,
               id_dtype=torch.int32, sm_scale=None, check_bwd=True, tol_o=TOL_O, tol_lse=TOL_LSE, window=0, prefix=0,
-              qpos=None, ceilings=None):
+              qpos=None, ceilings=None, copies=1):
+    """copies: the GPU gets the batch that many times over (more workgroups, hence other forms), and every copy is held to the oracle."""
     from flash_mi355 import attention, attention_with_lse, SCORE_FUNC_MODE1_DOC
     from oracle import attention_oracle as O
     g = torch.Generator().manual_seed(seed)
@@ -61,20 +62,22 @@ def _run_case(B, H, Hk, M, N, D, dtype, causal, doc, seed, ids_kind="uniform", p
         qpos = torch.from_numpy(qpos).to(torch.int32)
     print(f"case B{B} H{H}/{Hk} M{M} N{N} D{D} {dtype} causal={causal} doc={doc} seed={seed} ids={ids_kind} "
           f"window={window} prefix={prefix} qpos={None if qpos is None else tuple(qpos.shape)}", flush=True)
-    qposd = None if qpos is None else qpos.cuda()
+    more = lambda t: t.cuda().repeat(copies, *([1] * (t.dim() - 1)))
+    qposd = None if qpos is None else more(qpos)
 
-    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
-    eqd = eq.cuda() if eq is not None else None
-    ekd = ek.cuda() if ek is not None else None
+    qd, kd, vd = (more(t).requires_grad_(True) for t in (q, k, v))
+    eqd = more(eq) if eq is not None else None
+    ekd = more(ek) if ek is not None else None
     if eqd is not None and not per_head_ids:
-        eqd = eq[:, :1].contiguous().cuda().expand(B, H, M)
-        ekd = ek[:, :1].contiguous().cuda().expand(B, H, N)
+        eqd = more(eq[:, :1].contiguous()).expand(B * copies, H, M)
+        ekd = more(ek[:, :1].contiguous()).expand(B * copies, H, N)
     out, lse = attention_with_lse(qd.detach(), kd.detach(), vd.detach(), causal, sm_scale, eqd, ekd, mode,
                                   window=window, prefix=prefix, qpos=qposd)
     torch.cuda.synchronize()
     ref_o, ref_lse, ref_dq, ref_dk, ref_dv = O.attention_autograd(q, k, v, do, causal, sm_scale, eq, ek, mode,
                                                                    window=window, prefix=prefix, qpos=qpos)
     # rows without any kept key: O = 0, LSE = -inf on both sides
+    ref_o, ref_lse, ref_dq, ref_dk, ref_dv = (t.repeat(copies, *([1] * (t.dim() - 1))) for t in (ref_o, ref_lse, ref_dq, ref_dk, ref_dv))
     dead = torch.isinf(ref_lse)
     assert torch.equal(torch.isinf(lse.cpu()), dead)
     lse_err = (lse.cpu()[~dead] - ref_lse[~dead]).abs().max().item() if (~dead).any() else 0.0
@@ -85,7 +88,7 @@ def _run_case(B, H, Hk, M, N, D, dtype, causal, doc, seed, ids_kind="uniform", p
     if not check_bwd:
         return
     out2 = attention(qd, kd, vd, causal, sm_scale, eqd, ekd, mode, window=window, prefix=prefix, qpos=qposd)
-    out2.backward(do.cuda())
+    out2.backward(more(do))
     torch.cuda.synchronize()
     assert torch.equal(out2.detach(), out)
     for name, got, ref in (("dq", qd.grad, ref_dq), ("dk", kd.grad, ref_dk), ("dv", vd.grad, ref_dv)):
@@ -101,6 +104,12 @@ def _run_case(B, H, Hk, M, N, D, dtype, causal, doc, seed, ids_kind="uniform", p
         check_close(name, got, ref, tol_o * sharp * (ceilings or {}).get(name, 1.0))
 
 
+# Just beyond the problems whose backward takes the form for few workgroups (fa_bwd_form "small"): pairs of waves that poll (D = 128), waves that
+# own their keys (D = 64).  The lists below have such cases for every mask; test_dispatch_cpu.py holds them there.
+KEYS_CASES = [
+    (1, 8, 8, 1100, 1100, 128, torch.bfloat16, False, False), (1, 8, 8, 1100, 1100, 128, torch.bfloat16, True, False), (2, 16, 4, 700, 790, 128, torch.float16, True, False),
+    (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, True), (2, 8, 8, 545, 545, 64, torch.bfloat16, True, True), (2, 8, 8, 700, 705, 64, torch.float16, True, False),
+]
 CASES = [
     # B, H, Hk, M, N, D, dtype, causal, doc
     (1, 2, 2, 128, 128, 128, torch.bfloat16, False, False),
@@ -117,8 +126,9 @@ CASES = [
     (1, 2, 2, 256, 256, 16, torch.bfloat16, True, True),
     (2, 2, 1, 100, 300, 16, torch.float16, True, True),
     (1, 2, 2, 192, 192, 64, torch.bfloat16, False, False),
-    (1, 1, 1, 2048, 2048, 128, torch.bfloat16, False, False),  # long tile stream: the 128-key dk/dv form without ids
+    (1, 1, 1, 2048, 2048, 128, torch.bfloat16, False, False),  # long chains of few key tiles
     (1, 2, 1, 2100, 4300, 128, torch.float16, True, False),    # the same under a causal mask, grouped and ragged
+    *KEYS_CASES,
 ]
 
 
@@ -179,6 +189,10 @@ def test_mask_bit_exact():
         assert np.array_equal(got, ref)
 
 
+KEYS_BLOCK_CASES = [
+    (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, 0, 0.4, False), (2, 16, 4, 1000, 1130, 128, torch.float16, False, 0, 0.5, True),
+    (1, 8, 8, 1100, 1100, 128, torch.bfloat16, True, 400, 0.6, False), (2, 8, 8, 700, 700, 64, torch.bfloat16, True, 0, 0.5, False),
+]
 BLOCK_CASES = [
     # B, H, Hk, M, N, D, dtype, causal, window, density, broadcast (block map shared by batch and heads)
     (1, 2, 2, 512, 512, 128, torch.bfloat16, False, 0, 0.5, False),
@@ -189,12 +203,13 @@ BLOCK_CASES = [
     (1, 2, 1, 333, 520, 64, torch.float16, False, 0, 0.3, True),
     (1, 2, 2, 200, 200, 16, torch.bfloat16, True, 0, 0.5, False),
     (1, 2, 2, 640, 640, 32, torch.bfloat16, False, 0, 0.2, False),
-    (1, 1, 1, 2304, 2304, 128, torch.bfloat16, True, 0, 0.3, False),   # long stream: the 128-key dk/dv form
+    (1, 1, 1, 2304, 2304, 128, torch.bfloat16, True, 0, 0.3, False),   # long stream
     (1, 2, 2, 1024, 1024, 128, torch.bfloat16, True, 300, 0.7, False),  # with a sliding window
     (1, 2, 2, 192, 192, 128, torch.bfloat16, False, 0, 0.0, False),    # nothing kept at all
     (1, 2, 2, 300, 300, 64, torch.float32, True, 0, 0.5, False),       # the fp32 kernels
     (1, 4, 2, 200, 520, 128, torch.float32, False, 0, 0.4, True),
     (2, 2, 1, 450, 450, 32, torch.float32, True, 100, 0.6, False),
+    *KEYS_BLOCK_CASES,
 ]
 
 
@@ -819,6 +834,11 @@ def test_varlen_takes_boundaries_from_the_host_and_needs_key_boundaries_for_othe
         attention_varlen(q, k, v, cuq.cuda())
 
 
+COLS_BIG_CASES = [   # (enough workgroups for the column form at D >= 64; the other cases at these D may take the form for few)
+    (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "uniform", 0), (1, 16, 8, 300, 1700, 128, torch.float16, True, "uniform", 0), (1, 8, 8, 900, 2100, 128, torch.bfloat16, True, "uniform", 0),
+    (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "alllocal", 0), (1, 8, 8, 300, 1501, 64, torch.float16, True, "uniform", 0),
+    (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "uniform", 700), (1, 8, 8, 300, 1500, 128, torch.bfloat16, False, "uniform", 0),
+]
 COLS_CASES = [
     # B, H, Hk, M, N, D, dtype, causal, ids, window: more keys than queries, the queries' documents at the end
     (2, 2, 2, 300, 1500, 128, torch.bfloat16, True, "uniform", 0),     # one tile of global rows
@@ -832,6 +852,7 @@ COLS_CASES = [
     (1, 2, 2, 300, 1500, 128, torch.bfloat16, True, "uniform", 700),   # sliding window: global rows lose the far keys
     (1, 2, 2, 300, 1500, 128, torch.bfloat16, False, "uniform", 0),    # no causal mask
     (1, 2, 2, 64, 4100, 128, torch.bfloat16, True, "allglobal", 0),    # every row global: all key columns
+    *COLS_BIG_CASES,
 ]
 
 
@@ -976,6 +997,11 @@ def test_fp32_all_global_and_all_local_ids():
 
 # Sliding window and prefix-LM (causal masks the library adds; no counterpart in the reference):
 # checked against the oracle's closed form like every other case.
+KEYS_BAND_CASES = [
+    (1, 8, 8, 1088, 1088, 128, torch.bfloat16, False, 300, 0), (1, 8, 8, 1000, 1500, 128, torch.float16, False, 500, 0), (2, 16, 4, 800, 800, 128, torch.bfloat16, False, 65, 0),
+    (1, 8, 8, 1088, 1088, 128, torch.bfloat16, False, 0, 300), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, 300, 0), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, 0, 300),
+    (2, 8, 8, 700, 700, 64, torch.bfloat16, True, 100, 0), (2, 8, 8, 700, 700, 64, torch.bfloat16, False, 100, 0), (2, 8, 8, 700, 700, 64, torch.float16, False, 0, 200),
+]
 BAND_CASES = [
     # B, H, Hk, M, N, D, dtype, doc, window, prefix
     (1, 2, 2, 512, 512, 128, torch.bfloat16, False, 100, 0),
@@ -994,6 +1020,7 @@ BAND_CASES = [
     (1, 2, 2, 333, 333, 64, torch.float32, True, 50, 0),
     (1, 2, 2, 333, 333, 128, torch.float32, False, 0, 100),
     (1, 4, 2, 100, 260, 32, torch.float32, True, 0, 200),
+    *KEYS_BAND_CASES,
 ]
 
 
@@ -1054,9 +1081,11 @@ def test_p_crosses_the_wave_pair_as_fp16():
     cases found dK elements up to 19 % over the per-element bound (this case: 0.0206 against 0.02 at an exact
     value of -3.2081; grouped heads, local ids, window 876).  P <= 1 crosses as fp16 now, for either element
     type: 11 significant bits in the same two bytes.  The case sits at 0.65 of the bound."""
-    _run_case(1, 4, 2, 243, 1419, 128, torch.bfloat16, True, True, seed=5012, ids_kind="alllocal", window=876)
-    _run_case(2, 2, 1, 651, 617, 128, torch.bfloat16, False, True, seed=5086, ids_kind="alllocal")
-    _run_case(2, 4, 2, 248, 1297, 128, torch.bfloat16, True, True, seed=5210, ids_kind="alllocal", prefix=530)
+    # (the batch several times over: problems of these sizes take a form without pairs)
+    for copies in (1, 6):
+        _run_case(1, 4, 2, 243, 1419, 128, torch.bfloat16, True, True, seed=5012, ids_kind="alllocal", window=876, copies=copies)
+        _run_case(2, 2, 1, 651, 617, 128, torch.bfloat16, False, True, seed=5086, ids_kind="alllocal", copies=copies)
+        _run_case(2, 4, 2, 248, 1297, 128, torch.bfloat16, True, True, seed=5210, ids_kind="alllocal", prefix=530, copies=copies)
 
 
 FLOOR_CASES = [
