@@ -813,6 +813,7 @@ constexpr size_t dkdv_lds() { return 4 * 64 * (D < 32 ? 32 : D) * 2 + 2 * 1024 +
 //   ... no mask                0.68 [0.64, 0.73]  0.87 [.84, .88]  0.99 [.89, 1.08]  1.03 [.99, 1.05]  1.01 [.90, 1.05]  1.06  1.06
 //   ... block mask             0.53 [0.49, 0.64]  0.56 [.52, .63]  0.66 [.57, .79]  0.69 [.56, .90]  0.75 [.59, .93]  0.83  0.75, to 1024 0.85
 //       16 to 48 tiles                            0.69             0.99 [.91, 1.06] 0.97 [.82, 1.20] 0.94 [.89, 1.00] 0.96  1.00, to 768 1.01
+//       (few blocks on, 16 heads x 2011 with 14 % of them, 256 workgroups: 25 us -> 29)
 //   ... packed                 0.71 [0.68, 0.74]  0.68 [.67, .70]  0.70 [.67, .76]  0.73 [.68, .80]  0.80 [.69, .91]  0.79  0.84
 // Beyond the lines every tile is loaded for half the keys, and workgroups double: also with few tiles, 64/32 heads x 466 (256
 // workgroups, 8 tiles) 37 -> 43 us, a window of 67 keys (160, 4) 16 -> 19.  With ids the tiles are not known here.
@@ -821,8 +822,8 @@ static bool rows_form(const KArgs& a, int D, bool causal, bool doc) {
   const bool packed = a.ktab != nullptr, window = causal && a.win < 0x3fffffff;
   const int64_t wgs = int64_t(packed ? a.nKent : (a.N + 127) / 128) * a.B * a.Hk;
   const int tiles = dkdv_tiles(a, causal);   // (a sequence's are not known)
-  const int lim = a.G == 1 ? (packed ? kCUs * 3 / 2 : causal || a.bmask != nullptr ? kCUs : kCUs / 2)
-                           : a.bmask != nullptr ? (tiles < 48 ? kCUs : 4 * kCUs) : packed ? 2 * kCUs : !causal ? kCUs * 3 / 4 : window ? kCUs * 5 / 4 : 2 * kCUs;
+  const int lim = a.G == 1 ? (packed ? kCUs * 3 / 2 : a.bmask != nullptr ? (tiles < 48 ? kCUs * 3 / 4 : kCUs) : causal ? kCUs : kCUs / 2)
+                           : a.bmask != nullptr ? (tiles < 48 ? kCUs * 3 / 4 : 4 * kCUs) : packed ? 2 * kCUs : !causal ? kCUs * 3 / 4 : window ? kCUs * 5 / 4 : 2 * kCUs;
   if (wgs > lim) return false;
   if (!packed) return tiles >= std::max(16, 8 * a.G);
   const int rows = a.M / std::max(1, a.nKent - 1 - a.N / 128);   // of an average sequence (the table has an entry per 128 keys and one per sequence)
