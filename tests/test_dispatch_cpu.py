@@ -39,6 +39,12 @@ def test_the_small_form_stops_where_its_workgroups_share_cus(args, kw):
     assert dkdv_form(*args, **kw)[0] != "small"
 
 
+@pytest.mark.parametrize("args", [(1, 32, 8, 151, 614, 128, bf16, False), (2, 64, 16, 38, 149, 128, bf16, False), (3, 4, 1, 484, 1765, 128, bf16, False)])
+def test_the_small_form_stops_earlier_without_a_mask(args):
+    """D = 128, several query heads to a key head, 160 to 168 workgroups of 32 keys: 1.14 to 1.26 times the time of the other form."""
+    assert dkdv_form(*args)[0] == "keys"
+
+
 @pytest.mark.parametrize("args,kw", [
     ((1, 16, 16, 2425, 2425, 64, bf16, True), {}), ((1, 16, 16, 2021, 2021, 64, fp16, False), {}), ((2, 8, 8, 2854, 2854, 64, bf16, True), {"prefix": 100}),
     ((1, 16, 16, 2138, 2225, 64, fp16, True), {"kind": "block"}), ((1, 16, 16, 2011, 2011, 64, bf16, True), {"kind": "block"}), ((3, 16, 8, 2474, 2474, 64, bf16, False), {}),

@@ -394,12 +394,15 @@ int launch_cd(const KArgs& a, bool causal, bool doc, bool both, hipStream_t s) {
 //     (the line at two to a CU for all of them lost up to 1.4).
 //   D = 128, one workgroup to a CU, for its LDS.  One query head to a key head: kv to 64 0.91 [0.62, 1.09], to 96 0.95 [0.77, 1.06], to 128
 //     0.96 [0.60, 1.33], to 160 1.10 [0.78, 1.57].  Several, whose chains are longer, and then dq's workgroups of a group count as one:
-//     sum to 128 0.80 [0.49, 1.05], to 216 0.81 [0.55, 1.20], to 256 0.84 [0.70, 1.03], to 300 0.98 [0.65, 1.46].
-bool bwd_small(const KArgs& a, int D, bool doc) {
+//     sum to 128 0.80 [0.49, 1.05], to 216 0.81 [0.55, 1.20], to 256 0.84 [0.70, 1.03], to 300 0.98 [0.65, 1.46].  Without a mask all
+//     chains are equally long and none hides the others' second round: 8 key heads x 151 on 614 keys (160) 28 us, 32 here, 32 x 38 on
+//     149 (160) 15.5 : 19.5, 3 x 484 on 1765 (168) 59 : 67; kv to 128 0.80 [0.65, 0.93].
+bool bwd_small(const KArgs& a, int D, bool causal, bool doc) {
   if (D < 64) return false;
   const int64_t kv = dkdv_blocks(a, D, doc);
   if (D <= 64) return kv <= (a.G > 1 || (!doc && a.ktab != nullptr) ? kCUs * 3 / 2 : kCUs);
   if (a.G == 1) return kv <= 96;
+  if (!causal && !doc && a.bmask == nullptr && kv > kCUs / 2) return false;
   const int64_t dq = doc ? grid_blocks(launch_slots<GEO_DOC>(a), launch_groups<GEO_DOC>(a))
                          : geo_general(a) ? grid_blocks(launch_slots<GEO_GENERAL>(a), launch_groups<GEO_GENERAL>(a))
                                           : grid_blocks(launch_slots<GEO_PLAIN>(a), launch_groups<GEO_PLAIN>(a));

@@ -602,7 +602,7 @@ bool bwd_f32_in_one(const KArgs& a);
 int bwd_f32_shapes(const KArgs& a, bool doc);   // of dq's and dk/dv's workgroups, as FA_FORM_FP32 carries them
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 // problems that leave CUs idle (fa_bwd_small.hip): whether dk/dv takes its form there, and with dq in one launch or by itself
-bool bwd_small(const KArgs& a, int D, bool doc);
+bool bwd_small(const KArgs& a, int D, bool causal, bool doc);
 int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bool both, hipStream_t s);
 int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s);
 int launch_mask_dump(const KArgs& a, bool causal, bool doc, uint8_t* out, hipStream_t s);
