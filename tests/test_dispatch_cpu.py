@@ -64,6 +64,12 @@ def test_short_fp32_rows_are_not_cut_among_eight_waves(args, kw):
     assert form == "fp32" and dq != 0
 
 
+def test_fp32_shapes_without_a_mask_follow_the_rounds_of_workgroups():
+    """D = 128: 640 workgroups of 32 rows are three rounds of one to a CU or two of two, which take 1.9 times as long; 512 are two or one."""
+    assert dkdv_form(1, 40, 40, 490, 490, 128, f32, False) == ("fp32", 1, 1) and dkdv_form(1, 32, 32, 500, 500, 128, f32, False) == ("fp32", 2, 2)
+    assert dkdv_form(4, 1, 1, 1754, 1754, 64, f32, False)[1] is not True   # (440 workgroups of 32: two launches)
+
+
 def _kind(k):
     return k if k in ("doc", "heads", "qpos", "block") else "plain"
 

@@ -331,6 +331,7 @@ FP32_SHAPE_CASES = [
     (2, 16, 16, 330, 330, 64, True, "plain"), (2, 16, 8, 384, 400, 32, True, "window"),      # the second (of the forward the first)
     (2, 16, 16, 500, 501, 64, True, "plain"), (4, 16, 8, 545, 545, 64, True, "doc"), (1, 64, 64, 210, 270, 128, True, "prefix"),   # the second, dk/dv of the last the third
     (4, 16, 4, 530, 530, 16, False, "heads"), (2, 16, 16, 600, 333, 32, True, "qpos"), (2, 16, 16, 450, 450, 128, True, "block"),   # the second, dk/dv of the first the first
+    (1, 40, 40, 490, 490, 128, False, "plain"), (1, 32, 32, 500, 500, 128, False, "plain"),   # workgroups of equal length at D = 128: the second, the third
     (8, 32, 32, 31, 32, 64, True, "doc"), (4, 64, 64, 92, 92, 128, True, "doc"),             # short rows with ids, most of the plan's order empty: the third, the second
     (64, 64, 64, 49, 33, 16, False, "plain"), (32, 128, 64, 50, 65, 64, True, "plain"), (16, 64, 64, 257, 257, 16, True, "doc"),   # the third
     (8, 32, 32, 260, 260, 128, True, "doc"), (16, 32, 16, 130, 140, 128, True, "block"), (64, 64, 64, 63, 64, 32, True, "window"),

@@ -722,7 +722,7 @@ int launch(const KArgs& a, hipStream_t s) {
 template <int WHICH, int D> constexpr int kFewWaves = D == 128 && (WHICH == kDkdv || WHICH == kBoth) ? 4 : 8;
 inline int64_t clamped(int64_t x, int64_t lo, int64_t hi) { return x < lo ? lo : x > hi ? hi : x; }
 // 0, 1, 2: the columns of the table
-template <int WHICH, int MODE> int shape(const KArgs& a) {
+template <int WHICH, int MODE> int shape(const KArgs& a, int D, bool causal) {
   static_assert(WHICH != kBoth, "dq and dk/dv in one launch have one shape");
   constexpr bool IDS = WHICH != kDkdv && MODE == kDoc;
   const int64_t n = WHICH == kDkdv ? int64_t((a.N + kSB - 1) / kSB) * a.B * a.Hk : int64_t(((IDS ? a.Pp : a.M) + kSB - 1) / kSB) * a.B * a.H;
@@ -730,6 +730,12 @@ template <int WHICH, int MODE> int shape(const KArgs& a) {
   const int64_t chain = int64_t((std::min(other, MODE == kDoc ? other : a.win + kSB) + kSB - 1) / kSB) * (WHICH == kDkdv ? a.G : 1);
   if (IDS && chain <= 2) return 2;
   const int64_t few = WHICH == kFwd && !IDS ? 768 : clamped(16 * chain, 256, IDS ? 2048 : 768);
+  if (D == 128 && WHICH != kFwd && MODE == kPlain && !causal && n > few && chain >= 16) {
+    // Workgroups of equal length, one (the second shape) or two (the third) to a CU: whichever's rounds take less, two side by
+    // side 1.9 times as long as one (dq: 16 heads x 1810 437 : 415 us, four rounds or two; 24 x 1500 460 : 515, five or three).
+    const int64_t wgs = (n + 1) / 2, one = (wgs + kCUs - 1) / kCUs, two = (wgs + 2 * kCUs - 1) / (2 * kCUs);
+    return 19 * two < 10 * one ? 2 : 1;
+  }
   const int64_t many = WHICH == kFwd ? 16384 : IDS ? clamped(128 * chain, 2048, 16384) : clamped(64 * chain, 1024, 4096);
   return n <= few ? 0 : n < many ? 1 : 2;
 }
@@ -738,7 +744,7 @@ int launch_shape(const KArgs& a, hipStream_t s) {
   if constexpr (WHICH == kBoth) {
     return launch<WHICH, D, CAUSAL, MODE, 1, kFewWaves<WHICH, D>>(a, s);
   } else {
-    const int sh = shape<WHICH, MODE>(a);
+    const int sh = shape<WHICH, MODE>(a, D, CAUSAL);
     if (sh == 0) return launch<WHICH, D, CAUSAL, MODE, 1, kFewWaves<WHICH, D>>(a, s);
     if (sh == 1) return launch<WHICH, D, CAUSAL, MODE, 2, 4>(a, s);
     return launch<WHICH, D, CAUSAL, MODE, 2, 2>(a, s);
@@ -796,13 +802,15 @@ int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_
 
 // dq and dk/dv side by side in one launch, each forming delta itself: where the workgroups of both (32 rows or keys counted as
 // one, with ids the empty places of the plan's order too) are about as many as the CUs can hold.  2 x 4 heads x 512 rows with documents, D = 64, forward and backward: 64.9 us against
-// 69.0 with two launches.  At the line, 8 x 8 heads x 128, causal: 28.1 us against 26.2 and the gap between two launches.
+// 69.0 with two launches.  Up to three rounds of these workgroups of 16 rows, 8 heads
+// x 1024 111 us against 98 in two launches, 4 x 1754 174 : 149; 6 x 1024 (384) 88 : 96, 3 x 1500 (282) 111 : 132, 2 x 1024 (128) 36 : 54.
 bool bwd_f32_in_one(const KArgs& a) {
   const int64_t wgs = int64_t(((a.Pp > 0 ? a.Pp : a.M) + 31) / 32) * a.B * a.H + int64_t((a.N + 31) / 32) * a.B * a.Hk;
-  return wgs <= 2 * kCUs;
+  return wgs <= kCUs * 3 / 2;
 }
-int bwd_f32_shapes(const KArgs& a, bool doc) {
-  return doc ? 0x10 * shape<kDq, kDoc>(a) + 0x40 * shape<kDkdv, kDoc>(a) : 0x10 * shape<kDq, kPlain>(a) + 0x40 * shape<kDkdv, kPlain>(a);
+int bwd_f32_shapes(const KArgs& a, int D, bool causal, bool doc) {
+  auto both = [&](auto mode) { return 0x10 * shape<kDq, decltype(mode)::value>(a, D, causal) + 0x40 * shape<kDkdv, decltype(mode)::value>(a, D, causal); };
+  return doc ? both(IntC<kDoc>{}) : a.bmask != nullptr ? both(IntC<kBlock>{}) : both(IntC<kPlain>{});
 }
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kBoth>(a, D, causal, doc, s); }
 
