@@ -454,10 +454,7 @@ def test_dkdv_rows_split_over_two_waves(case):
         test_block_mask_parity((B, H, Hk, M, N, 64, dtype, causal, 0, 0.6, False))
         return
     from tests.test_gpu_parity import _run_case
-    # dk and dv add up the results of G heads, each rounded as one head's are: sqrt(G) of the bound for one
-    g = math.sqrt(H // Hk)
-    _run_case(B, H, Hk, M, N, 64, dtype, causal, False, seed=4, window=500 if kind == "window" else 0, prefix=270 if kind == "prefix" else 0,
-              ceilings={"dk": g, "dv": g})
+    _run_case(B, H, Hk, M, N, 64, dtype, causal, False, seed=4, window=500 if kind == "window" else 0, prefix=270 if kind == "prefix" else 0)
 
 
 # dk/dv by workgroups of 32 keys whose waves share the rows: blocks of rows and keys that are partly filled, heads of a group, one key, more
@@ -470,9 +467,10 @@ SMALL_BWD_CASES = [
     (1, 2, 1, 333, 77, 64, torch.float16, True, "qpos"), (1, 3, 1, 40, 800, 128, torch.bfloat16, False, "doc"),
     (2, 16, 16, 64, 700, 64, torch.bfloat16, True, "doc"), (1, 32, 16, 130, 900, 128, torch.bfloat16, True, "doc"), (1, 16, 16, 97, 800, 128, torch.float16, False, "heads"),
     (4, 16, 8, 300, 1100, 128, torch.bfloat16, True, "doc"), (8, 16, 16, 40, 801, 64, torch.float16, False, "doc"),
-    # (fp16: of four million elements of dq some lie between 2 and 4, where bf16 steps by 2^-6; half a step for the element and about as
-    # much from the roundings of O in delta and of the few large dS behind it are 0.016 and the tail of their sum passes 0.02)
-    (2, 32, 32, 520, 1033, 128, torch.float16, True, "doc"), (8, 32, 32, 33, 900, 64, torch.bfloat16, True, "doc"), (16, 16, 16, 20, 600, 128, torch.float16, True, "heads"),
+    # (bf16 at this size: of four million elements of dq some lie between 2 and 4, where bf16 steps by 2^-6; half a step for the element and
+    # about as much from the roundings of O in delta and of the few large dS behind it are 0.016, and the tail of their sum passes
+    # 0.02: 0.0201 at -2.5, the same bits as before the runs of key tiles changed.  Held to 1.05 of the bound; fp16 meets it plainly)
+    (2, 32, 32, 520, 1033, 128, torch.float16, True, "doc"), (2, 32, 32, 520, 1033, 128, torch.bfloat16, True, "doc"), (8, 32, 32, 33, 900, 64, torch.bfloat16, True, "doc"), (16, 16, 16, 20, 600, 128, torch.float16, True, "heads"),
 ]
 
 
@@ -485,7 +483,8 @@ def test_small_backward(case):
         return
     from tests.test_gpu_parity import _run_case
     _run_case(B, H, Hk, M, N, D, dtype, causal, kind in ("doc", "heads", "qpos"), seed=9, window=37 if kind == "window" else 0,
-              prefix=21 if kind == "prefix" else 0, per_head_ids=kind == "heads", qpos="random" if kind == "qpos" else None)
+              prefix=21 if kind == "prefix" else 0, per_head_ids=kind == "heads", qpos="random" if kind == "qpos" else None,
+              ceilings={"dq": 1.05} if (M, dtype) == (520, torch.bfloat16) else None)
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -532,8 +531,8 @@ def test_dkdv_rows_split_over_two_waves_packed(lens):
             x = slice(a, a + m)
             ref = O.attention_autograd(q[:, :, x], k[:, :, x], v[:, :, x], do[:, :, x], True, None, None, None, 0)[2:]
             for name, t, r in (("dq", qd, ref[0]), ("dk", kd, ref[1]), ("dv", vd, ref[2])):
-                # (dk, dv: sums over the heads of a group, each rounded by itself)
-                check_close(name, t.grad[x].transpose(0, 1)[None], r, TOL_ABS if name == "dq" else TOL_ABS * math.sqrt(H // Hk))
+                # (dk, dv: sums over the four heads of a group, each rounded by itself, up to twice one head's error; 0.98 of the plain bound measured)
+                check_close(name, t.grad[x].transpose(0, 1)[None], r, TOL_ABS if name == "dq" else 1.25 * TOL_ABS)
         a += m
 
 
@@ -611,8 +610,8 @@ def test_pipelined_dkdv(case):
     torch.cuda.synchronize()
     _, _, _, rdk, rdv = O.attention_autograd(q, k, v, do, causal, None, None, None, 0, window=window, prefix=prefix)
     # the bound of check_close is one head's: P and dS are rounded per (row, head), independently, and a sum over the G heads of a
-    # group carries sqrt(G) times that error
-    tol = TOL_ABS * math.sqrt(H // Hk)
+    # group carries up to sqrt(G) times that error (sixteen heads with a window of 100 measured 1.10 of the bound, all others less than 0.8)
+    tol = TOL_ABS * (1.25 if H // Hk >= 16 else 1.0)
     check_close("dk", dk, rdk, tol)
     check_close("dv", dv, rdv, tol)
 
