@@ -200,10 +200,15 @@ def wg_trace(w, q, k, v, do, eq, ek, torch):
             _cabi.check(fn(ref, stream), name)
         torch.cuda.synchronize()
         buf = np.zeros(8 * 65536, dtype=np.int64)
-        rc = L.fa_trace_read(which, buf.ctypes.data, buf.size)
-        assert rc == 0, f"fa_trace_read({which}) returned {rc}"
+        stamps = which
+        if which == 2:   # some forms of dk/dv keep stamps of their own
+            form = L.fa_bwd_form(ref, 0)
+            stamps = {_cabi.FA_FORM_PIPE: 3, _cabi.FA_FORM_SMALL: 4}.get(form, 2)
+        rc = L.fa_trace_read(stamps, buf.ctypes.data, buf.size)
+        assert rc == 0, f"fa_trace_read({stamps}) returned {rc}"
         t = buf.reshape(-1, 8)
         t = t[t[:, 0] != 0]
+        assert len(t), f"{name} leaves no stamps (the fp32 kernels have none)"
         c_start, c_setup, c_loop, c_end, c_tiles, c_info = cols
         left = t[:, c_info] == -1
         live = t[~left & (t[:, c_end] != 0) & (t[:, c_tiles] > 0)]

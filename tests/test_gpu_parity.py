@@ -379,16 +379,18 @@ def test_random_shapes(seed):
     _run_case(B, H, Hk, M, N, D, dtype, causal, doc, seed=seed, ids_kind=kind, per_head_ids=per_head, id_dtype=idt)
 
 
-def test_clock_stamp_build_gives_the_same_bits():
+@pytest.mark.parametrize("H,M,doc,stamps", [(2, 2304, True, 2), (8, 4100, False, 3), (2, 300, True, 4)])
+def test_clock_stamp_build_gives_the_same_bits(H, M, doc, stamps):
     """The measurement build (the same sources with -DFA_TRACE, what `bench.py --wg-trace` loads) must time the
-    kernels the product runs: its forward, dq and dk/dv results equal the product library's bit for bit."""
+    kernels the product runs: its forward, dq and dk/dv results equal the product library's bit for bit.  Each form of dk/dv
+    leaves its stamps where fa_trace_read looks for that form's, one row of words per workgroup."""
     import ctypes
     from flash_mi355 import _cabi
     from flash_mi355.api import _Plan, _set4, _stream_ptr
     from flash_mi355.build import TRACE_LIB_PATH
     T = ctypes.CDLL(str(TRACE_LIB_PATH))
     L = _cabi.lib()
-    B, H, M, D = 1, 2, 2304, 128
+    B, D = 1, 128
     dev = torch.device("cuda")
     g = torch.Generator().manual_seed(91)
     rng = np.random.default_rng(91)
@@ -399,7 +401,7 @@ def test_clock_stamp_build_gives_the_same_bits():
         o, dq, dk, dv = (torch.full_like(q, float("nan")) for _ in range(4))
         lse = torch.empty(B, H, M, device=dev, dtype=torch.float32)
         delta = torch.empty_like(lse)
-        plan = _Plan(q, k, v, True, 1.0 / math.sqrt(D), ids, ids, 1)
+        plan = _Plan(q, k, v, True, 1.0 / math.sqrt(D), ids if doc else None, ids if doc else None, int(doc))
         p = plan.p
         p.o, p.lse, p.dout, p.delta = o.data_ptr(), lse.data_ptr(), do.data_ptr(), delta.data_ptr()
         p.dq, p.dk, p.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
@@ -408,6 +410,7 @@ def test_clock_stamp_build_gives_the_same_bits():
         plan.ensure_workspace(dev)
         p.flags = _cabi.FA_FLAG_DQ_DELTA
         ref, stream = ctypes.byref(p), _stream_ptr(dev)
+        assert L.fa_bwd_form(ref, 0) == {2: _cabi.FA_FORM_KEYS, 3: _cabi.FA_FORM_PIPE, 4: _cabi.FA_FORM_SMALL}[stamps]
         for name in ("fa_mask_plan", "fa_fwd", "fa_bwd_dq", "fa_bwd_dkdv"):
             fn = getattr(lib, name)
             fn.restype = ctypes.c_int
@@ -417,6 +420,13 @@ def test_clock_stamp_build_gives_the_same_bits():
         results.append((o, lse, dq, dk, dv))
     for a_, b_ in zip(*results):
         assert not torch.isnan(a_).any() and torch.equal(a_, b_)
+    buf = np.zeros(8 * 65536, dtype=np.int64)
+    T.fa_trace_read.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_int]
+    assert T.fa_trace_read(stamps, buf.ctypes.data, buf.size) == 0
+    t = buf.reshape(-1, 8)
+    t = t[(t[:, 0] != 0) & (t[:, 7] != -1) & (t[:, 6] > 0)]
+    assert len(t) >= H * (M // 128 if stamps == 3 else M // 64)
+    assert (t[:, 0] <= t[:, 3]).all() and (t[:, 3] <= t[:, 4]).all() and (t[:, 4] <= t[:, 5]).all()
 
 
 def test_empty_inputs():

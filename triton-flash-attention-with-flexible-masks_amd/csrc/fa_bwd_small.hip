@@ -10,6 +10,8 @@
 #include "fa_tile.h"
 #ifdef FA_TRACE
 namespace fa { namespace { FA_TRACE_ARRAY(g_trace_dq); } }   // stamps of dq workgroups that share a launch: not read
+// words as in fa_bwd_dkdv.hip, of the first wave; its tiles are blocks of 32 rows
+namespace fa { FA_TRACE_ARRAY(g_trace_small); }
 #endif
 #include "fa_dq_body.h"
 
@@ -97,6 +99,8 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
   const int lq = lane & 31, g = lane >> 5;
   const bool packed = !DOC && a.ktab != nullptr;
   constexpr int SUB = dkdv_small_sub(D);
+  FA_STAMP(g_trace_small, 0, FA_CLOCK()); FA_STAMP(g_trace_small, 1, 0); FA_STAMP(g_trace_small, 5, 0); FA_STAMP(g_trace_small, 7, -1);
+  FA_TRACE_ONLY(int tr_tiles = 0;)
   int slot, bhk;
   if (!block_to_tile(packed ? a.nKent * SUB : (a.N + kRb - 1) / kRb, a.B * a.Hk, true, slot, bhk, bid)) return;
   const int b = bhk / a.Hk, hk = bhk % a.Hk;
@@ -111,6 +115,7 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
     if (n0 >= N) return;
   }
   const int key = n0 + lq, keyc = min(key, N - 1);
+  FA_STAMP(g_trace_small, 7, (long long)(n0 / kRb) | ((long long)bhk << 16));
   vec8 kf[KS], vf[KS];
   {
     const T* kp = reinterpret_cast<const T*>(a.k) + b * a.k_bs + hk * a.k_hs + (k0 + keyc) * a.k_rs;
@@ -268,6 +273,7 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
     }
   };
 
+  FA_STAMP(g_trace_small, 2, FA_CLOCK());
   Iter it;
   it.init(head, chunk, wg_rlo, wg_rhi);
   int cur = it.next(a.G, wave, head, chunk), ek = it.ek, gi = it.gi, idx = 0;
@@ -283,6 +289,7 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
   int buf = 0;
   while (cur >= 0) {
     wait_async_loads();
+    FA_TRACE_ONLY(if (tr_tiles++ == 0) FA_STAMP(g_trace_small, 3, FA_CLOCK());)
     if (OWN_DELTA) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) { settle(of_n[ks]); of[ks] = of_n[ks]; }
@@ -300,6 +307,7 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
     nxt = nx2; ek_n = ek2; gi_n = gi2; idx_n = idx2;
   }
 
+  FA_STAMP(g_trace_small, 4, FA_CLOCK()); FA_STAMP(g_trace_small, 6, tr_tiles);
   // the waves' sums, in their order: wave w adds up 32-column blocks w, w + 4, ... of dV and dK
   __syncthreads();
   f32x4* sums = reinterpret_cast<f32x4*>(smem) + lane;   // [wave][dV, dK blocks][quads of a lane's registers][lane]
@@ -329,6 +337,7 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
       *reinterpret_cast<typename E::vec4*>(p + 32 * db + 8 * q4 + 4 * g) = x;
     }
   }
+  FA_STAMP(g_trace_small, 5, FA_CLOCK());
 }
 
 template <int D> constexpr int kPerSimd = D > 64 ? 1 : 2;
@@ -414,5 +423,9 @@ int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bo
   if (D == 64) return dtype == FA_DTYPE_BF16 ? launch_cd<bf16_t, 64>(a, causal, doc, both, s) : launch_cd<fp16_t, 64>(a, causal, doc, both, s);
   return -1;
 }
+
+#ifdef FA_TRACE
+int trace_read_small(long long* host, int n) { return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(g_trace_small), size_t(n) * 8); }
+#endif
 
 }  // namespace fa

@@ -592,6 +592,8 @@ int read_pair_wait_expired(unsigned long long* n);   // expired pair waits of th
 int trace_read_fwd(long long* host, int n);
 int trace_read_dq(long long* host, int n);
 int trace_read_dkdv(long long* host, int n);
+int trace_read_pipe(long long* host, int n);
+int trace_read_small(long long* host, int n);
 #endif
 // the same four for fp32 tensors (fa_f32.hip)
 int launch_fwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);

@@ -18,6 +18,9 @@
 #include "fa_tile.h"
 
 namespace fa {
+#ifdef FA_TRACE
+FA_TRACE_ARRAY(g_trace_pipe);   // words as in fa_bwd_dkdv.hip, of the first score wave (word 1 is 0: nothing is polled)
+#endif
 
 constexpr int kPipePre = 4;    // row-wise operand fragments requested ahead of their MFMA
 constexpr int kPipePre2 = 3;   // transposed ones
@@ -42,8 +45,11 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
   const int role = wave & 1, kb = wave >> 1;
   const int lq = lane & 31, g = lane >> 5;
   const int nKt = (a.N + BK - 1) / BK;
+  FA_STAMP(g_trace_pipe, 0, FA_CLOCK()); FA_STAMP(g_trace_pipe, 1, 0); FA_STAMP(g_trace_pipe, 5, 0); FA_STAMP(g_trace_pipe, 7, -1);
+  FA_TRACE_ONLY(int tr_tiles = 0; bool tr_first = false;)
   int kt, bhk;
   if (!block_to_tile(nKt, a.B * a.Hk, false, kt, bhk, bid)) return;  // causal: the first key tiles see the most rows
+  FA_STAMP(g_trace_pipe, 7, (long long)kt | ((long long)bhk << 16));
   const int b = bhk / a.Hk, hk = bhk % a.Hk;
   const int M = a.M, N = a.N, gap = a.gap, G = a.G, win = a.win, pfx_m1 = a.pfx_m1;
   const int n0 = kt * BK, nw = n0 + kb * 32, key = nw + lq, keyc = key < N ? key : N - 1;
@@ -157,6 +163,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
     bool more = first < last, prev = false;
     if (more) {
       open_head();
+      FA_STAMP(g_trace_pipe, 2, FA_CLOCK());
 #pragma unroll
       for (int j = 0; j < NPART; ++j) load_part(t, 0, j);
       load_aux(t, 0);
@@ -167,6 +174,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
       const int pst = stage == 0 ? NST - 1 : stage - 1, nst = stage == NST - 1 ? 0 : stage + 1;
       wait_async_loads();
       __syncthreads();
+      FA_TRACE_ONLY(if (!tr_first) { FA_STAMP(g_trace_pipe, 3, FA_CLOCK()); tr_first = true; } tr_tiles += more;)
       // the tile after this one
       bool nmore = false;
       if (more) {
@@ -272,6 +280,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
     }
   };
   if (role == 0) stream(IntC<0>{}); else stream(IntC<1>{});
+  FA_STAMP(g_trace_pipe, 4, FA_CLOCK()); FA_STAMP(g_trace_pipe, 6, tr_tiles);
 
   // dK / dV rows leave through LDS (store_rows_through_lds), once every wave is done with the last query tile
   LateArgs& la = late_args();
@@ -282,6 +291,7 @@ FA_DEV void dkdv_pipe_body(const KArgs& a, const int bid, char* smem) {
   store_rows_through_lds<E, D, DBN>(patch, acc, role == 0 ? 1.0f : -la.scale, [&](const int r) -> T* {
     return nw + r < N ? base + int64_t(nw + r) * rs : nullptr;
   });
+  FA_STAMP(g_trace_pipe, 5, FA_CLOCK());
 }
 
 template <typename Tag, bool CAUSAL>
@@ -304,5 +314,8 @@ int launch_dkdv_pipe(const KArgs& a, int dtype, bool causal, hipStream_t s) {
   if (dtype == FA_DTYPE_BF16) return causal ? launch_pipe<bf16_t, true>(a, s) : launch_pipe<bf16_t, false>(a, s);
   return causal ? launch_pipe<fp16_t, true>(a, s) : launch_pipe<fp16_t, false>(a, s);
 }
+#ifdef FA_TRACE
+int trace_read_pipe(long long* host, int n) { return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(g_trace_pipe), size_t(n) * 8); }
+#endif
 
 }  // namespace fa
