@@ -106,7 +106,8 @@ extern "C" {
                                has used a P it cannot trust and REPORTS it by writing NaN into its 32 rows of dk
                                (dv is not affected).  A NaN in dk after a backward with finite inputs therefore
                                means "a pair wait expired", not an arithmetic overflow.  With this flag the poll
-                               budget is zero, so the report can be provoked without hanging or faulting anything.
+                               budget is zero, so the report can be provoked without hanging or faulting anything (and
+                               small problems, which take a form without pairs otherwise, take this one).
                                Accepted by fa_bwd_dkdv only; every other entry point refuses it (FA_ERR_MODE).
                                Every expiry is also counted, see fa_pair_wait_expired. */
 

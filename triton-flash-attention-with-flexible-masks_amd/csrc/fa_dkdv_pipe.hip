@@ -9,8 +9,8 @@
 // Neither waits for what the other does in the same step (P crosses behind the barrier of the tile stream: no flag, no polling),
 // and the stream goes on through the query heads of a group without draining.
 //
-// What bounds it: the power limit.  On random operands the clock settles at 1.9 GHz with the matrix pipes 48 % busy (3 stages x
-// 32 KB, 32 KB of P: one workgroup to a CU); on zeros the same launch takes 3.4 ms instead of 4.2.  Causal, 32 heads x 16384
+// What bounds it: the power limit first.  On random operands the clock settles at 2.10 GHz with the matrix pipes 51 % busy (counters,
+// causal, 32 heads x 16384 rows; 3 stages x 32 KB, 32 KB of P: one workgroup to a CU); on zeros the same launch takes 3.4 ms instead of 4.2.  Causal, 32 heads x 16384
 // rows, against the form in which the gradient wave polls for the P of its own tile: 4.51 -> 4.26, 4.42 -> 4.20, 4.84 -> 4.60 ms
 // on three cards; with the subtraction of delta in the accumulators (see fa_bwd_dkdv.hip) another 4.20 -> 3.95.
 // Steps of 32 rows (four stages) in workgroups of 128 or 64 keys: 4.60 ms against 4.26, and slower than the polling form with 64
