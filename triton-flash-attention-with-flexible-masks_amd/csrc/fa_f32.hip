@@ -736,7 +736,7 @@ template <int WHICH, int MODE> int shape(const KArgs& a, int D, bool causal) {
     const int64_t wgs = (n + 1) / 2, one = (wgs + kCUs - 1) / kCUs, two = (wgs + 2 * kCUs - 1) / (2 * kCUs);
     return 19 * two < 10 * one ? 2 : 1;
   }
-  const int64_t many = WHICH == kFwd ? 16384 : IDS ? clamped(128 * chain, 2048, 16384) : clamped(64 * chain, 1024, 4096);
+  const int64_t many = WHICH == kFwd ? (IDS && chain <= 6 ? 4096 : 16384) : IDS ? clamped(128 * chain, 2048, 16384) : clamped(64 * chain, 1024, 4096);
   return n <= few ? 0 : n < many ? 1 : 2;
 }
 template <int WHICH, int D, bool CAUSAL, int MODE>
