@@ -271,6 +271,10 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
       dv[i % DBN] = E::mfma32(dt[i], pf[i / DBN], dv[i % DBN]);
       dk[i % DBN] = E::mfma32(qt[i], sf[i / DBN], dk[i % DBN]);
     }
+    // Every read of this block ends up in a product above, so its wait stands above this line, and the loads that fill the buffer
+    // again stand below it.  (A wait of its own there, or behind the reads, cost 3 - 14 % of a long chain through the schedule
+    // around it.)
+    __builtin_amdgcn_sched_barrier(0);
   };
 
   FA_STAMP(g_trace_small, 2, FA_CLOCK());
@@ -296,7 +300,6 @@ FA_DEV void dkdv_small_body(const KArgs& a, const int bid, char* smem) {
     }
     int nx2 = -1, ek2 = 0, gi2 = 0, idx2 = 0;
     if (nxt >= 0) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads of the block before are done: its buffer is filled again
       load(nxt, gi_n, idx_n, mine + (buf ^ 1) * stage_bytes<D>());
       nx2 = it.next(a.G, wave, head, chunk); ek2 = it.ek; gi2 = it.gi;
       if (DOC && nx2 >= 0) idx2 = place(nx2, gi2);
