@@ -47,11 +47,20 @@ def test_the_small_form_stops_earlier_without_a_mask(args):
 
 @pytest.mark.parametrize("args,kw", [
     ((1, 16, 16, 2425, 2425, 64, bf16, True), {}), ((1, 16, 16, 2021, 2021, 64, fp16, False), {}), ((2, 8, 8, 2854, 2854, 64, bf16, True), {"prefix": 100}),
-    ((1, 16, 16, 2138, 2225, 64, fp16, True), {"kind": "block"}), ((1, 16, 16, 2011, 2011, 64, bf16, True), {"kind": "block"}), ((3, 16, 8, 2474, 2474, 64, bf16, False), {}),
+    ((1, 16, 16, 2138, 2225, 64, fp16, True), {"kind": "block"}), ((3, 16, 8, 2474, 2474, 64, bf16, False), {}),
 ])
 def test_rows_are_shared_only_where_cus_are_free(args, kw):
     """D = 64, 256 to 480 workgroups of 128 keys: 1.05 to 1.28 times the time of the form whose waves own their keys."""
     assert dkdv_form(*args, **kw)[0] == "keys"
+
+
+@pytest.mark.parametrize("args,kw", [
+    ((1, 16, 16, 2500, 2500, 64, bf16, False), {}), ((1, 6, 6, 6400, 6400, 64, bf16, True), {}), ((2, 64, 8, 3000, 3000, 64, fp16, True), {"window": 900}),
+    ((1, 16, 16, 2011, 2011, 64, bf16, True), {"kind": "block"}), ((1, 64, 8, 1302, 5000, 64, bf16, True), {"kind": "block"}),
+])
+def test_long_chains_share_their_rows_beyond_a_workgroup_to_a_cu(args, kw):
+    """... up to 512 workgroups (1024 with a block map), where every one of them walks many tiles."""
+    assert dkdv_form(*args, **kw)[0] == "rows"
 
 
 @pytest.mark.parametrize("args,kw", [

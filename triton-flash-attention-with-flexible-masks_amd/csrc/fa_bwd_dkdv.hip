@@ -819,13 +819,16 @@ constexpr size_t dkdv_lds() { return 4 * 64 * (D < 32 ? 32 : D) * 2 + 2 * 1024 +
 // workgroups, 8 tiles) 37 -> 43 us, a window of 67 keys (160, 4) 16 -> 19.  With ids the tiles are not known here.
 static bool rows_form(const KArgs& a, int D, bool causal, bool doc) {
   if (D != 64 || doc) return false;
-  const bool packed = a.ktab != nullptr, window = causal && a.win < 0x3fffffff;
+  const bool packed = a.ktab != nullptr, block = a.bmask != nullptr;
   const int64_t wgs = int64_t(packed ? a.nKent : (a.N + 127) / 128) * a.B * a.Hk;
-  const int tiles = dkdv_tiles(a, causal);   // (a sequence's are not known)
-  const int lim = a.G == 1 ? (packed ? kCUs * 3 / 2 : a.bmask != nullptr ? (tiles < 48 ? kCUs * 3 / 4 : kCUs) : causal ? kCUs : kCUs / 2)
-                           : a.bmask != nullptr ? (tiles < 48 ? kCUs * 3 / 4 : 4 * kCUs) : packed ? 2 * kCUs : !causal ? kCUs * 3 / 4 : window ? kCUs * 5 / 4 : 2 * kCUs;
-  if (wgs > lim) return false;
-  if (!packed) return tiles >= std::max(16, 8 * a.G);
+  if (wgs > (block ? 4 : 2) * kCUs) return false;
+  if (!packed) {
+    const int tiles = dkdv_tiles(a, causal);
+    if (tiles < std::max(16, 8 * a.G)) return false;
+    if (block) return a.G > 1 || tiles >= 48 || wgs <= kCUs;
+    if (!causal) return wgs <= kCUs * 3 / 2 && (a.G > 1 || tiles >= 48 || wgs <= kCUs / 2 || wgs > kCUs);
+    return a.G > 1 || tiles >= 48 || wgs <= kCUs * 9 / 8;
+  }
   const int rows = a.M / std::max(1, a.nKent - 1 - a.N / 128);   // of an average sequence (the table has an entry per 128 keys and one per sequence)
   return (rows / 64 + 1) * a.G >= (causal ? 16 : 8);
 }
