@@ -434,8 +434,8 @@ def test_backward_in_one_launch(case):
 # B, H, Hk, M, N, dtype, causal, kind
 ROWS_CASES = [
     (2, 32, 8, 1100, 1100, torch.bfloat16, True, "plain"), (2, 32, 8, 1100, 1090, torch.float16, False, "plain"), (2, 32, 8, 1100, 1100, torch.float16, True, "prefix"),
-    (4, 16, 4, 777, 900, torch.bfloat16, True, "window"), (4, 32, 8, 1100, 1100, torch.bfloat16, True, "window"), (2, 32, 8, 1100, 1100, torch.bfloat16, True, "block"),
-    (2, 8, 8, 1999, 2030, torch.bfloat16, True, "plain"), (1, 8, 8, 1999, 1900, torch.bfloat16, False, "plain"),
+    (4, 16, 4, 1100, 1111, torch.bfloat16, True, "window"), (4, 32, 8, 1100, 1100, torch.bfloat16, True, "window"), (2, 32, 8, 1100, 1100, torch.bfloat16, True, "block"),
+    (2, 8, 8, 1999, 2030, torch.bfloat16, True, "plain"), (1, 10, 10, 3100, 1900, torch.bfloat16, False, "plain"),
     (2, 128, 8, 1100, 1090, torch.float16, False, "plain"),
 ]
 # Sizes that stay with the form whose waves own their keys: short chains, or too many workgroups.
@@ -538,7 +538,7 @@ def test_dkdv_rows_split_over_two_waves_packed(lens):
 
 # A row of [B, L, H, D], or of a cache with room behind it, is read and written as one of [B, H, L, D]: the same bits, in every form of the backward.
 # B, H, Hk, M, N, D, causal, kind
-LAYOUT_CASES = [(1, 32, 32, 4100, 4100, 128, True, "pipe"), (2, 32, 8, 1100, 1100, 64, True, "rows"), (1, 8, 8, 1088, 1088, 128, True, "keys"), (2, 8, 8, 700, 700, 64, True, "keys"),
+LAYOUT_CASES = [(1, 32, 32, 4100, 4100, 128, True, "pipe"), (2, 32, 8, 1100, 1100, 64, True, "rows"), (1, 8, 8, 1088, 1088, 128, True, "keys"), (3, 8, 8, 700, 700, 64, True, "keys"),
                 (2, 4, 2, 333, 400, 128, True, "small"), (2, 4, 2, 333, 400, 64, False, "small")]
 
 

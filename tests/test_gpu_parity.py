@@ -108,7 +108,7 @@ def _run_case(B, H, Hk, M, N, D, dtype, causal, doc, seed, ids_kind="uniform", p
 # own their keys (D = 64).  The lists below have such cases for every mask; test_dispatch_cpu.py holds them there.
 KEYS_CASES = [
     (1, 8, 8, 1100, 1100, 128, torch.bfloat16, False, False), (1, 8, 8, 1100, 1100, 128, torch.bfloat16, True, False), (2, 16, 4, 700, 790, 128, torch.float16, True, False),
-    (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, True), (2, 8, 8, 545, 545, 64, torch.bfloat16, True, True), (2, 8, 8, 700, 705, 64, torch.float16, True, False),
+    (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, True), (4, 8, 8, 545, 545, 64, torch.bfloat16, True, True), (3, 8, 8, 700, 705, 64, torch.float16, True, False),
 ]
 CASES = [
     # B, H, Hk, M, N, D, dtype, causal, doc
@@ -191,7 +191,7 @@ def test_mask_bit_exact():
 
 KEYS_BLOCK_CASES = [
     (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, 0, 0.4, False), (2, 16, 4, 1000, 1130, 128, torch.float16, False, 0, 0.5, True),
-    (1, 8, 8, 1100, 1100, 128, torch.bfloat16, True, 400, 0.6, False), (2, 8, 8, 700, 700, 64, torch.bfloat16, True, 0, 0.5, False),
+    (1, 8, 8, 1100, 1100, 128, torch.bfloat16, True, 400, 0.6, False), (3, 8, 8, 700, 700, 64, torch.bfloat16, True, 0, 0.5, False),
 ]
 BLOCK_CASES = [
     # B, H, Hk, M, N, D, dtype, causal, window, density, broadcast (block map shared by batch and heads)
@@ -846,7 +846,7 @@ def test_varlen_takes_boundaries_from_the_host_and_needs_key_boundaries_for_othe
 
 COLS_BIG_CASES = [   # (enough workgroups for the column form at D >= 64; the other cases at these D may take the form for few)
     (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "uniform", 0), (1, 16, 8, 300, 1700, 128, torch.float16, True, "uniform", 0), (1, 8, 8, 900, 2100, 128, torch.bfloat16, True, "uniform", 0),
-    (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "alllocal", 0), (1, 8, 8, 300, 1501, 64, torch.float16, True, "uniform", 0),
+    (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "alllocal", 0), (2, 8, 8, 300, 1501, 64, torch.float16, True, "uniform", 0),
     (1, 8, 8, 300, 1500, 128, torch.bfloat16, True, "uniform", 700), (1, 8, 8, 300, 1500, 128, torch.bfloat16, False, "uniform", 0),
 ]
 COLS_CASES = [
@@ -1010,7 +1010,7 @@ def test_fp32_all_global_and_all_local_ids():
 KEYS_BAND_CASES = [
     (1, 8, 8, 1088, 1088, 128, torch.bfloat16, False, 300, 0), (1, 8, 8, 1000, 1500, 128, torch.float16, False, 500, 0), (2, 16, 4, 800, 800, 128, torch.bfloat16, False, 65, 0),
     (1, 8, 8, 1088, 1088, 128, torch.bfloat16, False, 0, 300), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, 300, 0), (1, 8, 8, 1088, 1088, 128, torch.bfloat16, True, 0, 300),
-    (2, 8, 8, 700, 700, 64, torch.bfloat16, True, 100, 0), (2, 8, 8, 700, 700, 64, torch.bfloat16, False, 100, 0), (2, 8, 8, 700, 700, 64, torch.float16, False, 0, 200),
+    (3, 8, 8, 700, 700, 64, torch.bfloat16, True, 100, 0), (3, 8, 8, 700, 700, 64, torch.bfloat16, False, 100, 0), (3, 8, 8, 700, 700, 64, torch.float16, False, 0, 200),
 ]
 BAND_CASES = [
     # B, H, Hk, M, N, D, dtype, doc, window, prefix

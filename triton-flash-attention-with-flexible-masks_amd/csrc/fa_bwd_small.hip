@@ -396,25 +396,38 @@ int launch_cd(const KArgs& a, bool causal, bool doc, bool both, hipStream_t s) {
 
 }  // namespace
 
-// Which problems: by the workgroups of 32 keys that they have (kv; packed sequences: as many as the plan's table holds).  The
-// whole backward in this form : in the next best one, geometric mean over random problems with all masks [smallest, largest]:
-//   D = 64, two workgroups to a CU    kv up to 128            to 192            to 256            to 320            to 384
-//     one query head to a key head    0.79 [0.68, 1.03]  0.88 [0.71, 1.07]  0.94 [0.59, 1.09]  1.04 [0.86, 1.33]  1.16 [0.90, 1.71]
-//     several                         0.74 [0.48, 0.96]  0.82 [0.49, 1.02]  0.86 [0.67, 1.13]  0.95 [0.53, 1.31]  1.01 [0.77, 1.47]
-//     packed sequences                0.75 [0.57, 0.98]  0.81 [0.55, 0.96]  0.84 [0.63, 1.00]  0.81 [0.65, 0.97]  0.90 [0.83, 1.08]
-//     With more, the workgroups share CUs and the longer chains of the other forms cost less than the rows that are read again
-//     (the line at two to a CU for all of them lost up to 1.4).
+// Which problems: by the workgroups of 32 keys that they have (kv; packed sequences: as many as the plan's table holds) and by the
+// blocks of 32 rows that one of them walks, over the heads of a group (half of them under a causal mask): its chain.  The whole
+// backward in this form : in the others, geometric mean over random problems [smallest, largest]:
+//   D = 64, two workgroups to a CU.  Up to one to a CU: 0.79 [0.68, 1.03] to kv 128, 0.88 [0.71, 1.07] to 192, 0.94 [0.59, 1.09] to 256.
+//     Beyond, short chains lose what the four waves add up at their end and what a second workgroup on the CU costs
+//       chain                      to 4               to 8               to 12              to 16              to 24
+//       causal, kv 320 - 384  1.07 [1.01, 1.24]  1.00 [0.80, 1.15]  0.84 [0.76, 1.12]  0.78 [0.63, 0.94]  0.73 [0.64, 0.83]
+//       kv 384 - 448          1.05 [1.03, 1.07]  1.20 [0.93, 1.54]  1.02 [0.95, 1.20]  0.93 [0.81, 1.19]  0.80 [0.73, 0.87]
+//       kv 448 - 512          1.28 [1.05, 1.39]  1.17 [0.98, 1.50]  1.04 [1.00, 1.18]  0.95 [0.85, 1.07]  0.92 [0.80, 1.11]
+//     (windows and block maps alike); without a mask, kv 352 - 512, 1.1 [0.92, 1.50] up to 32 blocks and 0.93 beyond; with the same ids on both
+//     sides 1.13 [1.01, 1.40] from kv 384 and up to 1.43 below for few rows, but 0.90 where the column form is the other one; packed
+//     sequences 0.81 [0.61, 1.27] throughout.
 //   D = 128, one workgroup to a CU, for its LDS.  One query head to a key head: kv to 64 0.91 [0.62, 1.09], to 96 0.95 [0.77, 1.06], to 128
 //     0.96 [0.60, 1.33], to 160 1.10 [0.78, 1.57].  Several, whose chains are longer, and then dq's workgroups of a group count as one:
 //     sum to 128 0.80 [0.49, 1.05], to 216 0.81 [0.55, 1.20], to 256 0.84 [0.70, 1.03], to 300 0.98 [0.65, 1.46].  Without a mask all
-//     chains are equally long and none hides the others' second round: 8 key heads x 151 on 614 keys (160) 28 us, 32 here, 32 x 38 on
-//     149 (160) 15.5 : 19.5, 3 x 484 on 1765 (168) 59 : 67; kv to 128 0.80 [0.65, 0.93].
+//     chains are equally long, and short ones do not make up for the second round of the workgroups that exceed the CUs: 8 key heads x 151
+//     rows on 614 keys (kv 160, chain 20) 27 us in the others, 32 here, 32 x 38 on 149 (160, 8) 15.5 : 19.5; 4 x 64/8 x 147 (160, 40) 48.7 : 40.4.
 bool bwd_small(const KArgs& a, int D, bool causal, bool doc) {
   if (D < 64) return false;
   const int64_t kv = dkdv_blocks(a, D, doc);
-  if (D <= 64) return kv <= (a.G > 1 || (!doc && a.ktab != nullptr) ? kCUs * 3 / 2 : kCUs);
+  const bool packed = !doc && a.ktab != nullptr, full = !causal && !doc && a.bmask == nullptr;
+  int chain = (a.M + kRb - 1) / kRb;
+  if (causal && !doc) chain = a.win < 0x3fffffff ? std::min(chain, a.win / kRb + 3) : (chain + 1) / 2;
+  const int64_t walked = int64_t(chain) * a.G;
+  if (D <= 64) {
+    if (kv > 2 * kCUs) return false;
+    if (kv <= kCUs || packed) return true;
+    if (doc) return !causal || a.qpos != nullptr || a.gap >= 128 || (kv <= kCUs * 3 / 2 && a.M > 150);   // (the first ones: next to the column form otherwise)
+    return full ? kv <= 352 || walked > 32 : 16 * walked >= kv - 320;
+  }
   if (a.G == 1) return kv <= 96;
-  if (!causal && !doc && a.bmask == nullptr && kv > kCUs / 2) return false;
+  if (full && !packed && kv > kCUs / 2 && walked <= 24) return false;
   const int64_t dq = doc ? grid_blocks(launch_slots<GEO_DOC>(a), launch_groups<GEO_DOC>(a))
                          : geo_general(a) ? grid_blocks(launch_slots<GEO_GENERAL>(a), launch_groups<GEO_GENERAL>(a))
                                           : grid_blocks(launch_slots<GEO_PLAIN>(a), launch_groups<GEO_PLAIN>(a));
