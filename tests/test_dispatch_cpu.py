@@ -87,6 +87,12 @@ def test_fp32_shapes_without_a_mask_follow_the_rounds_of_workgroups():
     assert dkdv_form(4, 1, 1, 1754, 1754, 64, f32, False)[1] is not True   # (440 workgroups of 32: two launches)
 
 
+def test_fp32_backward_in_one_launch_up_to_two_workgroups_to_a_cu():
+    """... under a causal mask, and without one where the chains are short; padded places of ids count against eight to a CU."""
+    assert dkdv_form(8, 8, 8, 128, 128, 64, f32, True) == ("fp32", True) and dkdv_form(4, 8, 8, 250, 250, 64, f32, False) == ("fp32", True)
+    assert dkdv_form(8, 8, 8, 129, 129, 64, f32, True)[1] is not True and dkdv_form(8, 32, 32, 29, 29, 64, f32, True, kind="doc")[1] is not True
+
+
 def _kind(k):
     return k if k in ("doc", "heads", "qpos", "block") else "plain"
 

@@ -696,8 +696,7 @@ int launch(const KArgs& a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Which of three shapes a launch takes, by the blocks of 16 rows (keys) that it has -- with ids those of the plan's padded order,
-// whose empty ones cost a workgroup each -- and by the blocks of the other side that one of them walks, its chain.  us (forward, dq, dk/dv):
+// Which of three shapes a launch takes, by the blocks of 16 rows (keys) that it has.  us (forward, dq, dk/dv):
 //                                          RB 1, SW 8 *       RB 2, SW 4         RB 2, SW 2
 //   D = 64  2 x 4 heads x 1024, causal (512)    22.6 35.6 37.2     28.2 36.9 46.1     48.9 63.5 79.8
 //           2 x 4 x 2048, documents  (1024)     33.6 43.4 54.6     61.1 79.0 46.2     108 140 60
@@ -714,30 +713,38 @@ int launch(const KArgs& a, hipStream_t s) {
 //           8 x 16 x 2048, causal    (16384)    1749 2763 3556     1232 2199 2728     1187 2008 2540
 //   * dk/dv at D = 128: SW 4, since one wave to a SIMD is all that its registers allow
 // Few blocks: the chain of one of them counts, so all waves share it.  Many: the work counts, and a block of 32 reads the
-// other side half as often; then also what a workgroup adds up at its end -- the more, the shorter the chain.  (Rows with ids:
-// the global ones among them walk all keys, the others a few blocks: the chain counts longer.)  Over 2000 random problems the
-// launches take 1.03, 1.03 and 1.02 times the best shape's time on average; with lines at fixed numbers of blocks (768 and 4096,
-// with ids 2048 and 16384, padding not counted) 1.06, 1.11 and 1.05, and many short rows with ids up to 2.5 times what they
-// took with tiles in LDS (8 x 32 heads x 32: dq 10.6 -> 26.6; 4 x 64 x 92, D = 128: forward 30 -> 59).
+// other side half as often; then also what a workgroup adds up at its end.  (Rows with ids: the global ones among them walk
+// all keys, the others a few blocks: the chain counts longer.)  Where a block walks few blocks of the other side, its chain, what a
+// workgroup adds up at its end counts earlier, and with ids every empty place of the plan's order costs a workgroup: exceptions below.
+// Many short rows without them, against tiles in LDS as before these kernels: 8 x 32 heads x 32 with ids, dq 10.6 -> 26.6; 4 x 64 x 92,
+// D = 128, with ids, forward 30 -> 59 (27 now); 2 x 64 x 209, D = 128, no mask, dk/dv 83 -> 108.  Of the launches of 2000 random problems 151
+// were slower than before these kernels without the exceptions, 50 with them, and 5 are slower than without (up to 1.16, launches of 10 us).
 template <int WHICH, int D> constexpr int kFewWaves = D == 128 && (WHICH == kDkdv || WHICH == kBoth) ? 4 : 8;
-inline int64_t clamped(int64_t x, int64_t lo, int64_t hi) { return x < lo ? lo : x > hi ? hi : x; }
 // 0, 1, 2: the columns of the table
 template <int WHICH, int MODE> int shape(const KArgs& a, int D, bool causal) {
   static_assert(WHICH != kBoth, "dq and dk/dv in one launch have one shape");
   constexpr bool IDS = WHICH != kDkdv && MODE == kDoc;
-  const int64_t n = WHICH == kDkdv ? int64_t((a.N + kSB - 1) / kSB) * a.B * a.Hk : int64_t(((IDS ? a.Pp : a.M) + kSB - 1) / kSB) * a.B * a.H;
-  const int other = WHICH == kDkdv ? a.M : a.N;
-  const int64_t chain = int64_t((std::min(other, MODE == kDoc ? other : a.win + kSB) + kSB - 1) / kSB) * (WHICH == kDkdv ? a.G : 1);
-  if (IDS && chain <= 2) return 2;
-  const int64_t few = WHICH == kFwd && !IDS ? 768 : clamped(16 * chain, 256, IDS ? 2048 : 768);
-  if (D == 128 && WHICH != kFwd && MODE == kPlain && !causal && n > few && chain >= 16) {
-    // Workgroups of equal length, one (the second shape) or two (the third) to a CU: whichever's rounds take less, two side by
-    // side 1.9 times as long as one (dq: 16 heads x 1810 437 : 415 us, four rounds or two; 24 x 1500 460 : 515, five or three).
-    const int64_t wgs = (n + 1) / 2, one = (wgs + kCUs - 1) / kCUs, two = (wgs + 2 * kCUs - 1) / (2 * kCUs);
-    return 19 * two < 10 * one ? 2 : 1;
+  const int64_t n = WHICH == kDkdv ? int64_t((a.N + kSB - 1) / kSB) * a.B * a.Hk : int64_t((a.M + kSB - 1) / kSB) * a.B * a.H;
+  const int64_t chain = WHICH == kDkdv ? int64_t((a.M + kSB - 1) / kSB) * a.G : (a.N + kSB - 1) / kSB;
+  constexpr int kFew = IDS ? 2048 : 768;
+  const int many = WHICH == kFwd || (IDS && D <= 64) ? 16384 : 4096;
+  if (IDS) {
+    const int64_t places = int64_t(a.Pp / kSB) * a.B * a.H;
+    if (chain <= 6 && places >= 2048) return 2;
+    if (n <= kFew && places >= std::max<int64_t>(WHICH == kFwd ? 4096 : 2048, 128 * chain)) return 1;
+  } else if (WHICH != kFwd && MODE != kBlock) {
+    if ((chain <= 3 && n >= 512) || (chain <= 8 && n >= 1024)) return 2;
+    if (MODE == kPlain && !causal) {   // workgroups of equal length
+      if (chain < 16 && n >= 1280) return 2;
+      if (D == 128 && a.G == 1 && n > kFew && n < many) {
+        // One (the second shape) or two (the third) to a CU: whichever's rounds take less, two side by side 1.9 times as long as
+        // one (dq: 16 heads x 1810 437 : 415 us, four rounds or two; 24 x 1500 460 : 515, five or three).
+        const int64_t wgs = (n + 1) / 2, one = (wgs + kCUs - 1) / kCUs, two = (wgs + 2 * kCUs - 1) / (2 * kCUs);
+        return 19 * two < 10 * one ? 2 : 1;
+      }
+    }
   }
-  const int64_t many = WHICH == kFwd ? (IDS && chain <= 6 ? 4096 : 16384) : IDS ? clamped(128 * chain, 2048, 16384) : clamped(64 * chain, 1024, 4096);
-  return n <= few ? 0 : n < many ? 1 : 2;
+  return n <= kFew ? 0 : n < many ? 1 : 2;
 }
 template <int WHICH, int D, bool CAUSAL, int MODE>
 int launch_shape(const KArgs& a, hipStream_t s) {
@@ -801,12 +808,14 @@ int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t 
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s) { return launch_d<kDkdv>(a, D, causal, doc, s); }
 
 // dq and dk/dv side by side in one launch, each forming delta itself: where the workgroups of both (32 rows or keys counted as
-// one, with ids the empty places of the plan's order too) are about as many as the CUs can hold.  2 x 4 heads x 512 rows with documents, D = 64, forward and backward: 64.9 us against
-// 69.0 with two launches.  Up to three rounds of these workgroups of 16 rows, 8 heads
-// x 1024 111 us against 98 in two launches, 4 x 1754 174 : 149; 6 x 1024 (384) 88 : 96, 3 x 1500 (282) 111 : 132, 2 x 1024 (128) 36 : 54.
-bool bwd_f32_in_one(const KArgs& a) {
-  const int64_t wgs = int64_t(((a.Pp > 0 ? a.Pp : a.M) + 31) / 32) * a.B * a.H + int64_t((a.N + 31) / 32) * a.B * a.Hk;
-  return wgs <= kCUs * 3 / 2;
+// one) are about as many as the CUs can hold.  2 x 4 heads x 512 rows with documents, D = 64, forward and backward: 64.9 us against
+// 69.0 with two launches.  At the line, 8 x 8 heads x 128, causal: 28.1 us against 26.2 and the gap between two launches.  Not
+// with ids where the empty places of the plan's order are more workgroups than that (8 x 32 x 29, 8192 of them, 1.5 times as long), nor
+// without a mask where the chains are long and equal and leave a last round half empty (4 x 1754, D = 64, 440 workgroups 174 : 149).
+bool bwd_f32_in_one(const KArgs& a, bool causal) {
+  const int64_t keys = int64_t((a.N + 31) / 32) * a.B * a.Hk, wgs = int64_t((a.M + 31) / 32) * a.B * a.H + keys;
+  if (wgs > 2 * kCUs || int64_t(a.Pp / 32) * a.B * a.H + keys > 8 * kCUs) return false;
+  return causal || wgs <= kCUs * 3 / 2 || std::min<int64_t>(a.N, int64_t(a.M) * a.G) <= 63 * kSB;
 }
 int bwd_f32_shapes(const KArgs& a, int D, bool causal, bool doc) {
   auto both = [&](auto mode) { return 0x10 * shape<kDq, decltype(mode)::value>(a, D, causal) + 0x40 * shape<kDkdv, decltype(mode)::value>(a, D, causal); };
