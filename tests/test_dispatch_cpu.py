@@ -85,6 +85,8 @@ def test_fp32_shapes_without_a_mask_follow_the_rounds_of_workgroups():
     """D = 128: 640 workgroups of 32 rows are three rounds of one to a CU or two of two, which take 1.9 times as long; 512 are two or one."""
     assert dkdv_form(1, 40, 40, 490, 490, 128, f32, False) == ("fp32", 1, 1) and dkdv_form(1, 32, 32, 500, 500, 128, f32, False) == ("fp32", 2, 2)
     assert dkdv_form(4, 1, 1, 1754, 1754, 64, f32, False)[1] is not True   # (440 workgroups of 32: two launches)
+    for args in ((2, 4, 1, 1219, 1219, 128), (1, 2, 2, 4240, 2436, 128), (3, 1, 1, 2419, 2419, 16)):   # (dk/dv's chains longer or shorter than dq's: one)
+        assert dkdv_form(*args, f32, False) == ("fp32", True)
 
 
 def test_fp32_backward_in_one_launch_up_to_two_workgroups_to_a_cu():

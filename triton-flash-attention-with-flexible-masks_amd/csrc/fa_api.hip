@@ -310,7 +310,7 @@ extern "C" int fa_pair_wait_expired(uint64_t* count) {
 // FA_FORM_* of the backward, or of dk/dv by itself
 static int bwd_form(const fa_params* p, const KArgs& a, bool whole) {
   const bool causal = p->causal != 0, doc = p->score_mode == FA_SCORE_MODE1_DOC;
-  if (p->dtype == FA_DTYPE_FP32) return FA_FORM_FP32 | (whole && bwd_f32_in_one(a, causal) ? FA_FORM_WITH_DQ : bwd_f32_shapes(a, p->D, causal, doc));
+  if (p->dtype == FA_DTYPE_FP32) return FA_FORM_FP32 | (whole && bwd_f32_in_one(a, p->D, causal) ? FA_FORM_WITH_DQ : bwd_f32_shapes(a, p->D, causal, doc));
   if ((p->flags & FA_FLAG_DEBUG_NO_PAIR_WAIT) == 0 && bwd_small(a, p->D, causal, doc)) return FA_FORM_SMALL | (whole ? FA_FORM_WITH_DQ : 0);
   const bool both = whole && bwd_in_one(a, p->D, causal, doc);
   return dkdv_form(a, p->D, causal, doc, both) | (both ? FA_FORM_WITH_DQ : 0);

@@ -600,7 +600,7 @@ int launch_fwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 int launch_bwd_delta_f32(const KArgs& a, int D, hipStream_t s);
 int launch_bwd_dq_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
-bool bwd_f32_in_one(const KArgs& a, bool causal);
+bool bwd_f32_in_one(const KArgs& a, int D, bool causal);
 int bwd_f32_shapes(const KArgs& a, int D, bool causal, bool doc);   // of dq's and dk/dv's workgroups, as FA_FORM_FP32 carries them
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
 // problems that leave CUs idle (fa_bwd_small.hip): whether dk/dv takes its form there, and with dq in one launch or by itself
