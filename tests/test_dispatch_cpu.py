@@ -32,7 +32,7 @@ def test_forms(args, kw, form):
 
 @pytest.mark.parametrize("args,kw", [
     ((4, 8, 8, 115, 429, 64, bf16, False), {}), ((1, 64, 64, 205, 205, 64, fp16, True), {"kind": "doc"}), ((1, 16, 16, 186, 989, 64, bf16, True), {"kind": "block"}),
-    ((4, 4, 4, 610, 1000, 64, fp16, True), {"window": 10}), ((2, 4, 4, 125, 1871, 64, bf16, True), {"prefix": 535}), ((1, 8, 8, 118, 1892, 64, bf16, True), {}),
+    ((2, 4, 4, 1711, 1870, 64, bf16, True), {"window": 100}), ((2, 4, 4, 125, 1871, 64, bf16, True), {"prefix": 535}), ((1, 8, 8, 118, 1892, 64, bf16, True), {}),
 ])
 def test_the_small_form_stops_where_its_workgroups_share_cus(args, kw):
     """D = 64, 340 to 512 workgroups of 32 keys with short chains of rows: 1.1 to 1.4 times the time of the form with 128 keys to a workgroup."""
@@ -40,7 +40,7 @@ def test_the_small_form_stops_where_its_workgroups_share_cus(args, kw):
 
 
 @pytest.mark.parametrize("args,kw", [((1, 8, 8, 1252, 1252, 64, bf16, True), {}), ((3, 2, 2, 1780, 1780, 64, bf16, True), {}), ((4, 64, 8, 470, 470, 64, bf16, True), {}),
-                                     ((1, 64, 8, 1856, 1856, 64, fp16, True), {"window": 62}), ((1, 4, 4, 2591, 3124, 64, bf16, True), {"kind": "doc"}),
+                                     ((1, 64, 8, 1856, 1856, 64, fp16, True), {"window": 62}), ((1, 8, 8, 96, 1925, 64, fp16, True), {"window": 51}), ((1, 4, 4, 2591, 3124, 64, bf16, True), {"kind": "doc"}),
                                      ((1, 16, 2, 2196, 2196, 64, fp16, True), {"kind": "packed", "nseq": 35}), ((4, 64, 8, 147, 147, 128, fp16, False), {})])
 def test_long_chains_keep_the_small_form(args, kw):
     """... up to two workgroups of 32 keys to a CU: 1.2 to 1.8 times faster than the other forms."""
@@ -64,7 +64,7 @@ def test_rows_are_shared_only_where_cus_are_free(args, kw):
 
 @pytest.mark.parametrize("args,kw", [
     ((1, 16, 16, 2500, 2500, 64, bf16, False), {}), ((1, 6, 6, 6400, 6400, 64, bf16, True), {}), ((2, 64, 8, 3000, 3000, 64, fp16, True), {"window": 900}),
-    ((1, 16, 16, 2011, 2011, 64, bf16, True), {"kind": "block"}), ((1, 64, 8, 1302, 5000, 64, bf16, True), {"kind": "block"}),
+    ((2, 4, 4, 1789, 6128, 64, bf16, True), {"window": 1156}), ((1, 16, 16, 2011, 2011, 64, bf16, True), {"kind": "block"}), ((1, 64, 8, 1302, 5000, 64, bf16, True), {"kind": "block"}),
 ])
 def test_long_chains_share_their_rows_beyond_a_workgroup_to_a_cu(args, kw):
     """... up to 512 workgroups (1024 with a block map), where every one of them walks many tiles."""

@@ -827,7 +827,7 @@ static bool rows_form(const KArgs& a, int D, bool causal, bool doc) {
     if (tiles < std::max(16, 8 * a.G)) return false;
     if (block) return a.G > 1 || tiles >= 48 || wgs <= kCUs;
     if (!causal) return wgs <= kCUs * 3 / 2 && (a.G > 1 || tiles >= 48 || wgs <= kCUs / 2 || wgs > kCUs);
-    return a.G > 1 || tiles >= 48 || wgs <= kCUs * 9 / 8;
+    return a.G > 1 || tiles >= 48 || wgs * seen_keys(a, causal) / std::max(1, a.N) <= kCUs * 9 / 8;   // (keys before a window: 2 x 4 x 1789 on 6128, window 1156, 35 : 38 us)
   }
   const int rows = a.M / std::max(1, a.nKent - 1 - a.N / 128);   // of an average sequence (the table has an entry per 128 keys and one per sequence)
   return (rows / 64 + 1) * a.G >= (causal ? 16 : 8);

@@ -603,6 +603,8 @@ int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_
 bool bwd_f32_in_one(const KArgs& a, int D, bool causal);
 int bwd_f32_shapes(const KArgs& a, int D, bool causal, bool doc);   // of dq's and dk/dv's workgroups, as FA_FORM_FP32 carries them
 int launch_bwd_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_t s);
+// keys that a row sees at all: workgroups of the others end at once
+inline int seen_keys(const KArgs& a, bool causal) { return causal && a.win < 0x3fffffff ? int(std::min<int64_t>(a.N, int64_t(a.M) + a.win + a.pfx_m1 + 1)) : a.N; }
 // problems that leave CUs idle (fa_bwd_small.hip): whether dk/dv takes its form there, and with dq in one launch or by itself
 bool bwd_small(const KArgs& a, int D, bool causal, bool doc);
 int launch_bwd_small(const KArgs& a, int dtype, int D, bool causal, bool doc, bool both, hipStream_t s);
