@@ -405,7 +405,8 @@ int launch_cd(const KArgs& a, bool causal, bool doc, bool both, hipStream_t s) {
 //       causal, kv 320 - 384  1.07 [1.01, 1.24]  1.00 [0.80, 1.15]  0.84 [0.76, 1.12]  0.78 [0.63, 0.94]  0.73 [0.64, 0.83]
 //       kv 384 - 448          1.05 [1.03, 1.07]  1.20 [0.93, 1.54]  1.02 [0.95, 1.20]  0.93 [0.81, 1.19]  0.80 [0.73, 0.87]
 //       kv 448 - 512          1.28 [1.05, 1.39]  1.17 [0.98, 1.50]  1.04 [1.00, 1.18]  0.95 [0.85, 1.07]  0.92 [0.80, 1.11]
-//     (windows, with the keys that are seen, and block maps alike); without a mask, kv 352 - 512, 1.1 [0.92, 1.50] up to 32 blocks and 0.93 beyond; with the same ids on both
+//     (windows, with the keys that are seen, and block maps alike), but keys that are twice the rows or more have equally long chains: one head to a
+//     key head, kv from 320 on, 1.18 [1.00, 1.41] for chains of 11 to 61 (4 heads x 425 rows on 3031 keys 18 us in the others, 25 here); without a mask, kv 352 - 512, 1.1 [0.92, 1.50] up to 32 blocks and 0.93 beyond; with the same ids on both
 //     sides 1.13 [1.01, 1.40] from kv 384 and up to 1.43 below for few rows, but 0.90 where the column form is the other one; packed
 //     sequences 0.81 [0.61, 1.27] throughout.
 //   D = 128, one workgroup to a CU, for its LDS.  One query head to a key head: kv to 64 0.91 [0.62, 1.09], to 96 0.95 [0.77, 1.06], to 128
@@ -424,6 +425,7 @@ bool bwd_small(const KArgs& a, int D, bool causal, bool doc) {
     if (kv > 2 * kCUs) return false;
     if (kv <= kCUs || packed) return true;
     if (doc) return !causal || a.qpos != nullptr || a.gap >= 128 || (kv <= kCUs * 3 / 2 && a.M > 150);   // (the first ones: next to the column form otherwise)
+    if (causal && a.G == 1 && a.N >= 2 * a.M && kv > 312 && a.win >= 0x3fffffff && a.bmask == nullptr) return false;
     return full ? kv <= 352 || walked > 32 : 16 * walked >= kv * seen_keys(a, causal) / std::max(1, a.N) - 320;
   }
   if (a.G == 1) return kv <= 96;
