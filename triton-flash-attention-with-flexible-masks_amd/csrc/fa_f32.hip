@@ -812,7 +812,7 @@ int launch_bwd_dkdv_f32(const KArgs& a, int D, bool causal, bool doc, hipStream_
 // 69.0 with two launches.  At the line, 8 x 8 heads x 128, causal: 28.1 us against 26.2 and the gap between two launches.  Not
 // with ids where the empty places of the plan's order are more workgroups than that (8 x 32 x 29, 8192 of them, 1.5 times as long), nor
 // without a mask where all chains are long and alike, as many rows as keys, and leave a last round half empty (4 x 1754, D = 64, 440
-// workgroups 174 : 149; 28 random problems 0.89).  Where dk/dv's are the longer ones or the shorter, for heads that share keys or other numbers of
+// workgroups 174 : 149; 17 random problems 0.89 [0.85, 0.97]).  Where dk/dv's are the longer ones or the shorter, for heads that share keys or other numbers of
 // rows, the two fill each other's gaps (2 x 4/1 x 1219, D = 128 312 : 395, 1 x 2 x 4240 on 2436 538 : 671).
 bool bwd_f32_in_one(const KArgs& a, int D, bool causal) {
   const int64_t keys = int64_t((a.N + 31) / 32) * a.B * a.Hk, wgs = int64_t((a.M + 31) / 32) * a.B * a.H + keys;
