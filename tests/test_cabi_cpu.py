@@ -144,6 +144,24 @@ def test_workspace_size():
     assert L.fa_workspace_plan_bytes(ctypes.byref(p)) == want - scratch
 
 
+@pytest.mark.parametrize("M,N,low", [(511, 4096, False), (512, 4096, True), (2000, 16384, True), (9000, 9000, True), (33000, 33000, False)])
+def test_workspace_does_not_depend_on_qpos(M, N, low):
+    """Rows with positions of their own take query tiles of 128 rows where others take 64; the arrival counters are as many for both."""
+    L = _cabi.lib()
+    buf = ctypes.create_string_buffer(4096)
+    p = _good_params(buf)
+    p.M, p.N, p.score_mode = M, N, 1
+    p.eq_stride[0], p.eq_stride[2], p.ek_stride[0], p.ek_stride[2] = M, 1, N, 1
+    want = [f(ctypes.byref(p)) for f in (L.fa_workspace_bytes, L.fa_workspace_plan_bytes)]
+    p.qpos = p.q
+    assert [f(ctypes.byref(p)) for f in (L.fa_workspace_bytes, L.fa_workspace_plan_bytes)] == want
+    r256 = lambda x: (x + 255) // 256 * 256
+    Pp, Mp, Np = r256(M) + 256, -(-M // 64) * 64, -(-N // 64) * 64
+    ids = r256(Mp * 4) + r256(Np * 4) + 3 * r256(Pp * 4) + r256(-(-Mp // 1024) * 4) + r256(32) + r256(Pp // 64 * 32) + r256(Np // 64 * 32)
+    tiles = min(64, -(-M // 128) + 1)
+    assert want[1] - ids == r256(p.H * tiles * (2 if low else 1) * 4)
+
+
 @pytest.mark.parametrize("M,N", [(1, 16384), (100, 9000), (3, 300), (2000, 16384), (4096, 4096)])
 def test_a_window_past_every_key_is_no_window(M, N):
     """Window sizes up to the largest int (callers that mean "none") shape the launch like window = 0: the form and the
@@ -209,7 +227,7 @@ def test_gpu_cases_reach_the_query_tiles_they_are_written_for(tmp_path):
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc")
     csrc = ROOT / "triton-flash-attention-with-flexible-masks_amd" / "csrc"
-    calls = [f"fa::doc_rows({c[0] * c[10].get('copies', 1)}, {c[1]}, {c[3]}, {c[5]})" for c in F.LOW_TILE_CASES]
+    calls = [f"fa::split_config({c[0] * c[10].get('copies', 1)}, {c[1]}, {c[3]}, {c[4]}, {c[5]}, {int('qpos' in c[10])}).rows" for c in F.LOW_TILE_CASES]
     calls += [f"fa::block_rows({c[0]}, {c[1]}, {c[3]}, {c[5]})" for c in F.LOW_BLOCK_CASES]
     calls += [f"fa::block_rows(1, {c[0]}, {c[2]}, 128, {f})" for c in F.LONG_BLOCK_CASES for f in ("true", "false")]
     src = tmp_path / "rows.hip"

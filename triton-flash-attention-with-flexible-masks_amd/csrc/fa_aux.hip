@@ -347,7 +347,7 @@ int launch_mask_plan(const fa_params* p, const WsLayout& w, hipStream_t s) {
     const int kend_min = p->prefix > 0 ? ((p->prefix < p->N ? p->prefix : p->N) - 1) / kSumRows + 1 : 0;
     const int* qpos = p->causal ? p->qpos : nullptr;
     int* sk_cnt = reinterpret_cast<int*>(ws + w.off_sk_cnt);
-    const int n_sk = p->B * p->H * w.split.tiles;
+    const int n_sk = w.nSk;
     if (p->M <= kPlanOneMax && p->N <= kPlanOneMax) {
       dim3 grid(w.Hk1 > w.Hq1 ? w.Hk1 : w.Hq1, p->B);
       if (i64)

@@ -66,11 +66,16 @@ constexpr int kCUs = 256;
 //     the backward's launches 0.87 - 1.0.  What loses beyond one workgroup to a CU are many heads of short rows (64 heads x 575 rows 20 -> 25 us,
 //     8 x 8 x 701 23 -> 31, 8 x 8 x 1024 on 8192 keys 77 -> 88), whose workgroups are mostly set-up; longer rows have global rows and
 //     documents of unequal length, which 64-row tiles even out (16 x 2544 45 -> 32, 16 x 1595 49 -> 29).
-constexpr int kLowLongRows = 1280;
+// Fewer than kLowMinRows rows keep tiles of 128: up to one workgroup to a CU they would gain 0.95 (D = 64) and 0.97 (D = 128) [0.82, 1.03] in the
+// kernels of a forward and backward, whose passes wait for the host there, and a row whose softmax is kept in two states is rounded
+// otherwise: dQ of 2 heads x 384 rows at a scale of 0.25, D = 128, comes out at 1.05 of the largest error that is allowed for (0.0595), with one
+// state at 0.72, at the same 2-norm.  Neither do rows with positions of their own (packed sequences with ids) take them: D = 128 0.94 - 1.17, D = 64
+// 0.88 - 1.05.
+constexpr int kLowLongRows = 1280, kLowMinRows = 512;
 inline int low_wgs(int D) { return D > 64 ? 2 * kCUs : kCUs * 5 / 2; }
-inline int doc_rows(int B, int H, int M, int D) {
+inline int doc_rows(int B, int H, int M, int D, bool own_pos = false) {
   const int64_t wgs = int64_t(B) * H * ((M + 127) / 128);
-  return wgs <= kCUs || (M >= kLowLongRows && wgs <= low_wgs(D)) ? 64 : 128;
+  return !own_pos && M >= kLowMinRows && (wgs <= kCUs || (M >= kLowLongRows && wgs <= low_wgs(D))) ? 64 : 128;
 }
 // dq under a block map at D = 128 takes them for long rows whatever their number: a tile of 128 rows visits the columns of two rows of blocks, and in
 // the six of seven (a quarter of the blocks on) that only one of them has on, half of its waves have nothing to do.  64 rows : 128, 16 - 32 heads x 6000 -
@@ -95,8 +100,8 @@ struct SplitCfg {
 // query block against a long packed key sequence) the chunks go down to kSplitMinTiles key tiles, up to
 // kSplitKMaxFew of them.  Never more splittable tiles than M rows can fill.
 constexpr uint64_t kSplitScratchBudget = uint64_t(128) << 20;   // bytes of sk_ml + sk_o
-inline SplitCfg split_config(int B, int H, int M, int N, int D, uint64_t budget = kSplitScratchBudget) {
-  SplitCfg c = {1, 0, doc_rows(B, H, M, D)};
+inline SplitCfg split_config(int B, int H, int M, int N, int D, bool own_pos, uint64_t budget = kSplitScratchBudget) {
+  SplitCfg c = {1, 0, doc_rows(B, H, M, D, own_pos)};
   const int nKs = (N + kSumRows - 1) / kSumRows;
   if (nKs < 2 * kSplitMinTiles) return c;   // no key range can be long enough to be cut
   const int qtiles = (M + 127) / 128 + 1;   // 128-row tiles of global rows a (batch, head) can have
@@ -523,6 +528,7 @@ struct WsLayout {
   int Pp;                 // length of the permuted order
   int nQs, nKs;
   int nCh;                // row chunks of the partition kernels
+  int nSk;                // arrival counters
   uint64_t off_eq32, off_ek32, off_perm, off_peq, off_ppos, off_cnt, off_qhdr, off_qsum, off_ksum;  // bytes
   uint64_t off_sk_cnt, off_sk_ml, off_sk_o, total;
   uint64_t plan_bytes;   // leading part that carries state from the plan to the kernels; the rest is scratch
@@ -552,10 +558,11 @@ inline WsLayout ws_layout(const fa_params* p, uint64_t split_budget = kSplitScra
   w.off_qsum = take(uint64_t(p->B) * w.Hq1 * w.nQs * sizeof(IdSummary));
   w.off_ksum = take(uint64_t(p->B) * w.Hk1 * w.nKs * sizeof(IdSummary));
   // scratch of the split tiles: only when a key range can be long enough to be cut
-  const SplitCfg sc = split_config(p->B, p->H, p->M, p->N, p->D, split_budget);
+  const SplitCfg sc = split_config(p->B, p->H, p->M, p->N, p->D, p->qpos != nullptr, split_budget);
   w.split = sc;
   const uint64_t nsk = uint64_t(p->B) * p->H * sc.tiles;
-  w.off_sk_cnt = take(nsk * 4);
+  w.nSk = int(nsk) * (sc.rows / doc_rows(p->B, p->H, p->M, p->D));   // as many with qpos as without: the layout does not depend on it
+  w.off_sk_cnt = take(uint64_t(w.nSk) * 4);
   w.plan_bytes = o;      // the counters (zeroed by the plan, left at zero by every kernel) are state
   w.off_sk_ml = take(nsk * sc.k * sc.rows * 2 * 4);
   w.off_sk_o = take(nsk * sc.k * sc.rows * uint64_t(p->D) * 4);
