@@ -144,7 +144,7 @@ def test_workspace_size():
     assert L.fa_workspace_plan_bytes(ctypes.byref(p)) == want - scratch
 
 
-@pytest.mark.parametrize("M,N,low", [(511, 4096, False), (512, 4096, True), (2000, 16384, True), (9000, 9000, True), (33000, 33000, False)])
+@pytest.mark.parametrize("M,N,low", [(511, 4096, False), (512, 4096, True), (2000, 16384, True), (12200, 12200, True), (12400, 12400, False), (33000, 33000, False)])
 def test_workspace_does_not_depend_on_qpos(M, N, low):
     """Rows with positions of their own take query tiles of 128 rows where others take 64; the arrival counters are as many for both."""
     L = _cabi.lib()

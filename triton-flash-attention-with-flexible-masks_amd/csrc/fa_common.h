@@ -60,12 +60,14 @@ constexpr int kCUs = 256;
 //     D = 128, forward      0.62 [0.56, 0.67]  0.69 [0.55, 0.83]  0.74 [.56, .98]  0.75 [.63, 1.04]  0.95 [.80, 1.09]  0.98
 //     D = 64,  forward      0.67 [0.61, 0.76]  0.67 [0.55, 0.75]  0.70 [.58, .85]  0.75 [.61, 0.95]  0.81 [.65, 0.94]  0.90 [.79, 1.08]
 //     the backward's launches 0.65 - 1.0 throughout.  (Bands of four blocks lose up to 1.25 between 160 and 512, full maps gain.)
-//   documents, forward
-//     D = 128               0.83 [0.64, 1.01]  0.79 [0.57, 0.98]  0.83 [.69, 1.18]  0.77 [.63, 1.07]  0.86 [.68, 1.10]  0.93 [.73, 1.18]
-//     D = 64                0.84 [0.74, 1.00]  0.83 [0.59, 1.05]  0.77 [.62, 1.05]  0.82 [.64, 1.25]  0.91 [.68, 1.26]  0.88
-//     the backward's launches 0.87 - 1.0.  What loses beyond one workgroup to a CU are many heads of short rows (64 heads x 575 rows 20 -> 25 us,
-//     8 x 8 x 701 23 -> 31, 8 x 8 x 1024 on 8192 keys 77 -> 88), whose workgroups are mostly set-up; longer rows have global rows and
-//     documents of unequal length, which 64-row tiles even out (16 x 2544 45 -> 32, 16 x 1595 49 -> 29).
+//   documents, kernels of a forward and backward [forward alone]
+//                     512 to 1279 rows, to 256               to 128                  to 256                  to 384                  to 512
+//     D = 128   0.94, 0.84 - 1.00 [.74 - 1.03]  0.91, 0.80 - 1.01       0.87, 0.76 - 0.94       0.95, 0.83 - 1.12       0.97, 0.80 - 1.06 [.68 - 1.24]
+//     D = 64    0.97, 0.93 - 1.04 [.78 - 1.04]  0.91, 0.82 - 0.98       0.93, 0.81 - 1.01       0.92, 0.77 - 1.09       0.89, 0.79 - 1.00 [.65 - 1.18]
+//     The line lies where tiles of 64 rows are all resident at once, two (D = 128) or three to a CU: beyond it documents without global rows, whose
+//     workgroups are mostly set-up, take a second round for nothing (8 heads x 7109 rows, D = 128, forward and backward 114 -> 121 us, 4 x 8 x 1289 on 4235
+//     keys 158 -> 176), which the host cannot tell from those that gain (12 x 5178 with a tenth of the rows global 164 -> 131).  Rows below
+//     kLowLongRows gain nothing from the third: D = 64 to 384 1.00 - 1.02.
 // Fewer than kLowMinRows rows keep tiles of 128: up to one workgroup to a CU they would gain 0.95 (D = 64) and 0.97 (D = 128) [0.82, 1.03] in the
 // kernels of a forward and backward, whose passes wait for the host there, and a row whose softmax is kept in two states is rounded
 // otherwise: dQ of 2 heads x 384 rows at a scale of 0.25, D = 128, comes out at 1.05 of the largest error that is allowed for (0.0595), with one
@@ -75,7 +77,7 @@ constexpr int kLowLongRows = 1280, kLowMinRows = 512;
 inline int low_wgs(int D) { return D > 64 ? 2 * kCUs : kCUs * 5 / 2; }
 inline int doc_rows(int B, int H, int M, int D, bool own_pos = false) {
   const int64_t wgs = int64_t(B) * H * ((M + 127) / 128);
-  return !own_pos && M >= kLowMinRows && (wgs <= kCUs || (M >= kLowLongRows && wgs <= low_wgs(D))) ? 64 : 128;
+  return !own_pos && M >= kLowMinRows && (wgs <= kCUs || (D <= 64 && M >= kLowLongRows && wgs <= kCUs * 3 / 2)) ? 64 : 128;
 }
 // dq under a block map at D = 128 takes them for long rows whatever their number: a tile of 128 rows visits the columns of two rows of blocks, and in
 // the six of seven (a quarter of the blocks on) that only one of them has on, half of its waves have nothing to do.  64 rows : 128, 16 - 32 heads x 6000 -
