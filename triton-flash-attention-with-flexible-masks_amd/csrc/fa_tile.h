@@ -675,11 +675,18 @@ FA_HD int launch_slots(const KArgs& a) { return MODE == GEO_DOC ? doc_tiles(a) +
 template <int MODE>
 FA_HD int launch_groups(const KArgs& a) { return MODE != GEO_GENERAL ? a.B * a.H : a.qtab != nullptr ? a.nHp : a.B * a.nHp; }
 inline bool geo_general(const KArgs& a) { return a.pack > 1 || a.dsplit > 1 || a.bm != 128 || a.qtab != nullptr; }
-// Workgroups of dq as the rules of the backward's forms count them: tiles of 128 rows, also where it takes twice as many of 64.
+// Workgroups of dq as the rules of the backward's forms count them, whose lines were measured with tiles of 128 rows: of those, also where dq takes
+// twice as many of 64 -- with ids, under a block map, and under a causal mask alone where 128-row tiles fill the CUs (fwd_config).  The tables of
+// bwd_small and bwd_in_one hold there too: counted in 64-row tiles, 1 x 16/2 x 2500 rows, D = 128, left the small form, 388 -> 470 us, 1 x 8/1 x 5156
+// 768 -> 965.
 inline int64_t dq_units(const KArgs& a, bool doc, bool grid) {
-  auto of = [&](int slots, int groups) { return int64_t(grid ? grid_blocks(slots, groups) : slots * groups); };
+  auto of = [&](int slots, int groups) { return grid ? int64_t(grid_blocks(slots, groups)) : int64_t(slots) * groups; };
   if (doc) return of(a.Pp / 128 + split_extra(a) * a.bm / 128, launch_groups<GEO_DOC>(a));
   if (a.bmask != nullptr) return of((a.M + 127) / 128, a.B * a.H);
+  if (a.qtab == nullptr) {
+    const int high = int((int64_t(a.M) * a.pack + 127) / 128);
+    if (a.bm == 64 && int64_t(high) * a.B * a.nHp >= kCUs) return of(high * a.dsplit, a.B * a.nHp);
+  }
   return geo_general(a) ? of(launch_slots<GEO_GENERAL>(a), launch_groups<GEO_GENERAL>(a)) : of(launch_slots<GEO_PLAIN>(a), launch_groups<GEO_PLAIN>(a));
 }
 
