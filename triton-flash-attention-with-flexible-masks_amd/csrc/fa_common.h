@@ -231,9 +231,10 @@ inline FwdCfg fwd_config(const fa_params* p, bool fwd = true) {   // fwd: for th
   //            816 to 950 rows                         1.06 [0.98, 1.14]  1.15 [1.06, 1.27]  1.17
   //   D = 64,  1024 rows and more   0.86 [0.80, 0.98]  0.87 [0.83, 0.94]  0.88 [0.80, 0.96]  0.87 [0.81, 0.93]  to 608 0.87, at 640 1.15
   // and the backward 0.96 of them [0.84, 1.08] (1 x 4 x 10787, D = 128, forward 204 -> 175 us, backward 521 -> 453).  Equal tiles
-  // lose what a 64-row tile costs more: no mask, D = 128 1.20 - 1.31; windows of up to half of the keys, D = 128 1.06 - 1.43, D = 64 from 448 on 0.94 - 1.24.
+  // lose what a 64-row tile costs more: no mask, D = 128 1.20 - 1.31; windows of up to half of the keys, D = 128 1.06 - 1.43, D = 64 from 448 on 0.94 - 1.24;
+  // prefixes, forward and backward, of a quarter of the keys 0.87 - 0.97 (D = 64 to 1.01), of half 1.00 - 1.08 (0.92 - 1.05), of three quarters 1.03 - 1.14.
   const int64_t wgs = c.tiles * bh;
-  const bool uneven = p->causal && (p->window <= 0 || p->window >= p->N) && p->N - p->M <= p->M / 2 && p->M >= 1024;
+  const bool uneven = p->causal && (p->window <= 0 || p->window >= p->N) && p->prefix <= p->N / 4 && p->N - p->M <= p->M / 2 && p->M >= 1024;
   if (wgs < kCUs || (uneven && wgs <= (p->D > 64 ? 2 * kCUs : kCUs * 9 / 4))) { c.bm = 64; c.tiles = int((rows + 63) / 64); }
   // a step: one 64-key tile; two workgroups to a CU
   if ((p->flags & FA_FLAG_SPLIT_KEYS) && c.tiles * bh < 2 * kCUs)
