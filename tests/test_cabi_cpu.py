@@ -231,14 +231,14 @@ def test_gpu_cases_reach_the_query_tiles_they_are_written_for(tmp_path):
     calls += [f"fa::block_rows({c[0]}, {c[1]}, {c[3]}, {c[5]})" for c in F.LOW_BLOCK_CASES]
     calls += [f"fa::block_rows(1, {c[0]}, {c[2]}, 128, {f})" for c in F.LONG_BLOCK_CASES for f in ("true", "false")]
     src = tmp_path / "rows.hip"
-    calls += [f"causal({c[0] * c[8]}, {c[1]}, {c[2]}, {c[3]}, {c[4]}, {c[5]}, {c[7]}, {sum(c[10:])})" for c in F.LOW_CAUSAL_CASES]
+    calls += [f"causal({c[0] * c[8]}, {c[1]}, {c[2]}, {c[3]}, {c[4]}, {c[5]}, {c[7]}, {sum(c[11:])})" for c in F.LOW_CAUSAL_CASES]
     src.write_text('''#include <cstdio>
 #include "fa_common.h"
 static int causal(int B, int H, int Hk, int M, int N, int D, int prefix, int window) {
   fa_params p = {};
   p.B = B; p.H = H; p.Hk = Hk; p.M = M; p.N = N; p.D = D; p.prefix = prefix; p.window = window; p.causal = 1; p.dtype = FA_DTYPE_BF16; p.flags = FA_FLAG_SPLIT_KEYS;
   const fa::FwdCfg f = fa::fwd_config(&p), b = fa::fwd_config(&p, false);
-  return f.bm == b.bm && !f.dec && f.split == 1 ? f.bm : 0;
+  return !f.dec && f.split == 1 && b.split == 1 ? 1000 * f.bm + b.bm : 0;
 }
 int main() { for (int r : {''' + ", ".join(calls) + '''}) printf("%d\\n", r); }
 ''')
@@ -246,7 +246,7 @@ int main() { for (int r : {''' + ", ".join(calls) + '''}) printf("%d\\n", r); }
     subprocess.run([hipcc, "--offload-host-only", "-std=c++17", "-O1", f"-I{csrc}", str(src), "-o", str(exe)], check=True, capture_output=True)
     got = list(map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()))
     assert got == [c[9] for c in F.LOW_TILE_CASES] + [c[11] for c in F.LOW_BLOCK_CASES] + [r for c in F.LONG_BLOCK_CASES for r in (128, c[5])] + \
-        [c[9] for c in F.LOW_CAUSAL_CASES]
+        [1000 * c[9] + c[10] for c in F.LOW_CAUSAL_CASES]
 
 
 @pytest.mark.parametrize("nseq,M,N,H,Hk,D,bm", [

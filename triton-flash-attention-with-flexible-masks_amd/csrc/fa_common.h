@@ -224,18 +224,31 @@ inline FwdCfg fwd_config(const fa_params* p, bool fwd = true) {   // fwd: for th
     return c;
   }
   c.tiles = int((rows + 127) / 128);
-  // 64-row tiles where 128-row ones leave CUs idle, and up to two of those to a CU where a causal mask makes them unequal: all are resident
-  // at once, and the launch waits for the longest.  64 rows : 128, forward, geometric mean over random problems [smallest, largest], by
-  // the tiles of 128 rows:                 to 320             to 384             to 448             to 512             to 640
-  //   D = 128, 1024 rows and more   0.85 [0.81, 1.01]  0.87 [0.83, 0.94]  0.91 [0.85, 0.97]  0.91 [0.88, 1.01]  1.08 [0.95, 1.21]
-  //            816 to 950 rows                         1.06 [0.98, 1.14]  1.15 [1.06, 1.27]  1.17
-  //   D = 64,  1024 rows and more   0.86 [0.80, 0.98]  0.87 [0.83, 0.94]  0.88 [0.80, 0.96]  0.87 [0.81, 0.93]  to 608 0.87, at 640 1.15
-  // and the backward 0.96 of them [0.84, 1.08] (1 x 4 x 10787, D = 128, forward 204 -> 175 us, backward 521 -> 453).  Equal tiles
+  // 64-row tiles where 128-row ones leave CUs idle, and up to nearly two of those to a CU where a causal mask makes them unequal: all are resident
+  // at once, and the launch waits for the longest.  64 rows : 128 by the tiles of 128 rows, geometric mean [smallest, largest]:
+  //                                                    to 320             to 384             to 448             to 512
+  //   D = 128, 2500 rows and more, forward     0.87 [0.85, 0.89]  0.89 [0.86, 0.91]  0.91 [0.88, 0.95]  0.97 [0.83, 1.12]
+  //                   forward and backward     0.90 [0.87, 0.93]  0.93 [0.90, 0.96]  0.95 [0.94, 0.98]  0.98 [0.89, 1.04]
+  //            1024 to 2048 rows, forward      0.96 [0.88, 1.01]  1.07 [1.05, 1.11]  1.14 [1.02, 1.20]  1.06 [1.05, 1.07]
+  //                   forward and backward     0.94 [0.91, 0.97]  1.01 [1.00, 1.01]  1.03 [1.01, 1.04]  0.99 [0.99, 1.00]
+  //   D = 64,  2500 rows and more, forward     0.85 [0.82, 0.89]  0.87 [0.84, 0.90]  0.88 [0.82, 0.90]  0.87 [0.81, 0.92], to 576 0.87
+  //              backward, as many keys        0.95 [0.82, 1.04]  0.92 [0.84, 1.03]  0.97 [0.91, 1.07]  0.92 [0.90, 0.95]
+  //              backward, up to a quarter more 1.00 [0.98, 1.01] 0.98 [0.93, 1.03]  1.05 [1.04, 1.07]  1.03 [0.92, 1.10]
+  //            1024 to 2048 rows, forward      0.92 [0.89, 0.96]  0.85 [0.83, 0.88]  0.95 [0.91, 1.02]  0.95 [0.95, 0.95]
+  //                             backward       1.03 [0.94, 1.14]  0.96 [0.91, 1.09]  1.00 [0.94, 1.11]  0.97 [0.97, 0.97]
+  // (1 x 4 x 12000, D = 128, forward and backward 747 -> 680 us.)  What loses to 512 at D = 128 are heads that the XCDs do not share evenly (5 x 12000 rows on
+  // 13200 keys 1044 -> 1087, 7 x 9000 682 -> 702).  Equal tiles
   // lose what a 64-row tile costs more: no mask, D = 128 1.20 - 1.31; windows of up to half of the keys, D = 128 1.06 - 1.43, D = 64 from 448 on 0.94 - 1.24;
-  // prefixes, forward and backward, of a quarter of the keys 0.87 - 0.97 (D = 64 to 1.01), of half 1.00 - 1.08 (0.92 - 1.05), of three quarters 1.03 - 1.14.
+  // prefixes, forward and backward, of a quarter of the keys 0.87 - 0.97 (D = 64 to 1.01), of half 1.00 - 1.08 (0.92 - 1.05), of three quarters 1.03 - 1.14;
+  // half as many keys again as rows 0.94 - 0.99, forward alone 0.87 - 1.03.
   const int64_t wgs = c.tiles * bh;
-  const bool uneven = p->causal && (p->window <= 0 || p->window >= p->N) && p->prefix <= p->N / 4 && p->N - p->M <= p->M / 2 && p->M >= 1024;
-  if (wgs < kCUs || (uneven && wgs <= (p->D > 64 ? 2 * kCUs : kCUs * 9 / 4))) { c.bm = 64; c.tiles = int((rows + 63) / 64); }
+  int64_t low = kCUs - 1;
+  if (p->causal && (p->window <= 0 || p->window >= p->N) && p->prefix <= p->N / 4 && p->N - p->M <= p->M / 4) {
+    if (p->M >= 2500) low = p->D > 64 ? kCUs * 7 / 4 : fwd || p->N - p->M <= p->M / 16 ? kCUs * 9 / 4 : kCUs * 3 / 2;
+    else if (p->M >= 1024 && p->D > 64) low = kCUs * 5 / 4;
+    else if (p->M >= 1024 && fwd) low = kCUs * 7 / 4;
+  }
+  if (wgs <= low) { c.bm = 64; c.tiles = int((rows + 63) / 64); }
   // a step: one 64-key tile; two workgroups to a CU
   if ((p->flags & FA_FLAG_SPLIT_KEYS) && c.tiles * bh < 2 * kCUs)
     c.split = pick_split(c.tiles * bh, (nk + 63) / 64, 2 * kCUs, 3.f, 4.f, 8);
