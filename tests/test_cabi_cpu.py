@@ -229,7 +229,7 @@ def test_gpu_cases_reach_the_query_tiles_they_are_written_for(tmp_path):
     csrc = ROOT / "triton-flash-attention-with-flexible-masks_amd" / "csrc"
     calls = [f"fa::split_config({c[0] * c[10].get('copies', 1)}, {c[1]}, {c[3]}, {c[4]}, {c[5]}, {int('qpos' in c[10])}).rows" for c in F.LOW_TILE_CASES]
     calls += [f"fa::block_rows({c[0]}, {c[1]}, {c[3]}, {c[5]})" for c in F.LOW_BLOCK_CASES]
-    calls += [f"fa::block_rows(1, {c[0]}, {c[2]}, 128, {f})" for c in F.LONG_BLOCK_CASES for f in ("true", "false")]
+    calls += [f"dq_block(1, {c[0]}, {c[2]}, {c[3]}, 128)" for c in F.LONG_BLOCK_CASES]
     src = tmp_path / "rows.hip"
     calls += [f"causal({c[0] * c[8]}, {c[1]}, {c[2]}, {c[3]}, {c[4]}, {c[5]}, {c[7]}, {sum(c[11:])})" for c in F.LOW_CAUSAL_CASES]
     src.write_text('''#include <cstdio>
@@ -240,12 +240,17 @@ static int causal(int B, int H, int Hk, int M, int N, int D, int prefix, int win
   const fa::FwdCfg f = fa::fwd_config(&p), b = fa::fwd_config(&p, false);
   return !f.dec && f.split == 1 && b.split == 1 ? 1000 * f.bm + b.bm : 0;
 }
+static int dq_block(int B, int H, int M, int N, int D) {
+  fa_params p = {};
+  p.B = B; p.H = p.Hk = H; p.M = M; p.N = N; p.D = D; p.score_mode = FA_SCORE_MODE2_BLOCK; p.dtype = FA_DTYPE_BF16;
+  return fa::fwd_config(&p, false).bm;
+}
 int main() { for (int r : {''' + ", ".join(calls) + '''}) printf("%d\\n", r); }
 ''')
     exe = tmp_path / "rows"
     subprocess.run([hipcc, "--offload-host-only", "-std=c++17", "-O1", f"-I{csrc}", str(src), "-o", str(exe)], check=True, capture_output=True)
     got = list(map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()))
-    assert got == [c[9] for c in F.LOW_TILE_CASES] + [c[11] for c in F.LOW_BLOCK_CASES] + [r for c in F.LONG_BLOCK_CASES for r in (128, c[5])] + \
+    assert got == [c[9] for c in F.LOW_TILE_CASES] + [c[11] for c in F.LOW_BLOCK_CASES] + [c[5] for c in F.LONG_BLOCK_CASES] + \
         [1000 * c[9] + c[10] for c in F.LOW_CAUSAL_CASES]
 
 

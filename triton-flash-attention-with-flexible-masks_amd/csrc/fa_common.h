@@ -79,15 +79,10 @@ inline int doc_rows(int B, int H, int M, int D, bool own_pos = false) {
   const int64_t wgs = int64_t(B) * H * ((M + 127) / 128);
   return !own_pos && M >= kLowMinRows && (wgs <= kCUs || (D <= 64 && M >= kLowLongRows && wgs <= kCUs * 3 / 2)) ? 64 : 128;
 }
-// dq under a block map at D = 128 takes them for long rows whatever their number: a tile of 128 rows visits the columns of two rows of blocks, and in
-// the six of seven (a quarter of the blocks on) that only one of them has on, half of its waves have nothing to do.  64 rows : 128, 16 - 32 heads x 6000 -
-// 16384 rows, 10 / 25 / 50 % on, dq 0.93 - 1.02 / 0.85 - 0.92 / 0.87 - 0.96, forward and backward together 0.97 - 1.01 / 0.96 - 1.0 / 0.96 - 1.0 (32 x 16384,
-// 25 % on: dq 934 -> 840 us, together 2764 -> 2703).  The forward gains nothing there (0.96 - 1.1), nor does D = 64 (0.92 - 1.05 together), and
-// of shorter rows those with many heads lose (2 x 32 x 5000, 10 % on: dq 147 -> 157).
-constexpr int kBlockLongRows = 6000;
-inline int block_rows(int B, int H, int M, int D, bool fwd = true) {
-  return int64_t(B) * H * ((M + 127) / 128) <= low_wgs(D) || (!fwd && D > 64 && M >= kBlockLongRows) ? 64 : 128;
-}
+// dq of long rows at D = 128 would gain under random maps (16 heads x 16384 rows, a quarter on, 479 -> 425 us), whose tiles of 128 rows visit the columns of
+// two unlike rows of blocks, and loses where neighbouring rows are alike: bands of 4 / 16 blocks 1.14 - 1.31 / 1.05 - 1.20, maps in pieces of 128 x 128
+// 1.00 - 1.15, full ones 1.02 - 1.09 (16 - 32 heads x 6016 - 16384 rows, causal and not, as many keys and twice as many).
+inline int block_rows(int B, int H, int M, int D) { return int64_t(B) * H * ((M + 127) / 128) <= low_wgs(D) ? 64 : 128; }
 struct SplitCfg {
   int k;      // chunks per tile (1: nothing is ever split)
   int tiles;  // global-row tiles per (batch, head) that can be split
@@ -205,7 +200,7 @@ inline FwdCfg fwd_config(const fa_params* p, bool fwd = true) {   // fwd: for th
     return c;
   }
   if (p->score_mode == FA_SCORE_MODE2_BLOCK && p->dtype != FA_DTYPE_FP32) {
-    c.bm = block_rows(p->B, p->H, p->M, p->D, fwd);
+    c.bm = block_rows(p->B, p->H, p->M, p->D);
     c.tiles = (p->M + c.bm - 1) / c.bm;
     return c;
   }
