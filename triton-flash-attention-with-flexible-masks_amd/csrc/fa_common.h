@@ -56,10 +56,18 @@ constexpr int kCUs = 256;
 // Forward and dq of masked problems with few query tiles take tiles of 64 rows, whose waves split every key tile in two
 // (QTileCtx::halved): twice the workgroups, each half as long, at about 1.3 times the instructions per pair.  By the workgroups that
 // tiles of 128 rows would make, all heads counted, 64-row tiles : 128, geometric mean over random problems [smallest, largest]:
-//   block map (10 - 50 % on)           to 128           to 256           to 384           to 512           to 640           to 768
-//     D = 128, forward      0.62 [0.56, 0.67]  0.69 [0.55, 0.83]  0.74 [.56, .98]  0.75 [.63, 1.04]  0.95 [.80, 1.09]  0.98
-//     D = 64,  forward      0.67 [0.61, 0.76]  0.67 [0.55, 0.75]  0.70 [.58, .85]  0.75 [.61, 0.95]  0.81 [.65, 0.94]  0.90 [.79, 1.08]
-//     the backward's launches 0.65 - 1.0 throughout.  (Bands of four blocks lose up to 1.25 between 160 and 512, full maps gain.)
+//   block map, kernels of a forward and backward [forward alone]
+//                                    to 128                    to 256                    to 384                    to 512
+//     D = 128, bands of 2 - 16     0.88, 0.83 - 0.92         1.02, 0.88 - 1.23         1.07, 0.90 - 1.18         1.13, 1.08 - 1.17 [1.25 - 1.41]
+//              128 x 128 pieces    0.89, 0.82 - 0.94         0.93, 0.85 - 0.99         0.99, 0.83 - 1.10         1.06, 1.03 - 1.11
+//              full                0.86, 0.83 - 0.90         0.89, 0.87 - 0.90         0.95, 0.90 - 1.02         0.99, 0.93 - 1.03
+//              random, 10 - 30 %   0.87, 0.84 - 0.90         0.88, 0.70 - 0.95                          [0.74, 0.56 - 1.04]
+//     D = 64,  bands               0.84, 0.79 - 0.90         0.98, 0.89 - 1.06         0.95, 0.88 - 1.05         1.10, 1.00 - 1.17 [1.06 - 1.29]
+//              128 x 128 pieces    0.88, 0.86 - 0.89         0.94, 0.90 - 0.99         0.94, 0.89 - 1.00         0.99, 0.93 - 1.05
+//              full                0.80, 0.79 - 0.81         0.92, 0.90 - 0.95         0.94, 0.91 - 0.98         0.94, 0.88 - 0.99
+//              random                                        0.94, 0.92 - 0.96         0.91, 0.87 - 0.98         0.95, 0.94 - 0.95
+//     The lines lie where narrow bands, whose workgroups are mostly set-up, begin to lose; the host cannot tell them from the others.  At D = 128 they do as soon
+//     as two 64-row tiles share a CU (18 heads x 1024 rows, bands of 2 blocks, forward 9.8 -> 11.4 us, backward 13.8 -> 18.7), at D = 64 when a fourth would.
 //   documents, kernels of a forward and backward [forward alone]
 //                     512 to 1279 rows, to 256               to 128                  to 256                  to 384                  to 512
 //     D = 128   0.94, 0.84 - 1.00 [.74 - 1.03]  0.91, 0.80 - 1.01       0.87, 0.76 - 0.94       0.95, 0.83 - 1.12       0.97, 0.80 - 1.06 [.68 - 1.24]
@@ -74,7 +82,6 @@ constexpr int kCUs = 256;
 // state at 0.72, at the same 2-norm.  Neither do rows with positions of their own (packed sequences with ids) take them: D = 128 0.94 - 1.17, D = 64
 // 0.88 - 1.05.
 constexpr int kLowLongRows = 1280, kLowMinRows = 512;
-inline int low_wgs(int D) { return D > 64 ? 2 * kCUs : kCUs * 5 / 2; }
 inline int doc_rows(int B, int H, int M, int D, bool own_pos = false) {
   const int64_t wgs = int64_t(B) * H * ((M + 127) / 128);
   return !own_pos && M >= kLowMinRows && (wgs <= kCUs || (D <= 64 && M >= kLowLongRows && wgs <= kCUs * 3 / 2)) ? 64 : 128;
@@ -82,7 +89,7 @@ inline int doc_rows(int B, int H, int M, int D, bool own_pos = false) {
 // dq of long rows at D = 128 would gain under random maps (16 heads x 16384 rows, a quarter on, 479 -> 425 us), whose tiles of 128 rows visit the columns of
 // two unlike rows of blocks, and loses where neighbouring rows are alike: bands of 4 / 16 blocks 1.14 - 1.31 / 1.05 - 1.20, maps in pieces of 128 x 128
 // 1.00 - 1.15, full ones 1.02 - 1.09 (16 - 32 heads x 6016 - 16384 rows, causal and not, as many keys and twice as many).
-inline int block_rows(int B, int H, int M, int D) { return int64_t(B) * H * ((M + 127) / 128) <= low_wgs(D) ? 64 : 128; }
+inline int block_rows(int B, int H, int M, int D) { return int64_t(B) * H * ((M + 127) / 128) <= (D > 64 ? kCUs / 2 : kCUs * 3 / 2) ? 64 : 128; }
 struct SplitCfg {
   int k;      // chunks per tile (1: nothing is ever split)
   int tiles;  // global-row tiles per (batch, head) that can be split
