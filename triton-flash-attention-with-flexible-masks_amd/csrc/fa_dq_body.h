@@ -139,8 +139,7 @@ FA_DEV void dq_body(const KArgs& a, const int bid, char* smem) {
       f32x16 s = zero, dp = dinit;
       mfma_phase();
       __builtin_amdgcn_sched_barrier(0);
-      // S and dP are accumulated alternately (an MFMA that accumulates onto the result of the MFMA
-      // issued right before it waits a full extra MFMA time), operands a few LDS reads ahead.
+      // S and dP are accumulated alternately, operands a few LDS reads ahead.
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const vec8 kf = lds_row8<E>(lk + lo.row[ks] + kb * 32 * DL * 2);

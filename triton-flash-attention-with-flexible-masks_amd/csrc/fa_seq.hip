@@ -71,8 +71,8 @@ FA_DEV float wave_sum(float v) {
 }
 
 // Block 0 writes the query tiles, block 1 the key tiles.  What bounds it: a chain of short phases in one workgroup, each the latency of a few LDS
-// accesses and a barrier.  32 sequences with 91 query and 998 key tiles 9.9 -> 6.5 us, 466 and 240 tiles 10.2 -> 8.2 (a chunked prefill of the first
-// 102.4 -> 97.8), against waves' scans through ds_bpermute, flat look-ups, two passes of atomics and whole entries of 64 bytes.
+// accesses and a barrier.  32 sequences with 91 query and 998 key tiles 8.6 -> 5.7 us (a chunked prefill of them 104.2 -> 101.8), 24 with 466 and
+// 240 tiles 9.9 -> 7.4, against waves' scans through ds_bpermute, flat look-ups, two passes of atomics and whole entries of 64 bytes.
 // BIG: more than kLdsSeqs sequences, their offsets in global memory (a kernel of its own: through a pointer to either, every access is a flat one).
 template <bool BIG>
 __global__ __launch_bounds__(kThreads) void seq_plan_kernel(const SeqPlanArgs p, int* __restrict__ spill) {
