@@ -254,6 +254,54 @@ int main() { for (int r : {''' + ", ".join(calls) + '''}) printf("%d\\n", r); }
         [1000 * c[9] + c[10] for c in F.LOW_CAUSAL_CASES]
 
 
+def test_64_row_tiles_leave_the_static_forward_its_sizes(tmp_path):
+    """fa_fwd_static takes what fits FA_STATIC_WS_BYTES with one arrival counter to 128 rows, whatever the tiles: its largest key ranges by the sizes of the
+    layout's parts, at each one below and above (with ids, with positions as well)."""
+    import os
+    import subprocess
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    csrc = ROOT / "triton-flash-attention-with-flexible-masks_amd" / "csrc"
+    cases = [(1, 1, 4096, 64), (1, 1, 8192, 128), (1, 2, 2000, 64), (1, 1, 700, 128), (2, 8, 3000, 64), (3, 32, 512, 64), (1, 1, 48000, 64), (1, 1, 300, 64)]
+    src = tmp_path / "static.hip"
+    src.write_text('''#include <cstdio>
+#include "fa_common.h"
+static bool fits(int B, int H, int M, int D, int N, bool own) {
+  fa_params p = {};
+  p.B = B; p.H = p.Hk = H; p.M = M; p.N = N; p.D = D; p.score_mode = FA_SCORE_MODE1_DOC;
+  if (own) p.qpos = &N;
+  const fa::WsLayout w = fa::ws_layout(&p, uint64_t(24) << 20);
+  return fa::fits_static(w) && w.total <= FA_STATIC_WS_BYTES + fa::kStaticMargin;
+}
+int main(int c, char** v) {
+  const int cases[][4] = {''' + ", ".join("{%d, %d, %d, %d}" % x for x in cases) + '''};
+  for (auto& x : cases) for (bool own : {false, true}) {
+    int lo = 1 << 14, hi = 1 << 24;
+    while (hi - lo > 1) { const int m = lo + (hi - lo) / 2; (fits(x[0], x[1], x[2], x[3], m, own) ? lo : hi) = m; }
+    fa_params p = {};
+    p.B = x[0]; p.H = p.Hk = x[1]; p.M = x[2]; p.N = lo; p.D = x[3]; p.score_mode = FA_SCORE_MODE1_DOC;
+    const fa::SplitCfg s = fa::split_config(p.B, p.H, p.M, p.N, p.D, own, uint64_t(24) << 20);
+    printf("%d %d %d %d\\n", lo, s.k, s.tiles * s.rows / 128, s.rows);
+  }
+}
+''')
+    exe = tmp_path / "static"
+    subprocess.run([hipcc, "--offload-host-only", "-std=c++17", "-O1", f"-I{csrc}", str(src), "-o", str(exe)], check=True, capture_output=True)
+    got = [tuple(map(int, l.split())) for l in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines()]
+    r256 = lambda x: (x + 255) // 256 * 256
+
+    def total(B, H, M, D, N, k, tiles):
+        Mp, Np, Pp = -(-M // 64) * 64, -(-N // 64) * 64, -(-M // 256) * 256 + 256
+        plan = r256(B * Mp * 4) + r256(B * Np * 4) + 3 * r256(B * Pp * 4) + r256(B * -(-Mp // 1024) * 4) + r256(B * 32) + r256(B * Pp // 64 * 32) + r256(B * Np // 64 * 32)
+        return plan + r256(B * H * tiles * 4) + r256(B * H * tiles * k * 128 * 2 * 4) + r256(B * H * tiles * k * 128 * D * 4)
+
+    for i, (N, k, tiles, _) in enumerate(got):
+        B, H, M, D = cases[i // 2]
+        assert total(B, H, M, D, N, k, tiles) <= 32 << 20 < total(B, H, M, D, N + 1, k, tiles), (cases[i // 2], N)
+    assert {r for _, _, _, r in got} == {64, 128} and all(got[i][0] == got[i + 1][0] for i in range(0, len(got), 2))
+
+
 @pytest.mark.parametrize("nseq,M,N,H,Hk,D,bm", [
     (600, 15000, 15000, 8, 8, 128, 64),      # many short sequences: not the form with one workgroup to a CU
     (600, 15000, 15000, 32, 32, 64, 64),

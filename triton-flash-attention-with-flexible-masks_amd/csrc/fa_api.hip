@@ -243,7 +243,7 @@ extern "C" int fa_fwd(const fa_params* p, void* stream) {
 // memsets or copies -- the array's name is a host-side stand-in, not a device address.
 // ---------------------------------------------------------------------------
 constexpr uint64_t kStaticSplitBudget = uint64_t(24) << 20;   // of FA_STATIC_WS_BYTES; the rest is for the plan
-static __device__ __align__(256) unsigned char scratch[FA_STATIC_WS_BYTES];
+static __device__ __align__(256) unsigned char scratch[FA_STATIC_WS_BYTES + kStaticMargin];
 static std::atomic<void*> g_scratch_ptr[64];
 
 static int static_scratch(void** out) {
@@ -277,11 +277,11 @@ extern "C" int fa_fwd_static(const fa_params* p, void* stream) {
   int rc = fa_validate(&q, 0);
   if (rc != FA_OK) return rc;
   const WsLayout w = ws_layout(&q, kStaticSplitBudget);
-  if (w.total > FA_STATIC_WS_BYTES) return FA_ERR_WORKSPACE;   // sizes beyond the static array
+  if (!fits_static(w)) return FA_ERR_WORKSPACE;   // sizes beyond the static array
   void* ws = nullptr;
   if (int e = static_scratch(&ws)) return finish(e);
   q.workspace = ws;
-  q.workspace_bytes = FA_STATIC_WS_BYTES;
+  q.workspace_bytes = FA_STATIC_WS_BYTES + kStaticMargin;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // the plan rewrites everything the kernels read (ids, order, summaries) and zeroes the arrival
   // counters with a kernel, so nothing of an earlier call's contents is ever looked at

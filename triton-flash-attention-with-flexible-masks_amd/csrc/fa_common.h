@@ -547,6 +547,7 @@ struct WsLayout {
   int nQs, nKs;
   int nCh;                // row chunks of the partition kernels
   int nSk;                // arrival counters
+  uint64_t low_bytes;     // what they take more than one to 128 rows would
   uint64_t off_eq32, off_ek32, off_perm, off_peq, off_ppos, off_cnt, off_qhdr, off_qsum, off_ksum;  // bytes
   uint64_t off_sk_cnt, off_sk_ml, off_sk_o, total;
   uint64_t plan_bytes;   // leading part that carries state from the plan to the kernels; the rest is scratch
@@ -581,12 +582,18 @@ inline WsLayout ws_layout(const fa_params* p, uint64_t split_budget = kSplitScra
   const uint64_t nsk = uint64_t(p->B) * p->H * sc.tiles;
   w.nSk = int(nsk) * (sc.rows / doc_rows(p->B, p->H, p->M, p->D));   // as many with qpos as without: the layout does not depend on it
   w.off_sk_cnt = take(uint64_t(w.nSk) * 4);
+  w.low_bytes = (o - w.off_sk_cnt) - ((nsk * sc.rows / 128 * 4 + 255) & ~uint64_t(255));
   w.plan_bytes = o;      // the counters (zeroed by the plan, left at zero by every kernel) are state
   w.off_sk_ml = take(nsk * sc.k * sc.rows * 2 * 4);
   w.off_sk_o = take(nsk * sc.k * sc.rows * uint64_t(p->D) * 4);
   w.total = o;
   return w;
 }
+
+// fa_fwd_static takes the problems whose layout fits FA_STATIC_WS_BYTES with one arrival counter to 128 rows; 64-row tiles have two, which lie in a margin of
+// the array (doc_rows: at most 384 tiles of 128 rows and one more to each of 96 (batch, head) pairs).
+constexpr uint64_t kStaticMargin = 4096;
+inline bool fits_static(const WsLayout& w) { return w.total - w.low_bytes <= FA_STATIC_WS_BYTES && w.low_bytes <= kStaticMargin; }
 
 // Layouts without a mask plan.  Mode 0 with FA_FLAG_SPLIT_KEYS: arrival counters (the part called plan) and partial
 // results.  Packed sequences: header, tile tables, counters, and partial results.
